@@ -210,12 +210,14 @@ __global__ __launch_bounds__(LD_THREADS, 4) void k_lmm_u8_dot(const uint8_t* __r
 
 	for(int k = tid; k < nPad * LD_SLOTS; k += THREADS) slots[k] = 0.0;
 
+	// the last thread of the matrix may hold fewer than RPT rows: it reads and looks up RPT codes all the same (see
+	// k_rmm_q1_u8) and multiplies what lies behind the last row by zero
 	int passLen = min(passRows, blockLen);
-	bool full = off + RPT <= passLen;
+	bool live = off < passLen;
 	const uint8_t* passBase = arena + (size_t) blockBeg;
-	uint32_t voff = full ? off : 0;
+	uint32_t voff = live ? off : 0;
 	CodeVec<1, RPT> ping[NB], pong[NB];
-	if(full) u8_load<RPT, NB>(ping, passBase, voff, arenaStride, 0, gLast);
+	if(live) u8_load<RPT, NB>(ping, passBase, voff, arenaStride, 0, gLast);
 
 	constexpr int TPT = (PER * 256 + THREADS - 1) / THREADS;
 	double stage[TPT];
@@ -235,14 +237,19 @@ __global__ __launch_bounds__(LD_THREADS, 4) void k_lmm_u8_dot(const uint8_t* __r
 	for(int pass = 0; pass < nPass; pass++) {
 		const int64_t passBeg = blockBeg + (int64_t) pass * passRows;
 		const int nextLen = pass + 1 < nPass ? min(passRows, blockLen - (pass + 1) * passRows) : 0;
-		const bool nfull = off + RPT <= nextLen;
+		const bool nlive = off < nextLen;
 		const uint8_t* nextBase = nextLen > 0 ? passBase + passRows : passBase;
-		const uint32_t noff = nfull ? off : 0;
+		const uint32_t noff = nlive ? off : 0;
 		double yv[RPT];
+		if(off + RPT <= passLen) {
 #pragma unroll
-		for(int i = 0; i < RPT; i++) yv[i] = full ? y[passBeg + off + i] : 0.0;
+			for(int i = 0; i < RPT; i++) yv[i] = y[passBeg + off + i];
+		}
+		else {
+#pragma unroll
+			for(int i = 0; i < RPT; i++) yv[i] = off + i < passLen ? y[passBeg + off + i] : 0.0;
+		}
 		for(int g0 = 0; g0 < nGroups; g0 += PER) {
-			const int nIn = min(PER, nGroups - g0);
 			__syncthreads();
 			int tidW = tid;
 			asm volatile("" : "+v"(tidW));
@@ -253,7 +260,7 @@ __global__ __launch_bounds__(LD_THREADS, 4) void k_lmm_u8_dot(const uint8_t* __r
 			}
 			__syncthreads();
 			fetch(g0 + PER < nGroups ? g0 + PER : 0);
-			if(full) {
+			if(live) {
 #pragma unroll
 				for(int s = 0; s < PER; s += 2 * NB) {
 					double sum[NB];
@@ -269,17 +276,9 @@ __global__ __launch_bounds__(LD_THREADS, 4) void k_lmm_u8_dot(const uint8_t* __r
 					for(int j = 0; j < NB; j++) unsafeAtomicAdd(mySlot + (g0 + s + NB + j) * LD_SLOTS, sum[j]);
 				}
 			}
-			else if(off < passLen) { // ragged end of the matrix
-				for(int g = 0; g < nIn; g++) {
-					const uint8_t* codes = arena + (size_t) (g0 + g) * arenaStride + passBeg;
-					double s = 0.0;
-					for(int i = 0; off + i < passLen; i++) s += y[passBeg + off + i] * tbl[g * 256 + codes[off + i]];
-					unsafeAtomicAdd(mySlot + (g0 + g) * LD_SLOTS, s);
-				}
-			}
 		}
 		passLen = nextLen;
-		full = nfull;
+		live = nlive;
 		passBase = nextBase;
 		voff = noff;
 	}

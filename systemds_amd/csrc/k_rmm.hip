@@ -281,13 +281,17 @@ __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restr
 	// partly filled wave, which has to store its rows untransposed
 	const int passRows = ((blockLen + nPass - 1) / nPass + 64 * RPT - 1) / (64 * RPT) * (64 * RPT);
 
+	// `live`: the thread holds at least one row of the pass. The last thread of the matrix may hold fewer than RPT: it
+	// reads and looks up RPT codes all the same (a stream's stride is a multiple of 256 bytes, so the bytes are there,
+	// and any byte finds an entry in a table of 256) and only its output is cut. (Rows taken one by one there cost the
+	// whole call about 1 us per group: 250,007 x 54 56 -> 21 us, 2,000,003 x 100 99 -> 58 us.)
 	int passLen = min(passRows, blockLen);
-	bool full = off + RPT <= passLen;
+	bool live = off < passLen;
 	const uint8_t* passBase = arena + (size_t) blockBeg; // uniform; a thread's codes start at passBase + off
-	uint32_t voff = full ? off : 0;
+	uint32_t voff = live ? off : 0;
 
 	CodeVec<1, RPT> ping[NB], pong[NB];
-	if(full) u8_load<RPT, NB>(ping, passBase, voff, arenaStride, 0, gLast);
+	if(live) u8_load<RPT, NB>(ping, passBase, voff, arenaStride, 0, gLast);
 
 	// the tables of the next slab are fetched into registers while the current slab is processed
 	constexpr int TPT = (U8_PER * 256 + THREADS - 1) / THREADS;
@@ -325,17 +329,16 @@ __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restr
 	for(int pass = 0; pass < nPass; pass++) {
 		const int64_t passBeg = blockBeg + (int64_t) pass * passRows;
 		// the first batch of the next pass is requested in the last batch slot of this pass; a
-		// thread without a full next pass requests valid but unused bytes instead, so that the
+		// thread without a row in the next pass requests valid but unused bytes instead, so that the
 		// number of loads in flight never depends on a branch
 		const int nextLen = pass + 1 < nPass ? min(passRows, blockLen - (pass + 1) * passRows) : 0;
-		const bool nfull = off + RPT <= nextLen;
+		const bool nlive = off < nextLen;
 		const uint8_t* nextBase = nextLen > 0 ? passBase + passRows : passBase; // uniform
-		const uint32_t noff = nfull ? off : 0; // without a next pass: everybody re-requests the same 16 bytes
+		const uint32_t noff = nlive ? off : 0; // without a next pass: everybody re-requests the same 16 bytes
 		double acc[RPT];
 #pragma unroll
 		for(int i = 0; i < RPT; i++) acc[i] = 0.0;
 		for(int g0 = 0; g0 < nGroups; g0 += U8_PER) {
-			const int nIn = min(U8_PER, nGroups - g0);
 			__syncthreads();
 			int tidW = tid;
 			asm volatile("" : "+v"(tidW));
@@ -346,7 +349,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restr
 			}
 			__syncthreads();
 			fetch(g0 + U8_PER < nGroups ? g0 + U8_PER : 0);
-			if(full) {
+			if(live) {
 #pragma unroll
 				for(int s = 0; s < U8_PER; s += 2 * NB) {
 					u8_load<RPT, NB>(pong, passBase, voff, arenaStride, g0 + s + NB, gLast);
@@ -355,14 +358,6 @@ __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restr
 					const bool wrap = gn >= nPad;
 					u8_load<RPT, NB>(ping, wrap ? nextBase : passBase, wrap ? noff : voff, arenaStride, wrap ? 0 : gn, gLast);
 					u8_consume<RPT, NB, LB, LN>(pong, tb + (s + NB) * 2048, acc);
-				}
-			}
-			else if(off < passLen) {
-				for(int g = 0; g < nIn; g++) {
-					const uint8_t* codes = arena + (size_t) (g0 + g) * arenaStride + passBeg;
-#pragma unroll
-					for(int i = 0; i < RPT; i++)
-						if(off + i < passLen) acc[i] += tbl[g * 256 + codes[off + i]];
 				}
 			}
 		}
@@ -412,7 +407,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restr
 				}
 		}
 		passLen = nextLen;
-		full = nfull;
+		live = nlive;
 		passBase = nextBase;
 		voff = noff;
 	}
