@@ -25,9 +25,10 @@
 #define CLA_CATCH_VOID CLA_CATCH_BODY(return, return)
 
 // Workspace of the entry point that allocates nothing (cla_rmm_dev_noalloc): the non-zero counter in the
-// first 256 bytes, then the pre-aggregated tables. One copy per GPU, held until the process ends. In host
+// first NNZ_BYTES, then the pre-aggregated tables. One copy per GPU, held until the process ends. In host
 // code the name is only a handle for hipGetSymbolAddress: kernels get the address looked up at cla_init.
-constexpr size_t CLA_SCRATCH_BYTES = (size_t) 4 << 20;
+constexpr size_t CLA_SCRATCH_TABLES = ((size_t) 4 << 20) - 256;
+constexpr size_t CLA_SCRATCH_BYTES = CLA_SCRATCH_TABLES + cla::NNZ_BYTES;
 static __device__ __align__(256) unsigned char scratch[CLA_SCRATCH_BYTES];
 
 namespace cla {
@@ -282,13 +283,14 @@ cla_handle cla_block_create(int64_t nRows, int32_t nCols) {
 	b->constV.assign((size_t) nCols, 0.0);
 	if(hipStreamCreate(&b->stream) != hipSuccess) { set_error("hipStreamCreate failed"); delete b; return nullptr; }
 	b->ownStream = true;
-	if(hipMalloc((void**) &b->dCounters, 8 * sizeof(unsigned long long)) != hipSuccess ||
-		hipHostMalloc((void**) &b->hCounters, 8 * sizeof(unsigned long long)) != hipSuccess) {
+	constexpr size_t counterBytes = NNZ_SLOTS * NNZ_BYTES + 2 * NNZ_STEP * sizeof(unsigned long long); // the counters, two ticket lines
+	if(hipMalloc((void**) &b->dCounters, counterBytes) != hipSuccess ||
+		hipHostMalloc((void**) &b->hCounters, NNZ_BYTES) != hipSuccess) {
 		set_error("allocating counters failed");
 		cla_block_free(b);
 		return nullptr;
 	}
-	if(hipMemset(b->dCounters, 0, 8 * sizeof(unsigned long long)) != hipSuccess) {
+	if(hipMemset(b->dCounters, 0, counterBytes) != hipSuccess) {
 		set_error("clearing counters failed");
 		cla_block_free(b);
 		return nullptr;
@@ -866,11 +868,16 @@ int cla_block_prepare(cla_handle b, uint32_t products, int32_t nColB, int32_t nR
 
 // sync: wait for the driver's kernels and return its non-zero count; otherwise leave the count in the
 // device counter (cla_block_nnz reads it on request) and return at once
-static int64_t finish_nnz(cla_block* b, bool sync = true) {
-	if(!sync) return 0;
-	CLA_HIP(hipMemcpyAsync(b->hCounters, b->dCounters + b->nnzSlot, sizeof(unsigned long long), hipMemcpyDeviceToHost, b->stream));
+static int64_t read_nnz(cla_block* b, const unsigned long long* dNnz) {
+	CLA_HIP(hipMemcpyAsync(b->hCounters, dNnz, NNZ_BYTES, hipMemcpyDeviceToHost, b->stream));
 	CLA_HIP(hipStreamSynchronize(b->stream));
-	return (int64_t) b->hCounters[0];
+	unsigned long long n = 0;
+	for(int i = 0; i < NNZ_WAYS; i++) n += b->hCounters[i * NNZ_STEP];
+	return (int64_t) n;
+}
+
+static int64_t finish_nnz(cla_block* b, bool sync = true) {
+	return sync ? read_nnz(b, b->nnz_counter(b->nnzSlot)) : 0;
 }
 
 static int64_t rmm_dev(cla_handle b, const double* dB, int32_t nColB, double* dOut, bool sync) {
@@ -911,12 +918,10 @@ int64_t cla_rmm_dev_noalloc(cla_handle b, const double* dB, int32_t nColB, doubl
 	unsigned long long* dNnz = (unsigned long long*) ws;
 	const bool profile = b->profile;
 	b->profile = false;
-	rc = launch_rmm(b, dB, nColB, dOut, dNnz, 0, (double*) (ws + 256), (CLA_SCRATCH_BYTES - 256) / sizeof(double));
+	rc = launch_rmm(b, dB, nColB, dOut, dNnz, 0, (double*) (ws + NNZ_BYTES), CLA_SCRATCH_TABLES / sizeof(double));
 	b->profile = profile;
 	if(rc) return rc;
-	CLA_HIP(hipMemcpyAsync(b->hCounters, dNnz, sizeof(unsigned long long), hipMemcpyDeviceToHost, b->stream));
-	CLA_HIP(hipStreamSynchronize(b->stream));
-	return (int64_t) b->hCounters[0];
+	return read_nnz(b, dNnz);
 	CLA_CATCH_CODE(int64_t)
 }
 
@@ -1076,7 +1081,7 @@ __global__ __launch_bounds__(256) void k_take_block(const double* __restrict__ G
 		out[idx] = v;
 		cnt += v != 0.0;
 	}
-	if(cnt) atomicAdd(nnz, (unsigned long long) cnt);
+	if(cnt) atomicAdd(nnz_way(nnz, 0), (unsigned long long) cnt);
 }
 
 // cbind(left, right) as a block of its own: the groups of `left` first, then those of `right` with
@@ -1329,7 +1334,7 @@ __global__ __launch_bounds__(256) void k_scatter_cols(const double* __restrict__
 		out[(size_t) i * n + colMap[j]] = v;
 		cnt += v != 0.0;
 	}
-	if(cnt) atomicAdd(nnz, (unsigned long long) cnt);
+	if(cnt) atomicAdd(nnz_way(nnz, 0), (unsigned long long) cnt);
 }
 
 // rs[i] += sum of Y[i, rows of the block]
@@ -1355,7 +1360,7 @@ __global__ __launch_bounds__(256) void k_const_cols(const double* __restrict__ r
 		out[(size_t) i * n + c] = v;
 		cnt += v != 0.0;
 	}
-	if(cnt) atomicAdd(nnz, (unsigned long long) cnt);
+	if(cnt) atomicAdd(nnz_way(nnz, 0), (unsigned long long) cnt);
 }
 
 // Cuts the block into chunks of whole groups of at most `width` columns, a block of its own each; the columns that
@@ -1406,7 +1411,7 @@ static int build_lmm_subs(cla_block* b, int width) {
 static int launch_lmm_chunked(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dNnz) {
 	if(b->lmmSubWidth < 0) return 1;
 	hipStream_t st = b->stream;
-	CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 	int width = b->lmmSubWidth ? b->lmmSubWidth : 64;
 	for(;;) {
 		if(b->lmmSubs.empty()) {
@@ -1455,7 +1460,7 @@ static int launch_lmm_chunked(cla_block* b, const double* dY, int p, double* dOu
 		CLA_HIP(hipStreamSynchronize(st));
 		clear_stats(b);
 		free_lmm_subs(b);
-		CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+		CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 		if(width == 16) { b->lmmSubWidth = -1; return 1; }
 		width /= 2;
 	}
@@ -1466,7 +1471,7 @@ static int launch_lmm_chunked(cla_block* b, const double* dY, int p, double* dOu
 		CLA_HIP(hipStreamSynchronize(st));
 		if(bad) { clear_stats(b); return 1; }
 	}
-	CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 	for(void* q : b->lmmSubs) {
 		LmmSub* sb = (LmmSub*) q;
 		const int k = sb->k;
@@ -1517,7 +1522,7 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 	int rc = ensure_stage(&b->dStageOut, &b->stageOutCap, n);
 	if(rc) return rc;
 	CLA_HIP(hipMemsetAsync(b->dStageOut, 0, n * sizeof(double), st));
-	CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 	for(int p0 = 0; p0 < p; p0 += 16) // 16 rows of Y per pass over the block
 		if((rc = launch_lmm_decode(b, dY + (size_t) p0 * b->nRows, std::min(16, p - p0), b->dStageOut + (size_t) p0 * b->nCols, dNnz))) {
 			if(rc == 1 && p0 == 0) return launch_lmm_chunked(b, dY, p, dOut, dNnz); // (nothing queued yet)
@@ -1533,7 +1538,7 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 		CLA_HIP(hipStreamSynchronize(st));
 		if(bad) { clear_stats(b); return 1; }
 	}
-	CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 	{
 		Prof pf(b, "k_take_block", ((int) n + 255) / 256, 256, 0, 0);
 		hipLaunchKernelGGL(k_take_block, dim3((unsigned) std::min(((int) n + 255) / 256, 1024)), dim3(256), 0, st, b->dStageOut, b->nCols, 0, 0, p,
@@ -1581,7 +1586,7 @@ int64_t cla_lmm_compressed_dev(cla_handle right, cla_handle left, double* dOut) 
 	if((rc = ensure_stage(&c->dStageOut, &c->stageOutCap, n * n))) return rc;
 	if((rc = launch_tsmm(c, c->dStageOut, c->dCounters))) return rc;
 	right->nnzSlot = 0;
-	CLA_HIP(hipMemsetAsync(right->dCounters, 0, sizeof(unsigned long long), right->stream));
+	CLA_HIP(hipMemsetAsync(right->dCounters, 0, NNZ_BYTES, right->stream));
 	const int nOut = left->nCols * right->nCols;
 	{
 		Prof pf(c, "k_take_block", (nOut + 255) / 256, 256, 0, 0);

@@ -59,10 +59,21 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
 	return v;
 }
 
-// Adds a per-thread count into a global 64-bit counter: one atomic per wave.
+// Where a wave (or, part 0, a whole block) adds its share of a non-zero count.
+__device__ __forceinline__ unsigned long long* nnz_way(unsigned long long* counter, unsigned part) {
+	return counter + ((blockIdx.x + part) % NNZ_WAYS) * NNZ_STEP;
+}
+
+// Clears a counter; called by one whole block of at least NNZ_WAYS threads.
+__device__ __forceinline__ void nnz_clear(unsigned long long* counter) {
+	if(threadIdx.x < NNZ_WAYS) counter[threadIdx.x * NNZ_STEP] = 0;
+}
+
+// Adds a per-thread count into a counter: one atomic per wave.
 __device__ __forceinline__ void count_add(unsigned long long* counter, int local) {
 	const int s = wave_sum_i32(local);
-	if((threadIdx.x & (WAVE - 1)) == 0 && s != 0) atomicAdd(counter, (unsigned long long) s);
+	if((threadIdx.x & (WAVE - 1)) == 0 && s != 0)
+		atomicAdd(nnz_way(counter, (blockDim.x / WAVE - 1) * blockIdx.x + threadIdx.x / WAVE), (unsigned long long) s);
 }
 
 // Tail of a left multiply whose kernel is the only one of the call: every block comes here behind its last add into
@@ -88,6 +99,7 @@ __device__ __forceinline__ void lmm_tail(unsigned* done, unsigned nBlocks, const
 	}
 	cnt = wave_sum_i32(cnt);
 	if((threadIdx.x & (WAVE - 1)) == 0) partS[threadIdx.x >> 6] = cnt;
+	nnz_clear(nnz);
 	__syncthreads();
 	if(threadIdx.x == 0) {
 		int s = 0;

@@ -21,6 +21,13 @@ constexpr int SDC_TILE = 1024;
 // Bytes allocated (and filled with 0x01) behind every uploaded array: list walkers read whole registers
 // from any byte position of an offset or code list without a bounds check.
 constexpr int UPLOAD_SLACK = 128;
+// A non-zero counter is NNZ_WAYS partial counts, one to a 128-byte line, that whoever reads it adds up. Atomic adds to
+// one address are served one after the other, 11.4 ns each on this device: with one word per counter the 4096 waves of
+// a mat-vec spent 47 us on it (X %*% v of 4,000,003 x 10: 59 us; 24 us on spread counters).
+constexpr int NNZ_WAYS = 64, NNZ_STEP = 16;
+constexpr int NNZ_SLOT = NNZ_WAYS * NNZ_STEP; // words of a counter
+constexpr size_t NNZ_BYTES = (size_t) NNZ_SLOT * 8;
+constexpr int NNZ_SLOTS = 4;                  // counters of a block (cla_block::nnzSlot)
 
 // Iterator state of an offset list in front of delta entry `idx`:
 // `row` = rows accumulated so far (last emitted row plus pending 0-entry skips),
@@ -206,14 +213,17 @@ struct cla_block {
 	uint32_t* dSdcPacked = nullptr;  // all listed groups' entries as (code << 16 | row inside its 4096-row tile), built on first use
 	int sdcPlanGroup = -2;
 	std::vector<int32_t> sdcList, sdcBinOff;
-	unsigned long long* dCounters = nullptr;   // 8 x u64: 0 - 3 non-zero counts, 6 and 7 ticket counters of the left multiply's and the Gram kernels' tails
+	unsigned long long* dCounters = nullptr;   // NNZ_SLOTS non-zero counters, then a line each for the ticket counters below
+	unsigned* lmm_ticket() { return (unsigned*) (dCounters + cla::NNZ_SLOTS * cla::NNZ_SLOT); }   // of the left multiply's tail
+	unsigned* gram_ticket() { return (unsigned*) (dCounters + cla::NNZ_SLOTS * cla::NNZ_SLOT + cla::NNZ_STEP); } // of the Gram kernels' tail
+	unsigned long long* nnz_counter(int slot) { return dCounters + (size_t) slot * cla::NNZ_SLOT; }
 	double* dGramAcc = nullptr;      // nCols x nCols, zero between calls: where the blocks of a one-kernel t(X) %*% X add (gram_tail)
 	unsigned long long* hCounters = nullptr;   // pinned
 
 	std::vector<cla::KernelStat> lastStats;
 	bool profile = false;            // bracket every kernel with HIP events on `stream`
 	cla::Options opt;
-	// Non-zero counter of the last driver call: index into dCounters. Slot 0 is cleared by the first
+	// Non-zero counter of the last driver call (nnz_counter). Slot 0 is cleared by the first
 	// kernel of a driver; the fused mat-vec kernel rotates over slots 1-3 instead (it counts into one
 	// and clears the next, so that no separate clearing step runs between two calls).
 	int nnzSlot = 0;

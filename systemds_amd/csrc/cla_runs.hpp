@@ -177,6 +177,7 @@ __device__ __forceinline__ void gram_tail(unsigned* done, unsigned nBlocks, doub
 	}
 	cnt = wave_sum_i32(cnt);
 	if((threadIdx.x & (WAVE - 1)) == 0) gramPartS[threadIdx.x >> 6] = cnt;
+	nnz_clear(nnz);
 	__syncthreads();
 	if(threadIdx.x == 0) {
 		int s = 0;

@@ -207,7 +207,7 @@ static int launch_aggregate_decompressed(cla_block* b, int op, int dir, double* 
 	const int64_t nRows = b->nRows;
 	hipStream_t st = b->stream;
 	clear_stats(b);
-	CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 	const int64_t chunkRows = std::min<int64_t>(nRows, std::max<int64_t>(AGG_CHUNK_ROWS,
 		((int64_t) 256 << 20) / ((int64_t) sizeof(double) * nCols) / AGG_CHUNK_ROWS * AGG_CHUNK_ROWS));
 	const int64_t nParts = (nRows + AGG_CHUNK_ROWS - 1) / AGG_CHUNK_ROWS;
@@ -299,7 +299,7 @@ int launch_aggregate(cla_block* b, int op, int dir, double* dOut, unsigned long 
 		return launch_rmm(b, b->dOnes, 1, dOut, dNnz, op == CLA_AGG_SUMSQ ? 1 : 0);
 	}
 	clear_stats(b);
-	CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 	int rc = ensure_counts(b);
 	if(rc) return rc;
 	// scratch: column aggregates | touched flags | partials of one uncompressed group at a time

@@ -693,7 +693,7 @@ int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	if(dNnz != nullptr) {
 		const int rc = ensure_gram_acc(b);
 		if(rc) return rc;
-		A.acc = b->dGramAcc; A.done = (unsigned*) (b->dCounters + 7); A.nnz = dNnz;
+		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
 	const size_t lds = b->gdrPlan->lds;
 	const int nChunks = (int) ((b->nRows + GDR_CH - 1) / GDR_CH);

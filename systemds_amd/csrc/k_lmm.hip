@@ -347,7 +347,7 @@ int launch_lmm(cla_block* b, const double* dY, int p, double* dOut, unsigned lon
 		return 0;
 	}
 	CLA_HIP(hipMemsetAsync(dPre, 0, sizeof(double) * ((size_t) p * b->totalVals + (size_t) p), st));
-	CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 	if(dot != 0 && (rc = run_preagg(b, dY, p, dPre, -1, dOut))) return rc;
 
 	int64_t rowsPerBlock = 256 * 1024;

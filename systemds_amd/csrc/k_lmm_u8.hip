@@ -338,7 +338,7 @@ int launch_lmm_u8_dot(cla_block* b, const double* dY, int p, double* dOut) {
 	CLA_HIP(allow_full_lds((const void*) kern));
 	const bool tail = b->lmmTailWanted; // (this kernel serves every group of the block)
 	hipLaunchKernelGGL(kern, dim3(grid, p), dim3(LD_THREADS), lds, b->stream, b->dArena, b->arenaStride, nG, b->dDictPad, dCol0, dY,
-		b->nRows, dOut, b->nCols, tail ? (unsigned*) (b->dCounters + 6) : nullptr, b->dCounters);
+		b->nRows, dOut, b->nCols, tail ? b->lmm_ticket() : nullptr, b->dCounters);
 	b->lmmTailDone = tail;
 	CLA_HIP(hipGetLastError());
 	return 0;

@@ -23,7 +23,7 @@ __global__ void k_preagg(const DGroup* __restrict__ groups, int nGroups, const d
 	unsigned long long* __restrict__ nnz, double* __restrict__ Tpad, int squares) {
 	const int g = blockIdx.y;
 	const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-	if(g == 0 && idx == 0) *nnz = 0; // the multiply kernels behind this one on the stream count into it
+	if(g == 0 && blockIdx.x == 0) nnz_clear(nnz); // the multiply kernels behind this one on the stream count into it
 	// Tpad (mat-vec on byte codes only): the same tables at a fixed stride of 256 entries, zero
 	// beyond nVals, so that the gather kernel copies a slab of tables without looking up offsets
 	if(Tpad != nullptr && g < nGroups && idx < 256 && idx >= groups[g].nVals) Tpad[(size_t) g * 256 + idx] = 0.0;
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restr
 	bool careful = false;
 	if(FUSED) {
 		static_assert(!FUSED || THREADS % 256 == 0, "a wave's table entries belong to one group");
-		if(blockIdx.x == 0 && tid == 0) *nnzNext = 0;
+		if(blockIdx.x == 0) nnz_clear(nnzNext);
 		int bad = 0;
 		for(int g = tid; g < nGroups; g += THREADS) bad |= !isfinite(v[col0[g]]);
 		careful = __syncthreads_or(bad) != 0;
@@ -572,13 +572,13 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 	const int32_t* dCol0 = fused ? (const int32_t*) (b->dDictPad + (size_t) nG * 256) : nullptr;
 	if(fused) {
 		b->nnzSlot = b->nnzRot;
-		dNnz = b->dCounters + b->nnzSlot;
+		dNnz = b->nnz_counter(b->nnzSlot);
 	}
 	// Blocks of single-column SDCZeros lists only: the row-list kernel makes its tables from the dictionaries and
 	// counts likewise into a counter that the call before has cleared: the only launch.
 	if(q == 1 && !squares && !noAlloc && !u8Path && b->opt.sdcRows && nRows > 0 && dNnz == b->dCounters && rows_fusable(b)) {
 		b->nnzSlot = b->nnzRot;
-		const int r = launch_rmm_sdc_rows(b, -1, 0, dOut, b->dCounters + b->nnzSlot, dB, b->dCounters + (b->nnzRot % 3 + 1));
+		const int r = launch_rmm_sdc_rows(b, -1, 0, dOut, b->nnz_counter(b->nnzSlot), dB, b->nnz_counter(b->nnzRot % 3 + 1));
 		if(r < 0) return r;
 		if(r == 0) {
 			b->nnzRot = b->nnzRot % 3 + 1;
@@ -609,7 +609,7 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 		const int pad16 = (nG + 15) / 16 * 16 - nG, pad20 = (nG + 19) / 20 * 20 - nG;
 		const int per = pad20 < pad16 ? 20 : 16;
 		const double* constTerm = constRow >= 0 ? tables + constRow : nullptr;
-		unsigned long long* nnzNext = fused ? b->dCounters + (b->nnzRot % 3 + 1) : nullptr;
+		unsigned long long* nnzNext = fused ? b->nnz_counter(b->nnzRot % 3 + 1) : nullptr;
 		Prof pf(b, "k_rmm_q1_u8", grid, THREADS, per * 256 * 8, bytes);
 #define U8_LAUNCH(PER, NBV, LB, LN, F)                                                                          \
 	hipLaunchKernelGGL((k_rmm_q1_u8<THREADS, PER, NBV, LB, LN, F>), dim3(grid), dim3(THREADS), 0, st, b->dArena, \

@@ -1558,7 +1558,7 @@ int launch_tsmm_decode(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	L.A.out = dOut;
 	if(dNnz != nullptr) {
 		if((rc = ensure_gram_acc(b))) return rc;
-		L.A.acc = b->dGramAcc; L.A.done = (unsigned*) (b->dCounters + 7); L.A.nnz = dNnz;
+		L.A.acc = b->dGramAcc; L.A.done = b->gram_ticket(); L.A.nnz = dNnz;
 	}
 	Prof pf(b, "k_tsmm_decode", L.grid, DEC_THREADS, (long) L.lds, (double) b->device_bytes_cached);
 	// a last column block of at most 4 columns: its rows on the 4 x 4 x 4 matrix instruction

@@ -657,7 +657,7 @@ int launch_lmm_sdc_lanes(cla_block* b, const double* dY, int p, double* dOut) {
 	hipLaunchKernelGGL(k_lmm_sdc_lanes, dim3((unsigned) (parts * nS), p), dim3(waves * 64), lds, b->stream, (const LaneDesc*) meta,
 		(const LaneSlab*) (meta + b->laneOff[0]), nS, (const double*) (meta + b->laneOff[1]), (const uint32_t*) (meta + b->laneOff[3]),
 		b->laneDictLds, (const uint32_t*) (meta + b->laneOff[4]), (const u32x4*) b->dLaneData, dY, b->nRows, nWin, dOut, b->nCols,
-		tail ? (unsigned*) (b->dCounters + 6) : nullptr, b->dCounters);
+		tail ? b->lmm_ticket() : nullptr, b->dCounters);
 	b->lmmTailDone = tail;
 	CLA_HIP(hipGetLastError());
 	return 0;

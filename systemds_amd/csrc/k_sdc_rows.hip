@@ -176,7 +176,7 @@ __global__ __launch_bounds__(RW_THREADS) void k_rmm_sdc_rows(const int32_t* __re
 			if(j * RW_THREADS + tid < nTbl) tbl[j * RW_THREADS + tid] = tv[j];
 	}
 	if(tid == 0) tbl[nTbl] = 0.0;
-	if(FUSE && blockIdx.x == 0 && tid == 0) *nnzNext = 0;
+	if(FUSE && blockIdx.x == 0) nnz_clear(nnzNext);
 	const double init = !ACC && constRow >= 0 ? T[constRow] : 0.0;
 	__syncthreads();
 	int cntNz = 0;

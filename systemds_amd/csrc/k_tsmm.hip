@@ -590,7 +590,7 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	clear_stats(b);
 	auto clear = [&]() -> int {
 		CLA_HIP(hipMemsetAsync(dOut, 0, sizeof(double) * (size_t) nCols * nCols, st));
-		CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+		CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 		return 0;
 	};
 	// Overlapping column groups (the result of an overlapping right multiply): every compressed form here
@@ -1011,7 +1011,7 @@ __global__ __launch_bounds__(256) void k_count_nnz2(const double* __restrict__ x
 	__syncthreads();
 	if(threadIdx.x == 0) {
 		const int s = part[0] + part[1] + part[2] + part[3];
-		if(s) atomicAdd(nnz, (unsigned long long) s);
+		if(s) atomicAdd(nnz_way(nnz, 0), (unsigned long long) s);
 	}
 }
 
@@ -1133,7 +1133,7 @@ __global__ __launch_bounds__(256) void k_dense_rmm(const double* __restrict__ D,
 	__syncthreads();
 	if(tid == 0) {
 		const int s = part[0] + part[1] + part[2] + part[3];
-		if(s) atomicAdd(nnz, (unsigned long long) s);
+		if(s) atomicAdd(nnz_way(nnz, 0), (unsigned long long) s);
 	}
 }
 
@@ -1191,7 +1191,7 @@ int launch_decompress(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	const int64_t nRows = b->nRows, n = nRows * b->nCols;
 	hipStream_t st = b->stream;
 	clear_stats(b);
-	CLA_HIP(hipMemsetAsync(dNnz, 0, sizeof(unsigned long long), st));
+	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
 	if(n == 0) return 0;
 	const int rc = launch_decompress_rows(b, 0, nRows, dOut);
 	if(rc) return rc;

@@ -556,3 +556,23 @@ def test_wide_right_multiply_through_decompressed_rows(cla, ora, q):
     assert_matches_truth(out, D, B, what=f"X %*% B through decompressed rows, {q} columns")
     assert_matches_truth(gather, D, B, what=f"X %*% B, gather kernels, {q} columns")
     assert nnz == np.count_nonzero(out) and nnz_g == np.count_nonzero(gather)
+
+
+@pytest.mark.parametrize("n_rows", [1, 1025, 70003])
+def test_counts_of_calls_in_turn(cla, n_rows):
+    """The non-zero counters are spread over partial counts: one driver's must not show in the next one's, whichever
+    way a driver clears them (in a kernel, by a fill, in the last block of a call)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows)
+    n_cols = 9
+    d = [np.where(rng.random((20, 1)) < 0.4, 0.0, rng.standard_normal((20, 1))) for _ in range(n_cols)]
+    specs = [synth.GroupSpec("ddc", np.array([c], np.int32), d[c], rng.integers(0, 20, n_rows).astype(np.uint8))
+             for c in range(n_cols)]
+    blk = cla.build_block(n_rows, n_cols, specs)
+    v, B, Y = rng.standard_normal((n_cols, 1)), rng.standard_normal((n_cols, 10)), rng.standard_normal((2, n_rows))
+    calls = [lambda: blk.rmm(B), lambda: blk.lmm(Y), lambda: blk.rmm(v), blk.tsmm, blk.decompress, lambda: blk.lmm(Y[:1]),
+             lambda: blk.mmchain(v), lambda: blk.rmm(v), lambda: blk.rmm(B), blk.tsmm, lambda: blk.aggregate("sum", "row")]
+    for k, call in enumerate(calls):
+        out, nnz = call()
+        assert nnz == np.count_nonzero(out), f"call {k}"
+    blk.close()
