@@ -122,7 +122,7 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *   lmm_joint       1 / 0: Y %*% X (16 rows of Y per pass) on a block that is not mostly offset lists in passes over the decoded
  *                   rows on the matrix cores; blocks of more than 64 columns, or whose code tiles exceed LDS together, go chunk of
  *                   columns by chunk (sub-blocks kept with the block); single-column byte-code blocks only from 13 rows of Y
- *                   on (the kernel reports non-finite values of Y and the host looks, i.e. waits for the stream once per call;
+ *                   on and up to 32768 rows (the kernel reports non-finite values of Y and the host looks, i.e. waits for the stream once per call;
  *                   such a Y takes the bin kernels)
  *   tsmm_one_kernel 1 / 0: t(X) %*% X of a whole block of at most 64 columns on the decoded Gram kernels as the call's only
  *                   kernel (its blocks add into an accumulator kept with the block, nCols x nCols doubles; the last block

@@ -629,6 +629,9 @@ int finish_finalize(cla_block* b, cla_block* arenaFrom, bool buildArena) {
 	else if(allDdc && buildArena) {
 		const size_t stride = (((size_t) b->nRows * cw) + 255) & ~(size_t) 255;
 		CLA_HIP(hipMalloc((void**) &b->dArena, stride * nG));
+		// (kernels read whole vectors of codes at the end of a stream: the bytes behind the last row are valid codes too)
+		if(stride > (size_t) b->nRows * cw)
+			CLA_HIP(hipMemset2DAsync(b->dArena + (size_t) b->nRows * cw, stride, 0, stride - (size_t) b->nRows * cw, nG, b->stream));
 		for(size_t i = 0; i < nG; i++) {
 			HostGroup& g = b->groups[i];
 			uint8_t* dst = b->dArena + i * stride;
@@ -1513,9 +1516,9 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 			}
 	}
 	if(nOther == 0 || nLists > nOther) return 1;
-	// single-column byte codes: the dot kernel takes a pass per row of Y, a twelfth of what a pass of the decode kernel
-	// over 16 rows of Y costs (C2: 0.21 against 2.5 ms)
-	if(dotForm && (p + 15) / 16 * 12 >= p) return 1;
+	// Single-column byte codes have kernels of their own (k_lmm_u8_dot, k_lmm_u8_vec), faster at every size. What keeps 13 rows
+	// of Y and more on few rows here is that this form is covered on byte codes there (30,011 x 100 by 14: 66 against 21 us).
+	if(dotForm && !(b->opt.lmmDisable & 1) && (p < 13 || b->nRows > 32768)) return 1;
 	if(b->nCols > 64) return launch_lmm_chunked(b, dY, p, dOut, dNnz);
 	hipStream_t st = b->stream;
 	const size_t n = (size_t) p * b->nCols;

@@ -179,8 +179,10 @@ struct cla_block {
 	std::vector<uint8_t*> expCodes;
 	bool expTried = false;
 	// all groups single-column DDC with byte codes: dictionaries at a fixed stride of 256 entries
-	// (zero beyond nVals) followed by the groups' column indexes; built on first use
+	// (zero beyond nVals) followed by the groups' column indexes and, from dictTOff on, by the dictionaries
+	// of 16 groups at a time as [code][16] (maxVals codes)
 	double* dDictPad = nullptr;
+	size_t dictTOff = 0;
 	int64_t dictPadBytes = 0;
 	// list of SDCZeros groups + prefix sums of their nVals, as the row-tile kernels read it;
 	// built on first use for all groups (sdcPlanGroup -1) or for one group (its index)
@@ -263,6 +265,7 @@ int launch_rmm_mfma(cla_block* b, const double* dB, int q, const double* dConstR
 	unsigned long long* dNnz);
 int launch_lmm_u8(cla_block* b, const double* dY, int p, double* dPre);
 int launch_lmm_u8_dot(cla_block* b, const double* dY, int p, double* dOut);
+int launch_lmm_u8_vec(cla_block* b, const double* dY, double* dOut);
 int launch_lmm_sdc_tiles(cla_block* b, const double* dY, int p, double* dPre, int onlyGroup, double* dOut);
 int launch_lmm_sdc_lanes(cla_block* b, const double* dY, int p, double* dOut);
 int sdc_plan_all(cla_block* b); // the list of the block's SDCZeros groups with entries (b->sdcList)

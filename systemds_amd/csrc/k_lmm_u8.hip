@@ -142,7 +142,8 @@ int launch_lmm_u8(cla_block* b, const double* dY, int p, double* dPre) {
 }
 
 // ---------------------------------------------------------------------------
-// The same blocks when every group has a single column: out[col_g] += sum_r Y[i, r] *
+// The same blocks when every group has a single column, one row of Y and many rows (fewer rows and more rows of Y:
+// k_lmm_u8_dot): out[col_g] += sum_r Y[r] *
 // dict_g[code_g[r]] directly, the mirror image of the mat-vec gather. Dictionaries of a slab
 // of groups sit in LDS at a fixed stride, a thread keeps 16 values of Y in registers, looks
 // up 16 dictionary values per group, multiplies and sums them and adds the sum into one of
@@ -182,7 +183,7 @@ __device__ __forceinline__ void u8_dot(const CodeVec<1, RPT> (&cv)[NB], const ch
 }
 
 template <int PER, int NB, int LB, int LN>
-__global__ __launch_bounds__(LD_THREADS, 4) void k_lmm_u8_dot(const uint8_t* __restrict__ arena, size_t arenaStride, int nGroups,
+__global__ __launch_bounds__(LD_THREADS, 4) void k_lmm_u8_vec(const uint8_t* __restrict__ arena, size_t arenaStride, int nGroups,
 	const double* __restrict__ dictPad, const int32_t* __restrict__ col0, const double* __restrict__ Y, int64_t nRows,
 	double* __restrict__ out, int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz) {
 	static_assert(PER % (2 * NB) == 0, "a slab holds whole ping/pong turns");
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(LD_THREADS, 4) void k_lmm_u8_dot(const uint8_t* __r
 	const int off = tid * RPT;
 	const int gLast = nGroups - 1;
 	const int nPad = (nGroups + PER - 1) / PER * PER;
-	const double* y = Y + (size_t) blockIdx.y * nRows;
+	const double* y = Y;
 
 	// shares of whole units of 64 * RPT rows that differ by at most one unit between blocks (see k_rmm_q1_u8)
 	constexpr int UNIT = 64 * RPT;
@@ -287,25 +288,30 @@ __global__ __launch_bounds__(LD_THREADS, 4) void k_lmm_u8_dot(const uint8_t* __r
 		double v = 0.0;
 #pragma unroll
 		for(int k = 0; k < LD_SLOTS; k++) v += slots[g * LD_SLOTS + k];
-		if(v != 0.0) unsafeAtomicAdd(&out[(size_t) blockIdx.y * nCols + col0[g]], v);
+		if(v != 0.0) unsafeAtomicAdd(&out[col0[g]], v);
 	}
-	lmm_tail(done, gridDim.x * gridDim.y, out, (int) gridDim.y * nCols, nnz);
+	lmm_tail(done, gridDim.x, out, nCols, nnz);
 }
 
 // All groups DDC with byte codes in one arena and one column each: the dictionaries at a fixed stride of
-// 256 entries (zero beyond nVals), followed by the groups' column indexes. Built once at finalize (200 KB
-// for 100 groups); the byte-code mat-vec and the dot-form left multiply read their slabs from it.
+// 256 entries (zero beyond nVals), followed by the groups' column indexes, followed by the dictionaries of 16
+// groups at a time as [code][16]. Built once at finalize (2 x 200 KB for 100 groups); the byte-code mat-vec and the
+// left multiplies read their slabs from it.
 int ensure_dict_pad(cla_block* b) {
 	const int nG = (int) b->groups.size();
 	if(b->dDictPad != nullptr || !(b->dArena && b->arenaWidth == 1 && b->maxVals <= 256 && nG > 0 && b->nRows > 0)) return 0;
 	for(int g = 0; g < nG; g++)
 		if(b->groups[g].d.nColG != 1) return 0;
-	std::vector<double> img((size_t) nG * 256 + (size_t) (nG + 1) / 2 + 1, 0.0);
+	const int nV = b->maxVals;
+	b->dictTOff = ((size_t) nG * 256 + (size_t) (nG + 1) / 2 + 1) & ~(size_t) 1; // (16-byte pieces)
+	std::vector<double> img(b->dictTOff + (size_t) (nG + 15) / 16 * nV * 16, 0.0);
 	int32_t* cols = (int32_t*) (img.data() + (size_t) nG * 256);
 	for(int g = 0; g < nG; g++) {
 		const HostGroup& H = b->groups[g];
 		std::copy(H.dict.begin(), H.dict.begin() + H.d.nVals, img.begin() + (size_t) g * 256);
 		cols[g] = H.cols[0];
+		double* t = img.data() + b->dictTOff + (size_t) (g / 16) * nV * 16 + g % 16;
+		for(int k = 0; k < H.d.nVals; k++) t[(size_t) k * 16] = H.dict[k];
 	}
 	CLA_HIP(hipMalloc((void**) &b->dDictPad, img.size() * sizeof(double)));
 	b->dictPadBytes = (int64_t) (img.size() * sizeof(double));
@@ -314,8 +320,8 @@ int ensure_dict_pad(cla_block* b) {
 	return 0;
 }
 
-// Returns 1 when the block is not eligible, 0 when the groups' contributions have been added to dOut.
-int launch_lmm_u8_dot(cla_block* b, const double* dY, int p, double* dOut) {
+// One row of Y. Returns 1 when the block is not eligible, 0 when the groups' contributions have been added to dOut.
+int launch_lmm_u8_vec(cla_block* b, const double* dY, double* dOut) {
 	const int nG = (int) b->groups.size();
 	if(!(b->dArena && b->arenaWidth == 1 && b->maxVals <= 256 && nG > 0 && b->nRows > 0)) return 1;
 	if(b->opt.lmmDisable & 1) return 1;
@@ -331,13 +337,13 @@ int launch_lmm_u8_dot(cla_block* b, const double* dY, int p, double* dOut) {
 	if(b->dDictPad == nullptr) return 1;
 	const int32_t* dCol0 = (const int32_t*) (b->dDictPad + (size_t) nG * 256);
 	const int perCU = 2;
-	const unsigned grid = (unsigned) std::min<int64_t>((b->nRows + 2047) / 2048, std::max(1, g_numCU * perCU / std::min(p, g_numCU * perCU)));
-	const double algo = (double) p * ((double) b->nRows * nG + (double) b->nRows * 8);
-	Prof pf(b, "k_lmm_u8_dot", (long) grid * p, LD_THREADS, (long) lds, algo);
-	auto kern = k_lmm_u8_dot<PER, 5, 4, 2>;
+	const unsigned grid = (unsigned) std::min<int64_t>((b->nRows + 2047) / 2048, g_numCU * perCU);
+	const double algo = (double) b->nRows * nG + (double) b->nRows * 8;
+	Prof pf(b, "k_lmm_u8_vec", grid, LD_THREADS, (long) lds, algo);
+	auto kern = k_lmm_u8_vec<PER, 5, 4, 2>;
 	CLA_HIP(allow_full_lds((const void*) kern));
 	const bool tail = b->lmmTailWanted; // (this kernel serves every group of the block)
-	hipLaunchKernelGGL(kern, dim3(grid, p), dim3(LD_THREADS), lds, b->stream, b->dArena, b->arenaStride, nG, b->dDictPad, dCol0, dY,
+	hipLaunchKernelGGL(kern, dim3(grid), dim3(LD_THREADS), lds, b->stream, b->dArena, b->arenaStride, nG, b->dDictPad, dCol0, dY,
 		b->nRows, dOut, b->nCols, tail ? b->lmm_ticket() : nullptr, b->dCounters);
 	b->lmmTailDone = tail;
 	CLA_HIP(hipGetLastError());

@@ -336,3 +336,24 @@ def test_repeated_calls_count_their_own_non_zeros(cla, ora):
     for got, Y in zip(outs, Ys):
         assert np.array_equal(got != 0, blk.lmm(Y)[0] != 0)
     blk.close()
+
+
+@pytest.mark.parametrize("n_rows,n_cols,n_vals", [(1, 1, 1), (63, 16, 2), (64, 17, 256), (65, 64, 7), (4097, 65, 256), (33333, 100, 200), (70001, 130, 3)])
+@pytest.mark.parametrize("p", [1, 4, 5, 12, 13, 16, 17, 33])
+def test_byte_codes_on_the_matrix_cores(cla, ora, n_rows, n_cols, n_vals, p):
+    """k_lmm_u8_dot at the edges of its tiles: units of 64 rows, column blocks of 16 groups, slabs of column blocks, every
+    number of rows of Y it is instantiated for and passes of 16."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows + p)
+    specs = [synth.GroupSpec("ddc", np.array([c], np.int32), rng.standard_normal((n_vals, 1)),
+                             rng.integers(0, n_vals, n_rows).astype(np.uint8)) for c in rng.permutation(n_cols)]
+    Y = rng.standard_normal((p, n_rows))
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, nnz = blk.lmm(Y)
+    names = {k["name"] for k in blk.stats()["kernels"]}
+    blk.close()
+    if p < 13 or n_rows > 32768:
+        assert names == {"k_lmm_u8_dot"}, names
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    assert_matches_truth(out, Y, D, what=f"{n_rows} x {n_cols}, {p} rows of Y")
+    assert nnz == np.count_nonzero(out)
