@@ -103,6 +103,7 @@ struct KernelStat {
 struct DecPlanCache;
 struct DirPlan;
 struct GdrPlan;
+struct GtPlan;
 
 } // namespace cla
 
@@ -197,6 +198,7 @@ struct cla_block {
 	cla::DecPlanCache* decPlans = nullptr; // decode kernels (k_rmm_decode.hip): plans per product shape, dropped by dec_plans_drop
 	cla::DirPlan* dirPlan = nullptr;     // plan of k_rmm_direct (dropped with the decode plans)
 	cla::GdrPlan* gdrPlan = nullptr;     // plan of k_tsmm_direct (likewise)
+	cla::GtPlan* gtPlan = nullptr;       // plan of k_gram_tiles (likewise)
 	void* dMfPlan = nullptr;         // matrix-core right multiply (k_rmm_mfma.hip): slab descriptors, column info, code streams, B row list
 	int mfState = 0;                 // 0 not planned yet, 1 ready, -1 not eligible
 	int mfNSlabs = 0, mfNColsAll = 0, mfWidth = 1, mfMaxKc = 0, mfNRowCol = 0, mfMaxDict = 0;
@@ -275,6 +277,8 @@ int launch_rmm_sdc_rows(cla_block* b, int constRow, int accumulate, double* dOut
 bool rows_fusable(cla_block* b);
 int launch_rmm_sdc_tiles(cla_block* b, int q, int constRow, int accumulate, double* dOut, unsigned long long* dNnz);
 int launch_tsmm_decode(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);
+int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);
+void gt_plan_drop(cla_block* b);
 int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);
 int ensure_gram_acc(cla_block* b); // the zeroed nCols x nCols accumulator of the one-kernel t(X) %*% X (a workspace kept with the block)
 int ensure_expanded(cla_block* b);

@@ -1,0 +1,397 @@
+// t(X) %*% X of a block whose groups are all DDC with one code width (one or two bytes), 13 to 128 columns, as the Gram
+// matrix of the decoded rows: every row is decoded once, into a tile of doubles in LDS that all waves multiply from.
+//
+// A workgroup of 8 waves (one per CU) takes a contiguous share of the rows in tiles of R = 32 m rows, two tile buffers in
+// LDS. Decoding is dealt by (16 columns, 32 rows): lane (k, c), k = lane / 16, c = lane % 16, holds 8 consecutive codes of
+// column c, looks them up (in LDS where the column block's dictionaries fit beside the tiles, [code][16 columns], else
+// straight in global memory) and writes the values to its rows of the tile. Multiplying: lane (k, c) reads X[row 4 s + k, 16 b + c],
+// which is both operands of v_mfma_f64_16x16x4 for column block b, so a step of 4 rows costs one LDS read per column block
+// for all its tiles. Up to 5 column blocks a wave keeps all tiles on or above the diagonal and the waves share the
+// tile's rows; from 6 on two waves share a set of rows and the tiles (the sums of 14 of 28 tiles take 112 registers).
+// A last column block of at most 8 columns goes through v_mfma_f64_4x4x4 (4 columns x 16, 17 cycles instead of 70).
+//
+// The stages of three tiles overlap: while a tile is multiplied, the values of the next one but one are looked up and the
+// codes behind those are on their way. One barrier per tile that waits for LDS only: loads stay in flight over it.
+//
+// Bound: the fp64 matrix pipe (70 cycles per tile and 4 rows).
+#include "../../include/cla_hip.h"
+#include "cla_device.hpp"
+#include "cla_runs.hpp"
+#include <algorithm>
+#include <cstring>
+
+namespace cla {
+
+constexpr int GT_THREADS = 512;
+typedef double f64x4_gt __attribute__((ext_vector_type(4)));
+
+// a decoded column
+struct GtCol {
+	int32_t dictOff;  // bytes from the dictionary base to its first value
+	int32_t stride;   // bytes from one code's value to the next one's
+	int32_t group;    // code stream
+	int32_t col;      // column of the block (-1: padding)
+};
+
+struct GtArgs {
+	const uint8_t* arena;
+	size_t arenaStride;
+	const GtCol* cols;       // NCB * 16
+	const double* dict;
+	const double* img;       // column blocks [0, nLds): imgV x 16 values each
+	int64_t nRows;
+	int nTiles, nLds, imgV, nCols;
+	double* acc;             // where the blocks add (upper triangle)
+	double* out;
+	unsigned* done;          // nullptr: no tail (acc is the caller's output)
+	unsigned long long* nnz;
+};
+
+__host__ __device__ constexpr int gt_m(int ncb) { return ncb == 1 ? 8 : ncb == 2 ? 3 : ncb <= 4 ? 2 : 1; } // 32 m rows per tile, m * ncb <= 8
+__host__ __device__ constexpr int gt_stride(int ncb) { return ncb * 16 + (ncb & 1 ? 0 : 16); } // doubles per row: rows 128 bytes apart in the banks
+
+// Barrier of the workgroup that waits for this wave's LDS accesses only.
+__device__ __forceinline__ void lds_barrier() {
+	asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+	__builtin_amdgcn_s_barrier();
+	asm volatile("" ::: "memory");
+}
+
+// NF full column blocks, then one of NN groups of 4 columns (NN = 0: none), W bytes per code
+template <int NF, int NN, int W>
+__global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
+	constexpr int NCB = NF + (NN ? 1 : 0), T = NF * (NF + 1) / 2;
+	constexpr int M = gt_m(NCB), R = 32 * M, S = gt_stride(NCB);
+	constexpr bool SPLIT = NF > 5;              // two waves share the tiles of a set of rows
+	constexpr int NK = SPLIT ? 2 * M : M;       // steps of 4 rows per wave and tile
+	constexpr int BUF = R * S;
+	// what a wave keeps of the T tiles and of the NCB products of a narrow group: SPLIT deals tiles [0, T0) and even
+	// column blocks to waves 0 - 3, the others to waves 4 - 7
+	constexpr int T0 = SPLIT ? T / 2 : T, TW = SPLIT ? T - T0 : T, NB = SPLIT ? (NCB + 1) / 2 : NCB;
+	extern __shared__ __attribute__((aligned(16))) double smem[]; // two tile buffers, the dictionaries
+	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int c = lane & 15, k = lane >> 4;
+	const int t0 = (int) ((int64_t) A.nTiles * blockIdx.x / gridDim.x), t1 = (int) ((int64_t) A.nTiles * (blockIdx.x + 1) / gridDim.x);
+
+	// this wave's part of the decoding: column block, 32 rows of the tile
+	const int myCb = wave % NCB, sub = wave / NCB;
+	const int mode = wave >= NCB * M || t0 >= t1 ? 0 : myCb < A.nLds ? 1 : 2; // nothing, dictionary in LDS, in global memory
+	const GtCol C = A.cols[myCb * 16 + c];
+	const uint8_t* stream = A.arena + (size_t) C.group * A.arenaStride;
+	const char* ldsDict = (const char*) (smem + 2 * BUF) + (size_t) myCb * A.imgV * 128 + c * 8;
+	const char* gDict = (const char*) A.dict;
+	const int64_t rowLast = (A.nRows - 1) & ~(int64_t) 7;
+	double* const put = smem + (sub * 32 + 8 * k) * S + myCb * 16 + c;
+
+	f64x4_gt acc[TW];
+	double nacc[NN ? NN : 1][NB];
+#pragma unroll
+	for(int t = 0; t < TW; t++) acc[t] = f64x4_gt{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+	for(int i = 0; i < (NN ? NN : 1); i++)
+#pragma unroll
+		for(int b = 0; b < NB; b++) nacc[i][b] = 0.0;
+
+	auto loop = [&](auto modeTag, auto halfTag) {
+		constexpr int MODE = decltype(modeTag)::value, HALF = decltype(halfTag)::value;
+		CodeVec<W, 8> codes;
+		double v[2][8];
+		auto load_codes = [&](int tile) {
+			if(MODE == 0) return;
+			const int64_t row = min((int64_t) min(tile, t1 - 1) * R + sub * 32 + 8 * k, rowLast);
+			if constexpr(W == 1) codes.raw.v = *(const u32x2*) (stream + row);
+			else codes.raw.v = *(const u32x4*) (stream + 2 * row);
+		};
+		auto look = [&](double (&d)[8]) {
+			if(MODE == 0) return;
+#pragma unroll
+			for(int t = 0; t < 8; t++) {
+				const uint32_t code = (uint32_t) codes.get(t);
+				if(MODE == 1) d[t] = *(const double*) (ldsDict + (code << 7));
+				else d[t] = *(const double*) (gDict + (uint32_t) (__umul24(code, (uint32_t) C.stride) + (uint32_t) C.dictOff));
+			}
+		};
+		auto write = [&](const double (&d)[8], int tile, int buf) {
+			if(MODE == 0) return;
+			double* p = put + buf * BUF;
+			if((int64_t) (tile + 1) * R <= A.nRows) {
+#pragma unroll
+				for(int t = 0; t < 8; t++) p[t * S] = d[t];
+			}
+			else { // zeros behind the last row of the matrix
+				const int64_t row = (int64_t) tile * R + sub * 32 + 8 * k;
+#pragma unroll
+				for(int t = 0; t < 8; t++) p[t * S] = row + t < A.nRows ? d[t] : 0.0;
+			}
+		};
+		auto multiply = [&](int buf) {
+			const double* x0 = smem + buf * BUF + ((SPLIT ? wave & 3 : wave) * 4 + k) * S;
+			double x[2][NCB], a[2][NN ? NN : 1];
+			auto read = [&](int j) {
+				const double* p = x0 + j * (SPLIT ? 16 : 32) * S;
+#pragma unroll
+				for(int b = 0; b < NCB; b++) x[j & 1][b] = p[16 * b + c];
+#pragma unroll
+				for(int i = 0; i < NN; i++) a[j & 1][i] = p[16 * NF + 4 * i + (lane & 3)];
+			};
+			read(0);
+#pragma unroll
+			for(int j = 0; j < NK; j++) {
+				if(j + 1 < NK) read(j + 1);
+				int t = 0;
+#pragma unroll
+				for(int p = 0; p < NF; p++)
+#pragma unroll
+					for(int q = p; q < NF; q++, t++)
+						if((t < T0) == (HALF == 0))
+							acc[t - HALF * T0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[j & 1][p], x[j & 1][q], acc[t - HALF * T0], 0, 0, 0);
+#pragma unroll
+				for(int i = 0; i < NN; i++)
+#pragma unroll
+					for(int b = 0; b < NCB; b++)
+						if(!SPLIT || (b & 1) == HALF)
+							nacc[i][SPLIT ? b / 2 : b] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[j & 1][i], x[j & 1][b], nacc[i][SPLIT ? b / 2 : b], 0, 0, 0);
+			}
+		};
+		load_codes(t0);
+		{
+			// the dictionaries of the first column blocks, 8 pieces of 16 bytes per thread requested together
+			const f64x2* src = (const f64x2*) A.img;
+			f64x2* dst = (f64x2*) (smem + 2 * BUF);
+			const int n = A.nLds * A.imgV * 8;
+			for(int i0 = tid; i0 < n; i0 += 8 * GT_THREADS) {
+				f64x2 d[8];
+#pragma unroll
+				for(int j = 0; j < 8; j++) d[j] = src[min(i0 + j * GT_THREADS, n - 1)];
+#pragma unroll
+				for(int j = 0; j < 8; j++)
+					if(i0 + j * GT_THREADS < n) dst[i0 + j * GT_THREADS] = d[j];
+			}
+		}
+		lds_barrier();
+		look(v[0]);
+		load_codes(t0 + 1);
+		look(v[1]);
+		load_codes(t0 + 2);
+		write(v[0], t0, 0);
+		lds_barrier();
+		auto step = [&](int tile, auto parity) {
+			constexpr int P = decltype(parity)::value;
+			look(v[P]);                    // of tile + 2
+			load_codes(tile + 3);
+			multiply(P);
+			write(v[P ^ 1], min(tile + 1, t1 - 1), P ^ 1); // (behind the last tile: values nobody reads)
+			lds_barrier();
+		};
+		using std::integral_constant;
+		for(int tile = t0; tile < t1; tile += 2) {
+			step(tile, integral_constant<int, 0>());
+			if(tile + 1 < t1) step(tile + 1, integral_constant<int, 1>());
+		}
+	};
+	if(t0 < t1) {
+		using std::integral_constant;
+		if(SPLIT && wave >= 4) {
+			if(mode == 0) loop(integral_constant<int, 0>(), integral_constant<int, 1>());
+			else if(mode == 1) loop(integral_constant<int, 1>(), integral_constant<int, 1>());
+			else loop(integral_constant<int, 2>(), integral_constant<int, 1>());
+		}
+		else {
+			if(mode == 0) loop(integral_constant<int, 0>(), integral_constant<int, 0>());
+			else if(mode == 1) loop(integral_constant<int, 1>(), integral_constant<int, 0>());
+			else loop(integral_constant<int, 2>(), integral_constant<int, 0>());
+		}
+	}
+
+	// the waves' sums of a tile, one set of rows after the other
+	double* sum = smem;
+	const int half = SPLIT ? wave >> 2 : 0, set = SPLIT ? wave & 3 : wave;
+	for(int s = 0; s < (SPLIT ? 4 : 8); s++) {
+		if(set == s) {
+#pragma unroll
+			for(int l = 0; l < TW; l++) {
+				const int t = l + half * T0;
+				if(half == 0 && l >= T0) continue;
+#pragma unroll
+				for(int i = 0; i < 4; i++) {
+					double* p = &sum[t * 256 + i * 64 + lane];
+					*p = s == 0 ? acc[l][i] : *p + acc[l][i];
+				}
+			}
+#pragma unroll
+			for(int i = 0; i < NN; i++)
+#pragma unroll
+				for(int l = 0; l < NB; l++) {
+					const int b = SPLIT ? 2 * l + half : l;
+					if(b >= NCB) continue;
+					double* p = &sum[T * 256 + (i * NCB + b) * 64 + lane];
+					*p = s == 0 ? nacc[i][l] : *p + nacc[i][l];
+				}
+		}
+		__syncthreads();
+	}
+	auto add = [&](int ca, int cb, double d) {
+		if(ca >= 0 && cb >= 0 && d != 0.0) unsafeAtomicAdd(&A.acc[(size_t) min(ca, cb) * A.nCols + max(ca, cb)], d);
+	};
+	for(int i = tid; i < T * 256; i += GT_THREADS) {
+		int t = i >> 8, p = 0;
+		while(t >= NF - p) { t -= NF - p; p++; }
+		const int q = p + t, r = ((i >> 6) & 3) * 4 + ((i & 63) >> 4), cc = i & 15;
+		if(p != q || r <= cc) add(A.cols[16 * p + r].col, A.cols[16 * q + cc].col, sum[i]);
+	}
+	for(int i = tid; i < NN * NCB * 64; i += GT_THREADS) {
+		const int g = i / (NCB * 64), b = i / 64 % NCB, r = 4 * g + ((i & 63) >> 4), cc = i & 15;
+		if(b < NF || r <= cc) add(A.cols[16 * NF + r].col, A.cols[16 * b + cc].col, sum[T * 256 + i]);
+	}
+	if(A.done != nullptr) {
+		__syncthreads();
+		gram_tail(A.done, gridDim.x, A.acc, A.out, A.nCols, A.nnz, (unsigned*) smem);
+	}
+}
+
+// ---- plan (kept with the block, dropped with the decode plans)
+
+struct GtPlan {
+	int rc = 0;       // 1: not of this kernel's shape
+	GtArgs A;
+	void* dImg = nullptr;
+	int64_t bytes = 0;
+	int nf = 0, nn = 0, w = 0;
+	size_t lds = 0;
+};
+
+static int gt_build_plan(cla_block* b, GtPlan& P) {
+	P.rc = 1;
+	const int n = b->nCols;
+	if(b->dArena == nullptr || b->arenaWidth > 2 || n < 13 || n > 128 || b->nRows == 0 || b->crossSplit > 0 || b->crossBlocks > 0) return 0;
+	std::vector<int> groupOf((size_t) n, -1);
+	for(size_t g = 0; g < b->groups.size(); g++)
+		for(int col : b->groups[g].cols) {
+			if(groupOf[col] >= 0) return 0; // overlapping groups
+			groupOf[col] = (int) g;
+		}
+	// columns in the groups' order, then those that only carry a constant
+	const int last = n - n / 16 * 16;
+	P.nn = last >= 1 && last <= 4 ? 1 : last >= 5 && last <= 8 ? 2 : 0;
+	P.nf = n / 16 + (last > 8 ? 1 : 0);
+	P.w = b->arenaWidth;
+	const int ncb = P.nf + (P.nn ? 1 : 0);
+	bool consts = false; // the dictionaries are copied with the constants added
+	for(int col = 0; col < n; col++) consts |= b->constV[col] != 0.0 || groupOf[col] < 0;
+	std::vector<GtCol> cols;
+	std::vector<double> dict;
+	std::vector<const double*> src; // host values of a column (nullptr: only a constant)
+	size_t total = 0;
+	for(size_t g = 0; g < b->groups.size(); g++) {
+		const HostGroup& H = b->groups[g];
+		const int nc = H.d.nColG;
+		for(int h = 0; h < nc; h++) {
+			cols.push_back(GtCol{(int32_t) ((total + h) * 8), nc * 8, (int32_t) g, H.cols[h]});
+			src.push_back(H.dict.data() + h);
+		}
+		if(consts)
+			for(size_t i = 0; i < H.dict.size(); i++) dict.push_back(H.dict[i] + b->constV[H.cols[i % nc]]);
+		total += H.dict.size();
+	}
+	for(int col = 0; col < n; col++)
+		if(groupOf[col] < 0) {
+			cols.push_back(GtCol{(int32_t) (total * 8), 0, 0, col});
+			src.push_back(nullptr);
+			dict.push_back(b->constV[col]);
+			total++;
+		}
+	if(total * 8 >= ((size_t) 1 << 31) || (int) cols.size() != n) return 0;
+	const int real = n;
+	while((int) cols.size() < ncb * 16) { GtCol p = cols[real - 1]; p.col = -1; cols.push_back(p); src.push_back(src[real - 1]); }
+	// column blocks whose dictionaries fit LDS beside the tiles
+	const size_t tileBytes = (size_t) 2 * 32 * gt_m(ncb) * gt_stride(ncb) * 8;
+	const size_t sumBytes = ((size_t) P.nf * (P.nf + 1) / 2 * 256 + (size_t) P.nn * ncb * 64) * 8;
+	const size_t room = (size_t) g_ldsPerBlock - tileBytes;
+	const int imgV = std::max(b->maxVals, 1);
+	const int nLds = (int) std::min<size_t>(ncb, room / ((size_t) imgV * 128));
+	P.lds = std::max(tileBytes + (size_t) nLds * imgV * 128, sumBytes);
+	if(P.lds > (size_t) g_ldsPerBlock) return 0;
+	std::vector<double> img((size_t) nLds * imgV * 16, 0.0);
+	for(int s = 0; s < nLds * 16; s++) {
+		const GtCol& C = cols[s];
+		const double add = b->constV[cols[std::min(s, real - 1)].col];
+		const int nV = src[s] ? b->groups[C.group].d.nVals : imgV;
+		for(int kk = 0; kk < nV; kk++)
+			img[((size_t) (s / 16) * imgV + kk) * 16 + s % 16] = (src[s] ? src[s][(size_t) kk * (C.stride / 8)] : 0.0) + add;
+	}
+	const size_t colBytes = cols.size() * sizeof(GtCol), imgBytes = img.size() * 8, dictBytes = consts ? dict.size() * 8 : 0;
+	std::vector<uint8_t> all(colBytes + imgBytes + dictBytes + 16, 0);
+	std::memcpy(all.data(), cols.data(), colBytes);
+	if(imgBytes) std::memcpy(all.data() + colBytes, img.data(), imgBytes);
+	if(dictBytes) std::memcpy(all.data() + colBytes + imgBytes, dict.data(), dictBytes);
+	uint8_t* d = nullptr;
+	CLA_HIP(hipMalloc((void**) &d, all.size()));
+	P.dImg = d;
+	P.bytes = (int64_t) all.size();
+	CLA_HIP(hipMemcpy(d, all.data(), all.size(), hipMemcpyHostToDevice));
+	GtArgs& A = P.A;
+	A.arena = b->dArena; A.arenaStride = b->arenaStride;
+	A.cols = (const GtCol*) d;
+	A.img = (const double*) (d + colBytes);
+	A.dict = consts ? (const double*) (d + colBytes + imgBytes) : b->dAllDict;
+	A.nRows = b->nRows;
+	A.nTiles = (int) ((b->nRows + 32 * gt_m(ncb) - 1) / (32 * gt_m(ncb)));
+	A.nLds = nLds; A.imgV = imgV; A.nCols = n;
+	P.rc = 0;
+	return 0;
+}
+
+void gt_plan_drop(cla_block* b) {
+	if(b->gtPlan == nullptr) return;
+	if(b->gtPlan->dImg) { (void) hipFree(b->gtPlan->dImg); b->derivedBytes -= b->gtPlan->bytes; }
+	delete b->gtPlan;
+	b->gtPlan = nullptr;
+}
+
+template <int NF, int NN>
+static int gt_launch(cla_block* b, const GtPlan& P, const GtArgs& A, unsigned grid) {
+	if(P.w == 1) {
+		CLA_HIP(allow_full_lds((const void*) k_gram_tiles<NF, NN, 1>));
+		hipLaunchKernelGGL((k_gram_tiles<NF, NN, 1>), dim3(grid), dim3(GT_THREADS), P.lds, b->stream, A);
+	}
+	else {
+		CLA_HIP(allow_full_lds((const void*) k_gram_tiles<NF, NN, 2>));
+		hipLaunchKernelGGL((k_gram_tiles<NF, NN, 2>), dim3(grid), dim3(GT_THREADS), P.lds, b->stream, A);
+	}
+	CLA_HIP(hipGetLastError());
+	return 0;
+}
+
+// Like launch_tsmm_decode: dNnz != nullptr: the call's only kernel, which writes dOut whole; else dOut (zeroed) gets the upper
+// triangle. Returns 1 when the block is not of this kernel's shape.
+int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz) {
+	if(b->gtPlan == nullptr) {
+		b->gtPlan = new GtPlan();
+		const int rc = gt_build_plan(b, *b->gtPlan);
+		if(b->gtPlan->dImg) b->derivedBytes += b->gtPlan->bytes;
+		if(rc < 0) { gt_plan_drop(b); return rc; }
+	}
+	const GtPlan& P = *b->gtPlan;
+	if(P.rc) return P.rc;
+	GtArgs A = P.A;
+	A.acc = dOut; A.out = dOut; A.done = nullptr; A.nnz = nullptr;
+	if(dNnz != nullptr) {
+		const int rc = ensure_gram_acc(b);
+		if(rc) return rc;
+		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
+	}
+	const unsigned grid = (unsigned) std::min(A.nTiles, g_numCU);
+	// (reported under the name of the form, the decoded Gram matrix, whichever of its kernels runs)
+	Prof pf(b, "k_tsmm_decode", grid, GT_THREADS, (long) P.lds, (double) b->device_bytes_cached);
+#define GT_CASE(NF) \
+	case NF: return P.nn == 0 ? gt_launch<NF, 0>(b, P, A, grid) : P.nn == 1 ? gt_launch<NF, 1>(b, P, A, grid) : gt_launch<NF, 2>(b, P, A, grid);
+	switch(P.nf) {
+		case 1: return P.nn == 0 ? gt_launch<1, 0>(b, P, A, grid) : P.nn == 1 ? gt_launch<1, 1>(b, P, A, grid) : gt_launch<1, 2>(b, P, A, grid);
+		GT_CASE(2) GT_CASE(3) GT_CASE(4) GT_CASE(5) GT_CASE(6) GT_CASE(7)
+		case 8: return gt_launch<8, 0>(b, P, A, grid);
+	}
+#undef GT_CASE
+	return 1;
+}
+
+} // namespace cla

@@ -981,6 +981,7 @@ void gdr_plan_drop(cla_block* b);
 void dec_plans_drop(cla_block* b) {
 	dir_plan_drop(b);
 	gdr_plan_drop(b);
+	gt_plan_drop(b);
 	if(b->decPlans == nullptr) return;
 	for(auto& e : b->decPlans->entries)
 		if(e.dImg) { (void) hipFree(e.dImg); b->derivedBytes -= e.bytes; }
@@ -1543,7 +1544,9 @@ int launch_tsmm_decode(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	if(b->groups.empty() || b->nRows == 0 || nCols > 64) return 1;
 	if(dNnz != nullptr && (b->crossBlocks > 0 || b->crossSplit > 0)) return 1; // (only a part of the Gram matrix is wanted: no one-kernel form)
 	{
-		const int rc = launch_tsmm_direct(b, dOut, dNnz);
+		int rc = launch_tsmm_direct(b, dOut, dNnz);
+		if(rc != 1) return rc;
+		rc = launch_gram_tiles(b, dOut, dNnz);
 		if(rc != 1) return rc;
 	}
 	const int NB = (nCols + 15) / 16;

@@ -644,6 +644,20 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	// accumulator kept with the block, and the last one to finish writes the output (both triangles) and the count of
 	// its non-zeros and clears the accumulator again: no fill in front of the kernel, no kernel behind it.
 	bool decodeTried = false;
+	// All-DDC blocks of 13 to 128 columns: every row decoded once (k_gram_tiles), whatever the number of groups
+	if(!forcePairs && split == 0 && b->crossBlocks == 0 && nRows > 0 && b->opt.tsmmMfma && (nCols <= 64 || b->opt.tsmmChunks)) {
+		if(!b->opt.tsmmOneKernel && (rc = clear())) return rc;
+		rc = nCols <= 64 && dense ? 1 : launch_gram_tiles(b, dOut, b->opt.tsmmOneKernel ? dNnz : nullptr);
+		if(rc < 0) return rc;
+		if(rc == 0) {
+			if(!b->opt.tsmmOneKernel) {
+				Prof pf(b, "k_tsmm_finish", 1, 256, 0, 0);
+				hipLaunchKernelGGL(k_tsmm_finish, dim3(1), dim3(256), 0, st, dOut, nCols, b->dConstV, b->dConstV, (double) nRows, 0, dNnz);
+				CLA_HIP(hipGetLastError());
+			}
+			return 0;
+		}
+	}
 	if(dense && nCols <= 64 && split == 0 && b->crossBlocks == 0 && nRows > 0 && b->opt.tsmmMfma && b->opt.tsmmOneKernel) {
 		decodeTried = true;
 		rc = launch_tsmm_decode(b, dOut, dNnz);
