@@ -10,6 +10,11 @@
 // tile's rows; from 6 on two waves share a set of rows and the tiles (the sums of 14 of 28 tiles take 112 registers).
 // A last column block of at most 8 columns goes through v_mfma_f64_4x4x4 (4 columns x 16, 17 cycles instead of 70).
 //
+// Two-byte codes of column pairs (co-coded groups): a wave's 64 lanes look up one group at 64 rows (below 64 rows per tile two
+// groups), a whole tuple of 16 bytes per lane, and write it to the lane's row of the tile. Dealt like the others the gathers
+// of 8 bytes bound the kernel: 10,000,000 x 50, 4096 tuples (Zipf), 1001 us; so 934, with the gathers spread between the
+// matrix instructions 692 (matrix pipe 496, gathers 400).
+//
 // The stages of three tiles overlap: while a tile is multiplied, the values of the next one but one are looked up and the
 // codes behind those are on their way. One barrier per tile that waits for LDS only: loads stay in flight over it.
 //
@@ -40,15 +45,19 @@ struct GtArgs {
 	const double* dict;
 	const double* img;       // column blocks [0, nLds): imgV x 16 values each
 	int64_t nRows;
-	int nTiles, nLds, imgV, nCols;
+	int nTiles, nLds, imgV, nCols, nGroups;
 	double* acc;             // where the blocks add (upper triangle)
 	double* out;
 	unsigned* done;          // nullptr: no tail (acc is the caller's output)
 	unsigned long long* nnz;
 };
 
-__host__ __device__ constexpr int gt_m(int ncb) { return ncb == 1 ? 8 : ncb == 2 ? 3 : ncb <= 4 ? 2 : 1; } // 32 m rows per tile, m * ncb <= 8
-__host__ __device__ constexpr int gt_stride(int ncb) { return ncb * 16 + (ncb & 1 ? 0 : 16); } // doubles per row: rows 128 bytes apart in the banks
+// How the codes are dealt: one-byte codes, two-byte codes, two-byte codes of column pairs (every group two columns)
+constexpr int GT_BYTE = 1, GT_SHORT = 2, GT_PAIR = 3;
+// 32 m rows per tile (m * ncb <= 8 where a wave decodes one part; pairs: whole waves of rows as far as LDS goes)
+__host__ __device__ constexpr int gt_m(int ncb, int kind) { return ncb == 1 ? 8 : ncb == 2 ? (kind == GT_PAIR ? 4 : 3) : ncb <= 4 ? 2 : 1; }
+// doubles per row: rows 128 bytes apart in the banks; pairs, written by row with 16 bytes per lane: 144 bytes apart
+__host__ __device__ constexpr int gt_stride(int ncb, int kind) { return kind == GT_PAIR ? ncb * 16 + (ncb & 1 ? 2 : 18) : ncb * 16 + (ncb & 1 ? 0 : 16); }
 
 // Barrier of the workgroup that waits for this wave's LDS accesses only.
 __device__ __forceinline__ void lds_barrier() {
@@ -57,11 +66,12 @@ __device__ __forceinline__ void lds_barrier() {
 	asm volatile("" ::: "memory");
 }
 
-// NF full column blocks, then one of NN groups of 4 columns (NN = 0: none), W bytes per code
-template <int NF, int NN, int W>
+// NF full column blocks, then one of NN groups of 4 columns (NN = 0: none)
+template <int NF, int NN, int KIND>
 __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 	constexpr int NCB = NF + (NN ? 1 : 0), T = NF * (NF + 1) / 2;
-	constexpr int M = gt_m(NCB), R = 32 * M, S = gt_stride(NCB);
+	constexpr int W = KIND == GT_BYTE ? 1 : 2;
+	constexpr int M = gt_m(NCB, KIND), R = 32 * M, S = gt_stride(NCB, KIND);
 	constexpr bool SPLIT = NF > 5;              // two waves share the tiles of a set of rows
 	constexpr int NK = SPLIT ? 2 * M : M;       // steps of 4 rows per wave and tile
 	constexpr int BUF = R * S;
@@ -92,26 +102,73 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 #pragma unroll
 		for(int b = 0; b < NB; b++) nacc[i][b] = 0.0;
 
+	// pairs: a wave decodes units of 64 lanes, one tuple each: UR rows of 64 / UR neighbouring groups
+	constexpr bool PAIR = KIND == GT_PAIR;
+	constexpr int UR = R < 64 ? R : 64, UG = 64 / UR, RB = R / UR;  // rows and groups of a unit, units that share a group
+	constexpr int NU = PAIR ? (NCB * 8 / UG * RB + 7) / 8 : 1;       // most units of a wave
+	const int uRow = lane & (UR - 1);
+	const int nUnits = ((A.nGroups + UG - 1) / UG * RB - wave + 7) / 8; // this wave's
+
 	auto loop = [&](auto modeTag, auto halfTag) {
 		constexpr int MODE = decltype(modeTag)::value, HALF = decltype(halfTag)::value;
-		CodeVec<W, 8> codes;
+		constexpr int U = PAIR ? NU - MODE : 0; // units of the wave (no branch around a load: it would wait for the load)
+		auto unit_row = [&](int i) { return (wave + 8 * i) % RB * UR; };
+		uint32_t pcode[2][U > 0 ? U : 1];
+		f64x2 pv[2][U > 0 ? U : 1];
+		const uint8_t* pstream[U > 0 ? U : 1];
+		const char* pdict[U > 0 ? U : 1];
+		double* pput[U > 0 ? U : 1];
+		if constexpr(PAIR) {
+#pragma unroll
+			for(int i = 0; i < U; i++) {
+				const int g = min((wave + 8 * i) / RB * UG + (UG > 1 ? lane / UR : 0), A.nGroups - 1); // (an odd last group: twice)
+				pstream[i] = A.arena + (size_t) g * A.arenaStride;
+				pdict[i] = gDict + A.cols[2 * g].dictOff;
+				pput[i] = smem + (unit_row(i) + uRow) * S + 2 * g;
+			}
+		}
+		CodeVec<W, 8> codes[2];
 		double v[2][8];
-		auto load_codes = [&](int tile) {
+		auto load_codes = [&](int tile, auto parity) { // (codes and values of a tile sit in the sets of its parity)
+			constexpr int Q = decltype(parity)::value;
+			if constexpr(PAIR) {
+#pragma unroll
+				for(int i = 0; i < U; i++) {
+					const int64_t row = min((int64_t) min(tile, t1 - 1) * R + unit_row(i) + uRow, A.nRows - 1);
+					pcode[Q][i] = *(const uint16_t*) (pstream[i] + 2 * row);
+				}
+				return;
+			}
 			if(MODE == 0) return;
 			const int64_t row = min((int64_t) min(tile, t1 - 1) * R + sub * 32 + 8 * k, rowLast);
-			if constexpr(W == 1) codes.raw.v = *(const u32x2*) (stream + row);
-			else codes.raw.v = *(const u32x4*) (stream + 2 * row);
+			if constexpr(W == 1) codes[Q].raw.v = *(const u32x2*) (stream + row);
+			else codes[Q].raw.v = *(const u32x4*) (stream + 2 * row);
 		};
-		auto look = [&](double (&d)[8]) {
-			if(MODE == 0) return;
-#pragma unroll
-			for(int t = 0; t < 8; t++) {
-				const uint32_t code = (uint32_t) codes.get(t);
-				if(MODE == 1) d[t] = *(const double*) (ldsDict + (code << 7));
-				else d[t] = *(const double*) (gDict + (uint32_t) (__umul24(code, (uint32_t) C.stride) + (uint32_t) C.dictOff));
+		constexpr int NL = PAIR ? U : MODE == 0 ? 0 : 8; // lookups per lane and tile
+		auto look_one = [&](int i, auto parity) {
+			constexpr int Q = decltype(parity)::value;
+			if constexpr(PAIR) pv[Q][i] = *(const f64x2*) (pdict[i] + (pcode[Q][i] << 4));
+			else {
+				const uint32_t code = (uint32_t) codes[Q].get(i);
+				if(MODE == 1) v[Q][i] = *(const double*) (ldsDict + (code << 7));
+				else v[Q][i] = *(const double*) (gDict + (uint32_t) (__umul24(code, (uint32_t) C.stride) + (uint32_t) C.dictOff));
 			}
 		};
+		auto look = [&](auto parity) {
+#pragma unroll
+			for(int i = 0; i < NL; i++) look_one(i, parity);
+		};
 		auto write = [&](const double (&d)[8], int tile, int buf) {
+			if constexpr(PAIR) { // (tile t goes from value set to buffer of the same parity)
+#pragma unroll
+				for(int i = 0; i < U; i++) {
+					const bool in = (int64_t) tile * R + unit_row(i) + uRow < A.nRows; // zeros behind the last row of the matrix
+					f64x2 x = buf == 0 ? pv[0][i] : pv[1][i];
+					x.x = in ? x.x : 0.0; x.y = in ? x.y : 0.0;
+					*(f64x2*) (pput[i] + buf * BUF) = x;
+				}
+				return;
+			}
 			if(MODE == 0) return;
 			double* p = put + buf * BUF;
 			if((int64_t) (tile + 1) * R <= A.nRows) {
@@ -124,7 +181,21 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 				for(int t = 0; t < 8; t++) p[t * S] = row + t < A.nRows ? d[t] : 0.0;
 			}
 		};
-		auto multiply = [&](int buf) {
+		// Multiplies the tile in a buffer. Two-byte codes: the lookups of the next tile but one are spread between the matrix
+		// instructions, so that the two pipes work side by side (all in front of them, the gathers hold up every wave first:
+		// 10,000,000 x 50 as pairs 934 instead of 692 us; byte codes, half of whose lookups go to LDS: 441 instead of 465 us).
+		constexpr bool SPREAD = KIND != GT_BYTE;
+		auto multiply = [&](int buf, auto parity) {
+			constexpr int NM = NK * ((HALF == 0 ? T0 : T - T0) + NN * (SPLIT ? (NCB + 1 - HALF) / 2 : NCB)); // matrix instructions
+			int at = 0, done = 0;
+			auto between = [&]() {
+				at++;
+				if(SPREAD && done < NL && done * NM < at * NL) {
+					__builtin_amdgcn_sched_barrier(0);
+					look_one(done++, parity);
+					__builtin_amdgcn_sched_barrier(0);
+				}
+			};
 			const double* x0 = smem + buf * BUF + ((SPLIT ? wave & 3 : wave) * 4 + k) * S;
 			double x[2][NCB], a[2][NN ? NN : 1];
 			auto read = [&](int j) {
@@ -143,17 +214,25 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 				for(int p = 0; p < NF; p++)
 #pragma unroll
 					for(int q = p; q < NF; q++, t++)
-						if((t < T0) == (HALF == 0))
+						if((t < T0) == (HALF == 0)) {
 							acc[t - HALF * T0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[j & 1][p], x[j & 1][q], acc[t - HALF * T0], 0, 0, 0);
+							between();
+						}
 #pragma unroll
 				for(int i = 0; i < NN; i++)
 #pragma unroll
 					for(int b = 0; b < NCB; b++)
-						if(!SPLIT || (b & 1) == HALF)
+						if(!SPLIT || (b & 1) == HALF) {
 							nacc[i][SPLIT ? b / 2 : b] = __builtin_amdgcn_mfma_f64_4x4x4f64(a[j & 1][i], x[j & 1][b], nacc[i][SPLIT ? b / 2 : b], 0, 0, 0);
+							between();
+						}
 			}
+#pragma unroll
+			for(int i = 0; i < NL; i++)
+				if(SPREAD && i >= done) look_one(i, parity); // (more lookups than matrix instructions)
 		};
-		load_codes(t0);
+		using std::integral_constant;
+		load_codes(t0, integral_constant<int, 0>());
 		{
 			// the dictionaries of the first column blocks, 8 pieces of 16 bytes per thread requested together
 			const f64x2* src = (const f64x2*) A.img;
@@ -169,21 +248,20 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 			}
 		}
 		lds_barrier();
-		look(v[0]);
-		load_codes(t0 + 1);
-		look(v[1]);
-		load_codes(t0 + 2);
+		load_codes(t0 + 1, integral_constant<int, 1>());
+		look(integral_constant<int, 0>());
+		load_codes(t0 + 2, integral_constant<int, 0>());
+		look(integral_constant<int, 1>());
 		write(v[0], t0, 0);
 		lds_barrier();
 		auto step = [&](int tile, auto parity) {
 			constexpr int P = decltype(parity)::value;
-			look(v[P]);                    // of tile + 2
-			load_codes(tile + 3);
-			multiply(P);
+			if(!SPREAD) look(parity);      // of tile + 2
+			load_codes(tile + 3, integral_constant<int, P ^ 1>());
+			multiply(P, parity);
 			write(v[P ^ 1], min(tile + 1, t1 - 1), P ^ 1); // (behind the last tile: values nobody reads)
 			lds_barrier();
 		};
-		using std::integral_constant;
 		for(int tile = t0; tile < t1; tile += 2) {
 			step(tile, integral_constant<int, 0>());
 			if(tile + 1 < t1) step(tile + 1, integral_constant<int, 1>());
@@ -191,7 +269,16 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 	};
 	if(t0 < t1) {
 		using std::integral_constant;
-		if(SPLIT && wave >= 4) {
+		if constexpr(PAIR) {
+			auto units = [&](auto halfTag) {
+				if(nUnits >= NU) loop(integral_constant<int, 0>(), halfTag);
+				else if(nUnits == NU - 1) loop(integral_constant<int, 1>(), halfTag);
+				else loop(integral_constant<int, 2>(), halfTag);
+			};
+			if(SPLIT && wave >= 4) units(integral_constant<int, 1>());
+			else units(integral_constant<int, 0>());
+		}
+		else if(SPLIT && wave >= 4) {
 			if(mode == 0) loop(integral_constant<int, 0>(), integral_constant<int, 1>());
 			else if(mode == 1) loop(integral_constant<int, 1>(), integral_constant<int, 1>());
 			else loop(integral_constant<int, 2>(), integral_constant<int, 1>());
@@ -256,7 +343,7 @@ struct GtPlan {
 	GtArgs A;
 	void* dImg = nullptr;
 	int64_t bytes = 0;
-	int nf = 0, nn = 0, w = 0;
+	int nf = 0, nn = 0, kind = 0;
 	size_t lds = 0;
 };
 
@@ -274,7 +361,12 @@ static int gt_build_plan(cla_block* b, GtPlan& P) {
 	const int last = n - n / 16 * 16;
 	P.nn = last >= 1 && last <= 4 ? 1 : last >= 5 && last <= 8 ? 2 : 0;
 	P.nf = n / 16 + (last > 8 ? 1 : 0);
-	P.w = b->arenaWidth;
+	bool pairs = b->arenaWidth == 2 && n == 2 * (int) b->groups.size();
+	for(const HostGroup& H : b->groups) pairs &= H.d.nColG == 2;
+	// Column pairs whose dictionaries LDS cannot hold: a unit's lanes all look up one group, 16 bytes at a time. The lanes
+	// share the lines of the frequent tuples, and each lookup gives two columns: 62.9 M tuples of 24 dictionaries of 4096
+	// (Zipf) take 99 us of gathers like this, 170 us as 8 bytes per column with 8 groups per instruction.
+	P.kind = b->arenaWidth == 1 ? GT_BYTE : pairs ? GT_PAIR : GT_SHORT;
 	const int ncb = P.nf + (P.nn ? 1 : 0);
 	bool consts = false; // the dictionaries are copied with the constants added
 	for(int col = 0; col < n; col++) consts |= b->constV[col] != 0.0 || groupOf[col] < 0;
@@ -304,11 +396,11 @@ static int gt_build_plan(cla_block* b, GtPlan& P) {
 	const int real = n;
 	while((int) cols.size() < ncb * 16) { GtCol p = cols[real - 1]; p.col = -1; cols.push_back(p); src.push_back(src[real - 1]); }
 	// column blocks whose dictionaries fit LDS beside the tiles
-	const size_t tileBytes = (size_t) 2 * 32 * gt_m(ncb) * gt_stride(ncb) * 8;
+	const size_t tileBytes = (size_t) 2 * 32 * gt_m(ncb, P.kind) * gt_stride(ncb, P.kind) * 8;
 	const size_t sumBytes = ((size_t) P.nf * (P.nf + 1) / 2 * 256 + (size_t) P.nn * ncb * 64) * 8;
 	const size_t room = (size_t) g_ldsPerBlock - tileBytes;
 	const int imgV = std::max(b->maxVals, 1);
-	const int nLds = (int) std::min<size_t>(ncb, room / ((size_t) imgV * 128));
+	const int nLds = P.kind == GT_PAIR ? 0 : (int) std::min<size_t>(ncb, room / ((size_t) imgV * 128));
 	P.lds = std::max(tileBytes + (size_t) nLds * imgV * 128, sumBytes);
 	if(P.lds > (size_t) g_ldsPerBlock) return 0;
 	std::vector<double> img((size_t) nLds * imgV * 16, 0.0);
@@ -335,8 +427,8 @@ static int gt_build_plan(cla_block* b, GtPlan& P) {
 	A.img = (const double*) (d + colBytes);
 	A.dict = consts ? (const double*) (d + colBytes + imgBytes) : b->dAllDict;
 	A.nRows = b->nRows;
-	A.nTiles = (int) ((b->nRows + 32 * gt_m(ncb) - 1) / (32 * gt_m(ncb)));
-	A.nLds = nLds; A.imgV = imgV; A.nCols = n;
+	A.nTiles = (int) ((b->nRows + 32 * gt_m(ncb, P.kind) - 1) / (32 * gt_m(ncb, P.kind)));
+	A.nLds = nLds; A.imgV = imgV; A.nCols = n; A.nGroups = (int) b->groups.size();
 	P.rc = 0;
 	return 0;
 }
@@ -350,14 +442,9 @@ void gt_plan_drop(cla_block* b) {
 
 template <int NF, int NN>
 static int gt_launch(cla_block* b, const GtPlan& P, const GtArgs& A, unsigned grid) {
-	if(P.w == 1) {
-		CLA_HIP(allow_full_lds((const void*) k_gram_tiles<NF, NN, 1>));
-		hipLaunchKernelGGL((k_gram_tiles<NF, NN, 1>), dim3(grid), dim3(GT_THREADS), P.lds, b->stream, A);
-	}
-	else {
-		CLA_HIP(allow_full_lds((const void*) k_gram_tiles<NF, NN, 2>));
-		hipLaunchKernelGGL((k_gram_tiles<NF, NN, 2>), dim3(grid), dim3(GT_THREADS), P.lds, b->stream, A);
-	}
+	const auto kern = P.kind == GT_BYTE ? k_gram_tiles<NF, NN, GT_BYTE> : P.kind == GT_SHORT ? k_gram_tiles<NF, NN, GT_SHORT> : k_gram_tiles<NF, NN, GT_PAIR>;
+	CLA_HIP(allow_full_lds((const void*) kern));
+	hipLaunchKernelGGL(kern, dim3(grid), dim3(GT_THREADS), P.lds, b->stream, A);
 	CLA_HIP(hipGetLastError());
 	return 0;
 }

@@ -1,0 +1,89 @@
+"""t(X) %*% X of all-DDC blocks on k_gram_tiles: the edges of its tiles (rows and columns), its three ways of decoding,
+dictionaries beside the tiles and behind them, constants added to the columns."""
+import numpy as np
+import pytest
+
+from parity import assert_matches_truth
+
+pytestmark = pytest.mark.gpu
+
+
+def check(cla, ora, specs, n_rows, n_cols, what):
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, nnz = blk.tsmm()
+    names = {k["name"] for k in blk.stats()["kernels"]}
+    blk.close()
+    assert names == {"k_tsmm_decode"}, names
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    assert np.array_equal(out, out.T)
+    assert_matches_truth(out, D.T, D, what=what)
+    assert nnz == np.count_nonzero(out)
+
+
+def columns(synth, rng, n_rows, n_cols, n_vals, dtype, width):
+    order = rng.permutation(n_cols).astype(np.int32)
+    return [synth.GroupSpec("ddc", order[c:c + width], rng.standard_normal((n_vals, len(order[c:c + width]))),
+                            rng.integers(0, n_vals, n_rows).astype(dtype)) for c in range(0, n_cols, width)]
+
+
+@pytest.mark.parametrize("n_cols", [65, 68, 72, 73, 80, 81, 88, 96, 97, 100, 112, 113, 120, 127, 128])
+@pytest.mark.parametrize("n_rows", [1, 31, 33, 8191, 40009])
+def test_byte_codes(cla, ora, n_cols, n_rows):
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_cols + n_rows)
+    check(cla, ora, columns(synth, rng, n_rows, n_cols, 200, np.uint8, 1), n_rows, n_cols, f"{n_rows} x {n_cols}, bytes")
+
+
+@pytest.mark.parametrize("n_cols", [14, 16, 18, 20, 24, 26, 32, 34, 40, 42, 48, 50, 64, 66, 70, 74, 82, 90, 98, 106, 114, 128])
+@pytest.mark.parametrize("n_rows,n_vals", [(1, 300), (65, 4096), (16387, 2500)])
+def test_column_pairs(cla, ora, n_cols, n_rows, n_vals):
+    """Groups of two columns, two-byte codes: one group per instruction, whole tuples (every number of units that a wave can miss)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_cols + n_rows)
+    specs = columns(synth, rng, n_rows, n_cols, n_vals, np.uint16, 2)
+    if n_cols <= 64:  # narrow blocks of few groups come here when their codes exceed the direct kernel's tables
+        blk = cla.build_block(n_rows, n_cols, specs).set_option("tsmm_route", 2)
+        out, nnz = blk.tsmm()
+        blk.close()
+        D = ora.np_decompress(specs, n_rows, n_cols)
+        assert_matches_truth(out, D.T, D, what=f"{n_rows} x {n_cols}, pairs")
+        assert nnz == np.count_nonzero(out)
+        return
+    check(cla, ora, specs, n_rows, n_cols, f"{n_rows} x {n_cols}, pairs")
+
+
+@pytest.mark.parametrize("n_cols,width,n_vals", [(66, 1, 300), (99, 3, 1000), (101, 2, 4096), (128, 1, 260)])
+def test_two_byte_codes(cla, ora, n_cols, width, n_vals):
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_cols)
+    check(cla, ora, columns(synth, rng, 12345, n_cols, n_vals, np.uint16, width), 12345, n_cols, f"{n_cols} columns, width {width}")
+
+
+@pytest.mark.parametrize("dtype,width,n_vals", [(np.uint8, 1, 17), (np.uint16, 2, 700)])
+def test_constant_columns_and_offsets(cla, ora, dtype, width, n_vals):
+    """Columns that only carry a constant, and a constant added to decoded columns: the dictionaries are copied with it."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(5)
+    n_rows, n_cols = 9001, 70
+    specs = columns(synth, rng, n_rows, n_cols - 2, n_vals, dtype, width)
+    specs.append(synth.GroupSpec("const", np.array([n_cols - 2, n_cols - 1], np.int32), np.array([[2.5, -1.0]])))
+    specs.append(synth.GroupSpec("const", np.array([0, 7], np.int32), np.array([[1.5, 0.25]])))
+    check(cla, ora, specs, n_rows, n_cols, "constants")
+
+
+def test_infinities_and_nan_stay_in_their_cells(cla, ora):
+    from systemds_amd import synth
+    rng = np.random.default_rng(6)
+    n_rows, n_cols = 5003, 68
+    specs = columns(synth, rng, n_rows, n_cols, 300, np.uint16, 2)
+    specs[3].dict[5, 0] = np.inf
+    specs[9].dict[7, 1] = np.nan
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, _ = blk.tsmm()
+    blk.close()
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    with np.errstate(invalid="ignore"):
+        want = D.T @ D
+    ok = np.isfinite(want)
+    assert np.array_equal(np.isfinite(out), ok)
+    assert np.allclose(out[ok], want[ok], rtol=0, atol=1e-11 * n_rows)  # n_rows terms of size about 1, eps 1.1e-16
