@@ -115,7 +115,7 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *                   the decompressed rows times a wide B)
  *   rmm_direct      1 / 0: X %*% B on blocks of plain streams with codes read straight from global memory, 16 columns of B per pass
  *                   (0: at most 16 columns of B on the tile kernel on the matrix cores, wider B per row and group)
- *   lmm_disable     bit 0 dot form on byte codes, bit 1 byte-code bin kernel
+ *   lmm_disable     bit 0 dot forms on byte codes and (one row of Y) on two-byte codes, bit 1 byte-code bin kernel
  *   sdc_packed      1 / 0: packed SDCZeros lists for the mat-vecs
  *   sdc_lanes       1 / 0: SDCZeros mat-vecs on lane-major copies of the lists, one lane per group
  *   sdc_rows        1 / 0: SDCZeros X %*% v on row lists (the lists transposed), one lane per row
@@ -195,7 +195,7 @@ int64_t cla_block_nnz(cla_handle h);
 /* CLALibLeftMultBy.leftMultByMatrix (C/lib/CLALibLeftMultBy.java:126-145,
  * 286-346): out[nRowY x nCols] = Y %*% X, Y is nRowY x nRows.
  * The _dev_async form returns without waiting except where the block takes the one-pass kernel on the decoded rows
- * (option lmm_joint, blocks that are neither byte-code DDC nor mostly offset lists): that kernel reports a value
+ * (option lmm_joint, blocks that are neither byte-code DDC nor mostly offset lists, nor, for one row of Y, two-byte DDC of one or two columns per group): that kernel reports a value
  * of Y that is not finite, the host reads the flag (one wait for the block's stream per call) and such a Y takes
  * the bin kernels. The same holds for cla_mmchain_dev_async, whose second half is this product. */
 int64_t cla_lmm(cla_handle h, const double* Y, int32_t nRowY, double* out);

@@ -59,6 +59,13 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
 	return v;
 }
 
+// Barrier of the workgroup that waits for this wave's LDS accesses only.
+__device__ __forceinline__ void lds_barrier() {
+	asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+	__builtin_amdgcn_s_barrier();
+	asm volatile("" ::: "memory");
+}
+
 // Where a wave (or, part 0, a whole block) adds its share of a non-zero count.
 __device__ __forceinline__ unsigned long long* nnz_way(unsigned long long* counter, unsigned part) {
 	return counter + ((blockIdx.x + part) % NNZ_WAYS) * NNZ_STEP;

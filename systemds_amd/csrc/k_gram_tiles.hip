@@ -59,13 +59,6 @@ __host__ __device__ constexpr int gt_m(int ncb, int kind) { return ncb == 1 ? 8 
 // doubles per row: rows 128 bytes apart in the banks; pairs, written by row with 16 bytes per lane: 144 bytes apart
 __host__ __device__ constexpr int gt_stride(int ncb, int kind) { return kind == GT_PAIR ? ncb * 16 + (ncb & 1 ? 2 : 18) : ncb * 16 + (ncb & 1 ? 0 : 16); }
 
-// Barrier of the workgroup that waits for this wave's LDS accesses only.
-__device__ __forceinline__ void lds_barrier() {
-	asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-	__builtin_amdgcn_s_barrier();
-	asm volatile("" ::: "memory");
-}
-
 // NF full column blocks, then one of NN groups of 4 columns (NN = 0: none)
 template <int NF, int NN, int KIND>
 __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {

@@ -335,6 +335,7 @@ int launch_lmm(cla_block* b, const double* dY, int p, double* dOut, unsigned lon
 	int dot = 1;
 	if(p == 1 && nRows > 1500000) dot = launch_lmm_u8_vec(b, dY, dOut);
 	if(dot == 1 && nRows > 0) dot = launch_lmm_u8_dot(b, dY, p, dOut);
+	if(dot == 1 && nRows > 0 && p == 1) dot = launch_lmm_q1_short(b, dY, dOut);
 	if(dot < 0) return dot;
 	if(dot != 0 && nRows > 0 && b->lmmTailWanted && b->opt.sdcLanes && !b->dictNonFinite && b->hasSdc && !b->hasUnc && !b->hasRle) {
 		bool onlyLists = true;

@@ -621,6 +621,10 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 		if(fused) b->nnzRot = b->nnzRot % 3 + 1;
 		return 0;
 	}
+	if(q == 1) {
+		const int r = launch_rmm_q1_short(b, tables, constRow, dOut, dNnz);
+		if(r <= 0) return r;
+	}
 	if(q == 1 && b->dArena && b->q1LdsBytes > 0) {
 		const int cw = b->arenaWidth;
 		const int threads = b->q1Threads, rpt = cw == 4 ? 8 : 16;
@@ -643,9 +647,8 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 		else if(threads == 1024) LAUNCH_Q1(CWV, RPTV, 1024);                     \
 		else LAUNCH_Q1(CWV, RPTV, 256);                                          \
 	} while(0)
-		if(cw == 1) { if(rpt == 8) LAUNCH_Q1_T(1, 8); else LAUNCH_Q1_T(1, 16); }
-		else if(cw == 2) { if(rpt == 8) LAUNCH_Q1_T(2, 8); else LAUNCH_Q1_T(2, 16); }
-		else { if(rpt == 8) LAUNCH_Q1_T(4, 8); else LAUNCH_Q1_T(4, 16); }
+		if(cw == 1) LAUNCH_Q1_T(1, 16); // (two-byte codes: k_rmm_q1_short)
+		else LAUNCH_Q1_T(4, 8);
 #undef LAUNCH_Q1_T
 #undef LAUNCH_Q1
 		CLA_HIP(hipGetLastError());
