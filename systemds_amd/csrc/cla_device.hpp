@@ -66,6 +66,9 @@ __device__ __forceinline__ void lds_barrier() {
 	asm volatile("" ::: "memory");
 }
 
+// (rounded like the kernel of its own that follows where the product does not do it)
+__device__ __forceinline__ double row_op(double sum, double w, int minus) { return minus ? sum - w : __dmul_rn(sum, w); }
+
 // Where a wave (or, part 0, a whole block) adds its share of a non-zero count.
 __device__ __forceinline__ unsigned long long* nnz_way(unsigned long long* counter, unsigned part) {
 	return counter + ((blockIdx.x + part) % NNZ_WAYS) * NNZ_STEP;

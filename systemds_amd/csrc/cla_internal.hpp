@@ -100,6 +100,11 @@ struct KernelStat {
 	float ms = -1.f;
 };
 
+// What the multiply chain does to the sum of a row on its way out: nothing (w == nullptr), times w or minus w.
+struct RowOp {
+	const double* w = nullptr;
+	int minus = 0;
+};
 struct DecPlanCache;
 struct DirPlan;
 struct GdrPlan;
@@ -170,6 +175,10 @@ struct cla_block {
 	double* dStageOut = nullptr; size_t stageOutCap = 0;
 	void* dScratch = nullptr;   size_t scratchCap = 0;
 	double* dChain = nullptr;   size_t chainCap = 0;   // X %*% v inside the multiply chain
+	// While the chain's right multiply is queued: what happens to each of its sums (RowOp). A kernel that does it on the way
+	// out sets chainOpDone; else a kernel of its own follows.
+	cla::RowOp chainOp;
+	bool chainOpDone = false;
 	// exact code counts of all dictionary-coded groups (totalVals int32, group g at tblOff[g]),
 	// computed on the first TSMM and kept, like the reference's cached counts
 	// (CG/AColGroupValue.java getCounts)

@@ -248,11 +248,12 @@ __device__ __forceinline__ void u8_consume(const CodeVec<1, RPT> (&cv)[NB], cons
 // entries are bit-identical to the pre-aggregation kernel's). `Tpad` is then the padded dictionary
 // image (256 entries per group, zero beyond nVals), `col0` the groups' columns. Block 0 clears
 // *nnzNext, the counter of the next call, so that no clearing step runs between two calls.
-template <int THREADS, int U8_PER, int U8_NB, int LB, int LN, bool FUSED>
+// OP: a row's sum goes out times the row's weight or minus it (RowOp).
+template <int THREADS, int U8_PER, int U8_NB, int LB, int LN, bool FUSED, bool OP>
 __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restrict__ arena, size_t arenaStride,
 	int nGroups, const double* __restrict__ Tpad, const double* __restrict__ constTerm,
 	double* __restrict__ out, int64_t nRows, unsigned long long* __restrict__ nnz,
-	const int32_t* __restrict__ col0, const double* __restrict__ v, unsigned long long* __restrict__ nnzNext) {
+	const int32_t* __restrict__ col0, const double* __restrict__ v, unsigned long long* __restrict__ nnzNext, const RowOp op) {
 	__shared__ double tbl[U8_PER * 256];
 	__shared__ double wbufAll[(THREADS / 64) * 64 * 8]; // per-wave transpose buffers of the epilogue
 	const char* tb = (const char*) tbl;
@@ -378,6 +379,12 @@ __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restr
 			double* obase = out + passBeg + (int64_t) wave * 64 * RPT;
 #pragma unroll
 			for(int h = 0; h < 2; h++) {
+				double wv[OP ? 8 : 1];
+				if constexpr(OP) {
+					const double* wbase = op.w + passBeg + (int64_t) wave * 64 * RPT;
+#pragma unroll
+					for(int j = 0; j < 8; j++) wv[j] = __builtin_nontemporal_load(wbase + ((j * 64 + lane) >> 3) * RPT + h * 8 + (lane & 7));
+				}
 #pragma unroll
 				for(int i = 0; i < 8; i++) {
 					const double v = acc[h * 8 + i] + cadd;
@@ -390,7 +397,9 @@ __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restr
 #pragma unroll
 				for(int j = 0; j < 8; j++) {
 					const int t = j * 64 + lane, sl = t >> 3, i = t & 7;
-					__builtin_nontemporal_store(wbuf[sl * 8 + (i ^ ((sl >> 2) & 7))], obase + sl * RPT + h * 8 + i);
+					double res = wbuf[sl * 8 + (i ^ ((sl >> 2) & 7))];
+					if constexpr(OP) res = row_op(res, wv[j], op.minus);
+					__builtin_nontemporal_store(res, obase + sl * RPT + h * 8 + i);
 				}
 				__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 				__builtin_amdgcn_wave_barrier();
@@ -401,7 +410,8 @@ __global__ __launch_bounds__(THREADS, 4) void k_rmm_q1_u8(const uint8_t* __restr
 #pragma unroll
 			for(int i = 0; i < RPT; i++)
 				if(off + i < passLen) {
-					const double v = acc[i] + cadd;
+					double v = acc[i] + cadd;
+					if constexpr(OP) v = row_op(v, op.w[passBeg + off + i], op.minus);
 					cnt += v != 0.0;
 					out[passBeg + off + i] = v;
 				}
@@ -611,12 +621,17 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 		const double* constTerm = constRow >= 0 ? tables + constRow : nullptr;
 		unsigned long long* nnzNext = fused ? b->nnz_counter(b->nnzRot % 3 + 1) : nullptr;
 		Prof pf(b, "k_rmm_q1_u8", grid, THREADS, per * 256 * 8, bytes);
+		const RowOp op = b->chainOp;
+#define U8_LAUNCH_OP(PER, NBV, LB, LN, F, O)                                                                    \
+	hipLaunchKernelGGL((k_rmm_q1_u8<THREADS, PER, NBV, LB, LN, F, O>), dim3(grid), dim3(THREADS), 0, st, b->dArena, \
+		b->arenaStride, nG, F ? b->dDictPad : dTpad, constTerm, dOut, nRows, dNnz, dCol0, dB, nnzNext, op)
 #define U8_LAUNCH(PER, NBV, LB, LN, F)                                                                          \
-	hipLaunchKernelGGL((k_rmm_q1_u8<THREADS, PER, NBV, LB, LN, F>), dim3(grid), dim3(THREADS), 0, st, b->dArena, \
-		b->arenaStride, nG, F ? b->dDictPad : dTpad, constTerm, dOut, nRows, dNnz, dCol0, dB, nnzNext)
+	do { if(op.w != nullptr) U8_LAUNCH_OP(PER, NBV, LB, LN, F, true); else U8_LAUNCH_OP(PER, NBV, LB, LN, F, false); } while(0)
 		if(per == 20) { if(fused) U8_LAUNCH(20, 5, 4, 2, true); else U8_LAUNCH(20, 5, 4, 2, false); }
 		else { if(fused) U8_LAUNCH(16, 4, 8, 2, true); else U8_LAUNCH(16, 4, 8, 2, false); }
 #undef U8_LAUNCH
+#undef U8_LAUNCH_OP
+		b->chainOpDone = op.w != nullptr;
 		CLA_HIP(hipGetLastError());
 		if(fused) b->nnzRot = b->nnzRot % 3 + 1;
 		return 0;

@@ -145,12 +145,13 @@ __global__ __launch_bounds__(RB_THREADS) void k_rows_build(const DGroup* __restr
 // FUSE (blocks of single-column lists only, nothing to add): the kernel makes the tables itself, T being the block's
 // dictionaries and u the vector: table value = dictionary value * u[column]; block 0 clears *nnzNext, the counter of
 // the next call, so that no other kernel runs in a call.
-template <bool ACC, bool FUSE>
+// OP: a row's sum goes out times the row's weight or minus it (RowOp); the weights are requested a quarter ahead.
+template <bool ACC, bool FUSE, bool OP>
 __global__ __launch_bounds__(RW_THREADS) void k_rmm_sdc_rows(const int32_t* __restrict__ tblIndex, int nTbl,
 	const uint2* __restrict__ hdr, const uint32_t* __restrict__ perm, const uint32_t* __restrict__ data,
 	const double* __restrict__ T, int constRow, double* __restrict__ out, int64_t nRows, int nQuarters,
 	unsigned long long* __restrict__ nnz, const int32_t* __restrict__ tblCol, const double* __restrict__ u,
-	unsigned long long* __restrict__ nnzNext) {
+	unsigned long long* __restrict__ nnzNext, const RowOp op) {
 	extern __shared__ double smemD[];
 	double* tbl = smemD;                 // nTbl values and a 0.0
 	const int tid = threadIdx.x, lane = tid & 63;
@@ -187,6 +188,7 @@ __global__ __launch_bounds__(RW_THREADS) void k_rmm_sdc_rows(const int32_t* __re
 		uint2 h;
 		uint32_t p;
 		double start[RW_F];
+		double w[OP ? RW_F : 1];
 	};
 	// (a vector load although the address is uniform: a scalar load is counted with the LDS reads, whose waits would
 	// then wait for it too)
@@ -203,6 +205,7 @@ __global__ __launch_bounds__(RW_THREADS) void k_rmm_sdc_rows(const int32_t* __re
 #pragma unroll
 		for(int j = 0; j < RW_F; j++) {
 			A.start[j] = init;
+			if(OP) A.w[j] = __builtin_nontemporal_load(op.w + min((int64_t) qt * RW_Q + j * 64 + lane, nRows - 1));
 			if(ACC) A.start[j] = out[min((int64_t) qt * RW_Q + j * 64 + lane, nRows - 1)]; // (a template parameter: a load under a run-time branch is waited for at the branch's end)
 		}
 	};
@@ -251,7 +254,8 @@ __global__ __launch_bounds__(RW_THREADS) void k_rmm_sdc_rows(const int32_t* __re
 #pragma unroll
 		for(int j = 0; j < RW_F; j++) {
 			const int64_t r = (int64_t) qt * RW_Q + j * 64 + lane;
-			const double res = A.start[j] + back[j * 64 + lane];
+			double res = A.start[j] + back[j * 64 + lane];
+			if(OP) res = row_op(res, A.w[j], op.minus);
 			if(r < nRows) {
 				cntNz += res != 0.0;
 				__builtin_nontemporal_store(res, &out[r]);
@@ -377,15 +381,19 @@ int launch_rmm_sdc_rows(cla_block* b, int constRow, int accumulate, double* dOut
 	double algo = (double) b->nRows * 8 * (accumulate ? 2 : 1);
 	for(int g : b->sdcList) algo += (double) b->groups[g].d.nDeltas * b->groups[g].d.deltaWidth + (double) b->groups[g].d.nOffsets * b->groups[g].d.codeWidth;
 	Prof pf(b, "k_rmm_sdc_rows", (long) grid, RW_THREADS, (long) lds, algo);
+	const RowOp op = b->chainOp; // (the lists come last: with what other groups have written a row's sum is complete)
 	auto go = [&](auto kernel) {
 		CLA_HIP(allow_full_lds((const void*) kernel));
 		hipLaunchKernelGGL(kernel, dim3(grid), dim3(RW_THREADS), lds, b->stream, (const int32_t*) meta, b->rowsTbl,
 			(const uint2*) (meta + b->rowsOff[0]), (const uint32_t*) (meta + b->rowsOff[1]), (const uint32_t*) b->dRowsData,
 			dU ? (const double*) b->dAllDict : (const double*) b->dTables, constRow, dOut, b->nRows, nQuarters, dNnz,
-			(const int32_t*) (meta + b->rowsColOff), dU, nnzNext);
+			(const int32_t*) (meta + b->rowsColOff), dU, nnzNext, op);
 		return 0;
 	};
-	if((rc = dU ? go(k_rmm_sdc_rows<false, true>) : accumulate ? go(k_rmm_sdc_rows<true, false>) : go(k_rmm_sdc_rows<false, false>))) return rc;
+	if(op.w != nullptr) rc = dU ? go(k_rmm_sdc_rows<false, true, true>) : accumulate ? go(k_rmm_sdc_rows<true, false, true>) : go(k_rmm_sdc_rows<false, false, true>);
+	else rc = dU ? go(k_rmm_sdc_rows<false, true, false>) : accumulate ? go(k_rmm_sdc_rows<true, false, false>) : go(k_rmm_sdc_rows<false, false, false>);
+	if(rc) return rc;
+	b->chainOpDone = op.w != nullptr;
 	CLA_HIP(hipGetLastError());
 	return 0;
 }

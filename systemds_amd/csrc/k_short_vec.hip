@@ -30,7 +30,7 @@ typedef double f64x2_sv __attribute__((ext_vector_type(2), aligned(8)));
 template <int NU>
 __global__ __launch_bounds__(SV_THREADS) void k_rmm_q1_short(const uint8_t* __restrict__ arena, size_t arenaStride, int nGroups, int gs,
 	const int32_t* __restrict__ tblOff, const double* __restrict__ T, int constIdx, double* __restrict__ out, int64_t nRows,
-	unsigned long long* __restrict__ nnz) {
+	unsigned long long* __restrict__ nnz, const RowOp op) {
 	extern __shared__ double tbl[]; // two buffers
 	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int64_t n4 = (nRows + 3) / 4;
@@ -102,6 +102,10 @@ __global__ __launch_bounds__(SV_THREADS) void k_rmm_q1_short(const uint8_t* __re
 #pragma unroll
 			for(int i = 0; i < 4; i++) acc[j][i] += cadd;
 		}
+		if(op.w != nullptr) {
+#pragma unroll
+			for(int i = 0; i < 4; i++) acc[j][i] = row_op(acc[j][i], op.w[min(row + i, nRows - 1)], op.minus);
+		}
 		if(row + 4 <= nRows) {
 #pragma unroll
 			for(int i = 0; i < 4; i += 2) {
@@ -125,7 +129,7 @@ __global__ __launch_bounds__(SV_THREADS) void k_rmm_q1_short(const uint8_t* __re
 constexpr int SV_NB = 13;
 __global__ __launch_bounds__(256) void k_rmm_q1_short_rows(const uint8_t* __restrict__ arena, size_t arenaStride, int nGroups,
 	const int32_t* __restrict__ tblOff, const double* __restrict__ T, int constIdx, double* __restrict__ out, int64_t nRows,
-	unsigned long long* __restrict__ nnz) {
+	unsigned long long* __restrict__ nnz, const RowOp op) {
 	const int64_t row = (int64_t) blockIdx.x * 256 + threadIdx.x;
 	const uint8_t* at = arena + 2 * min(row, nRows - 1);
 	double acc = 0.0;
@@ -141,6 +145,7 @@ __global__ __launch_bounds__(256) void k_rmm_q1_short_rows(const uint8_t* __rest
 			if(g0 + j < nGroups) acc += v[j];
 	}
 	if(constIdx >= 0) acc += T[constIdx];
+	if(op.w != nullptr) acc = row_op(acc, op.w[min(row, nRows - 1)], op.minus);
 	if(row < nRows) out[row] = acc;
 	count_add(nnz, row < nRows && acc != 0.0);
 }
@@ -150,13 +155,14 @@ __global__ __launch_bounds__(256) void k_rmm_q1_short_rows(const uint8_t* __rest
 int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double* dOut, unsigned long long* dNnz) {
 	const int nG = (int) b->groups.size();
 	if(b->dArena == nullptr || b->arenaWidth != 2 || nG == 0 || b->nRows == 0 || b->maxVals > SV_BUF) return 1;
+	b->chainOpDone = b->chainOp.w != nullptr;
 	// Up to 400,000 rows (where both take 29 us at 25 groups, 15 at 10) straight from global memory: 20,000 x 50 11 against 27 us,
 	// 200,000 x 50 18 against 28; beyond, the form with the tables in LDS: 700,000 x 50 31 against 43, 1,500,000 x 6 14 against 26.
 	if(b->nRows <= 400000) {
 		const unsigned grid = (unsigned) ((b->nRows + 255) / 256);
 		Prof pf(b, "k_rmm_q1_ddc", grid, 256, 0, (double) b->nRows * (2 * nG + 8) + (double) b->totalVals * 8);
 		hipLaunchKernelGGL(k_rmm_q1_short_rows, dim3(grid), dim3(256), 0, b->stream, b->dArena, b->arenaStride, nG, b->dTblOff, tables,
-			constIdx, dOut, b->nRows, dNnz);
+			constIdx, dOut, b->nRows, dNnz, b->chainOp);
 		CLA_HIP(hipGetLastError());
 		return 0;
 	}
@@ -173,7 +179,7 @@ int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double
 	do {                                                                                                                     \
 		CLA_HIP(allow_full_lds((const void*) k_rmm_q1_short<NU>));                                                           \
 		hipLaunchKernelGGL(k_rmm_q1_short<NU>, dim3(grid), dim3(SV_THREADS), lds, b->stream, b->dArena, b->arenaStride, nG, gs, \
-			b->dTblOff, tables, constIdx, dOut, b->nRows, dNnz);                                                             \
+			b->dTblOff, tables, constIdx, dOut, b->nRows, dNnz, b->chainOp);                                                             \
 	} while(0)
 	if(nu <= 1) SV_LAUNCH(1);
 	else if(nu == 2) SV_LAUNCH(2);
