@@ -1542,8 +1542,7 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 		CLA_HIP(hipStreamSynchronize(st));
 		if(bad) { clear_stats(b); return 1; }
 	}
-	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
-	{
+	{ // (the counter is still zero: the kernel writes nothing but that flag into it)
 		Prof pf(b, "k_take_block", ((int) n + 255) / 256, 256, 0, 0);
 		hipLaunchKernelGGL(k_take_block, dim3((unsigned) std::min(((int) n + 255) / 256, 1024)), dim3(256), 0, st, b->dStageOut, b->nCols, 0, 0, p,
 			b->nCols, dOut, dNnz);

@@ -1,0 +1,77 @@
+// Blocks of a few "varying" columns (one value per row behind a plain stream) next to run-length columns: the plan that the
+// kernels on decoded rows with lane = row share (k_gram_direct.hip, k_lmm_direct.hip).
+#pragma once
+#include "cla_runs.hpp"
+
+namespace cla {
+
+struct GdrCol {            // 24 bytes
+	int32_t ringOff;       // bytes from the start of a ring buffer: the column's code / value of the chunk's first row
+	int32_t base8;         // bytes from the LDS base: the column's values by tuple
+	int32_t stride;        // bytes per row of the stream in the ring
+	int32_t col;           // column of the matrix
+	int32_t pad[2];
+};
+struct GdrStream {         // what the ring holds per chunk: bpr * GDR_CH consecutive bytes of each stream
+	const uint8_t* src;
+	int32_t bpr;           // bytes per row
+	int32_t piece0;        // first 16-byte piece of the stream in a ring buffer
+};
+struct GdrArgs {
+	const GdrCol* cols;
+	const double* vals;    // values of the code columns by tuple, constants added: the head of LDS as it is
+	const RunCol* runs;
+	const GdrStream* streams;
+	int nV, n2, n12, nR, nStreams; // columns [0, n2) two-byte codes, [n2, n12) one-byte codes, [n12, nV) dense
+	int packed;            // every code column has a stream of its own and the dense columns are one uncompressed group: the ring is columns in order
+	int valDoubles;        // even
+	int ringBytes;         // one ring buffer
+	int64_t nRows;
+	double* out;
+	int nCols;
+	double* acc;               // the call's only kernel: the blocks add here and the last one writes out (gram_tail)
+	unsigned* done;            // its ticket counter (nullptr: the blocks add into out, the caller fills and finishes)
+	unsigned long long* nnz;
+};
+
+// A varying column as the left multiply reads it: straight from its stream.
+struct LdCol {
+	const uint8_t* src;    // its code (or value) of row 0
+	int32_t stride;        // bytes per row; 0: a filler
+	int32_t base8;         // bytes from the LDS base: values by tuple
+	uint32_t mask;         // of a code; 0: a filler, which looks a zero up
+	int32_t col;           // column of the matrix, -1: a filler
+};
+
+struct LdCols { LdCol c[12]; };
+
+struct GdrPlan {
+	int rc = 1;            // 0 usable, 1 the block does not qualify
+	void* dImg = nullptr;
+	int64_t bytes = 0;
+	size_t lds = 0;
+	GdrArgs A;
+	LdCols ld;             // ldNC code columns (fillers behind the real ones), ldND dense ones; ldNC == 0: no such form
+	int ldNC = 0, ldND = 0;
+};
+
+// A block's copy of the values into LDS: 16-byte pieces, several requested together (one dictionary after the other, each a
+// round trip to memory, took 15 us of a call).
+template <int THREADS>
+__device__ __forceinline__ void gdr_copy_vals(double* smem, const double* __restrict__ vals, int valDoubles) {
+	const f64x2* src = (const f64x2*) vals;
+	const int n = valDoubles / 2;
+	for(int i0 = threadIdx.x; i0 < n; i0 += 8 * THREADS) {
+		f64x2 d[8];
+#pragma unroll
+		for(int j = 0; j < 8; j++) d[j] = src[min(i0 + j * THREADS, n - 1)];
+#pragma unroll
+		for(int j = 0; j < 8; j++)
+			if(i0 + j * THREADS < n) ((f64x2*) smem)[i0 + j * THREADS] = d[j];
+	}
+}
+
+// The block's plan, built on first use; P.rc says whether it qualifies. Negative: an error.
+int gdr_plan(cla_block* b, const GdrPlan*& P);
+
+} // namespace cla

@@ -289,6 +289,7 @@ int launch_tsmm_decode(cla_block* b, double* dOut, unsigned long long* dNnz = nu
 int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double* dOut, unsigned long long* dNnz);
 int lmm_q1_short_groups(const cla_block* b);
 int launch_lmm_q1_short(cla_block* b, const double* dY, double* dOut);
+int launch_lmm_direct(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dBad);
 int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);
 void gt_plan_drop(cla_block* b);
 int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);

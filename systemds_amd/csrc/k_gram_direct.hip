@@ -23,7 +23,7 @@
 // that bypass the registers (two chunks in flight while one is read): a wave is alone on its SIMD (the sums
 // take most of the register file), so nothing else would hide the memory latency.
 #include "../../include/cla_hip.h"
-#include "cla_runs.hpp"
+#include "cla_gdr.hpp"
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -40,48 +40,6 @@ constexpr int GDR_CH = 128;                  // rows per chunk of the wave's str
 constexpr int GDR_NBUF = 4;                  // ring buffers per wave: one being read, three in flight
 constexpr int GDR_REBASE = 128;             // chunks between two rebases of the run-length columns' running sums (a power of two)
 constexpr int GDR_NI = 8;                    // at most this many 1 KB pieces per chunk and wave (8 KB per ring buffer)
-
-struct GdrCol {            // 24 bytes
-	int32_t ringOff;       // bytes from the start of a ring buffer: the column's code / value of the chunk's first row
-	int32_t base8;         // bytes from the LDS base: the column's values by tuple
-	int32_t stride;        // bytes per row of the stream in the ring
-	int32_t col;           // column of the matrix
-	int32_t pad[2];
-};
-struct GdrStream {         // what the ring holds per chunk: bpr * GDR_CH consecutive bytes of each stream
-	const uint8_t* src;
-	int32_t bpr;           // bytes per row
-	int32_t piece0;        // first 16-byte piece of the stream in a ring buffer
-};
-struct GdrDict {           // values of one varying column by tuple: add + src[t * nC + h] for t < n, add up to fill
-	const double* src;
-	double add;
-	int32_t n, nC, h, off, fill, pad;
-};
-struct GdrArgs {
-	const GdrCol* cols;
-	const GdrDict* dicts;
-	const RunCol* runs;
-	const GdrStream* streams;
-	int nDicts, nV, n2, n12, nR, nStreams; // columns [0, n2) two-byte codes, [n2, n12) one-byte codes, [n12, nV) dense
-	int packed;            // every code column has a stream of its own and the dense columns are one uncompressed group: the ring is columns in order
-	int valDoubles;        // values by tuple
-	int ringBytes;         // one ring buffer
-	int64_t nRows;
-	double* out;
-	int nCols;
-	double* acc;               // the call's only kernel: the blocks add here and the last one writes out (gram_tail)
-	unsigned* done;            // its ticket counter (nullptr: the blocks add into out, the caller fills and finishes)
-	unsigned long long* nnz;
-};
-
-struct GdrPlan {
-	int rc = 1;            // 0 usable, 1 the block does not qualify
-	void* dImg = nullptr;
-	int64_t bytes = 0;
-	size_t lds = 0;
-	GdrArgs A;
-};
 
 // One piece of up to 1 KB global -> LDS without registers: lane l fetches 16 bytes from its own address, they land at
 // the (wave-uniform) LDS address + 16 l. Written as assembly on purpose: the compiler then does not know of the LDS
@@ -134,12 +92,7 @@ __global__ __launch_bounds__(GDR_THREADS) void k_tsmm_direct(const GdrArgs A) {
 	const uint32_t ringBytes = (uint32_t) A.ringBytes;
 	const uint32_t ring0 = (uint32_t) ((A.valDoubles + GDR_NP * GDR_NP + GDR_WAVES * GDR_WDOUBLES) * 8) + (uint32_t) wave * GDR_NBUF * ringBytes;
 
-	for(int d = 0; d < A.nDicts; d++) {
-		const GdrDict D = A.dicts[d];
-		const double* __restrict__ src = as_global(D.src);
-#pragma unroll 8
-		for(int t = tid; t < D.fill; t += GDR_THREADS) smem[D.off + t] = D.add + (t < D.n ? src[(size_t) t * D.nC + D.h] : 0.0);
-	}
+	gdr_copy_vals<GDR_THREADS>(smem, A.vals, A.valDoubles);
 	for(int i = tid; i < GDR_NP * GDR_NP; i += GDR_THREADS) gramS[i] = 0.0;
 	__syncthreads();
 
@@ -539,10 +492,9 @@ static int gdr_build_plan(cla_block* b, GdrPlan& P) {
 	if(b->nRows <= 0 || b->nRows >= ((int64_t) 1 << 31) - 2 * GDR_CH || b->nCols > 64) return 0;
 	struct Src { const uint8_t* src; int bpr; std::vector<GdrCol> cols; };
 	std::vector<Src> srcs[3]; // streams by class: two-byte codes, one-byte codes, dense rows
-	std::vector<GdrDict> dicts;
+	std::vector<double> vals; // by tuple: the column's constant plus the dictionary's value
 	std::vector<RunCol> runs;
 	std::vector<char> seen((size_t) b->nCols, 0);
-	size_t valD = 0;
 	int covered = 0;
 	for(int g = 0; g < nG; g++) {
 		const DGroup& G = b->groups[g].d;
@@ -586,9 +538,8 @@ static int gdr_build_plan(cla_block* b, GdrPlan& P) {
 		if(((uintptr_t) src & 15) != 0) return 0;
 		Src S{src, cls == 0 ? 2 : 1, {}};
 		for(int h = 0; h < G.nColG; h++) {
-			dicts.push_back(GdrDict{G.dict, b->constV[hc[h]], G.nVals, G.nColG, h, (int32_t) valD, fill, 0});
-			S.cols.push_back(GdrCol{0, (int32_t) (8 * valD), S.bpr, hc[h], {0, 0}});
-			valD += (size_t) fill;
+			S.cols.push_back(GdrCol{0, (int32_t) (8 * vals.size()), S.bpr, hc[h], {0, 0}});
+			for(int t = 0; t < fill; t++) vals.push_back(b->constV[hc[h]] + (t < G.nVals ? b->groups[g].dict[(size_t) t * G.nColG + h] : 0.0));
 		}
 		srcs[cls].push_back(S);
 		covered += G.nColG;
@@ -621,9 +572,8 @@ static int gdr_build_plan(cla_block* b, GdrPlan& P) {
 	const int nR = (int) runs.size();
 	// the kernel without compile-time code widths exists for even numbers of code columns: a filler column reads
 	// the ring's first two bytes, masks them away and looks a zero up
-	const size_t zeroAt = valD;
-	valD += 2;
-	dicts.push_back(GdrDict{nullptr, 0.0, 0, 1, 0, (int32_t) zeroAt, 2, 0}); // two zeros
+	const size_t zeroAt = vals.size();
+	vals.resize((vals.size() + 3) & ~(size_t) 1, 0.0); // two zeros and an even number
 	int nFill = 0;
 	if(nCode >= 1 && (nCode & 1)) {
 		all.insert(all.begin() + nCode, GdrCol{0, (int32_t) (8 * zeroAt), 2, -1, {0, 0}});
@@ -631,14 +581,32 @@ static int gdr_build_plan(cla_block* b, GdrPlan& P) {
 	}
 	const int nV = (int) all.size();
 	if(nCode < 1 || nV > GDR_VMAX || nR > RC_MAX || pieces > GDR_NI * 64) return 0;
-	valD = (valD + 1) & ~(size_t) 1;
+	const size_t valD = vals.size();
 	const int ringBytes = pieces * 16;
 	P.lds = (valD + GDR_NP * GDR_NP + (size_t) GDR_WAVES * GDR_WDOUBLES) * 8 + (size_t) GDR_WAVES * GDR_NBUF * ringBytes;
 	if(P.lds > (size_t) std::min(g_ldsPerBlock, 160 * 1024) - 1024) return 0;
-	const size_t colBytes = all.size() * sizeof(GdrCol), dictBytes = dicts.size() * sizeof(GdrDict), runBytes = runs.size() * sizeof(RunCol);
+	const size_t colBytes = all.size() * sizeof(GdrCol), dictBytes = valD * sizeof(double), runBytes = runs.size() * sizeof(RunCol);
 	const size_t streamBytes = streams.size() * sizeof(GdrStream);
-	std::vector<uint8_t> img(dictBytes + runBytes + streamBytes + colBytes + 16, 0); // (structs with pointers first: 8-byte aligned)
-	if(dictBytes) std::memcpy(img.data(), dicts.data(), dictBytes);
+	// the same columns as the left multiply wants them: straight from their streams, filled up to a shape it exists for
+	std::vector<LdCol> ld;
+	{
+		const int nD = nV - nCode - nFill;
+		P.ldND = nD == 0 ? 0 : nD <= 2 ? 2 : 4;
+		P.ldNC = nCode <= 4 ? 4 : nCode <= 8 ? 8 : nCode <= 10 && P.ldND == 2 ? 10 : 12;
+		if(nD <= 4 && P.ldNC + P.ldND <= GDR_VMAX) {
+			for(int k = 0; k < 3; k++) {
+				for(const Src& S : srcs[k])
+					for(const GdrCol& C : S.cols) // (dense: ringOff is the column's place in the row)
+						ld.push_back(LdCol{S.src + (k == 2 ? C.ringOff : 0), k == 2 ? C.stride : S.bpr, C.base8, k == 0 ? 0xffffu : 0xffu, C.col});
+				if(k == 1)
+					while((int) ld.size() < P.ldNC) ld.push_back(LdCol{ld[0].src, ld[0].stride, (int32_t) (8 * zeroAt), 0u, -1});
+			}
+			while((int) ld.size() < P.ldNC + P.ldND) ld.push_back(LdCol{nullptr, 0, 0, 0u, -1}); // (src: a zero, below)
+		}
+	}
+	if(ld.empty()) P.ldNC = 0;
+	std::vector<uint8_t> img(dictBytes + runBytes + streamBytes + colBytes + 24, 0); // (structs with pointers first: 8-byte aligned)
+	std::memcpy(img.data(), vals.data(), dictBytes);
 	if(runBytes) std::memcpy(img.data() + dictBytes, runs.data(), runBytes);
 	std::memcpy(img.data() + dictBytes + runBytes, streams.data(), streamBytes);
 	std::memcpy(img.data() + dictBytes + runBytes + streamBytes, all.data(), colBytes);
@@ -646,12 +614,15 @@ static int gdr_build_plan(cla_block* b, GdrPlan& P) {
 	CLA_HIP(hipMalloc((void**) &d, img.size() + 64));
 	P.dImg = d;
 	P.bytes = (int64_t) img.size() + 64;
+	for(size_t i = 0; i < ld.size(); i++) {
+		P.ld.c[i] = ld[i];
+		if(ld[i].src == nullptr) P.ld.c[i].src = d + dictBytes + runBytes + streamBytes + colBytes; // a zero
+	}
 	CLA_HIP(hipMemcpy(d, img.data(), img.size(), hipMemcpyHostToDevice));
-	P.A.dicts = (const GdrDict*) d;
+	P.A.vals = (const double*) d;
 	P.A.runs = (const RunCol*) (d + dictBytes);
 	P.A.streams = (const GdrStream*) (d + dictBytes + runBytes);
 	P.A.cols = (const GdrCol*) (d + dictBytes + runBytes + streamBytes);
-	P.A.nDicts = (int) dicts.size();
 	P.A.nStreams = (int) streams.size();
 	P.A.nV = nV; P.A.nR = nR;
 	P.A.n2 = 0; P.A.n12 = 0;
@@ -674,10 +645,7 @@ void gdr_plan_drop(cla_block* b) {
 	b->gdrPlan = nullptr;
 }
 
-// dOut (nCols x nCols, zeroed) += upper triangle of t(D) %*% D of the decoded rows, constants included. Returns 1
-// when the block is not of this kernel's shape (the caller takes the tile kernel on the matrix cores).
-int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz) {
-	if(!b->opt.tsmmDirect || b->crossSplit > 0 || b->crossBlocks > 0) return 1;
+int gdr_plan(cla_block* b, const GdrPlan*& P) {
 	if(b->gdrPlan == nullptr) {
 		int rc = ensure_expanded(b);
 		if(rc) return rc;
@@ -686,8 +654,18 @@ int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz) {
 		if(rc < 0) { gdr_plan_drop(b); return rc; }
 		if(b->gdrPlan->dImg) b->derivedBytes += b->gdrPlan->bytes;
 	}
-	if(b->gdrPlan->rc) return b->gdrPlan->rc;
-	GdrArgs A = b->gdrPlan->A;
+	P = b->gdrPlan;
+	return 0;
+}
+
+// dOut (nCols x nCols, zeroed) += upper triangle of t(D) %*% D of the decoded rows, constants included. Returns 1
+// when the block is not of this kernel's shape (the caller takes the tile kernel on the matrix cores).
+int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz) {
+	if(!b->opt.tsmmDirect || b->crossSplit > 0 || b->crossBlocks > 0) return 1;
+	const GdrPlan* P = nullptr;
+	if(const int rc = gdr_plan(b, P)) return rc;
+	if(P->rc) return P->rc;
+	GdrArgs A = P->A;
 	A.out = dOut;
 	A.acc = nullptr; A.done = nullptr; A.nnz = nullptr;
 	if(dNnz != nullptr) {
@@ -695,7 +673,7 @@ int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz) {
 		if(rc) return rc;
 		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
-	const size_t lds = b->gdrPlan->lds;
+	const size_t lds = P->lds;
 	const int nChunks = (int) ((b->nRows + GDR_CH - 1) / GDR_CH);
 	const unsigned grid = (unsigned) std::max(1, std::min((nChunks + GDR_WAVES - 1) / GDR_WAVES, g_numCU * (lds <= 76 * 1024 ? 2 : 1)));
 	Prof pf(b, "k_tsmm_direct", grid, GDR_THREADS, (long) lds, (double) b->device_bytes_cached);

@@ -1516,6 +1516,10 @@ int launch_rmm_decode(cla_block* b, const double* dB, int q, const double* dCons
 int launch_lmm_decode(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dBad) {
 	const int nCols = b->nCols;
 	if(b->groups.empty() || b->nRows == 0 || nCols > 64 || p < 1 || p > 16) return 1;
+	{
+		const int rc = launch_lmm_direct(b, dY, p, dOut, dBad);
+		if(rc != 1) return rc;
+	}
 	const int NB = (nCols + 15) / 16;
 	DecLaunch L;
 	bool flat = false;

@@ -1,0 +1,63 @@
+"""Y %*% X on k_lmm_direct (a few streamed columns next to run-length columns): every number of rows of Y per pass and of code
+and dense columns it is filled up to, row counts at the edges of its steps, run ends at every place of a step."""
+import numpy as np
+import pytest
+
+from parity import assert_matches_truth
+
+pytestmark = pytest.mark.gpu
+
+
+def block(synth, rng, n_rows, n_rle, n_short, n_byte, n_sdc, n_dense, mean_run=400):
+    order = list(rng.permutation(n_rle + n_short + n_byte + n_sdc + n_dense).astype(np.int32))
+    specs = []
+    for _ in range(n_rle):
+        starts = np.flatnonzero(rng.random(n_rows) < 1.0 / mean_run)
+        codes = np.repeat(rng.integers(-1, 32, len(starts) + 1), np.diff(np.concatenate(([0], starts, [n_rows]))))  # -1: rows that no run covers
+        ptr, rle = synth.encode_rle(codes, 32)
+        specs.append(synth.GroupSpec("rle", np.array([order.pop()], np.int32), rng.standard_normal((32, 1)), ptr=ptr, rle=rle))
+    for k in range(n_short + n_byte):
+        v, t = (700, np.uint16) if k < n_short else (9, np.uint8)
+        specs.append(synth.GroupSpec("ddc", np.array([order.pop()], np.int32), rng.standard_normal((v, 1)), rng.integers(0, v, n_rows).astype(t)))
+    for _ in range(n_sdc):
+        rows = np.flatnonzero(rng.random(n_rows) < 0.1)
+        rows = rows if len(rows) else np.array([0])
+        deltas, first, last, n = synth.encode_offsets(rows)
+        specs.append(synth.GroupSpec("sdc", np.array([order.pop()], np.int32), rng.standard_normal((16, 1)), rng.integers(0, 16, n).astype(np.uint8),
+                                     np.array([1.0]), deltas, first, last, n))
+    if n_dense:
+        specs.append(synth.GroupSpec("unc", np.sort(np.array(order, np.int32)), dense=rng.standard_normal((n_rows, n_dense))))
+    return specs, n_rle + n_short + n_byte + n_sdc + n_dense
+
+
+def check(cla, ora, specs, n_cols, n_rows, p, what, rng, direct=True):
+    Y = rng.standard_normal((p, n_rows))
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, nnz = blk.lmm(Y)
+    ran = [k["name"] for k in blk.stats()["kernels"]]
+    tile, _ = blk.set_option("tsmm_direct", 0).lmm(Y)
+    blk.close()
+    assert "k_lmm_decode" in ran, ran
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    assert_matches_truth(out, Y, D, what=what)
+    assert_matches_truth(tile, Y, D, what=what + ", tile kernel")
+    assert nnz == np.count_nonzero(out)
+
+
+@pytest.mark.parametrize("shape", [(8, 8, 0, 2, 2), (2, 2, 0, 1, 1), (0, 3, 2, 0, 0), (5, 4, 3, 1, 0), (1, 0, 1, 2, 4), (8, 6, 4, 2, 0), (3, 5, 1, 2, 3), (2, 8, 0, 0, 0), (1, 3, 1, 0, 2)])
+@pytest.mark.parametrize("p", [1, 2, 3, 4, 5, 6, 7, 8, 11, 16, 17])
+def test_shapes(cla, ora, shape, p):
+    from systemds_amd import synth
+    rng = np.random.default_rng(p)
+    n_rows = 70003
+    specs, n_cols = block(synth, rng, n_rows, *shape)
+    check(cla, ora, specs, n_cols, n_rows, p, f"{shape}, {p} rows", rng)
+
+
+@pytest.mark.parametrize("n_rows", [1, 2, 3, 63, 64, 127, 128, 129, 131, 255, 1030, 16383, 16384, 40005])
+@pytest.mark.parametrize("p,mean_run", [(3, 400), (6, 70), (8, 30)])
+def test_row_edges(cla, ora, n_rows, p, mean_run):
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows)
+    specs, n_cols = block(synth, rng, n_rows, 4, 3, 2, 1, 2, mean_run)
+    check(cla, ora, specs, n_cols, n_rows, p, f"{n_rows} rows", rng)
