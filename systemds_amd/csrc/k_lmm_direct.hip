@@ -185,6 +185,11 @@ __global__ __launch_bounds__(LD_THREADS, 2) void k_lmm_direct(const GdrArgs A, c
 				for(int i = 0; i < P; i++)
 #pragma unroll
 					for(int h = 0; h < R; h++) y[h][i] = row + h < nRows ? y[h][i] : 0.0;
+				// (the value beside such a zero as well: the last row, which stands in for the rows behind it, may hold an infinity)
+#pragma unroll
+				for(int c = 0; c < ND; c++)
+#pragma unroll
+					for(int h = 0; h < R; h++) xd[h][c] = row + h < nRows ? xd[h][c] : 0.0;
 			}
 #pragma unroll
 			for(int h = 0; h < R; h++) { // (one row after the other: both rows' values do not fit the registers next to the sums)
@@ -199,6 +204,7 @@ __global__ __launch_bounds__(LD_THREADS, 2) void k_lmm_direct(const GdrArgs A, c
 					uint32_t code = w & C.mask;
 					if(TAIL) code = row + h < nRows ? code : 0u; // (behind the last row: never an index)
 					x[c] = *(const double*) (ldsBytes + C.base8 + (code << 3));
+					if(TAIL) x[c] = row + h < nRows ? x[c] : 0.0; // (a column's constant may be infinite)
 				}
 #pragma unroll
 				for(int c = 0; c < NC; c++)

@@ -61,3 +61,34 @@ def test_row_edges(cla, ora, n_rows, p, mean_run):
     rng = np.random.default_rng(n_rows)
     specs, n_cols = block(synth, rng, n_rows, 4, 3, 2, 1, 2, mean_run)
     check(cla, ora, specs, n_cols, n_rows, p, f"{n_rows} rows", rng)
+
+
+@pytest.mark.parametrize("n_rows", [63, 65, 129, 70003])
+@pytest.mark.parametrize("p", [1, 6, 8])
+def test_infinities_in_the_last_row(cla, ora, n_rows, p):
+    """An infinity in the last row of a dense column and an infinite constant under a dictionary column reach their own column as
+    they do row by row: the rows that fill up the last step do not multiply them by zero."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows + p)
+    specs, n_cols = block(synth, rng, n_rows, 2, 2, 1, 1, 2)
+    specs[-1].dense[-1, 0], specs[-1].dense[-1, 1] = np.inf, -np.inf
+    Y = rng.random((p, n_rows)) + 0.5
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, nnz = blk.lmm(Y)
+    blk.close()
+    dense = specs[-1].cols
+    assert np.all(out[:, dense[0]] == np.inf) and np.all(out[:, dense[1]] == -np.inf)
+    rest = np.setdiff1d(np.arange(n_cols), dense)
+    assert_matches_truth(out[:, rest], Y, D[:, rest], what=f"{n_rows} rows")
+    assert nnz == np.count_nonzero(out)
+
+    specs, n_cols = block(synth, rng, n_rows, 0, 3, 1, 0, 0)
+    specs.append(synth.GroupSpec("const", np.array([specs[0].cols[0]], np.int32), np.array([[np.inf]])))
+    D = ora.np_decompress(specs[:-1], n_rows, n_cols)
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, _ = blk.lmm(Y)
+    blk.close()
+    rest = np.setdiff1d(np.arange(n_cols), specs[0].cols)
+    assert np.all(out[:, specs[0].cols] == np.inf)
+    assert_matches_truth(out[:, rest], Y, D[:, rest], what=f"{n_rows} rows, constant")
