@@ -3,10 +3,11 @@
 //
 // Lane = two consecutive rows, read straight from their streams: a wave takes 128 rows at a time. A varying column is looked up
 // in LDS once for all P rows of Y: acc[i][c] += y_i x_c, lane-private sums reduced over the lanes once at the end. A
-// run-length column is constant between two run ends, so by summation by parts (k_gram_direct.hip)
-//   sum_r y_i v_a = v_a(now) S_i(now) + sum over a's run ends of (v_a before - v_a behind) S_i(at that row),
-// S_i the running sum of y_i: only where a run ends is anything done for it. The lanes fold their P running sums eight to one
-// first, so that a run end adds one value per lane to the column's cells in LDS.
+// run-length column is never looked up per row: the rows between two run ends (of any column) are a stretch on which all of
+// them are constant, and a stretch adds its sums of y times the columns' values. The lanes fold their P sums eight to one first,
+// so that a stretch adds one value per lane to each column's cell in LDS.
+// (Not by summation by parts, which adds only where a column's own run ends, its value's step times the sum of y so far: rows on
+// which the column is zero enter such sums and must cancel again. A y of 1e14 on one of them left an error of 4e-7 of the sum of |y||x|.)
 //
 // Why not the tile kernel on the matrix cores (k_lmm_decode, which it precedes): Y %*% X has as few multiply-adds as P times
 // the columns per row and is bound by its streams; the tiles went through LDS twice, the matrix instruction pads both P and the
@@ -25,7 +26,7 @@ namespace cla {
 constexpr int LD_THREADS = 512;
 constexpr int LD_WAVES = LD_THREADS / WAVE;
 constexpr int LD_PMAX = 8;
-constexpr int LD_REBASE = 128;              // steps between two rebases of the running sums (a power of two)
+constexpr int LD_REBASE = 128;              // most steps that a stretch's sums run over (a power of two)
 constexpr int LD_WDOUBLES = 64 + 32 + RC_MAX * 64; // per wave: window values, window ends, the run-length columns' cells
 
 typedef double f64x2_ld __attribute__((ext_vector_type(2), aligned(8))); // (a row of Y starts at any multiple of 8 bytes)
@@ -109,38 +110,26 @@ __global__ __launch_bounds__(LD_THREADS, 2) void k_lmm_direct(const GdrArgs A, c
 			for(int i = 0; i < 2; i++) u[i] = (fb1 ? w[2 * i + 1] : w[2 * i]) + xchg2(fb1 ? w[2 * i] : w[2 * i + 1]);
 			return (fb2 ? u[1] : u[0]) + xchg4(fb2 ? u[0] : u[1]);
 		};
-		auto bcast_f64 = [](double v, int src) {
-			int p[2];
-			__builtin_memcpy(p, &v, 8);
-			p[0] = __builtin_amdgcn_readlane(p[0], src);
-			p[1] = __builtin_amdgcn_readlane(p[1], src);
-			double r;
-			__builtin_memcpy(&r, p, 8);
-			return r;
-		};
-		// the runs that end at row e (el(i): the running sums with the rows in front of e)
-		auto event = [&](int32_t e, auto el) __attribute__((always_inline)) {
-			const double vOld = rc.val;
-			unsigned mm = (unsigned) (__ballot(rc.end == e) >> RC_LANE0) & ((1u << RC_MAX) - 1u); // (cursor lanes only)
-			rc.advance(e, lane);
-			const double step = vOld - rc.val;
+		// A stretch of rows on which every run-length column is constant ends (el(i): the lane's sums of y over it): each column
+		// takes its value times the stretch's sums. (Unused cursors hold the value 0.)
+		auto stretch = [&](auto el) __attribute__((always_inline)) {
 			const double f = fold(el);
-			while(mm != 0) {
-				const int a = __builtin_ctz(mm);
-				mm &= mm - 1;
-				cells[64 * a] = __builtin_fma(f, bcast_f64(step, RC_LANE0 + a), cells[64 * a]);
-			}
-		};
-		auto rebase = [&]() __attribute__((always_inline)) {
-			if(nR > 0) {
-				const double f = fold([&](int i) __attribute__((always_inline)) { return S[i]; });
-				for(int a = 0; a < nR; a++) cells[64 * a] = __builtin_fma(f, rc.value(a), cells[64 * a]);
-			}
+			bad |= !(__builtin_fabs(f) <= 1.7976931348623157e308); // (a value of y that is not finite stays in its sum)
+			auto take = [&](auto a0Tag) __attribute__((always_inline)) { // four columns, their cells requested together
+				constexpr int a0 = decltype(a0Tag)::value;
+				double h[4];
 #pragma unroll
-			for(int i = 0; i < P; i++) {
-				bad |= !(__builtin_fabs(S[i]) <= 1.7976931348623157e308); // (a value of y that is not finite stays in its sum)
-				S[i] = 0.0;
-			}
+				for(int a = 0; a < 4; a++) h[a] = cells[64 * (a0 + a)];
+#pragma unroll
+				for(int a = 0; a < 4; a++) cells[64 * (a0 + a)] = __builtin_fma(f, rc.value(a0 + a), h[a]);
+			};
+			if(nR > 0) take(std::integral_constant<int, 0>());
+			if(nR > 4) take(std::integral_constant<int, 4>());
+		};
+		auto restart = [&]() __attribute__((always_inline)) {
+			stretch([&](int i) __attribute__((always_inline)) { return S[i]; });
+#pragma unroll
+			for(int i = 0; i < P; i++) S[i] = 0.0;
 		};
 
 		// the word that holds the lane's codes, for streams of two bytes and of one, and the place in it
@@ -221,9 +210,16 @@ __global__ __launch_bounds__(LD_THREADS, 2) void k_lmm_direct(const GdrArgs A, c
 					for(int i = 0; i < P; i++) asm volatile("" : "+v"(acc[c][i]));
 				__builtin_amdgcn_sched_barrier(0);
 			}
-			while(eNext < s0 + LD_CH) { // (uniform) runs that end inside the step
+			while(eNext < s0 + LD_CH) { // (uniform) runs that end inside the step: the rows in front of the end leave the sums
 				const bool m0 = row < eNext, m1 = row + 1 < eNext;
-				event(eNext, [&](int i) __attribute__((always_inline)) { return S[i] + (R == 1 ? (m0 ? y[0][i] : 0.0) : (m0 ? y[0][i] : 0.0) + (m1 ? y[R - 1][i] : 0.0)); });
+				stretch([&](int i) __attribute__((always_inline)) { return S[i] + (R == 1 ? (m0 ? y[0][i] : 0.0) : (m0 ? y[0][i] : 0.0) + (m1 ? y[R - 1][i] : 0.0)); });
+#pragma unroll
+				for(int i = 0; i < P; i++) {
+					S[i] = 0.0;
+					y[0][i] = m0 ? 0.0 : y[0][i];
+					if(R > 1) y[R - 1][i] = m1 ? 0.0 : y[R - 1][i];
+				}
+				rc.advance(eNext, lane);
 				eNext = rc.next_end();
 			}
 #pragma unroll
@@ -233,11 +229,11 @@ __global__ __launch_bounds__(LD_THREADS, 2) void k_lmm_direct(const GdrArgs A, c
 		for(int chB = ch0; chB < chFull; chB += LD_REBASE) {
 			const int chE = min(chB + LD_REBASE, chFull);
 			for(int ch = chB; ch < chE; ch++) chunk(ch, std::false_type());
-			rebase();
+			restart();
 		}
 		if(chFull < ch1) {
 			chunk(chFull, std::true_type());
-			rebase();
+			restart();
 		}
 		if(__ballot(bad) != 0 && lane == 0) atomicOr(badY, 1ull);
 

@@ -92,3 +92,28 @@ def test_infinities_in_the_last_row(cla, ora, n_rows, p):
     rest = np.setdiff1d(np.arange(n_cols), specs[0].cols)
     assert np.all(out[:, specs[0].cols] == np.inf)
     assert_matches_truth(out[:, rest], Y, D[:, rest], what=f"{n_rows} rows, constant")
+
+
+@pytest.mark.parametrize("big", [1e14, 1e200, -1e290])
+@pytest.mark.parametrize("p,mean_run", [(1, 3000), (4, 400), (6, 90)])
+def test_large_values_where_a_run_length_column_is_zero(cla, ora, big, p, mean_run):
+    """Y may be of any size on rows that no run covers or whose value is zero: such rows leave no trace in the column's sums
+    (each cell within 1e-12 of |Y| %*% |X|, to which they add nothing)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(p)
+    n_rows = 40005
+    specs, n_cols = block(synth, rng, n_rows, 5, 3, 1, 1, 1, mean_run)
+    row = np.arange(n_rows)
+    specs[0].ptr, specs[0].rle = synth.encode_rle(np.where(row < 5000, -1, 3), 32)         # one run behind rows that none covers
+    specs[1].ptr, specs[1].rle = synth.encode_rle(np.where(row // 137 % 2 == 0, 2, 3), 32)  # every other run is of zeros
+    specs[1].dict[2] = 0.0
+    Y = rng.standard_normal((p, n_rows))
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    zero = np.flatnonzero((D[:, specs[0].cols[0]] == 0.0) & (D[:, specs[1].cols[0]] == 0.0))
+    Y[:, [0, 17, zero[-1]] + list(rng.choice(zero, 5))] = big
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, nnz = blk.lmm(Y)
+    blk.close()
+    for c in range(n_cols):  # (a column at a time: the largest output of one is no scale for another)
+        assert_matches_truth(out[:, c:c + 1], Y, D[:, c:c + 1], what=f"column {c}, y of {big}")
+    assert nnz == np.count_nonzero(out)
