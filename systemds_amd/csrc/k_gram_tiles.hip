@@ -461,8 +461,7 @@ int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz) {
 		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
 	const unsigned grid = (unsigned) std::min(A.nTiles, g_numCU);
-	// (reported under the name of the form, the decoded Gram matrix, whichever of its kernels runs)
-	Prof pf(b, "k_tsmm_decode", grid, GT_THREADS, (long) P.lds, (double) b->device_bytes_cached);
+	Prof pf(b, "k_gram_tiles", grid, GT_THREADS, (long) P.lds, (double) b->device_bytes_cached);
 #define GT_CASE(NF) \
 	case NF: return P.nn == 0 ? gt_launch<NF, 0>(b, P, A, grid) : P.nn == 1 ? gt_launch<NF, 1>(b, P, A, grid) : gt_launch<NF, 2>(b, P, A, grid);
 	switch(P.nf) {

@@ -276,8 +276,7 @@ int launch_lmm_direct(cla_block* b, const double* dY, int p, double* dOut, unsig
 		const int rows = WAVE * ld_rows(nc + nd, ph);
 		const int nChunks = (int) ((b->nRows + rows - 1) / rows);
 		const unsigned grid = (unsigned) std::max(1, std::min((nChunks + LD_WAVES - 1) / LD_WAVES, g_numCU));
-		// (reported under the name of the form, Y times the decoded rows, whichever of its kernels runs)
-		Prof pf(b, "k_lmm_decode", grid, LD_THREADS, (long) lds, (double) b->device_bytes_cached + (double) b->nRows * ph * 8);
+		Prof pf(b, "k_lmm_direct", grid, LD_THREADS, (long) lds, (double) b->device_bytes_cached + (double) b->nRows * ph * 8);
 		bool launched = false;
 #define LD_CASE_P(NCV, NDV, PV)                                                                                                \
 	if(!launched && nc == NCV && nd == NDV && ph == PV) {                                                                      \

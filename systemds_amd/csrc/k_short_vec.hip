@@ -151,7 +151,6 @@ __global__ __launch_bounds__(256) void k_rmm_q1_short_rows(const uint8_t* __rest
 }
 
 // Returns 1 when the block is not eligible. `tables`: dict x v of all groups and, at constIdx, the constants' term.
-// (Reported under the name of the form, the mat-vec gather on tables, whichever kernel runs.)
 int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double* dOut, unsigned long long* dNnz) {
 	const int nG = (int) b->groups.size();
 	if(b->dArena == nullptr || b->arenaWidth != 2 || nG == 0 || b->nRows == 0 || b->maxVals > SV_BUF) return 1;
@@ -160,7 +159,7 @@ int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double
 	// 200,000 x 50 18 against 28; beyond, the form with the tables in LDS: 700,000 x 50 31 against 43, 1,500,000 x 6 14 against 26.
 	if(b->nRows <= 400000) {
 		const unsigned grid = (unsigned) ((b->nRows + 255) / 256);
-		Prof pf(b, "k_rmm_q1_ddc", grid, 256, 0, (double) b->nRows * (2 * nG + 8) + (double) b->totalVals * 8);
+		Prof pf(b, "k_rmm_q1_short_rows", grid, 256, 0, (double) b->nRows * (2 * nG + 8) + (double) b->totalVals * 8);
 		hipLaunchKernelGGL(k_rmm_q1_short_rows, dim3(grid), dim3(256), 0, b->stream, b->dArena, b->arenaStride, nG, b->dTblOff, tables,
 			constIdx, dOut, b->nRows, dNnz, b->chainOp);
 		CLA_HIP(hipGetLastError());
@@ -174,7 +173,7 @@ int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double
 	const int64_t perWave = ((n4 + grid - 1) / grid + SV_WAVES - 1) / SV_WAVES;
 	const int nu = (int) ((perWave + WAVE - 1) / WAVE);
 	const size_t lds = (size_t) 2 * SV_BUF * 8;
-	Prof pf(b, "k_rmm_q1_ddc", grid, SV_THREADS, (long) lds, (double) b->nRows * (2 * nG + 8) + (double) b->totalVals * 8);
+	Prof pf(b, "k_rmm_q1_short", grid, SV_THREADS, (long) lds, (double) b->nRows * (2 * nG + 8) + (double) b->totalVals * 8);
 #define SV_LAUNCH(NU)                                                                                                        \
 	do {                                                                                                                     \
 		CLA_HIP(allow_full_lds((const void*) k_rmm_q1_short<NU>));                                                           \

@@ -8,12 +8,14 @@ from parity import assert_matches_truth
 pytestmark = pytest.mark.gpu
 
 
-def check(cla, ora, specs, n_rows, n_cols, what):
+def check(cla, ora, specs, n_rows, n_cols, what, options=()):
     blk = cla.build_block(n_rows, n_cols, specs)
+    for key, value in options:
+        blk.set_option(key, value)
     out, nnz = blk.tsmm()
     names = {k["name"] for k in blk.stats()["kernels"]}
     blk.close()
-    assert names == {"k_tsmm_decode"}, names
+    assert names == {"k_gram_tiles"}, names
     D = ora.np_decompress(specs, n_rows, n_cols)
     assert np.array_equal(out, out.T)
     assert_matches_truth(out, D.T, D, what=what)
@@ -26,7 +28,7 @@ def columns(synth, rng, n_rows, n_cols, n_vals, dtype, width):
                             rng.integers(0, n_vals, n_rows).astype(dtype)) for c in range(0, n_cols, width)]
 
 
-@pytest.mark.parametrize("n_cols", [65, 68, 72, 73, 80, 81, 88, 96, 97, 100, 112, 113, 120, 127, 128])
+@pytest.mark.parametrize("n_cols", [13, 16, 17, 20, 24, 25, 33, 40, 48, 52, 64, 65, 68, 72, 73, 80, 81, 88, 96, 97, 100, 112, 113, 120, 127, 128])
 @pytest.mark.parametrize("n_rows", [1, 31, 33, 8191, 40009])
 def test_byte_codes(cla, ora, n_cols, n_rows):
     from systemds_amd import synth
@@ -41,15 +43,7 @@ def test_column_pairs(cla, ora, n_cols, n_rows, n_vals):
     from systemds_amd import synth
     rng = np.random.default_rng(n_cols + n_rows)
     specs = columns(synth, rng, n_rows, n_cols, n_vals, np.uint16, 2)
-    if n_cols <= 64:  # narrow blocks of few groups come here when their codes exceed the direct kernel's tables
-        blk = cla.build_block(n_rows, n_cols, specs).set_option("tsmm_route", 2)
-        out, nnz = blk.tsmm()
-        blk.close()
-        D = ora.np_decompress(specs, n_rows, n_cols)
-        assert_matches_truth(out, D.T, D, what=f"{n_rows} x {n_cols}, pairs")
-        assert nnz == np.count_nonzero(out)
-        return
-    check(cla, ora, specs, n_rows, n_cols, f"{n_rows} x {n_cols}, pairs")
+    check(cla, ora, specs, n_rows, n_cols, f"{n_rows} x {n_cols}, pairs", [("tsmm_route", 2)])  # (few groups: decoded all the same)
 
 
 @pytest.mark.parametrize("n_cols,width,n_vals", [(66, 1, 300), (99, 3, 1000), (101, 2, 4096), (128, 1, 260)])

@@ -183,14 +183,14 @@ def test_byte_code_block_with_non_finite_dictionary_values(cla, ora):
 @pytest.mark.parametrize("p", [1, 2, 5, 8, 16, 17, 40])
 def test_mixed_block_takes_one_decoded_pass(cla, ora, p):
     """C5's shape (RLE, two-byte DDC, offset lists with a default, dense columns): Y %*% X in one pass over the decoded
-    rows on the matrix cores, Y as the other operand (`k_lmm_decode`); with the option off the bin kernels give the
-    same cells."""
+    rows on the matrix cores, Y as the other operand (`k_lmm_decode`, here also for the rows of Y that `k_lmm_direct`
+    would serve: option tsmm_direct); with the option off the bin kernels give the same cells."""
     from systemds_amd import synth
     c = synth.config5(scale=400)
     n_rows, n_cols = c["n_rows"], c["n_cols"]
     Y = np.random.default_rng(p).standard_normal((p, n_rows))
     D = ora.np_decompress(c["groups"], n_rows, n_cols)
-    blk = cla.build_block(n_rows, n_cols, c["groups"])
+    blk = cla.build_block(n_rows, n_cols, c["groups"]).set_option("tsmm_direct", 0)
     try:
         out, nnz = blk.lmm(Y)
         blk.profile(True)

@@ -506,12 +506,12 @@ def test_wide_right_multiply_in_passes_of_the_tile_kernel(cla, ora, q):
 
 
 @pytest.mark.parametrize("n_vals,n_groups", [(1000, 20), (1900, 11)])
-def test_mat_vec_on_two_byte_codes_with_large_dictionaries(cla, ora, n_vals, n_groups):
-    """Single-column DDC groups with two-byte codes whose tables fit a slab of 8 only in blocks of 512 threads (1000
-    values) or 1024 threads (1900 values): X %*% v stays on the slab kernel with its tables in LDS."""
+@pytest.mark.parametrize("n_rows,kernel", [(70003, "k_rmm_q1_short_rows"), (400003, "k_rmm_q1_short")])
+def test_mat_vec_on_two_byte_codes_with_large_dictionaries(cla, ora, n_vals, n_groups, n_rows, kernel):
+    """Single-column DDC groups with two-byte codes whose tables do not fit LDS together: X %*% v on few rows straight from
+    global memory, on many with the tables of two groups at a time in LDS."""
     from systemds_amd import synth
     rng = np.random.default_rng(n_vals)
-    n_rows = 70003
     specs = [synth.GroupSpec("ddc", np.array([c], np.int32), rng.standard_normal((n_vals, 1)), rng.integers(0, n_vals, n_rows).astype(np.uint16))
              for c in range(n_groups)]
     v = rng.standard_normal((n_groups, 1))
@@ -523,7 +523,7 @@ def test_mat_vec_on_two_byte_codes_with_large_dictionaries(cla, ora, n_vals, n_g
         names = [k["name"] for k in blk.stats()["kernels"]]
     finally:
         blk.close()
-    assert "k_rmm_q1_ddc" in names, names
+    assert kernel in names, names
     assert_matches_truth(out, D, v, what=f"X %*% v, {n_vals} values per column")
     assert nnz == np.count_nonzero(out)
 

@@ -188,7 +188,7 @@ def test_decoded_gram_with_a_narrow_last_column_block(cla, ora, n_cols, big_dict
     check_tsmm(cla, ora, specs, n_rows, n_cols, f"{n_cols} columns, narrow {narrow}", {"tsmm_route": 2, "tsmm_narrow": narrow})
 
 
-@pytest.mark.parametrize("shape", ["decode", "direct"])
+@pytest.mark.parametrize("shape", ["tiles", "decode", "direct"])
 def test_decoded_gram_is_one_kernel_per_call(cla, ora, shape):
     """A block of at most 64 columns that the decoded Gram kernels take runs as one kernel per call: the blocks add
     into an accumulator kept with the block and the last one writes the output, mirrored, counts its non-zeros and
@@ -197,18 +197,18 @@ def test_decoded_gram_is_one_kernel_per_call(cla, ora, shape):
     between them."""
     import devmem
     from systemds_amd import synth
-    if shape == "decode":
+    if shape == "tiles":
         c = synth.config3(scale=100)
         specs, n_rows, n_cols = c["groups"], c["n_rows"], c["n_cols"]
-        kernel = "k_tsmm_decode"
-    else:
+        kernel = "k_gram_tiles"
+    else: # ("decode": the tile kernel on the other kernel's blocks)
         from test_gpu_gram_direct import stream_block
         n_rows = 70003
         specs, n_cols = stream_block(21, n_rows)
-        kernel = "k_tsmm_direct"
+        kernel = "k_tsmm_" + shape
     D = ora.np_decompress(specs, n_rows, n_cols)
     scale = np.abs(D).T @ np.abs(D)
-    blk = cla.build_block(n_rows, n_cols, specs)
+    blk = cla.build_block(n_rows, n_cols, specs).set_option("tsmm_direct", 0 if shape == "decode" else 1)
     try:
         first, nnz = blk.tsmm()
         blk.profile(True)
