@@ -53,6 +53,7 @@ struct GdrPlan {
 	GdrArgs A;
 	LdCols ld;             // ldNC code columns (fillers behind the real ones), ldND dense ones; ldNC == 0: no such form
 	int ldNC = 0, ldND = 0;
+	int64_t runEnds = 0;   // of the run-length groups that are followed by run (inside the matrix)
 };
 
 // A block's copy of the values into LDS: 16-byte pieces, several requested together (one dictionary after the other, each a

@@ -519,6 +519,7 @@ static int gdr_build_plan(cla_block* b, GdrPlan& P) {
 		if(G.type == G_RLE && !haveStream) {
 			for(int h = 0; h < G.nColG; h++) runs.push_back(RunCol{G.runStart, G.runCode, G.dict, b->constV[hc[h]], G.nRuns, G.nColG, h, hc[h]});
 			covered += G.nColG;
+			P.runEnds += std::max(G.nRuns - 1, 0);
 			continue;
 		}
 		const uint8_t* src;

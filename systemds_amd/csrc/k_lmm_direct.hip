@@ -267,6 +267,11 @@ int launch_lmm_direct(cla_block* b, const double* dY, int p, double* dOut, unsig
 	// A pass costs 14 us before its first row; the tile kernel takes 16 rows of Y in one (500,000 x 11 by 11 rows 40 against 47 us,
 	// 100,003 x 20 by 6 29 against 20; 5,000,011 x 20 by 16 332 against 247).
 	if(passes > 1 && b->nRows <= (int64_t) 500000 * (passes - 1)) return 1;
+	// A run end takes 0.24 - 0.32 ns of a pass (by 1 and 6 rows of Y, all waves together), the tile kernel hardly notices it. One to six rows
+	// and a pass is where they meet, whatever the number of run-length columns and of rows: 3,000,017 rows by 6 of Y, 8 run-length
+	// columns of mean run 24 381 against 279 us, 48 235 against 334; 4 of 16 284 against 233, of 24 216 against 256; 2 of 8 296 against
+	// 209, of 12 217 against 219; 300,007 rows, 4 of 16 76 against 69, of 24 66 against 75.
+	if(P->runEnds * passes * 6 > b->nRows) return 1;
 	const size_t lds = ((size_t) P->A.valDoubles + LD_PMAX * (nc + nd + RC_MAX) + (size_t) LD_WAVES * LD_WDOUBLES) * 8;
 	if(lds > (size_t) std::min(g_ldsPerBlock, 160 * 1024)) return 1;
 	for(int k = 0, p0 = 0; k < passes; k++) {

@@ -78,6 +78,17 @@ def test_shapes(cla, ora, shape, p):
     check(cla, ora, specs, n_cols, n_rows, p, f"{shape}, {p} rows", rng)
 
 
+@pytest.mark.parametrize("p,mean_run,kernel", [(6, 8, "k_lmm_decode"), (6, 40, "k_lmm_decode"), (6, 60, "k_lmm_direct"), (1, 8, "k_lmm_decode")])
+def test_many_short_runs_take_the_tile_kernel(cla, ora, p, mean_run, kernel):
+    """Eight run-length columns of short runs next to too few other bytes for one-code-per-row copies: a run end for every row
+    or two is what the tile kernel does better (run ends are counted once per column, so 8 of mean run 48 lie at the rule's edge)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(mean_run)
+    n_rows = 100003
+    specs, n_cols = block(synth, rng, n_rows, 8, 0, 2, 0, 0, mean_run)
+    check(cla, ora, specs, n_cols, n_rows, p, f"runs of {mean_run}", rng, [kernel])
+
+
 @pytest.mark.parametrize("n_rows,p", [(500003, 7), (500003, 11), (1000003, 13), (1000003, 16), (500001, 8)])
 @pytest.mark.parametrize("shape", [(2, 4, 0, 4, 1), (1, 2, 1, 1, 2)])
 def test_passes_over_many_rows(cla, ora, n_rows, p, shape):
