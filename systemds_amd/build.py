@@ -93,6 +93,20 @@ def build_c_driver(verbose=True):
     return C_DRIVER
 
 
+ALLOC_DRIVER = os.path.join(ROOT, "tests", "cla_alloc_driver")
+
+
+def build_alloc_driver(verbose=True):
+    """The test driver that makes host allocations inside the library fail (tests/cla_alloc_driver.cpp)."""
+    cxx = os.environ.get("CXX", "g++")
+    cmd = [cxx, "-O1", "-std=c++17", "-Wall", "-Wextra", "-rdynamic", "-I" + INCLUDE, ALLOC_DRIVER + ".cpp", "-o", ALLOC_DRIVER,
+           "-L" + HERE, "-lclahip", "-Wl,-rpath,$ORIGIN/../systemds_amd", "-ldl"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    return ALLOC_DRIVER
+
+
 def build_jni(verbose=True):
     """The JNI shim (jni/cla_jni.c) when a JDK is present ($JAVA_HOME/include/jni.h); returns None otherwise."""
     jh = os.environ.get("JAVA_HOME")
@@ -113,5 +127,6 @@ if __name__ == "__main__":
     if "--no-host" not in sys.argv:
         build_host()
         build_c_driver()
+        build_alloc_driver()
         build_jni()
     sys.exit(0)

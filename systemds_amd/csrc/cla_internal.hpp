@@ -100,10 +100,12 @@ struct KernelStat {
 	float ms = -1.f;
 };
 
-// What the multiply chain does to the sum of a row on its way out: nothing (w == nullptr), times w or minus w.
+// What the multiply chain does to the sum of a row on its way out: nothing (w == nullptr), times w or minus w. The chain hands
+// it to its right multiply; a launcher whose kernel does it sets `done`, else a kernel of its own follows.
 struct RowOp {
 	const double* w = nullptr;
 	int minus = 0;
+	bool done = false;
 };
 struct DecPlanCache;
 struct DirPlan;
@@ -175,10 +177,6 @@ struct cla_block {
 	double* dStageOut = nullptr; size_t stageOutCap = 0;
 	void* dScratch = nullptr;   size_t scratchCap = 0;
 	double* dChain = nullptr;   size_t chainCap = 0;   // X %*% v inside the multiply chain
-	// While the chain's right multiply is queued: what happens to each of its sums (RowOp). A kernel that does it on the way
-	// out sets chainOpDone; else a kernel of its own follows.
-	cla::RowOp chainOp;
-	bool chainOpDone = false;
 	// exact code counts of all dictionary-coded groups (totalVals int32, group g at tblOff[g]),
 	// computed on the first TSMM and kept, like the reference's cached counts
 	// (CG/AColGroupValue.java getCounts)
@@ -268,7 +266,7 @@ int launch_counts(cla_block* b, int group, int32_t* dCounts);
 int reorder_ddc_by_count(cla_block* b, int group);
 int launch_sdc_build(cla_block* b, HostGroup& g);
 int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned long long* dNnz, int squares = 0,
-	double* ws = nullptr, size_t wsDoubles = 0);
+	double* ws = nullptr, size_t wsDoubles = 0, RowOp* op = nullptr);
 int launch_tables(cla_block* b, const double* dB, int q); // dict x B of every group (+ constV x B) into b->dTables
 int launch_aggregate(cla_block* b, int op, int dir, double* dOut, unsigned long long* dNnz);
 int ensure_counts(cla_block* b);
@@ -281,12 +279,12 @@ int launch_lmm_sdc_tiles(cla_block* b, const double* dY, int p, double* dPre, in
 int launch_lmm_sdc_lanes(cla_block* b, const double* dY, int p, double* dOut);
 int sdc_plan_all(cla_block* b); // the list of the block's SDCZeros groups with entries (b->sdcList)
 int launch_rmm_sdc_lanes(cla_block* b, int constRow, int accumulate, double* dOut, unsigned long long* dNnz);
-int launch_rmm_sdc_rows(cla_block* b, int constRow, int accumulate, double* dOut, unsigned long long* dNnz, const double* dU = nullptr,
-	unsigned long long* nnzNext = nullptr);
+int launch_rmm_sdc_rows(cla_block* b, int constRow, int accumulate, double* dOut, unsigned long long* dNnz, RowOp* op,
+	const double* dU = nullptr, unsigned long long* nnzNext = nullptr);
 bool rows_fusable(cla_block* b);
-int launch_rmm_sdc_tiles(cla_block* b, int q, int constRow, int accumulate, double* dOut, unsigned long long* dNnz);
+int launch_rmm_sdc_tiles(cla_block* b, int q, int constRow, int accumulate, double* dOut, unsigned long long* dNnz, RowOp* op);
 int launch_tsmm_decode(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);
-int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double* dOut, unsigned long long* dNnz);
+int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double* dOut, unsigned long long* dNnz, RowOp* op);
 int lmm_q1_short_groups(const cla_block* b);
 int launch_lmm_q1_short(cla_block* b, const double* dY, double* dOut);
 int launch_lmm_direct(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dBad);

@@ -410,19 +410,15 @@ int launch_mmchain(cla_block* b, const double* dV, const double* dW, int ctype, 
 	double* tmp = b->dChain;
 	int rc;
 	// (the weights are read where X %*% v writes its rows: a pass of its own over 10 M rows takes 40 us)
-	b->chainOp = RowOp{ctype == 0 ? nullptr : dW, ctype == 2};
-	b->chainOpDone = false;
-	rc = launch_rmm(b, dV, 1, tmp, dNnz);
-	const bool done = b->chainOpDone;
-	b->chainOp = RowOp();
-	b->chainOpDone = false;
-	if(rc) return rc;
+	RowOp op;
+	if(ctype != 0) { op.w = dW; op.minus = ctype == 2; }
+	if((rc = launch_rmm(b, dV, 1, tmp, dNnz, 0, nullptr, 0, &op))) return rc;
 	b->nnzSlot = 0; // the left multiply below counts the result's non-zeros into dNnz
 	std::vector<KernelStat> first;
 	first.swap(b->lastStats);
-	if(ctype == 1 && !done && nRows > 0)
+	if(ctype == 1 && !op.done && nRows > 0)
 		hipLaunchKernelGGL(k_mul_inplace, dim3((unsigned) ((nRows + 255) / 256)), dim3(256), 0, b->stream, tmp, dW, nRows);
-	if(ctype == 2 && !done && nRows > 0)
+	if(ctype == 2 && !op.done && nRows > 0)
 		hipLaunchKernelGGL(k_sub_inplace, dim3((unsigned) ((nRows + 255) / 256)), dim3(256), 0, b->stream, tmp, dW, nRows);
 	rc = launch_lmm(b, tmp, 1, dOut, dNnz);
 	b->lastStats.insert(b->lastStats.begin(), first.begin(), first.end());

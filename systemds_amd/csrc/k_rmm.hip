@@ -550,8 +550,9 @@ int launch_tables(cla_block* b, const double* dB, int q) {
 // ws != nullptr: a workspace of wsDoubles doubles that the caller owns takes the place of the block's table
 // buffer and nothing is allocated: kernels that need a derived format or a buffer of their own are left
 // out (the tables then always come from the pre-aggregation kernel), and a block that needs them is refused.
+// op: what the multiply chain does to the row sums (RowOp), where a kernel that can do it serves the block.
 int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned long long* dNnz, int squares, double* ws,
-	size_t wsDoubles) {
+	size_t wsDoubles, RowOp* op) {
 	const int nG = (int) b->groups.size();
 	const int64_t nRows = b->nRows;
 	hipStream_t st = b->stream;
@@ -588,7 +589,7 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 	// counts likewise into a counter that the call before has cleared: the only launch.
 	if(q == 1 && !squares && !noAlloc && !u8Path && b->opt.sdcRows && nRows > 0 && dNnz == b->dCounters && rows_fusable(b)) {
 		b->nnzSlot = b->nnzRot;
-		const int r = launch_rmm_sdc_rows(b, -1, 0, dOut, b->nnz_counter(b->nnzSlot), dB, b->nnz_counter(b->nnzRot % 3 + 1));
+		const int r = launch_rmm_sdc_rows(b, -1, 0, dOut, b->nnz_counter(b->nnzSlot), op, dB, b->nnz_counter(b->nnzRot % 3 + 1));
 		if(r < 0) return r;
 		if(r == 0) {
 			b->nnzRot = b->nnzRot % 3 + 1;
@@ -621,23 +622,23 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 		const double* constTerm = constRow >= 0 ? tables + constRow : nullptr;
 		unsigned long long* nnzNext = fused ? b->nnz_counter(b->nnzRot % 3 + 1) : nullptr;
 		Prof pf(b, "k_rmm_q1_u8", grid, THREADS, per * 256 * 8, bytes);
-		const RowOp op = b->chainOp;
+		const RowOp rowOp = op != nullptr ? *op : RowOp();
 #define U8_LAUNCH_OP(PER, NBV, LB, LN, F, O)                                                                    \
 	hipLaunchKernelGGL((k_rmm_q1_u8<THREADS, PER, NBV, LB, LN, F, O>), dim3(grid), dim3(THREADS), 0, st, b->dArena, \
-		b->arenaStride, nG, F ? b->dDictPad : dTpad, constTerm, dOut, nRows, dNnz, dCol0, dB, nnzNext, op)
+		b->arenaStride, nG, F ? b->dDictPad : dTpad, constTerm, dOut, nRows, dNnz, dCol0, dB, nnzNext, rowOp)
 #define U8_LAUNCH(PER, NBV, LB, LN, F)                                                                          \
-	do { if(op.w != nullptr) U8_LAUNCH_OP(PER, NBV, LB, LN, F, true); else U8_LAUNCH_OP(PER, NBV, LB, LN, F, false); } while(0)
+	do { if(rowOp.w != nullptr) U8_LAUNCH_OP(PER, NBV, LB, LN, F, true); else U8_LAUNCH_OP(PER, NBV, LB, LN, F, false); } while(0)
 		if(per == 20) { if(fused) U8_LAUNCH(20, 5, 4, 2, true); else U8_LAUNCH(20, 5, 4, 2, false); }
 		else { if(fused) U8_LAUNCH(16, 4, 8, 2, true); else U8_LAUNCH(16, 4, 8, 2, false); }
 #undef U8_LAUNCH
 #undef U8_LAUNCH_OP
-		b->chainOpDone = op.w != nullptr;
 		CLA_HIP(hipGetLastError());
+		if(op != nullptr) op->done = true;
 		if(fused) b->nnzRot = b->nnzRot % 3 + 1;
 		return 0;
 	}
 	if(q == 1) {
-		const int r = launch_rmm_q1_short(b, tables, constRow, dOut, dNnz);
+		const int r = launch_rmm_q1_short(b, tables, constRow, dOut, dNnz, op);
 		if(r <= 0) return r;
 	}
 	if(q == 1 && b->dArena && b->q1LdsBytes > 0) {
@@ -728,7 +729,7 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 			hipLaunchKernelGGL(k_rmm_rows, grid, dim3(256), 0, st, b->dGroups, nG, tables, dB, q, constRow, dOut, nRows);
 		}
 		if(anySdc) {
-			const int r = launch_rmm_sdc_tiles(b, q, constRow, anyRowGroup ? 1 : 0, dOut, dNnz);
+			const int r = launch_rmm_sdc_tiles(b, q, constRow, anyRowGroup ? 1 : 0, dOut, dNnz, op);
 			if(r < 0) return r;
 			if(r == 0) needNnzPass = false;
 			else {

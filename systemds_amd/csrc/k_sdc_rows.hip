@@ -369,8 +369,8 @@ static int rows_plan(cla_block* b) {
 // X %*% u of all listed groups (tables in b->dTables). Returns 1 when the lists do not fit (tables beyond LDS or
 // 16-bit positions, rows with too many entries), 0 when done. dU != nullptr: the kernel makes the tables itself
 // (rows_fusable said it can) and clears *nnzNext.
-int launch_rmm_sdc_rows(cla_block* b, int constRow, int accumulate, double* dOut, unsigned long long* dNnz, const double* dU,
-	unsigned long long* nnzNext) {
+int launch_rmm_sdc_rows(cla_block* b, int constRow, int accumulate, double* dOut, unsigned long long* dNnz, RowOp* op,
+	const double* dU, unsigned long long* nnzNext) {
 	int rc = rows_plan(b);
 	if(rc) return rc;
 	if(b->rowsState != 1 || (dU != nullptr && !b->rowsFusable)) return 1;
@@ -381,20 +381,20 @@ int launch_rmm_sdc_rows(cla_block* b, int constRow, int accumulate, double* dOut
 	double algo = (double) b->nRows * 8 * (accumulate ? 2 : 1);
 	for(int g : b->sdcList) algo += (double) b->groups[g].d.nDeltas * b->groups[g].d.deltaWidth + (double) b->groups[g].d.nOffsets * b->groups[g].d.codeWidth;
 	Prof pf(b, "k_rmm_sdc_rows", (long) grid, RW_THREADS, (long) lds, algo);
-	const RowOp op = b->chainOp; // (the lists come last: with what other groups have written a row's sum is complete)
+	const RowOp rowOp = op != nullptr ? *op : RowOp(); // (the lists come last: with what other groups have written a row's sum is complete)
 	auto go = [&](auto kernel) {
 		CLA_HIP(allow_full_lds((const void*) kernel));
 		hipLaunchKernelGGL(kernel, dim3(grid), dim3(RW_THREADS), lds, b->stream, (const int32_t*) meta, b->rowsTbl,
 			(const uint2*) (meta + b->rowsOff[0]), (const uint32_t*) (meta + b->rowsOff[1]), (const uint32_t*) b->dRowsData,
 			dU ? (const double*) b->dAllDict : (const double*) b->dTables, constRow, dOut, b->nRows, nQuarters, dNnz,
-			(const int32_t*) (meta + b->rowsColOff), dU, nnzNext, op);
+			(const int32_t*) (meta + b->rowsColOff), dU, nnzNext, rowOp);
 		return 0;
 	};
-	if(op.w != nullptr) rc = dU ? go(k_rmm_sdc_rows<false, true, true>) : accumulate ? go(k_rmm_sdc_rows<true, false, true>) : go(k_rmm_sdc_rows<false, false, true>);
+	if(rowOp.w != nullptr) rc = dU ? go(k_rmm_sdc_rows<false, true, true>) : accumulate ? go(k_rmm_sdc_rows<true, false, true>) : go(k_rmm_sdc_rows<false, false, true>);
 	else rc = dU ? go(k_rmm_sdc_rows<false, true, false>) : accumulate ? go(k_rmm_sdc_rows<true, false, false>) : go(k_rmm_sdc_rows<false, false, false>);
 	if(rc) return rc;
-	b->chainOpDone = op.w != nullptr;
 	CLA_HIP(hipGetLastError());
+	if(op != nullptr) op->done = true;
 	return 0;
 }
 

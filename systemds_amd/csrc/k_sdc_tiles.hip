@@ -566,14 +566,14 @@ int launch_lmm_sdc_tiles(cla_block* b, const double* dY, int p, double* dPre, in
 }
 
 // Returns 1 if the tile kernel cannot be used (caller falls back), 0 when done.
-int launch_rmm_sdc_tiles(cla_block* b, int q, int constRow, int accumulate, double* dOut, unsigned long long* dNnz) {
+int launch_rmm_sdc_tiles(cla_block* b, int q, int constRow, int accumulate, double* dOut, unsigned long long* dNnz, RowOp* op) {
 	int32_t *dList = nullptr, *dBinOff = nullptr;
 	int rc = sdc_plan(b, -1, &dList, &dBinOff);
 	if(rc) return rc;
 	struct { const std::vector<int32_t>&list, &binOff; } plan{b->sdcList, b->sdcBinOff};
 	if(plan.list.empty() || b->nRows == 0) return 1;
 	if(q == 1 && b->opt.sdcRows) { // one lane per row on row lists
-		const int r = launch_rmm_sdc_rows(b, constRow, accumulate, dOut, dNnz);
+		const int r = launch_rmm_sdc_rows(b, constRow, accumulate, dOut, dNnz, op);
 		if(r <= 0) return r;
 	}
 	if(q == 1 && b->opt.sdcLanes) { // one lane per group on lane-major lists

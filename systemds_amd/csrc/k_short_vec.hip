@@ -151,18 +151,19 @@ __global__ __launch_bounds__(256) void k_rmm_q1_short_rows(const uint8_t* __rest
 }
 
 // Returns 1 when the block is not eligible. `tables`: dict x v of all groups and, at constIdx, the constants' term.
-int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double* dOut, unsigned long long* dNnz) {
+int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double* dOut, unsigned long long* dNnz, RowOp* op) {
 	const int nG = (int) b->groups.size();
 	if(b->dArena == nullptr || b->arenaWidth != 2 || nG == 0 || b->nRows == 0 || b->maxVals > SV_BUF) return 1;
-	b->chainOpDone = b->chainOp.w != nullptr;
+	const RowOp rowOp = op != nullptr ? *op : RowOp();
 	// Up to 400,000 rows (where both take 29 us at 25 groups, 15 at 10) straight from global memory: 20,000 x 50 11 against 27 us,
 	// 200,000 x 50 18 against 28; beyond, the form with the tables in LDS: 700,000 x 50 31 against 43, 1,500,000 x 6 14 against 26.
 	if(b->nRows <= 400000) {
 		const unsigned grid = (unsigned) ((b->nRows + 255) / 256);
 		Prof pf(b, "k_rmm_q1_short_rows", grid, 256, 0, (double) b->nRows * (2 * nG + 8) + (double) b->totalVals * 8);
 		hipLaunchKernelGGL(k_rmm_q1_short_rows, dim3(grid), dim3(256), 0, b->stream, b->dArena, b->arenaStride, nG, b->dTblOff, tables,
-			constIdx, dOut, b->nRows, dNnz, b->chainOp);
+			constIdx, dOut, b->nRows, dNnz, rowOp);
 		CLA_HIP(hipGetLastError());
+		if(op != nullptr) op->done = true;
 		return 0;
 	}
 	const int gs = 2 * b->maxVals <= SV_BUF ? 2 : 1;
@@ -178,7 +179,7 @@ int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double
 	do {                                                                                                                     \
 		CLA_HIP(allow_full_lds((const void*) k_rmm_q1_short<NU>));                                                           \
 		hipLaunchKernelGGL(k_rmm_q1_short<NU>, dim3(grid), dim3(SV_THREADS), lds, b->stream, b->dArena, b->arenaStride, nG, gs, \
-			b->dTblOff, tables, constIdx, dOut, b->nRows, dNnz, b->chainOp);                                                             \
+			b->dTblOff, tables, constIdx, dOut, b->nRows, dNnz, rowOp);                                                               \
 	} while(0)
 	if(nu <= 1) SV_LAUNCH(1);
 	else if(nu == 2) SV_LAUNCH(2);
@@ -186,6 +187,7 @@ int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double
 	else SV_LAUNCH(4);
 #undef SV_LAUNCH
 	CLA_HIP(hipGetLastError());
+	if(op != nullptr) op->done = true;
 	return 0;
 }
 

@@ -1,0 +1,111 @@
+/*
+ * Test driver of libclahip.so's behaviour when host memory runs out inside a call: its own operator new fails the k-th
+ * allocation that the library makes during cla_mmchain, k = 0, 1, ... until the call gets through. Each failure has to
+ * come back as an error code, and the block has to answer the next plain X %*% v as if nothing had happened (the weights
+ * of the failed chain must not show in it).
+ *
+ * Prints "ALLOC-DRIVER OK" at the end; exit code 0 only then.
+ */
+#include <dlfcn.h>
+#include <stdint.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+#include <new>
+#include <vector>
+#include "cla_hip.h"
+
+static thread_local long allocLeft = -1; // allocations of the library until one fails; -1: none does
+static thread_local bool allocFailed = false;
+
+// Allocations of other libraries (the HIP runtime's among them) always succeed: the caller's code must lie in libclahip.so.
+static bool from_library(void* ret) {
+	Dl_info info;
+	return dladdr(ret, &info) && info.dli_fname && strstr(info.dli_fname, "libclahip");
+}
+
+__attribute__((noinline)) void* operator new(size_t n) {
+	if(allocLeft >= 0 && from_library(__builtin_return_address(0)) && allocLeft-- == 0) {
+		allocFailed = true;
+		throw std::bad_alloc();
+	}
+	if(void* p = malloc(n ? n : 1)) return p;
+	throw std::bad_alloc();
+}
+__attribute__((noinline)) void operator delete(void* p) noexcept { free(p); }
+__attribute__((noinline)) void operator delete(void* p, size_t) noexcept { free(p); }
+
+static const int64_t N = 1031;
+enum { COLS = 3 };
+
+// kind 0: byte codes, 1: two-byte codes, 2: offset lists of every third row
+static cla_handle make_block(int kind, std::vector<double>& X) {
+	cla_handle h = cla_block_create(N, COLS);
+	X.assign((size_t) N * COLS, 0.0);
+	for(int32_t c = 0; h && c < COLS; c++) {
+		double dict[7];
+		for(int k = 0; k < 7; k++) dict[k] = 0.5 + k + 10 * c;
+		int rc;
+		if(kind == 2) {
+			std::vector<uint8_t> codes, deltas;
+			for(int64_t r = c; r < N; r += 3) {
+				codes.push_back((uint8_t) (r % 7));
+				if(r > c) deltas.push_back(3);
+				X[(size_t) r * COLS + c] = dict[r % 7];
+			}
+			rc = cla_block_add_sdc(h, &c, 1, dict, 7, nullptr, codes.data(), 1, deltas.data(), 1, (int32_t) deltas.size(), c,
+				(int32_t) (c + 3 * (int64_t) (codes.size() - 1)), (int32_t) codes.size());
+		}
+		else {
+			std::vector<uint8_t> bytes;
+			std::vector<uint16_t> words;
+			for(int64_t r = 0; r < N; r++) {
+				const int k = (int) ((r * 5 + c) % 7);
+				bytes.push_back((uint8_t) k);
+				words.push_back((uint16_t) k);
+				X[(size_t) r * COLS + c] = dict[k];
+			}
+			rc = cla_block_add_ddc(h, &c, 1, dict, 7, kind == 0 ? (const void*) bytes.data() : (const void*) words.data(), kind + 1);
+		}
+		if(rc < 0) { fprintf(stderr, "add: %s\n", cla_last_error()); return nullptr; }
+	}
+	if(!h || cla_block_finalize(h) < 0) { fprintf(stderr, "block: %s\n", cla_last_error()); return nullptr; }
+	return h;
+}
+
+int main() {
+	if(cla_init(0) < 0) { fprintf(stderr, "cla_init: %s\n", cla_last_error()); return 2; }
+	int fails = 0, thrown = 0;
+	for(int kind = 0; kind < 3; kind++)
+		for(int ctype = 1; ctype <= 2; ctype++)
+			for(long k = 0;; k++) {
+				std::vector<double> X, w((size_t) N), out((size_t) N);
+				cla_handle h = make_block(kind, X);
+				if(!h) return 2;
+				if(kind == 2 && cla_block_prepare(h, CLA_PRODUCT_RMM | CLA_PRODUCT_LMM, 1, 1) < 0) return 2; // (the lists' copies are no part of this)
+				const double v[COLS] = {1.0, 0.25, -2.0};
+				for(int64_t r = 0; r < N; r++) w[(size_t) r] = 3.0 + (double) (r % 5);
+				double chain[COLS];
+				allocFailed = false;
+				allocLeft = k;
+				const int64_t rc = cla_mmchain(h, v, w.data(), ctype, chain);
+				allocLeft = -1;
+				if(allocFailed) thrown++;
+				if(allocFailed && rc >= 0) { printf("kind %d, allocation %ld failed without an error\n", kind, k); fails++; }
+				if(!allocFailed && rc < 0) { printf("kind %d: %s\n", kind, cla_last_error()); fails++; }
+				if(cla_rmm(h, v, 1, out.data()) < 0) { printf("kind %d: rmm: %s\n", kind, cla_last_error()); fails++; }
+				int64_t bad = 0;
+				for(int64_t r = 0; r < N; r++) { // (small multiples of 1/8: exact)
+					double s = 0;
+					for(int c = 0; c < COLS; c++) s += X[(size_t) r * COLS + c] * v[c];
+					bad += out[(size_t) r] != s;
+				}
+				if(bad) { printf("kind %d, type %d, allocation %ld: %lld rows of the next X %%*%% v are wrong\n", kind, ctype, k, (long long) bad); fails++; }
+				cla_block_free(h);
+				if(!allocFailed) break;
+			}
+	printf("%d failed allocations\n", thrown);
+	if(fails || thrown < 4) { printf("FAIL\n"); return 1; }
+	printf("ALLOC-DRIVER OK\n");
+	return 0;
+}

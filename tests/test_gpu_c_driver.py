@@ -9,6 +9,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+ALLOC_DRIVER = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cla_alloc_driver")
 DRIVER = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cla_c_driver")
 
 
@@ -20,3 +21,13 @@ def test_c_driver(n_rows):
     print(r.stderr)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "C-DRIVER OK" in r.stdout and "FAIL" not in r.stdout
+
+
+def test_allocation_failures_leave_no_state():
+    """Host memory runs out at every place inside cla_mmchain in turn: an error code each time, and no trace of the chain's
+    weights in the next X %*% v of the block."""
+    assert os.path.exists(ALLOC_DRIVER), "tests/cla_alloc_driver not built: run __graft_entry__.build()"
+    r = subprocess.run([ALLOC_DRIVER], capture_output=True, text=True, timeout=110)
+    print(r.stdout)
+    print(r.stderr)
+    assert r.returncode == 0 and "ALLOC-DRIVER OK" in r.stdout, r.stdout + r.stderr
