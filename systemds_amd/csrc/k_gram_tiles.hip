@@ -1,7 +1,7 @@
 // t(X) %*% X of a block whose groups are all DDC with one code width (one or two bytes), 13 to 128 columns, as the Gram
 // matrix of the decoded rows: every row is decoded once, into a tile of doubles in LDS that all waves multiply from.
 //
-// A workgroup of 8 waves (one per CU) takes a contiguous share of the rows in tiles of R = 32 m rows, two tile buffers in
+// A workgroup of 8 waves (one per CU or two, gt_blocks_per_cu) takes a contiguous share of the rows in tiles of R = 32 m rows, two tile buffers in
 // LDS. Decoding is dealt by (16 columns, 32 rows): lane (k, c), k = lane / 16, c = lane % 16, holds 8 consecutive codes of
 // column c, looks them up (in LDS where the column block's dictionaries fit beside the tiles, [code][16 columns], else
 // straight in global memory) and writes the values to its rows of the tile. Multiplying: lane (k, c) reads X[row 4 s + k, 16 b + c],
@@ -338,7 +338,20 @@ struct GtPlan {
 	int64_t bytes = 0;
 	int nf = 0, nn = 0, kind = 0;
 	size_t lds = 0;
+	int perCU = 1;    // blocks per CU, one after the other where LDS holds one
 };
+
+// Blocks per CU. A wave adds up its part of the block's rows in one chain, whose error grows with its length (like terms drift). Where
+// k_tsmm_decode ran twice as many waves' sums side by side, two blocks share a CU's rows: diagonal cells of 4,000,000 rows of 7 values,
+// rms relative error 20 columns 1.2e-14 -> 7.4e-15 (k_tsmm_decode 7.1e-15), 38 1.3e-14 -> 7.6e-15 (7.6e-15), 100 2.3e-14 -> 1.2e-14
+// (1.0e-14); column pairs of 300 tuples, 20 columns 4.1e-15 -> 2.0e-15 (2.1e-15). A second block costs 8 - 23 us where it starts behind the first
+// (2,000,003 rows of 256 values: 20 columns 73 -> 81 us, 100 columns 438 -> 461; 10,000,000 x 20 of 7 values, side by side: 280 -> 239).
+static int gt_blocks_per_cu(int nf, int nn, int kind, int nTiles) {
+	if(nTiles < 16 * g_numCU) return 1; // (short chains: below 1e-15 with one block)
+	if(nf > 5) return 2;
+	const int ncb = nf + (nn ? 1 : 0);
+	return kind == GT_PAIR ? (nf == 1 && nn < 2) || ncb == 3 ? 2 : 1 : ncb <= 3 ? 2 : 1;
+}
 
 static int gt_build_plan(cla_block* b, GtPlan& P) {
 	P.rc = 1;
@@ -421,6 +434,7 @@ static int gt_build_plan(cla_block* b, GtPlan& P) {
 	A.dict = consts ? (const double*) (d + colBytes + imgBytes) : b->dAllDict;
 	A.nRows = b->nRows;
 	A.nTiles = (int) ((b->nRows + 32 * gt_m(ncb, P.kind) - 1) / (32 * gt_m(ncb, P.kind)));
+	P.perCU = gt_blocks_per_cu(P.nf, P.nn, P.kind, A.nTiles);
 	A.nLds = nLds; A.imgV = imgV; A.nCols = n; A.nGroups = (int) b->groups.size();
 	P.rc = 0;
 	return 0;
@@ -460,7 +474,7 @@ int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz) {
 		if(rc) return rc;
 		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
-	const unsigned grid = (unsigned) std::min(A.nTiles, g_numCU);
+	const unsigned grid = (unsigned) std::min(A.nTiles, g_numCU * P.perCU);
 	Prof pf(b, "k_gram_tiles", grid, GT_THREADS, (long) P.lds, (double) b->device_bytes_cached);
 #define GT_CASE(NF) \
 	case NF: return P.nn == 0 ? gt_launch<NF, 0>(b, P, A, grid) : P.nn == 1 ? gt_launch<NF, 1>(b, P, A, grid) : gt_launch<NF, 2>(b, P, A, grid);
