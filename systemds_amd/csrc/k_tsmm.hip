@@ -296,27 +296,28 @@ __global__ __launch_bounds__(256) void k_tsmm_self(const DGroup* __restrict__ gr
 	if(G.type == G_UNC) return;
 	const int32_t* counts = countsAll + G.tblOff;
 	const int nC = G.nColG, tid = threadIdx.x;
-	for(int i = 0; i < nC; i++) {
-		for(int j = i; j <= nC; j++) { // j == nC: column sum of column i
-			double s = 0.0;
-			for(int k = tid; k < G.nVals; k += 256) {
-				const double v = G.dict[(size_t) k * nC + i] * (double) counts[k];
-				s += j < nC ? v * G.dict[(size_t) k * nC + j] : v;
-			}
-			s = wave_sum_f64(s);
-			if((tid & 63) == 0) red[tid >> 6] = s;
-			__syncthreads();
-			if(tid == 0) {
-				const double tot = red[0] + red[1] + red[2] + red[3];
-				if(j < nC) {
-					const int r = G.cols[i], c = G.cols[j];
-					unsafeAtomicAdd(&out[(size_t) min(r, c) * nCols + max(r, c)], tot);
-				}
-				else
-					unsafeAtomicAdd(&colSum[G.cols[i]], tot);
-			}
-			__syncthreads();
+	int i = 0, j = blockIdx.x; // cell (i, j), j = i .. nC of row i; j == nC: column sum of column i
+	for(;; j += gridDim.x) {
+		while(i < nC && j > nC) { j += i - nC; i++; } // (the next row's cells start at i + 1)
+		if(i >= nC) return;
+		double s = 0.0;
+		for(int k = tid; k < G.nVals; k += 256) {
+			const double v = G.dict[(size_t) k * nC + i] * (double) counts[k];
+			s += j < nC ? v * G.dict[(size_t) k * nC + j] : v;
 		}
+		s = wave_sum_f64(s);
+		if((tid & 63) == 0) red[tid >> 6] = s;
+		__syncthreads();
+		if(tid == 0) {
+			const double tot = red[0] + red[1] + red[2] + red[3];
+			if(j < nC) {
+				const int r = G.cols[i], c = G.cols[j];
+				unsafeAtomicAdd(&out[(size_t) min(r, c) * nCols + max(r, c)], tot);
+			}
+			else
+				unsafeAtomicAdd(&colSum[G.cols[i]], tot);
+		}
+		__syncthreads();
 	}
 }
 
@@ -644,8 +645,12 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	// accumulator kept with the block, and the last one to finish writes the output (both triangles) and the count of
 	// its non-zeros and clears the accumulator again: no fill in front of the kernel, no kernel behind it.
 	bool decodeTried = false;
-	// All-DDC blocks of 13 to 128 columns: every row decoded once (k_gram_tiles), whatever the number of groups
-	if(!forcePairs && split == 0 && b->crossBlocks == 0 && nRows > 0 && b->opt.tsmmMfma && (nCols <= 64 || b->opt.tsmmChunks)) {
+	// All-DDC blocks of 13 to 128 columns: every row decoded once (k_gram_tiles), from two groups on. A single group needs no row at all:
+	// its cells are exact counts times dictionary products (22 us at 20 columns, 28 at 64, 56 at 128, on 40,000,000 rows as on 200,003;
+	// decoded, 10,000,000 x 20 take 290 us). Several groups need a pass over the rows per pair: 10,000,000 rows, 2 groups of 8 columns
+	// (256 tuples) 442 us against 157 decoded, 3 of 8 806 / 317, 4 of 4 552 / 159, 4 of 8 1573 / 354, 2 of 50 4012 / 1947; the two meet
+	// only for two narrow groups on 40,000,000 rows (2 of 7 columns 537 / 578, 2 of 8 1209 / 587, 3 of 5 866 / 574).
+	if(nPairs > 0 && !forcePairs && split == 0 && b->crossBlocks == 0 && nRows > 0 && b->opt.tsmmMfma && (nCols <= 64 || b->opt.tsmmChunks)) {
 		if(!b->opt.tsmmOneKernel && (rc = clear())) return rc;
 		rc = nCols <= 64 && dense ? 1 : launch_gram_tiles(b, dOut, b->opt.tsmmOneKernel ? dNnz : nullptr);
 		if(rc < 0) return rc;
@@ -731,8 +736,13 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	CLA_HIP(hipMemsetAsync(dColSum, 0, sizeof(double) * (size_t) nCols, st));
 	if((rc = ensure_counts(b))) return rc;
 	if(nG > 0) {
-		Prof pf(b, "k_tsmm_self", nG, 256, 0, 0);
-		hipLaunchKernelGGL(k_tsmm_self, dim3(1, nG), dim3(256), 0, st, b->dGroups, b->dCountsAll, dOut, nCols, dColSum);
+		// a block per cell, several cells in turn where there are many (one block per group took 0.8 us a cell: 64 columns 1.7 ms)
+		int maxCols = 1;
+		for(auto& g : b->groups) maxCols = std::max(maxCols, g.d.nColG);
+		const int64_t cells = (int64_t) maxCols * (maxCols + 3) / 2;
+		const dim3 grid((unsigned) std::min<int64_t>(cells, std::max(1, 8 * g_numCU / nG)), (unsigned) nG);
+		Prof pf(b, "k_tsmm_self", (long) grid.x * nG, 256, 0, 0);
+		hipLaunchKernelGGL(k_tsmm_self, grid, dim3(256), 0, st, b->dGroups, b->dCountsAll, dOut, nCols, dColSum);
 	}
 	const int nTiles = (int) ((nRows + TT - 1) / TT);
 	// Pairs of DDC groups with one or two columns each, equal code width and both dictionaries

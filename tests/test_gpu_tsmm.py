@@ -243,3 +243,27 @@ def test_decoded_gram_is_one_kernel_per_call(cla, ora, shape):
         blk.close()
     assert_matches_truth(first, D.T, D, what=f"{shape}: one kernel per call")
     assert nnz == np.count_nonzero(first)
+
+
+@pytest.mark.parametrize("n_cols,n_vals,dtype", [(13, 100, np.uint8), (20, 5, np.uint8), (64, 100, np.uint8), (100, 300, np.uint16), (128, 20, np.uint8)])
+def test_one_group_of_many_columns_is_counts_times_dictionary(cla, n_cols, n_vals, dtype):
+    """A block of one dictionary group is not decoded: counts times products of dictionary values, to a few units in the last
+    place of the exact sums (256 partial sums of n_vals / 256 terms, added up in a tree of 6 levels and one of 4 terms, products and
+    counts rounded: 14 + n_vals / 256 roundings at most)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_cols)
+    n_rows = 1_000_003
+    codes = np.minimum(rng.integers(0, n_vals, n_rows), rng.integers(0, n_vals, n_rows)).astype(dtype)
+    d = rng.standard_normal((n_vals, n_cols))
+    perm = np.arange(n_cols, dtype=np.int32)[::-1].copy()
+    blk = cla.build_block(n_rows, n_cols, [synth.GroupSpec("ddc", perm, d, codes)])
+    out, nnz = blk.tsmm()
+    names = [k["name"] for k in blk.stats()["kernels"]]
+    blk.close()
+    assert names == ["k_tsmm_self", "k_tsmm_finish"], names
+    n = np.bincount(codes, minlength=n_vals).astype(np.longdouble)
+    L = d.astype(np.longdouble)
+    exact, scale = (L * n[:, None]).T @ L, (np.abs(L) * n[:, None]).T @ np.abs(L)
+    got = out[np.ix_(perm, perm)]
+    assert np.array_equal(out, out.T) and nnz == np.count_nonzero(out)
+    assert np.all(np.abs(got - exact) <= (14 + n_vals / 256) * 2.0 ** -53 * scale)
