@@ -4,9 +4,10 @@
 // A wave takes 64 rows of X and up to 4 column blocks of 16 groups. Lane (k, c), k = lane / 16, c = lane % 16, reads 16
 // codes of group c of a column block (rows 16 k .. 16 k + 15 of the 64) with one 16-byte load and looks them up in the
 // column block's dictionaries in LDS, one row of each quarter per step: the looked-up values are the B operand (4 rows x 16
-// columns) of the matrix instruction as they come, and the A operand is Y at the same rows, read straight from global
-// memory, 8 consecutive values per lane. The sums stay in registers over all rows of the block: one LDS add per wave and
-// cell at the end, where k_lmm_u8_vec adds once per thread and group for every row of Y.
+// columns) of the matrix instruction as they come, and the A operand is Y at the same rows. The sums stay in registers over
+// all rows of the block: one LDS add per wave and cell at the end, where k_lmm_u8_vec adds once per thread and group.
+// A unit's 64 rows are a chain of additions of their own (one chain over a wave's share drifts where the terms are alike: a row
+// of like values times columns of 7 values, 4,000,000 rows, 1.7e-14 relative error instead of 5e-16; 0.8 % of the time).
 // Up to 12 rows of Y go through v_mfma_f64_4x4x4 (four 4 x 4 x 4 products, 4 rows of Y each: 17 - 19 cycles per 4 rows of Y),
 // more through v_mfma_f64_16x16x4 (70 cycles for 16).
 //
@@ -89,11 +90,20 @@ __device__ __forceinline__ void lmm_mfma_rows(double* smem, double* yLds, const 
 		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 	};
 
-	double acc[NCB][NI]; // [.][0 .. 3]: the four values of the 16 x 16 form
+	double acc[NCB][NI], tot[NCB][NI]; // of a unit's rows, of the units in front of it; [.][0 .. 3]: the four values of the 16 x 16 form
 #pragma unroll
 	for(int cb = 0; cb < NCB; cb++)
 #pragma unroll
-		for(int i = 0; i < NI; i++) acc[cb][i] = 0.0;
+		for(int i = 0; i < NI; i++) acc[cb][i] = tot[cb][i] = 0.0;
+	auto next_unit = [&]() {
+#pragma unroll
+		for(int cb = 0; cb < NCB; cb++)
+#pragma unroll
+			for(int i = 0; i < NI; i++) {
+				tot[cb][i] += acc[cb][i];
+				acc[cb][i] = 0.0;
+			}
+	};
 
 	const char* tb = (const char*) smem + c * 8;
 	const int cbBytes = nVals * 128;
@@ -162,6 +172,7 @@ __device__ __forceinline__ void lmm_mfma_rows(double* smem, double* yLds, const 
 		work(codes[0], integral_constant<int, 1>());
 #pragma unroll
 		for(int cb = 0; cb < NCB; cb++) codes[0][cb] = codes[1][cb];
+		next_unit();
 	}
 	// (outside the loop: a load under a condition makes the compiler wait for all loads in flight)
 	if(tail && wave == NW - 1) {
@@ -173,6 +184,7 @@ __device__ __forceinline__ void lmm_mfma_rows(double* smem, double* yLds, const 
 		work(codes[0], integral_constant<int, 0>());
 		put_y(1);
 		work(codes[0], integral_constant<int, 1>());
+		next_unit();
 	}
 
 	__syncthreads();
@@ -181,7 +193,7 @@ __device__ __forceinline__ void lmm_mfma_rows(double* smem, double* yLds, const 
 #pragma unroll
 	for(int cb = 0; cb < NCB; cb++)
 #pragma unroll
-		for(int i = 0; i < NI; i++) unsafeAtomicAdd(&smem[(cb * NI + i) * 64 + lane], acc[cb][i]);
+		for(int i = 0; i < NI; i++) unsafeAtomicAdd(&smem[(cb * NI + i) * 64 + lane], tot[cb][i]);
 	__syncthreads();
 }
 
@@ -219,7 +231,7 @@ __global__ __launch_bounds__(LM_THREADS, 2) void k_lmm_u8_dot(const uint8_t* __r
 // Returns 1 when the block is not eligible, 0 when the groups' contributions have been added to dOut.
 int launch_lmm_u8_dot(cla_block* b, const double* dY, int p, double* dOut) {
 	const int nG = (int) b->groups.size();
-	if(b->dDictPad == nullptr || b->dictNonFinite || (b->opt.lmmDisable & 1)) return 1; // (non-finite: see launch_lmm_u8_dot)
+	if(b->dDictPad == nullptr || b->dictNonFinite || (b->opt.lmmDisable & 1)) return 1; // (non-finite dictionary values: the reference sums Y per tuple first, see launch_lmm_joint)
 	const int nCb = (nG + 15) / 16, nPass = (p + 15) / 16;
 	const int nV = b->maxVals;
 	const int ni = p > 12 ? 4 : (p + 3) / 4; // (also the last rows of a larger p: the passes share one launch)
