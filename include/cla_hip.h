@@ -107,7 +107,9 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  * same product: the reference likewise holds several variants per product, e.g. the pre-aggregating and
  * the decompressing right multiply, CG/ColGroupDDC.java:647-692). The defaults are the tuned dispatch.
  *   tsmm_route      0 cost model, 1 one pass per pair of groups, 2 decoded Gram matrix
- *   tsmm_chunks     1 / 0: more than 64 columns as pairs of column chunks
+ *   tsmm_chunks     1 / 0: more than 64 columns decoded: all-DDC blocks of up to 128 at once, others as pairs of column chunks
+ *   tsmm_direct     1 / 0: blocks of a few streamed columns next to run-length columns on the vector unit, both t(X) %*% X and
+ *                   Y %*% X (0: both on the decoded tiles)
  *   tsmm_wide_dense 0 / 1, tsmm_mfma 1 / 0, tsmm_pair_dot 1 / 0
  *   tsmm_narrow     1 / 0: decoded Gram matrix with a last column block of at most 4 columns on the 4x4x4 matrix instruction
  *   expand_streams  1 / 0: one code per row for small RLE / SDCZeros groups (set before the first multiply)
@@ -120,11 +122,11 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *   sdc_lanes       1 / 0: SDCZeros mat-vecs on lane-major copies of the lists, one lane per group
  *   sdc_rows        1 / 0: SDCZeros X %*% v on row lists (the lists transposed), one lane per row
  *   lmm_joint       1 / 0: Y %*% X (16 rows of Y per pass) on a block that is not mostly offset lists in passes over the decoded
- *                   rows on the matrix cores; blocks of more than 64 columns, or whose code tiles exceed LDS together, go chunk of
- *                   columns by chunk (sub-blocks kept with the block); single-column byte-code blocks only from 13 rows of Y
- *                   on and up to 32768 rows (the kernel reports non-finite values of Y and the host looks, i.e. waits for the stream once per call;
+ *                   rows, on the vector unit (see tsmm_direct) or on the matrix cores; blocks of more than 64 columns, or whose code tiles exceed LDS together, go chunk of
+ *                   columns by chunk (sub-blocks kept with the block); not single-column byte-code blocks, except with bit 0 of
+ *                   lmm_disable (the kernel reports non-finite values of Y and the host looks, i.e. waits for the stream once per call;
  *                   such a Y takes the bin kernels)
- *   tsmm_one_kernel 1 / 0: t(X) %*% X of a whole block of at most 64 columns on the decoded Gram kernels as the call's only
+ *   tsmm_one_kernel 1 / 0: t(X) %*% X of a whole block of at most 64 columns (all-DDC: 128) on the decoded Gram kernels as the call's only
  *                   kernel (its blocks add into an accumulator kept with the block, nCols x nCols doubles; the last block
  *                   to finish writes the output, mirrored, and the count of its non-zeros and clears the accumulator)
  *                   instead of a fill of the output in front of the kernel and a mirror-and-count kernel behind it

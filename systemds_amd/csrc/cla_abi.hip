@@ -1516,9 +1516,9 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 			}
 	}
 	if(nOther == 0 || nLists > nOther) return 1;
-	// Single-column byte codes have kernels of their own (k_lmm_u8_dot, k_lmm_u8_vec), faster at every size. What keeps 13 rows
-	// of Y and more on few rows here is that this form is covered on byte codes there (30,011 x 100 by 14: 66 against 21 us).
-	if(dotForm && !(b->opt.lmmDisable & 1) && (p < 13 || b->nRows > 32768)) return 1;
+	// Single-column byte codes have kernels of their own (k_lmm_u8_dot, k_lmm_u8_vec), faster at every size and number of rows of Y
+	// (20,011 rows by 20 of Y, 1 column 14 against 43 us, 60 of 256 values 27 against 117, 30,011 x 100 by 14 21 against 66).
+	if(dotForm && !(b->opt.lmmDisable & 1)) return 1;
 	if(p == 1 && lmm_q1_short_groups(b) > 0) return 1; // k_lmm_q1_short
 	if(b->nCols > 64) return launch_lmm_chunked(b, dY, p, dOut, dNnz);
 	hipStream_t st = b->stream;
