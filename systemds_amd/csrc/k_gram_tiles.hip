@@ -33,7 +33,7 @@ typedef double f64x4_gt __attribute__((ext_vector_type(4)));
 // a decoded column
 struct GtCol {
 	int32_t dictOff;  // bytes from the dictionary base to its first value
-	int32_t stride;   // bytes from one code's value to the next one's
+	int32_t stride;   // bytes from one code's value to the next one's (0: a column that only carries a constant)
 	int32_t group;    // code stream
 	int32_t col;      // column of the block (-1: padding)
 };
@@ -50,6 +50,7 @@ struct GtArgs {
 	double* out;
 	unsigned* done;          // nullptr: no tail (acc is the caller's output)
 	unsigned long long* nnz;
+	int skipOwn;             // cells inside a group and of columns without one come from the code counts (k_tsmm_self)
 };
 
 // How the codes are dealt: one-byte codes, two-byte codes, two-byte codes of column pairs (every group two columns)
@@ -310,18 +311,21 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 		}
 		__syncthreads();
 	}
-	auto add = [&](int ca, int cb, double d) {
+	auto add = [&](int ia, int ib, double d) {
+		const GtCol Ca = A.cols[ia], Cb = A.cols[ib];
+		if(A.skipOwn && (Ca.group == Cb.group || Ca.stride == 0 || Cb.stride == 0)) return;
+		const int ca = Ca.col, cb = Cb.col;
 		if(ca >= 0 && cb >= 0 && d != 0.0) unsafeAtomicAdd(&A.acc[(size_t) min(ca, cb) * A.nCols + max(ca, cb)], d);
 	};
 	for(int i = tid; i < T * 256; i += GT_THREADS) {
 		int t = i >> 8, p = 0;
 		while(t >= NF - p) { t -= NF - p; p++; }
 		const int q = p + t, r = ((i >> 6) & 3) * 4 + ((i & 63) >> 4), cc = i & 15;
-		if(p != q || r <= cc) add(A.cols[16 * p + r].col, A.cols[16 * q + cc].col, sum[i]);
+		if(p != q || r <= cc) add(16 * p + r, 16 * q + cc, sum[i]);
 	}
 	for(int i = tid; i < NN * NCB * 64; i += GT_THREADS) {
 		const int g = i / (NCB * 64), b = i / 64 % NCB, r = 4 * g + ((i & 63) >> 4), cc = i & 15;
-		if(b < NF || r <= cc) add(A.cols[16 * NF + r].col, A.cols[16 * b + cc].col, sum[T * 256 + i]);
+		if(b < NF || r <= cc) add(16 * NF + r, 16 * b + cc, sum[T * 256 + i]);
 	}
 	if(A.done != nullptr) {
 		__syncthreads();
@@ -339,6 +343,8 @@ struct GtPlan {
 	int nf = 0, nn = 0, kind = 0;
 	size_t lds = 0;
 	int perCU = 1;    // blocks per CU, one after the other where LDS holds one
+	const int32_t* constCols = nullptr; // columns without a group whose constant is not zero
+	int nConst = 0;
 };
 
 // Blocks per CU. A wave adds up its part of the block's rows in one chain, whose error grows with its length (like terms drift). Where
@@ -418,10 +424,15 @@ static int gt_build_plan(cla_block* b, GtPlan& P) {
 			img[((size_t) (s / 16) * imgV + kk) * 16 + s % 16] = (src[s] ? src[s][(size_t) kk * (C.stride / 8)] : 0.0) + add;
 	}
 	const size_t colBytes = cols.size() * sizeof(GtCol), imgBytes = img.size() * 8, dictBytes = consts ? dict.size() * 8 : 0;
-	std::vector<uint8_t> all(colBytes + imgBytes + dictBytes + 16, 0);
+	std::vector<int32_t> constCols;
+	for(int col = 0; col < n; col++)
+		if(groupOf[col] < 0 && b->constV[col] != 0.0) constCols.push_back(col);
+	const size_t constBytes = constCols.size() * sizeof(int32_t);
+	std::vector<uint8_t> all(colBytes + imgBytes + dictBytes + constBytes + 16, 0);
 	std::memcpy(all.data(), cols.data(), colBytes);
 	if(imgBytes) std::memcpy(all.data() + colBytes, img.data(), imgBytes);
 	if(dictBytes) std::memcpy(all.data() + colBytes + imgBytes, dict.data(), dictBytes);
+	if(constBytes) std::memcpy(all.data() + colBytes + imgBytes + dictBytes, constCols.data(), constBytes);
 	uint8_t* d = nullptr;
 	CLA_HIP(hipMalloc((void**) &d, all.size()));
 	P.dImg = d;
@@ -432,6 +443,8 @@ static int gt_build_plan(cla_block* b, GtPlan& P) {
 	A.cols = (const GtCol*) d;
 	A.img = (const double*) (d + colBytes);
 	A.dict = consts ? (const double*) (d + colBytes + imgBytes) : b->dAllDict;
+	P.constCols = (const int32_t*) (d + colBytes + imgBytes + dictBytes);
+	P.nConst = (int) constCols.size();
 	A.nRows = b->nRows;
 	A.nTiles = (int) ((b->nRows + 32 * gt_m(ncb, P.kind) - 1) / (32 * gt_m(ncb, P.kind)));
 	P.perCU = gt_blocks_per_cu(P.nf, P.nn, P.kind, A.nTiles);
@@ -456,9 +469,23 @@ static int gt_launch(cla_block* b, const GtPlan& P, const GtArgs& A, unsigned gr
 	return 0;
 }
 
+static int gt_launch_shape(cla_block* b, const GtPlan& P, const GtArgs& A, unsigned grid) {
+	Prof pf(b, "k_gram_tiles", grid, GT_THREADS, (long) P.lds, (double) b->device_bytes_cached);
+#define GT_CASE(NF) \
+	case NF: return P.nn == 0 ? gt_launch<NF, 0>(b, P, A, grid) : P.nn == 1 ? gt_launch<NF, 1>(b, P, A, grid) : gt_launch<NF, 2>(b, P, A, grid);
+	switch(P.nf) {
+		case 1: return P.nn == 0 ? gt_launch<1, 0>(b, P, A, grid) : P.nn == 1 ? gt_launch<1, 1>(b, P, A, grid) : gt_launch<1, 2>(b, P, A, grid);
+		GT_CASE(2) GT_CASE(3) GT_CASE(4) GT_CASE(5) GT_CASE(6) GT_CASE(7)
+		case 8: return gt_launch<8, 0>(b, P, A, grid);
+	}
+#undef GT_CASE
+	return 1;
+}
+
 // Like launch_tsmm_decode: dNnz != nullptr: the call's only kernel, which writes dOut whole; else dOut (zeroed) gets the upper
-// triangle. Returns 1 when the block is not of this kernel's shape.
-int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz) {
+// triangle. ownByCounts: cells inside a group are exact code counts times dictionary products, as on the way by pairs of groups (one
+// more kernel in front). Returns 1 when the block is not of this kernel's shape.
+int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz, bool ownByCounts) {
 	if(b->gtPlan == nullptr) {
 		b->gtPlan = new GtPlan();
 		const int rc = gt_build_plan(b, *b->gtPlan);
@@ -474,17 +501,14 @@ int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz) {
 		if(rc) return rc;
 		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
+	A.skipOwn = ownByCounts;
+	if(ownByCounts)
+		if(const int rc = launch_tsmm_self(b, A.acc, nullptr, b->hasConst ? b->dConstV : nullptr, P.constCols, P.nConst)) return rc;
 	const unsigned grid = (unsigned) std::min(A.nTiles, g_numCU * P.perCU);
-	Prof pf(b, "k_gram_tiles", grid, GT_THREADS, (long) P.lds, (double) b->device_bytes_cached);
-#define GT_CASE(NF) \
-	case NF: return P.nn == 0 ? gt_launch<NF, 0>(b, P, A, grid) : P.nn == 1 ? gt_launch<NF, 1>(b, P, A, grid) : gt_launch<NF, 2>(b, P, A, grid);
-	switch(P.nf) {
-		case 1: return P.nn == 0 ? gt_launch<1, 0>(b, P, A, grid) : P.nn == 1 ? gt_launch<1, 1>(b, P, A, grid) : gt_launch<1, 2>(b, P, A, grid);
-		GT_CASE(2) GT_CASE(3) GT_CASE(4) GT_CASE(5) GT_CASE(6) GT_CASE(7)
-		case 8: return gt_launch<8, 0>(b, P, A, grid);
-	}
-#undef GT_CASE
-	return 1;
+	const int rc = gt_launch_shape(b, P, A, grid);
+	if(rc && ownByCounts && dNnz != nullptr) // (nothing behind the counts' kernel clears the accumulator then)
+		(void) hipMemsetAsync(b->dGramAcc, 0, (size_t) A.nCols * A.nCols * sizeof(double), b->stream);
+	return rc;
 }
 
 } // namespace cla

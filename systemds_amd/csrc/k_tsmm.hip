@@ -289,36 +289,62 @@ static void launch_pair_dot_cw(int nct, int ncs, dim3 grid, size_t lds, hipStrea
 
 // Self term (AColGroupCompressed.tsmmDense) + column sums of the group:
 // out[cols[i], cols[j]] += sum_k cnt[k] d[k,i] d[k,j], j >= i; colSum[cols[j]] += sum_k cnt[k] d[k,j]
-__global__ __launch_bounds__(256) void k_tsmm_self(const DGroup* __restrict__ groups, const int32_t* __restrict__ countsAll,
-	double* __restrict__ out, int nCols, double* __restrict__ colSum) {
+// A block per cell and group, several cells in turn where there are many (one block per group took 0.8 us a cell: 64 columns 1.7 ms).
+// constV != nullptr: of the decoded columns, constants added, the cells of columns that only carry a constant (constCols) among them
+// (blocks nGroups of grid.y those of two such columns); then there is no colSum.
+__global__ __launch_bounds__(256) void k_tsmm_self(const DGroup* __restrict__ groups, int nGroups, const int32_t* __restrict__ countsAll,
+	double* __restrict__ out, int nCols, double* __restrict__ colSum, const double* __restrict__ constV, const int32_t* __restrict__ constCols,
+	int nConst, double nRows) {
 	__shared__ double red[4];
+	const int tid = threadIdx.x;
+	auto add = [&](int r, int c, double v) { unsafeAtomicAdd(&out[(size_t) min(r, c) * nCols + max(r, c)], v); };
+	if((int) blockIdx.y == nGroups) {
+		for(int k = blockIdx.x * 256 + tid; k < nConst * nConst; k += gridDim.x * 256) {
+			const int r = constCols[k / nConst], c = constCols[k % nConst];
+			if(r <= c) add(r, c, constV[r] * constV[c] * nRows);
+		}
+		return;
+	}
 	const DGroup G = dgroup(groups + (blockIdx.y));
 	if(G.type == G_UNC) return;
 	const int32_t* counts = countsAll + G.tblOff;
-	const int nC = G.nColG, tid = threadIdx.x;
+	const int nC = G.nColG;
 	int i = 0, j = blockIdx.x; // cell (i, j), j = i .. nC of row i; j == nC: column sum of column i
 	for(;; j += gridDim.x) {
 		while(i < nC && j > nC) { j += i - nC; i++; } // (the next row's cells start at i + 1)
 		if(i >= nC) return;
+		const double ci = constV ? constV[G.cols[i]] : 0.0, cj = constV && j < nC ? constV[G.cols[j]] : 0.0;
 		double s = 0.0;
 		for(int k = tid; k < G.nVals; k += 256) {
-			const double v = G.dict[(size_t) k * nC + i] * (double) counts[k];
-			s += j < nC ? v * G.dict[(size_t) k * nC + j] : v;
+			const double v = (G.dict[(size_t) k * nC + i] + ci) * (double) counts[k];
+			s += j < nC ? v * (G.dict[(size_t) k * nC + j] + cj) : v;
 		}
 		s = wave_sum_f64(s);
 		if((tid & 63) == 0) red[tid >> 6] = s;
 		__syncthreads();
-		if(tid == 0) {
-			const double tot = red[0] + red[1] + red[2] + red[3];
-			if(j < nC) {
-				const int r = G.cols[i], c = G.cols[j];
-				unsafeAtomicAdd(&out[(size_t) min(r, c) * nCols + max(r, c)], tot);
-			}
-			else
-				unsafeAtomicAdd(&colSum[G.cols[i]], tot);
-		}
+		const double tot = red[0] + red[1] + red[2] + red[3];
+		if(tid == 0 && j < nC) add(G.cols[i], G.cols[j], tot);
+		if(tid == 0 && j == nC && colSum) unsafeAtomicAdd(&colSum[G.cols[i]], tot);
+		if(j == nC)
+			for(int k = tid; k < nConst; k += 256) add(G.cols[i], constCols[k], tot * constV[constCols[k]]);
 		__syncthreads();
 	}
+}
+
+// out (upper triangle) += the cells that exact code counts give (k_tsmm_self).
+int launch_tsmm_self(cla_block* b, double* out, double* colSum, const double* constV, const int32_t* constCols, int nConst) {
+	const int nG = (int) b->groups.size();
+	if(const int rc = ensure_counts(b)) return rc;
+	if(nG == 0) return 0;
+	int maxCols = 1;
+	for(auto& g : b->groups) maxCols = std::max(maxCols, g.d.nColG);
+	const int64_t cells = (int64_t) maxCols * (maxCols + 3) / 2;
+	const dim3 grid((unsigned) std::min<int64_t>(cells, std::max(1, 8 * g_numCU / nG)), (unsigned) (nG + (nConst > 0)));
+	Prof pf(b, "k_tsmm_self", (long) grid.x * grid.y, 256, 0, 0);
+	hipLaunchKernelGGL(k_tsmm_self, grid, dim3(256), 0, b->stream, b->dGroups, nG, b->dCountsAll, out, b->nCols, colSum, constV, constCols,
+		nConst, (double) b->nRows);
+	CLA_HIP(hipGetLastError());
+	return 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -641,6 +667,9 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	// More than 64 columns: the decoded Gram matrices of pairs of 32-column chunks (about 1.4 ms per pair of
 	// chunks on 10M rows) against one pass per pair of groups (3-16 us each): chunks when there are a hundred
 	// times more pairs of groups than pairs of chunks, or when there is no per-pair form.
+	const int64_t mAll = (nCols + 31) / 32, mLeft = split > 0 ? std::max<int64_t>(1, mAll / 2) : 0;
+	const int64_t nJoints = split > 0 ? mLeft * std::max<int64_t>(1, mAll - mLeft) : mAll * (mAll - 1) / 2;
+	const bool chunkCheaper = !forcePairs && pairsFit && nPairs >= 100 * nJoints;
 	// The decoded Gram matrix of a whole block of at most 64 columns as the call's only kernel: its blocks add into an
 	// accumulator kept with the block, and the last one to finish writes the output (both triangles) and the count of
 	// its non-zeros and clears the accumulator again: no fill in front of the kernel, no kernel behind it.
@@ -650,9 +679,13 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	// decoded, 10,000,000 x 20 take 290 us). Several groups need a pass over the rows per pair: 10,000,000 rows, 2 groups of 8 columns
 	// (256 tuples) 442 us against 157 decoded, 3 of 8 806 / 317, 4 of 4 552 / 159, 4 of 8 1573 / 354, 2 of 50 4012 / 1947; the two meet
 	// only for two narrow groups on 40,000,000 rows (2 of 7 columns 537 / 578, 2 of 8 1209 / 587, 3 of 5 866 / 574).
+	// Blocks that went by pairs of groups otherwise keep what those are exact in: cells inside a group (and of columns without one) from
+	// the code counts, one small kernel in front (rms relative error on 4,000,003 rows of like terms, 5 groups of 4 columns of 16 tuples
+	// 5.0e-15 decoded, 7.5e-17 by counts, 99 -> 100 us; 2 of 50 columns 2.1e-15, 1.0e-16, 851 -> 859; 300,007 rows, 3 of 8 25 -> 27).
+	const bool ownByCounts = !dense && !(nCols > 64 && chunkCheaper);
 	if(nPairs > 0 && !forcePairs && split == 0 && b->crossBlocks == 0 && nRows > 0 && b->opt.tsmmMfma && (nCols <= 64 || b->opt.tsmmChunks)) {
 		if(!b->opt.tsmmOneKernel && (rc = clear())) return rc;
-		rc = nCols <= 64 && dense ? 1 : launch_gram_tiles(b, dOut, b->opt.tsmmOneKernel ? dNnz : nullptr);
+		rc = nCols <= 64 && dense ? 1 : launch_gram_tiles(b, dOut, b->opt.tsmmOneKernel ? dNnz : nullptr, ownByCounts);
 		if(rc < 0) return rc;
 		if(rc == 0) {
 			if(!b->opt.tsmmOneKernel) {
@@ -669,9 +702,6 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz) {
 		if(rc <= 0) return rc;
 	}
 	if((rc = clear())) return rc;
-	const int64_t mAll = (nCols + 31) / 32, mLeft = split > 0 ? std::max<int64_t>(1, mAll / 2) : 0;
-	const int64_t nJoints = split > 0 ? mLeft * std::max<int64_t>(1, mAll - mLeft) : mAll * (mAll - 1) / 2;
-	const bool chunkCheaper = !forcePairs && pairsFit && nPairs >= 100 * nJoints;
 	if((dense || chunkCheaper) && nCols > 64 && nRows > 0 && b->opt.tsmmChunks) {
 		// decoded Gram matrices of pairs of column chunks
 		rc = launch_tsmm_chunked(b, dOut);
@@ -734,16 +764,7 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	double* dColSum = (double*) b->dScratch;
 	int4* dPairs = (int4*) ((char*) b->dScratch + sumBytes);
 	CLA_HIP(hipMemsetAsync(dColSum, 0, sizeof(double) * (size_t) nCols, st));
-	if((rc = ensure_counts(b))) return rc;
-	if(nG > 0) {
-		// a block per cell, several cells in turn where there are many (one block per group took 0.8 us a cell: 64 columns 1.7 ms)
-		int maxCols = 1;
-		for(auto& g : b->groups) maxCols = std::max(maxCols, g.d.nColG);
-		const int64_t cells = (int64_t) maxCols * (maxCols + 3) / 2;
-		const dim3 grid((unsigned) std::min<int64_t>(cells, std::max(1, 8 * g_numCU / nG)), (unsigned) nG);
-		Prof pf(b, "k_tsmm_self", (long) grid.x * nG, 256, 0, 0);
-		hipLaunchKernelGGL(k_tsmm_self, grid, dim3(256), 0, st, b->dGroups, b->dCountsAll, dOut, nCols, dColSum);
-	}
+	if((rc = launch_tsmm_self(b, dOut, dColSum, nullptr, nullptr, 0))) return rc;
 	const int nTiles = (int) ((nRows + TT - 1) / TT);
 	// Pairs of DDC groups with one or two columns each, equal code width and both dictionaries
 	// in LDS take the dot-form kernel (one launch per shape); the others the pre-aggregate kernel.

@@ -15,7 +15,7 @@ def check(cla, ora, specs, n_rows, n_cols, what, options=()):
     out, nnz = blk.tsmm()
     names = {k["name"] for k in blk.stats()["kernels"]}
     blk.close()
-    assert names == {"k_gram_tiles"}, names
+    assert names - {"k_tsmm_self"} == {"k_gram_tiles"}, names  # (few wide groups: cells inside a group from the code counts)
     D = ora.np_decompress(specs, n_rows, n_cols)
     assert np.array_equal(out, out.T)
     assert_matches_truth(out, D.T, D, what=what)
@@ -104,6 +104,6 @@ def test_sums_of_like_terms(cla, n_cols, width, n_vals, dtype, bound):
     out, _ = blk.tsmm()
     names = {k["name"] for k in blk.stats()["kernels"]}
     blk.close()
-    assert names == {"k_gram_tiles"}, names
+    assert names - {"k_tsmm_self"} == {"k_gram_tiles"}, names  # (few wide groups: cells inside a group from the code counts)
     rel = np.diag(out) / exact - 1.0
     assert np.sqrt((rel ** 2).mean()) < bound, np.sqrt((rel ** 2).mean())

@@ -267,3 +267,47 @@ def test_one_group_of_many_columns_is_counts_times_dictionary(cla, n_cols, n_val
     got = out[np.ix_(perm, perm)]
     assert np.array_equal(out, out.T) and nnz == np.count_nonzero(out)
     assert np.all(np.abs(got - exact) <= (14 + n_vals / 256) * 2.0 ** -53 * scale)
+
+
+@pytest.mark.parametrize("one_kernel", [1, 0])
+@pytest.mark.parametrize("n_groups,width,n_vals,dtype", [(2, 8, 5, np.uint8), (5, 4, 16, np.uint8), (3, 8, 300, np.uint16), (2, 50, 20, np.uint8)])
+@pytest.mark.parametrize("const", [False, True])
+def test_cells_inside_a_wide_group_are_counts_times_dictionary(cla, n_groups, width, n_vals, dtype, const, one_kernel):
+    """A block of a few wide groups is decoded for the cells between its groups; those inside a group, and those of columns
+    that only carry a constant, are code counts times products of dictionary values, to a few units in the last place (as
+    for a single group, and a rounding each for the two constants and the last product; positive values, so that a chain of additions over the rows drifts)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_groups * width)
+    n_rows = 2_000_003
+    n_cols = n_groups * width + (2 if const else 0)
+    cols = rng.permutation(n_cols).astype(np.int32)
+    codes = [np.minimum(rng.integers(0, n_vals, n_rows), rng.integers(0, n_vals, n_rows)).astype(dtype) for _ in range(n_groups)]
+    dicts = [1 + rng.random((n_vals, width)) for _ in range(n_groups)]
+    parts = [cols[g * width:(g + 1) * width] for g in range(n_groups)]
+    specs = [synth.GroupSpec("ddc", parts[g], dicts[g], codes[g]) for g in range(n_groups)]
+    if const:
+        specs.append(synth.GroupSpec("const", cols[n_groups * width:], np.array([[1.3, 0.7]])))
+    blk = cla.build_block(n_rows, n_cols, specs).set_option("tsmm_one_kernel", one_kernel)
+    for _ in range(2):  # (the accumulator is zero again behind a call)
+        out, nnz = blk.tsmm()
+        names = [k["name"] for k in blk.stats()["kernels"]]
+        assert names == ["k_tsmm_self", "k_gram_tiles"] + ([] if one_kernel else ["k_tsmm_finish"]), names
+        assert np.array_equal(out, out.T) and nnz == n_cols * n_cols
+        eps = (17 + n_vals / 256) * 2.0 ** -53
+        sums = []
+        for g in range(n_groups):
+            n, L = np.bincount(codes[g], minlength=n_vals).astype(np.longdouble), dicts[g].astype(np.longdouble)
+            exact = (L * n[:, None]).T @ L
+            assert np.all(np.abs(out[np.ix_(parts[g], parts[g])] - exact) <= eps * exact), g
+            sums.append(n @ L)
+            for h in range(g):
+                joint = np.bincount(codes[g].astype(np.int64) * n_vals + codes[h], minlength=n_vals * n_vals).reshape(n_vals, n_vals)
+                exact = L.T @ joint.astype(np.longdouble) @ dicts[h].astype(np.longdouble)
+                assert np.all(np.abs(out[np.ix_(parts[g], parts[h])] - exact) <= 1e-13 * exact), (g, h)
+        if const:
+            c, w = cols[n_groups * width:], np.array([1.3, 0.7]).astype(np.longdouble)
+            assert np.all(np.abs(out[np.ix_(c, c)] - n_rows * np.outer(w, w)) <= eps * n_rows * np.outer(w, w))
+            for g in range(n_groups):
+                exact = np.outer(sums[g], w)
+                assert np.all(np.abs(out[np.ix_(parts[g], c)] - exact) <= eps * exact), g
+    blk.close()
