@@ -290,6 +290,7 @@ int launch_lmm_q1_short(cla_block* b, const double* dY, double* dOut);
 int launch_lmm_direct(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dBad);
 int launch_tsmm_self(cla_block* b, double* out, double* colSum, const double* constV, const int32_t* constCols, int nConst);
 int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr, bool ownByCounts = false);
+int gram_tiles_behind_decode(const cla_block* b);
 void gt_plan_drop(cla_block* b);
 int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);
 int ensure_gram_acc(cla_block* b); // the zeroed nCols x nCols accumulator of the one-kernel t(X) %*% X (a workspace kept with the block)

@@ -482,6 +482,28 @@ static int gt_launch_shape(cla_block* b, const GtPlan& P, const GtArgs& A, unsig
 	return 1;
 }
 
+// Where k_tsmm_decode stays the better kernel: two-byte codes of blocks that are not all column pairs, up to 48 columns, whose dictionaries
+// do not fit beside the tiles of one column block or exceed an XCD's L2 by far. 1: there; 2: there if it holds all dictionaries in LDS.
+// Both in us: 16 columns of 890 values, which its smaller tiles leave room for, 150,003 rows 21.7 / 22.6 here, 250,007 24 / 27, 1,000,003
+// 40 / 63, 4,000,003 106 / 203 (100,003: 20.4 / 13.6 at 700 values); dictionaries in global memory, up to its second turn of tiles, 16 of
+// 20,000 values, 50,003 rows 18.9 / 19.3, 100,003 21.4 / 23.0, 200,003 27.7 / 30.9, 400,003 48 / 43; past the L2, 16 of 60,000 values
+// 70,001 rows 32 / 38, 1,000,003 139 / 149, 20 of 60,000 206 / 216 (100,003: 41 / 41), 32 of 30,000 200,003 rows 70 / 76, 300,007
+// 129 / 102, 1,000,003 269 / 293, 48 of 60,000 200,003 rows 161 / 171, 300,007 277 / 266, 1,000,003 683 / 732; 64 columns of 60,000 1148 / 1002. Pairs of 60,000 tuples stay within 4 %.
+int gram_tiles_behind_decode(const cla_block* b) {
+	const int n = b->nCols;
+	if(b->dArena == nullptr || b->arenaWidth != 2 || n < 13 || n > 48) return 0;
+	bool pairs = n == 2 * (int) b->groups.size();
+	size_t bytes = 0;
+	for(const HostGroup& H : b->groups) { pairs &= H.d.nColG == 2; bytes += H.dict.size() * 8; }
+	if(pairs) return 0;
+	const int64_t rows = b->nRows;
+	if(bytes > ((size_t) 4 << 20) && rows > 150000 && rows <= 250000) return 1;
+	if(bytes > ((size_t) 6 << 20)) return rows > (n <= 16 ? 60000 : n <= 32 && bytes > ((size_t) 9 << 20) ? 90000 : 500000);
+	if(n > 16 || (size_t) b->maxVals * 128 + (size_t) 64 * gt_m(1, GT_SHORT) * gt_stride(1, GT_SHORT) * 8 <= (size_t) g_ldsPerBlock) return 0;
+	if(bytes <= 120 * 1024) return rows > 150000 ? 2 : 0;
+	return bytes <= ((size_t) 4 << 20) && rows > 60000 && rows <= 250000;
+}
+
 // Like launch_tsmm_decode: dNnz != nullptr: the call's only kernel, which writes dOut whole; else dOut (zeroed) gets the upper
 // triangle. ownByCounts: cells inside a group are exact code counts times dictionary products, as on the way by pairs of groups (one
 // more kernel in front). Returns 1 when the block is not of this kernel's shape.

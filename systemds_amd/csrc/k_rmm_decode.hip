@@ -1547,12 +1547,16 @@ int launch_tsmm_decode(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	const int nCols = b->nCols;
 	if(b->groups.empty() || b->nRows == 0 || nCols > 64) return 1;
 	if(dNnz != nullptr && (b->crossBlocks > 0 || b->crossSplit > 0)) return 1; // (only a part of the Gram matrix is wanted: no one-kernel form)
-	{
-		int rc = launch_tsmm_direct(b, dOut, dNnz);
-		if(rc != 1) return rc;
-		rc = launch_gram_tiles(b, dOut, dNnz);
-		if(rc != 1) return rc;
+	int rc = launch_tsmm_direct(b, dOut, dNnz);
+	if(rc != 1) return rc;
+	int behind = gram_tiles_behind_decode(b); // k_gram_tiles only if this kernel does not take the block
+	if(behind == 2) {
+		DecLaunch L;
+		bool flat = false;
+		if((rc = gram_prepare(b, L, flat)) < 0) return rc;
+		behind = rc == 0 && !flat;
 	}
+	if(!behind && (rc = launch_gram_tiles(b, dOut, dNnz)) != 1) return rc;
 	const int NB = (nCols + 15) / 16;
 	// only the product of the first crossBlocks column blocks with the others is wanted (a pair of column chunks
 	// whose own Gram matrices nobody reads): shapes 1 x 1, 1 x 2, 2 x 1, 2 x 2 blocks, anything else in full
@@ -1560,7 +1564,8 @@ int launch_tsmm_decode(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	if(XB < 1 || XB > 2 || NB - XB < 1 || NB - XB > 2) XB = 0;
 	DecLaunch L;
 	bool flat = false;
-	int rc = gram_prepare(b, L, flat);
+	rc = gram_prepare(b, L, flat);
+	if(rc == 1 && behind) return launch_gram_tiles(b, dOut, dNnz);
 	if(rc) return rc;
 	L.A.out = dOut;
 	if(dNnz != nullptr) {

@@ -107,3 +107,25 @@ def test_sums_of_like_terms(cla, n_cols, width, n_vals, dtype, bound):
     assert names - {"k_tsmm_self"} == {"k_gram_tiles"}, names  # (few wide groups: cells inside a group from the code counts)
     rel = np.diag(out) / exact - 1.0
     assert np.sqrt((rel ** 2).mean()) < bound, np.sqrt((rel ** 2).mean())
+
+
+@pytest.mark.parametrize("n_rows,n_cols,n_vals,kernel", [
+    (150_000, 13, 900, "k_gram_tiles"), (150_001, 13, 900, "k_tsmm_decode"), (400_001, 16, 890, "k_tsmm_decode"),  # dictionaries in LDS there
+    (400_001, 16, 700, "k_gram_tiles"),                                                                          # ... and here
+    (60_000, 16, 3000, "k_gram_tiles"), (60_001, 16, 3000, "k_tsmm_decode"), (250_001, 14, 3000, "k_gram_tiles"),  # in global memory
+    (60_001, 13, 61000, "k_tsmm_decode"), (90_001, 17, 50000, "k_gram_tiles"), (150_001, 17, 50000, "k_tsmm_decode"),  # past the L2
+    (250_001, 17, 50000, "k_gram_tiles"), (500_001, 17, 50000, "k_tsmm_decode")])
+def test_two_byte_codes_where_the_older_kernel_is_faster(cla, n_rows, n_cols, n_vals, kernel):
+    """The rule that leaves two-byte blocks to k_tsmm_decode, at its lines; t(X) %*% X against exact integers (dictionaries of
+    whole numbers, whose products and sums stay below 2^53)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows + n_cols)
+    codes = rng.integers(0, n_vals, (n_cols, n_rows)).astype(np.uint16)
+    dicts = rng.integers(-1000, 1000, (n_cols, n_vals)).astype(np.float64)
+    blk = cla.build_block(n_rows, n_cols, [synth.GroupSpec("ddc", np.array([c], np.int32), dicts[c][:, None], codes[c]) for c in range(n_cols)])
+    out, nnz = blk.tsmm()
+    names = [k["name"] for k in blk.stats()["kernels"]]
+    blk.close()
+    assert names == [kernel], names
+    D = np.stack([dicts[c][codes[c]] for c in range(n_cols)])
+    assert np.array_equal(out, D @ D.T) and nnz == np.count_nonzero(out)
