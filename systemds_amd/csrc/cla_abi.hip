@@ -672,7 +672,7 @@ int finish_finalize(cla_block* b, cla_block* arenaFrom, bool buildArena) {
 				if(per >= 8) b->q1Threads = 1024;
 			}
 		}
-		if(nG > 0 && per >= 8) {
+		if(b->dArena != nullptr && b->arenaWidth != 2 && per >= 8) { // (two-byte codes have kernels of their own, k_short_vec.hip)
 			for(size_t i = 0; i < nG; i += per) {
 				const size_t j = std::min(nG, i + (size_t) per);
 				bool uniform = true;

@@ -663,7 +663,7 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 		else if(threads == 1024) LAUNCH_Q1(CWV, RPTV, 1024);                     \
 		else LAUNCH_Q1(CWV, RPTV, 256);                                          \
 	} while(0)
-		if(cw == 1) LAUNCH_Q1_T(1, 16); // (two-byte codes: k_rmm_q1_short)
+		if(cw == 1) LAUNCH_Q1_T(1, 16); // (two-byte codes have no slabs)
 		else LAUNCH_Q1_T(4, 8);
 #undef LAUNCH_Q1_T
 #undef LAUNCH_Q1
