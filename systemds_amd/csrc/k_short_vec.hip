@@ -155,9 +155,14 @@ int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double
 	const int nG = (int) b->groups.size();
 	if(b->dArena == nullptr || b->arenaWidth != 2 || nG == 0 || b->nRows == 0 || b->maxVals > SV_BUF) return 1;
 	const RowOp rowOp = op != nullptr ? *op : RowOp();
-	// Up to 400,000 rows (where both take 29 us at 25 groups, 15 at 10) straight from global memory: 20,000 x 50 11 against 27 us,
-	// 200,000 x 50 18 against 28; beyond, the form with the tables in LDS: 700,000 x 50 31 against 43, 1,500,000 x 6 14 against 26.
-	if(b->nRows <= 400000) {
+	// Few rows straight from global memory: 20,000 x 50 11 against 27 us, 200,000 x 50 18 against 28. Its lookups slow down as the tables
+	// grow: up to 1000 tuples the two meet between 300 and 400 thousand rows (30 groups of 700 23 / 30 at 200,003, 35 / 31 at 399,001),
+	// from there on at 300,000 (30 of 1100 31.7 / 31.4, of 4000 42 / 33; 90 of 4000 399,001 rows 147 / 78). Tables that come one at a time
+	// (more than 4096 tuples) cost the form with the tables in LDS twice the time, and k_rmm_rows has its range between the two from a few groups on, up to
+	// 450,000 rows: 90 of 8000 tuples 350,003 rows 157 straight / 129 there / 146 in LDS, 30 of 4500 399,001 rows 57 / 44 / 55, 499,001
+	// 65 / 54 / 55 (90 of 4500 172 / 154 / 143; 2 of 4500 399,001 rows 14 / 10 / 11).
+	if(b->nRows > 300000 && b->nRows <= 450000 && 2 * b->maxVals > SV_BUF && nG >= 8) return 1;
+	if(b->nRows <= (b->maxVals <= 1000 ? 400000 : 300000)) {
 		const unsigned grid = (unsigned) ((b->nRows + 255) / 256);
 		Prof pf(b, "k_rmm_q1_short_rows", grid, 256, 0, (double) b->nRows * (2 * nG + 8) + (double) b->totalVals * 8);
 		hipLaunchKernelGGL(k_rmm_q1_short_rows, dim3(grid), dim3(256), 0, b->stream, b->dArena, b->arenaStride, nG, b->dTblOff, tables,

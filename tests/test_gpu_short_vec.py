@@ -62,3 +62,24 @@ def test_non_finite_vector(cla, ora):
     y[0, 5] = np.nan
     assert np.all(np.isnan(blk.lmm(y)[0]))
     blk.close()
+
+
+@pytest.mark.parametrize("n_rows,n_groups,n_vals,kernel", [
+    (300000, 3, 1001, "k_rmm_q1_short_rows"), (300001, 3, 1000, "k_rmm_q1_short_rows"), (300001, 3, 1001, "k_rmm_q1_short"), (400001, 3, 300, "k_rmm_q1_short"),
+    (300000, 8, 4097, "k_rmm_q1_short_rows"), (300001, 8, 4097, "k_rmm_rows"), (300001, 7, 4097, "k_rmm_q1_short"), (300001, 8, 4096, "k_rmm_q1_short"),
+    (450000, 8, 4097, "k_rmm_rows"), (450001, 8, 4097, "k_rmm_q1_short")])
+def test_which_kernel_multiplies_by_a_vector(cla, ora, n_rows, n_groups, n_vals, kernel):
+    """X %*% v on both sides of the lines between its kernels, bit for bit against the oracle, and the chain with weights (which
+    k_rmm_rows leaves to a kernel of its own) against exact sums."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_vals)
+    specs = block(synth, rng, n_rows, n_groups, 1, n_vals)
+    v, w = rng.standard_normal((n_groups, 1)), rng.random((n_rows, 1))
+    blk = cla.build_block(n_rows, n_groups, specs)
+    out, nnz = blk.rmm(v)
+    assert kernel in [k["name"] for k in blk.stats()["kernels"]]
+    ref, rnnz = ora.rmm(ora.Groups(specs, n_rows, n_groups), v, 1)
+    assert np.array_equal(out, ref) and nnz == rnnz
+    chain, _ = blk.mmchain(v, w, 1)
+    blk.close()
+    assert_matches_truth(chain.reshape(1, -1), (w * ref).reshape(1, -1), ora.np_decompress(specs, n_rows, n_groups), what="weighted chain")
