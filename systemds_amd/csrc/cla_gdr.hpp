@@ -72,6 +72,32 @@ __device__ __forceinline__ void gdr_copy_vals(double* smem, const double* __rest
 	}
 }
 
+// The value of lane ^ 1, ^ 2 or ^ 4 on the vector unit.
+template <int CTRL>
+__device__ __forceinline__ double gdr_dpp(double v) {
+	int p[2];
+	__builtin_memcpy(p, &v, 8);
+	p[0] = __builtin_amdgcn_update_dpp(0, p[0], CTRL, 0xf, 0xf, false);
+	p[1] = __builtin_amdgcn_update_dpp(0, p[1], CTRL, 0xf, 0xf, false);
+	double r;
+	__builtin_memcpy(&r, p, 8);
+	return r;
+}
+__device__ __forceinline__ double gdr_xchg1(double v) { return gdr_dpp<0xB1>(v); }
+__device__ __forceinline__ double gdr_xchg2(double v) { return gdr_dpp<0x4E>(v); }
+__device__ __forceinline__ double gdr_xchg4(double v) { // banks 0 and 2 from the bank above, 1 and 3 from the bank below
+	int p[2];
+	__builtin_memcpy(p, &v, 8);
+#pragma unroll
+	for(int h = 0; h < 2; h++) {
+		int r = __builtin_amdgcn_update_dpp(0, p[h], 0x104, 0xf, 0x5, false); // row_shl:4
+		p[h] = __builtin_amdgcn_update_dpp(r, p[h], 0x114, 0xf, 0xA, false);   // row_shr:4
+	}
+	double r;
+	__builtin_memcpy(&r, p, 8);
+	return r;
+}
+
 // The block's plan, built on first use; P.rc says whether it qualifies. Negative: an error.
 int gdr_plan(cla_block* b, const GdrPlan*& P);
 

@@ -214,51 +214,27 @@ __global__ __launch_bounds__(GDR_THREADS) void k_tsmm_direct(const GdrArgs A) {
 			asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(hi) : "v"(p[1]));
 		};
 		const bool fb0 = (lane & 1) != 0, fb1 = (lane & 2) != 0, fb2 = (lane & 4) != 0;
-		auto dpp_f64 = [](double v, auto ctrlTag) __attribute__((always_inline)) {
-			constexpr int ctrl = decltype(ctrlTag)::value;
-			int p[2];
-			__builtin_memcpy(p, &v, 8);
-			p[0] = __builtin_amdgcn_update_dpp(0, p[0], ctrl, 0xf, 0xf, false);
-			p[1] = __builtin_amdgcn_update_dpp(0, p[1], ctrl, 0xf, 0xf, false);
-			double r;
-			__builtin_memcpy(&r, p, 8);
-			return r;
-		};
-		auto xchg1 = [&](double v) __attribute__((always_inline)) { return dpp_f64(v, std::integral_constant<int, 0xB1>()); }; // lane ^ 1
-		auto xchg2 = [&](double v) __attribute__((always_inline)) { return dpp_f64(v, std::integral_constant<int, 0x4E>()); }; // lane ^ 2
-		auto xchg4 = [&](double v) __attribute__((always_inline)) { // lane ^ 4: banks 0 and 2 from the bank above, 1 and 3 from the bank below
-			int p[2];
-			__builtin_memcpy(p, &v, 8);
-#pragma unroll
-			for(int h = 0; h < 2; h++) {
-				int r = __builtin_amdgcn_update_dpp(0, p[h], 0x104, 0xf, 0x5, false); // row_shl:4
-				p[h] = __builtin_amdgcn_update_dpp(r, p[h], 0x114, 0xf, 0xA, false);   // row_shr:4
-			}
-			double r;
-			__builtin_memcpy(&r, p, 8);
-			return r;
-		};
 		// fold0 / fold1 of the running sums el(c), c < NV
 		auto fold = [&](double& f0, double& f1, auto el) __attribute__((always_inline)) {
 			double w[4], u[2];
 #pragma unroll
 			for(int j = 0; j < 4; j++) {
 				const double lo = 2 * j < NV ? el(2 * j < NV ? 2 * j : 0) : 0.0, hi = 2 * j + 1 < NV ? el(2 * j + 1 < NV ? 2 * j + 1 : 0) : 0.0;
-				w[j] = (fb0 ? hi : lo) + xchg1(fb0 ? lo : hi);
+				w[j] = (fb0 ? hi : lo) + gdr_xchg1(fb0 ? lo : hi);
 			}
 #pragma unroll
-			for(int i = 0; i < 2; i++) u[i] = (fb1 ? w[2 * i + 1] : w[2 * i]) + xchg2(fb1 ? w[2 * i] : w[2 * i + 1]);
-			f0 = (fb2 ? u[1] : u[0]) + xchg4(fb2 ? u[0] : u[1]);
+			for(int i = 0; i < 2; i++) u[i] = (fb1 ? w[2 * i + 1] : w[2 * i]) + gdr_xchg2(fb1 ? w[2 * i] : w[2 * i + 1]);
+			f0 = (fb2 ? u[1] : u[0]) + gdr_xchg4(fb2 ? u[0] : u[1]);
 			f1 = 0.0;
 			if(NV > 8) {
 				double w1[2];
 #pragma unroll
 				for(int j = 0; j < 2; j++) {
 					const double lo = 8 + 2 * j < NV ? el(8 + 2 * j < NV ? 8 + 2 * j : 0) : 0.0, hi = 9 + 2 * j < NV ? el(9 + 2 * j < NV ? 9 + 2 * j : 0) : 0.0;
-					w1[j] = (fb0 ? hi : lo) + xchg1(fb0 ? lo : hi);
+					w1[j] = (fb0 ? hi : lo) + gdr_xchg1(fb0 ? lo : hi);
 				}
-				const double u1 = (fb1 ? w1[1] : w1[0]) + xchg2(fb1 ? w1[0] : w1[1]);
-				const double t1 = u1 + xchg4(u1); // (lanes k and k ^ 4 hold the same column: one of them keeps it)
+				const double u1 = (fb1 ? w1[1] : w1[0]) + gdr_xchg2(fb1 ? w1[0] : w1[1]);
+				const double t1 = u1 + gdr_xchg4(u1); // (lanes k and k ^ 4 hold the same column: one of them keeps it)
 				f1 = fb2 ? 0.0 : t1;
 			}
 		};

@@ -74,41 +74,17 @@ __global__ __launch_bounds__(LD_THREADS, 2) void k_lmm_direct(const GdrArgs A, c
 		bool bad = false;
 
 		const bool fb0 = (lane & 1) != 0, fb1 = (lane & 2) != 0, fb2 = (lane & 4) != 0;
-		auto dpp_f64 = [](double v, auto ctrlTag) __attribute__((always_inline)) {
-			constexpr int ctrl = decltype(ctrlTag)::value;
-			int p[2];
-			__builtin_memcpy(p, &v, 8);
-			p[0] = __builtin_amdgcn_update_dpp(0, p[0], ctrl, 0xf, 0xf, false);
-			p[1] = __builtin_amdgcn_update_dpp(0, p[1], ctrl, 0xf, 0xf, false);
-			double r;
-			__builtin_memcpy(&r, p, 8);
-			return r;
-		};
-		auto xchg1 = [&](double v) __attribute__((always_inline)) { return dpp_f64(v, std::integral_constant<int, 0xB1>()); }; // lane ^ 1
-		auto xchg2 = [&](double v) __attribute__((always_inline)) { return dpp_f64(v, std::integral_constant<int, 0x4E>()); }; // lane ^ 2
-		auto xchg4 = [&](double v) __attribute__((always_inline)) { // lane ^ 4
-			int p[2];
-			__builtin_memcpy(p, &v, 8);
-#pragma unroll
-			for(int h = 0; h < 2; h++) {
-				int r = __builtin_amdgcn_update_dpp(0, p[h], 0x104, 0xf, 0x5, false); // row_shl:4
-				p[h] = __builtin_amdgcn_update_dpp(r, p[h], 0x114, 0xf, 0xA, false);   // row_shr:4
-			}
-			double r;
-			__builtin_memcpy(&r, p, 8);
-			return r;
-		};
 		// lane k of every group of eight: the group's sum of el(k), k < P
 		auto fold = [&](auto el) __attribute__((always_inline)) {
 			double w[4], u[2];
 #pragma unroll
 			for(int j = 0; j < 4; j++) {
 				const double lo = 2 * j < P ? el(2 * j < P ? 2 * j : 0) : 0.0, hi = 2 * j + 1 < P ? el(2 * j + 1 < P ? 2 * j + 1 : 0) : 0.0;
-				w[j] = (fb0 ? hi : lo) + xchg1(fb0 ? lo : hi);
+				w[j] = (fb0 ? hi : lo) + gdr_xchg1(fb0 ? lo : hi);
 			}
 #pragma unroll
-			for(int i = 0; i < 2; i++) u[i] = (fb1 ? w[2 * i + 1] : w[2 * i]) + xchg2(fb1 ? w[2 * i] : w[2 * i + 1]);
-			return (fb2 ? u[1] : u[0]) + xchg4(fb2 ? u[0] : u[1]);
+			for(int i = 0; i < 2; i++) u[i] = (fb1 ? w[2 * i + 1] : w[2 * i]) + gdr_xchg2(fb1 ? w[2 * i] : w[2 * i + 1]);
+			return (fb2 ? u[1] : u[0]) + gdr_xchg4(fb2 ? u[0] : u[1]);
 		};
 		// A stretch of rows on which every run-length column is constant ends (el(i): the lane's sums of y over it): each column
 		// takes its value times the stretch's sums. (Unused cursors hold the value 0.)
