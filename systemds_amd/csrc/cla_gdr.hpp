@@ -51,6 +51,8 @@ struct GdrPlan {
 	int64_t bytes = 0;
 	size_t lds = 0;
 	GdrArgs A;
+	int spread = -1;       // 1: a varying column next to run-length columns spans too many magnitudes for summation by parts; -1: not looked at yet
+	bool codeSpread = false; // the same of the columns behind codes, from their dictionaries
 	LdCols ld;             // ldNC code columns (fillers behind the real ones), ldND dense ones; ldNC == 0: no such form
 	int ldNC = 0, ldND = 0;
 	int64_t runEnds = 0;   // of the run-length groups that are followed by run (inside the matrix)

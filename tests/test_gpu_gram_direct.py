@@ -154,6 +154,43 @@ def test_non_finite_run_length_values_take_the_tile_kernel(cla, ora):
     assert nnz == np.count_nonzero(out)
 
 
+@pytest.mark.parametrize("kind", ["infinity", "dense", "dictionary", "zeros"])
+def test_values_of_many_magnitudes_next_to_run_length_columns(cla, ora, kind):
+    """Summation by parts takes every row of a varying column into its sums, also those on which a run-length column is zero: a
+    column with values far above the others (a marker of 1e14 on uncovered rows, an infinity) goes to the tile kernel, which
+    forms every row's cells; many zeros among ordinary values do not count as a wide span."""
+    n_rows = 70003
+    specs, n_cols = stream_block(41, n_rows, n_rle=3, n_u16=2, n_u8=1, n_sdc=1, n_dense=2)
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    rle = next(s.cols[0] for k, s in enumerate(specs) if k == 1)  # (some of its runs have no value)
+    uncovered = np.flatnonzero(D[:, rle] == 0.0)
+    dense = next(s for s in specs if s.type == "unc")
+    ddc = next(s for s in specs if s.type == "ddc")
+    if kind == "infinity":
+        dense.dense[np.flatnonzero(np.all(D[:, :3] != 0.0, axis=1))[7], 0] = np.inf
+    elif kind == "dense":
+        dense.dense[uncovered[::3], 1] = 1e14
+    elif kind == "dictionary":
+        ddc.dict[5, 0] = 1e14
+        ddc.codes[ddc.codes == 5] = 6
+        ddc.codes[uncovered[::50]] = 5
+    else:
+        dense.dense[::2, 0] = 0.0
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, nnz = blk.tsmm()
+    names = [k["name"] for k in blk.stats()["kernels"]]
+    blk.close()
+    assert ("k_tsmm_direct" in names) == (kind == "zeros"), names
+    with np.errstate(invalid="ignore", over="ignore"):
+        truth = (D.T.astype(np.longdouble) @ D.astype(np.longdouble)).astype(np.float64)
+        scale = np.abs(D).T @ np.abs(D)
+        fin = np.isfinite(truth)
+        assert np.array_equal(np.isnan(out), np.isnan(truth)) and np.array_equal(out[np.isinf(truth)], truth[np.isinf(truth)])
+        assert np.all(np.abs(out - truth)[fin] <= 1e-12 * scale[fin])
+    assert nnz == np.count_nonzero(out)
+
+
 def test_long_runs_keep_no_expanded_copy(cla):
     """A run-length group whose runs are long gets no one-code-per-row copy: the block's derived bytes stay far below
     one byte per row and group."""
