@@ -122,10 +122,10 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *   sdc_lanes       1 / 0: SDCZeros mat-vecs on lane-major copies of the lists, one lane per group
  *   sdc_rows        1 / 0: SDCZeros X %*% v on row lists (the lists transposed), one lane per row
  *   lmm_joint       1 / 0: Y %*% X (16 rows of Y per pass) on a block that is not mostly offset lists in passes over the decoded
- *                   rows, on the vector unit (see tsmm_direct) or on the matrix cores; blocks of more than 64 columns, or whose code tiles exceed LDS together, go chunk of
- *                   columns by chunk (sub-blocks kept with the block); not single-column byte-code blocks, except with bit 0 of
- *                   lmm_disable (the kernel reports non-finite values of Y and the host looks, i.e. waits for the stream once per call;
- *                   such a Y takes the bin kernels)
+ *                   rows, on the vector unit (see tsmm_direct) or on the matrix cores; blocks of more than 64 columns, or
+ *                   whose code tiles exceed LDS together, go chunk of columns by chunk (sub-blocks kept with the block);
+ *                   not single-column byte-code blocks, except with bit 0 of lmm_disable (the kernel reports non-finite
+ *                   values of Y and the host looks, i.e. waits for the stream once per call; such a Y takes the bin kernels)
  *   tsmm_one_kernel 1 / 0: t(X) %*% X of a whole block of at most 64 columns (all-DDC: 128) on the decoded Gram kernels as the call's only
  *                   kernel (a few wide DDC groups: behind the kernel of the cells inside a group; its blocks add into an accumulator kept with the block, nCols x nCols doubles; the last block
  *                   to finish writes the output, mirrored, and the count of its non-zeros and clears the accumulator)
@@ -197,9 +197,9 @@ int64_t cla_block_nnz(cla_handle h);
 /* CLALibLeftMultBy.leftMultByMatrix (C/lib/CLALibLeftMultBy.java:126-145,
  * 286-346): out[nRowY x nCols] = Y %*% X, Y is nRowY x nRows.
  * The _dev_async form returns without waiting except where the block takes the one-pass kernel on the decoded rows
- * (option lmm_joint, blocks that are neither byte-code DDC nor mostly offset lists, nor, for one row of Y, two-byte DDC of one or two columns per group): that kernel reports a value
- * of Y that is not finite, the host reads the flag (one wait for the block's stream per call) and such a Y takes
- * the bin kernels. The same holds for cla_mmchain_dev_async, whose second half is this product. */
+ * (option lmm_joint, blocks that are neither byte-code DDC nor mostly offset lists, nor, for one row of Y, two-byte DDC
+ * of one or two columns per group): that kernel reports a value of Y that is not finite, the host reads the flag (one
+ * wait for the block's stream per call) and such a Y takes the bin kernels. The same holds for cla_mmchain_dev_async, whose second half is this product. */
 int64_t cla_lmm(cla_handle h, const double* Y, int32_t nRowY, double* out);
 int64_t cla_lmm_dev(cla_handle h, const double* dY, int32_t nRowY, double* dOut);
 int cla_lmm_dev_async(cla_handle h, const double* dY, int32_t nRowY, double* dOut);

@@ -18,7 +18,8 @@
 // The stages of three tiles overlap: while a tile is multiplied, the values of the next one but one are looked up and the
 // codes behind those are on their way. One barrier per tile that waits for LDS only: loads stay in flight over it.
 //
-// Bound: the fp64 matrix pipe (70 cycles per tile and 4 rows).
+// Bound: the fp64 matrix pipe (70 cycles per tile and 4 rows): busy 72 % of the time at 2,000,003 x 100 byte codes (vector issue 12 %,
+// LDS 19 %, vector memory path 38 %), 69 % at 10,000,000 x 50 column pairs, where the gathers keep the vector memory path busy 64 %.
 #include "../../include/cla_hip.h"
 #include "cla_device.hpp"
 #include "cla_runs.hpp"

@@ -16,7 +16,7 @@
 // Y goes through LDS: as the matrix operand wants it, neighbouring lanes hold different rows of Y, and the vector memory
 // path serves such a load one lane a cycle (it was busy 70 - 80 % of the kernel and 2,000,003 x 100 by 8 rows took 118 us).
 //
-// Bound: matrix and vector issue (they do not overlap on a SIMD): per 64 rows and column block 16 lookups of two vector
+// Bound: matrix and vector issue (they do not overlap on a SIMD; 55 and 35 % of the time by 8 rows of Y, LDS 40 %): per 64 rows and column block 16 lookups of two vector
 // instructions and 16 x ceil(p / 4) matrix instructions of 17 cycles; under that HBM (codes once, Y once per slab of 4
 // column blocks). Measured (before: a pass of k_lmm_u8_vec per row of Y): 2,000,003 x 100 by 8 rows of Y 343 -> 104 us
 // (3.1 TB/s), 8,000,001 x 100 by 16 2075 -> 641 us, 70,014 x 54 by 4 91 -> 15 us.

@@ -5,8 +5,8 @@
 //   k_lmm_q1_short   t(y) %*% X: the dictionaries of a few groups in LDS, every looked-up tuple times y into registers
 //
 // A lookup straight in global memory costs the vector memory path a cycle per lane and line (62.9 M lookups: 76 us for 8
-// bytes, 99 us for tuples of 16 bytes, one group at a time; 170 us with several groups per instruction); from LDS the same
-// take 25 us and 60 us. So a block holds what its lookups need in LDS: the right multiply owns rows and walks the groups (its
+// bytes, 99 us for tuples of 16 bytes, one group at a time; 170 us with several groups per instruction); the whole kernels with
+// lookups in LDS take 40 and 39 us on as many. So a block holds what its lookups need in LDS: the right multiply owns rows and walks the groups (its
 // sums stay in registers), the left multiply owns groups and walks the rows (its sums are one cell per column).
 #include "../../include/cla_hip.h"
 #include "cla_device.hpp"
@@ -24,7 +24,8 @@ typedef double f64x2_sv __attribute__((ext_vector_type(2), aligned(8)));
 // X %*% v: a block owns a share of the rows, lane l of a wave 4 consecutive rows of each of its NU units of 256. For every
 // pair of groups (GS = 1: every group) the tables come through registers into the LDS buffer that the pair before does not
 // use, while that pair is looked up. Groups are added in list order, as the reference does.
-// Bound: LDS lookups and the tables' way through L2 (all tables once per 16,384 rows at most), about 1 us per group below that.
+// Bound: the vector memory path (its address unit is busy 71 % of the time at 2,500,009 x 50: 8 bytes of codes per lane and group,
+// and all tables once per 16,384 rows at most), LDS 39 %, vector issue 31 %; about 1 us per group below that.
 // 2,500,009 x 50 (25 groups of 4096 tuples) 191 -> 44 us (a thread per row and group before), of 1000 tuples 101 -> 43
 // (slabs of eight tables, reloaded by every block of 4096 rows); 8,000,000 x 50 703 -> 123.
 template <int NU>
@@ -126,6 +127,8 @@ __global__ __launch_bounds__(SV_THREADS) void k_rmm_q1_short(const uint8_t* __re
 
 // The same on few rows: a thread per row looks its groups up straight in global memory, SV_NB at a time.
 // Bound: latency (codes, then values, per batch), then the vector memory path, a cycle per lane and line.
+// (8, 10, 13, 16, 25 at a time: 25 groups of 4096 tuples, 20,003 rows 13.0, 12.4, 12.1, 12.6, 11.9 us, 300,000 rows 37.0, 36.4, 36.0,
+// 37.1, 36.1; 30 groups of 700 24.7, 26.0, 27.7, 27.1, 31.2; places behind the last group look the last one up again.)
 constexpr int SV_NB = 13;
 __global__ __launch_bounds__(256) void k_rmm_q1_short_rows(const uint8_t* __restrict__ arena, size_t arenaStride, int nGroups,
 	const int32_t* __restrict__ tblOff, const double* __restrict__ T, int constIdx, double* __restrict__ out, int64_t nRows,
@@ -198,7 +201,8 @@ int launch_rmm_q1_short(cla_block* b, const double* tables, int constIdx, double
 
 // t(y) %*% X: a block owns a slab of at most GS groups and a share of the rows. A wave takes 512 rows at a time, lane l the
 // rows 2 l and 2 l + 1 of each 128 (whole lines of y and of the codes per instruction), the next 512 on their way meanwhile.
-// Bound: LDS lookups of 8 NC bytes; y comes once per slab from L2 or the memory-side cache. 2,500,009 x 50, 4096 tuples, 278 -> 42 us
+// Bound: LDS lookups of 8 NC bytes (busy 71 % of the time, more than half of it bank conflicts; vector memory path 54 %, vector
+// issue 34 %); y comes once per slab from L2 or the memory-side cache. 2,500,009 x 50, 4096 tuples, 278 -> 42 us
 // (rows decoded into tiles for the matrix cores before, with a wait for the host's look at y), 20,000 x 50 62 -> 11.
 template <int NC, int GS>
 __global__ __launch_bounds__(SV_THREADS) void k_lmm_q1_short(const DGroup* __restrict__ groups, const uint8_t* __restrict__ arena,
