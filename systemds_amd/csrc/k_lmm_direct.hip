@@ -15,8 +15,9 @@
 //
 // More rows of Y than 6 (8 where at most 8 columns vary) take passes (the sums of 12 columns by 6 rows are 144 registers; two
 // waves per SIMD; what spills from two rows per lane there cost 60 of 154 us, so such shapes take one).
-// Bound: HBM (Y once, the streams once per pass), 14 us of start and end. 5,000,011 x 20 (8 run-length, 8 two-byte, 2 offset-list,
-// 2 dense columns) by 6 rows of Y 274 -> 92 us (410 MB: 4.5 TB/s), by 1 259 -> 54, by 16 332 -> 247; 1,250,000 rows by 6 86 -> 35.
+// Bound: HBM (Y once, the streams once per pass; vector memory path 67 % busy, vector issue 40 %), 14 us of start and end. 5,000,011 x
+// 20 (8 run-length, 8 two-byte, 2 offset-list, 2 dense columns) by 6 rows of Y 88 us (414 MB: 4.7 TB/s). Calls, with the host's look at
+// the flag: by 6 301 -> 114 us, by 1 284 -> 77, by 16 361 -> 269; 1,250,000 rows by 6 110 -> 59.
 #include "../../include/cla_hip.h"
 #include "cla_gdr.hpp"
 #include <algorithm>

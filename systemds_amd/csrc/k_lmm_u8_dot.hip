@@ -18,8 +18,8 @@
 //
 // Bound: matrix and vector issue (they do not overlap on a SIMD; 55 and 35 % of the time by 8 rows of Y, LDS 40 %): per 64 rows and column block 16 lookups of two vector
 // instructions and 16 x ceil(p / 4) matrix instructions of 17 cycles; under that HBM (codes once, Y once per slab of 4
-// column blocks). Measured (before: a pass of k_lmm_u8_vec per row of Y): 2,000,003 x 100 by 8 rows of Y 343 -> 104 us
-// (3.1 TB/s), 8,000,001 x 100 by 16 2075 -> 641 us, 70,014 x 54 by 4 91 -> 15 us.
+// column blocks). Measured (before: a pass of k_lmm_u8_vec per row of Y): 2,000,003 x 100 by 8 rows of Y 346 -> 105 us
+// (3.1 TB/s), 8,000,001 x 100 by 16 2199 -> 742 us, 70,014 x 54 by 4 92 -> 15.5 us.
 #include "../../include/cla_hip.h"
 #include "cla_device.hpp"
 #include <algorithm>
