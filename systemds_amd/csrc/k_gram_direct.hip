@@ -463,10 +463,11 @@ __global__ __launch_bounds__(GDR_THREADS) void k_tsmm_direct(const GdrArgs A) {
 
 // Summation by parts lets every row of a varying column enter sums that a run-length column with the value 0 there has to cancel
 // again, so a value of x far above the others costs them their last bits (1e14 among normal ones: 4e-7 of the sum of |v||x|; an
-// infinity: NaN). A column qualifies while its largest value is within 2^GDR_SPREAD of all but a sixteenth of its nonzero ones: then
-// an uncovered row's share of the error is below that of a thousand covered ones. (Normal values span 2^7 by this measure,
-// log-normal ones of sigma 2 and 50 M rows 2^16.)
-constexpr int GDR_SPREAD = 16;
+// infinity: NaN). A column qualifies while its largest value is within 2^GDR_SPREAD of all but a sixteenth of its nonzero ones: the
+// 16 or so run ends of a column between two rebases each round at 2^-53 of such a value at most, 4 x 2^-33 of an ordinary one
+// together, below 1e-12 of the sum from five hundred covered rows on. (Normal values span 2^7 by this measure, log-normal ones of
+// sigma 2 and 50 M rows 2^20, counts up to a million 2^20.)
+constexpr int GDR_SPREAD = 20;
 constexpr int GDR_BINS = 2048; // exponents of a double; the last one: infinities and NaN
 
 // The exponents of |x| counted, column c of a dense group: bins[c][exponent].
