@@ -127,7 +127,8 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *                   not single-column byte-code blocks, except with bit 0 of lmm_disable (the kernel reports non-finite
  *                   values of Y and the host looks, i.e. waits for the stream once per call; such a Y takes the bin kernels)
  *   tsmm_one_kernel 1 / 0: t(X) %*% X of a whole block of at most 64 columns (all-DDC: 128) on the decoded Gram kernels as the call's only
- *                   kernel (a few wide DDC groups: behind the kernel of the cells inside a group; its blocks add into an accumulator kept with the block, nCols x nCols doubles; the last block
+ *                   kernel (a few wide DDC groups: behind the kernel of the cells inside a group; its blocks add into an
+ *                   accumulator kept with the block, nCols x nCols doubles; the last block
  *                   to finish writes the output, mirrored, and the count of its non-zeros and clears the accumulator)
  *                   instead of a fill of the output in front of the kernel and a mirror-and-count kernel behind it
  *   ddc_reorder     1 / 0 (read by cla_block_finalize): the block's copy of a DDC group with two- or four-byte codes and a

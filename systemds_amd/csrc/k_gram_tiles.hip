@@ -525,12 +525,16 @@ int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz, bool
 		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
 	A.skipOwn = ownByCounts;
-	if(ownByCounts)
-		if(const int rc = launch_tsmm_self(b, A.acc, nullptr, b->hasConst ? b->dConstV : nullptr, P.constCols, P.nConst)) return rc;
 	const unsigned grid = (unsigned) std::min(A.nTiles, g_numCU * P.perCU);
-	const int rc = gt_launch_shape(b, P, A, grid);
-	if(rc && ownByCounts && dNnz != nullptr) // (nothing behind the counts' kernel clears the accumulator then)
-		(void) hipMemsetAsync(b->dGramAcc, 0, (size_t) A.nCols * A.nCols * sizeof(double), b->stream);
+	// (where k_gram_tiles does not follow, an exception on the way included, nothing clears what the counts' kernel has added)
+	struct Clear {
+		cla_block* b;
+		bool on;
+		~Clear() { if(on) (void) hipMemsetAsync(b->dGramAcc, 0, (size_t) b->nCols * b->nCols * sizeof(double), b->stream); }
+	} clear{b, ownByCounts && dNnz != nullptr};
+	int rc = 0;
+	if(ownByCounts && (rc = launch_tsmm_self(b, A.acc, nullptr, b->hasConst ? b->dConstV : nullptr, P.constCols, P.nConst))) return rc;
+	if((rc = gt_launch_shape(b, P, A, grid)) == 0) clear.on = false;
 	return rc;
 }
 

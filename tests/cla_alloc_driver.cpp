@@ -2,7 +2,8 @@
  * Test driver of libclahip.so's behaviour when host memory runs out inside a call: its own operator new fails the k-th
  * allocation that the library makes during cla_mmchain, k = 0, 1, ... until the call gets through. Each failure has to
  * come back as an error code, and the block has to answer the next plain X %*% v as if nothing had happened (the weights
- * of the failed chain must not show in it).
+ * of the failed chain must not show in it). The same for cla_tsmm of a block of two wide groups, whose kernels add into an
+ * accumulator that the block keeps: the next t(X) %*% X must hold nothing of the failed one.
  *
  * Prints "ALLOC-DRIVER OK" at the end; exit code 0 only then.
  */
@@ -73,6 +74,46 @@ static cla_handle make_block(int kind, std::vector<double>& X) {
 	return h;
 }
 
+// t(X) %*% X of two groups of 8 columns with each allocation of the library failing in turn.
+static int gram_failures(int& thrown) {
+	enum { W = 8, M = 2 * W };
+	int fails = 0;
+	for(long k = 0;; k++) {
+		cla_handle h = cla_block_create(N, M);
+		std::vector<double> X((size_t) N * M), dict(7 * W), out(M * M);
+		for(int g = 0; h && g < 2; g++) {
+			std::vector<uint8_t> codes((size_t) N);
+			int32_t cols[W];
+			for(int c = 0; c < W; c++) cols[c] = g * W + c;
+			for(int i = 0; i < 7 * W; i++) dict[(size_t) i] = 1 + i % 13 + g;
+			for(int64_t r = 0; r < N; r++) {
+				codes[(size_t) r] = (uint8_t) ((r * (3 + g)) % 7);
+				for(int c = 0; c < W; c++) X[(size_t) r * M + g * W + c] = dict[(size_t) codes[(size_t) r] * W + c];
+			}
+			if(cla_block_add_ddc(h, cols, W, dict.data(), 7, codes.data(), 1) < 0) return 1;
+		}
+		if(!h || cla_block_finalize(h) < 0) { printf("gram block: %s\n", cla_last_error()); return 1; }
+		allocFailed = false;
+		allocLeft = k;
+		const int64_t rc = cla_tsmm(h, out.data());
+		allocLeft = -1;
+		if(allocFailed) thrown++;
+		if(allocFailed && rc >= 0) { printf("gram: allocation %ld failed without an error\n", k); fails++; }
+		if(!allocFailed && rc < 0) { printf("gram: %s\n", cla_last_error()); fails++; }
+		if(cla_tsmm(h, out.data()) < 0) { printf("gram: %s\n", cla_last_error()); fails++; }
+		int bad = 0;
+		for(int i = 0; i < M; i++)
+			for(int j = 0; j < M; j++) { // (whole numbers: exact)
+				double s = 0;
+				for(int64_t r = 0; r < N; r++) s += X[(size_t) r * M + i] * X[(size_t) r * M + j];
+				bad += out[(size_t) i * M + j] != s;
+			}
+		if(bad) { printf("gram, allocation %ld: %d cells of the next t(X) %%*%% X are wrong\n", k, bad); fails++; }
+		cla_block_free(h);
+		if(!allocFailed) return fails;
+	}
+}
+
 int main() {
 	if(cla_init(0) < 0) { fprintf(stderr, "cla_init: %s\n", cla_last_error()); return 2; }
 	int fails = 0, thrown = 0;
@@ -104,8 +145,10 @@ int main() {
 				cla_block_free(h);
 				if(!allocFailed) break;
 			}
-	printf("%d failed allocations\n", thrown);
-	if(fails || thrown < 4) { printf("FAIL\n"); return 1; }
+	int gramThrown = 0;
+	fails += gram_failures(gramThrown);
+	printf("%d + %d failed allocations\n", thrown, gramThrown);
+	if(fails || thrown < 4 || gramThrown < 2) { printf("FAIL\n"); return 1; }
 	printf("ALLOC-DRIVER OK\n");
 	return 0;
 }
