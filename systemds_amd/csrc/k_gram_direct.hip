@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <vector>
 
 namespace cla {
@@ -494,13 +495,13 @@ static bool gdr_spread(const unsigned long long* bins) {
 
 // P.spread, from the dense columns and P.codeSpread.
 static int gdr_look(cla_block* b, GdrPlan& P) {
-	P.spread = P.codeSpread ? 1 : 0;
+	int spread = P.codeSpread ? 1 : 0;
 	for(const HostGroup& H : b->groups) {
-		if(P.spread || P.A.nR == 0) return 0;
+		if(spread || P.A.nR == 0) break;
 		if(H.d.type != G_UNC) continue;
 		std::vector<unsigned long long> bins((size_t) H.d.nColG * GDR_BINS, 0);
 		const int rc = ensure_scratch(b, bins.size() * sizeof(bins[0]));
-		if(rc) { P.spread = -1; return rc; }
+		if(rc) return rc;
 		unsigned long long* d = (unsigned long long*) b->dScratch;
 		CLA_HIP(hipMemsetAsync(d, 0, bins.size() * sizeof(bins[0]), b->stream));
 		hipLaunchKernelGGL(k_exponents, dim3((unsigned) std::min<int64_t>((b->nRows + 2047) / 2048, 2 * g_numCU), (unsigned) H.d.nColG), dim3(256), 0, b->stream,
@@ -508,8 +509,9 @@ static int gdr_look(cla_block* b, GdrPlan& P) {
 		CLA_HIP(hipGetLastError());
 		CLA_HIP(hipMemcpyAsync(bins.data(), d, bins.size() * sizeof(bins[0]), hipMemcpyDeviceToHost, b->stream));
 		CLA_HIP(hipStreamSynchronize(b->stream));
-		for(int c = 0; c < H.d.nColG; c++) P.spread |= gdr_spread(&bins[(size_t) c * GDR_BINS]);
+		for(int c = 0; c < H.d.nColG; c++) spread |= gdr_spread(&bins[(size_t) c * GDR_BINS]);
 	}
+	P.spread = spread; // (only now: a call that fails on the way looks again)
 	return 0;
 }
 
@@ -681,10 +683,14 @@ int gdr_plan(cla_block* b, const GdrPlan*& P) {
 	if(b->gdrPlan == nullptr) {
 		int rc = ensure_expanded(b);
 		if(rc) return rc;
-		b->gdrPlan = new GdrPlan();
-		rc = gdr_build_plan(b, *b->gdrPlan);
-		if(rc < 0) { gdr_plan_drop(b); return rc; }
-		if(b->gdrPlan->dImg) b->derivedBytes += b->gdrPlan->bytes;
+		std::unique_ptr<GdrPlan> plan(new GdrPlan()); // (the block's only when it is complete)
+		rc = gdr_build_plan(b, *plan);
+		if(rc < 0) {
+			if(plan->dImg) (void) hipFree(plan->dImg);
+			return rc;
+		}
+		if(plan->dImg) b->derivedBytes += plan->bytes;
+		b->gdrPlan = plan.release();
 	}
 	P = b->gdrPlan;
 	return 0;

@@ -25,6 +25,7 @@
 #include "cla_runs.hpp"
 #include <algorithm>
 #include <cstring>
+#include <memory>
 
 namespace cla {
 
@@ -510,10 +511,14 @@ int gram_tiles_behind_decode(const cla_block* b) {
 // more kernel in front). Returns 1 when the block is not of this kernel's shape.
 int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz, bool ownByCounts) {
 	if(b->gtPlan == nullptr) {
-		b->gtPlan = new GtPlan();
-		const int rc = gt_build_plan(b, *b->gtPlan);
-		if(b->gtPlan->dImg) b->derivedBytes += b->gtPlan->bytes;
-		if(rc < 0) { gt_plan_drop(b); return rc; }
+		std::unique_ptr<GtPlan> plan(new GtPlan()); // (the block's only when it is complete: half a plan would refuse the block for good)
+		const int rc = gt_build_plan(b, *plan);
+		if(rc < 0) {
+			if(plan->dImg) (void) hipFree(plan->dImg);
+			return rc;
+		}
+		if(plan->dImg) b->derivedBytes += plan->bytes;
+		b->gtPlan = plan.release();
 	}
 	const GtPlan& P = *b->gtPlan;
 	if(P.rc) return P.rc;

@@ -101,6 +101,9 @@ static int gram_failures(int& thrown) {
 		if(allocFailed && rc >= 0) { printf("gram: allocation %ld failed without an error\n", k); fails++; }
 		if(!allocFailed && rc < 0) { printf("gram: %s\n", cla_last_error()); fails++; }
 		if(cla_tsmm(h, out.data()) < 0) { printf("gram: %s\n", cla_last_error()); fails++; }
+		char stats[2048] = "";
+		(void) cla_stats(h, stats, sizeof(stats));
+		if(!strstr(stats, "k_gram_tiles")) { printf("gram, allocation %ld: the next call took another kernel: %s\n", k, stats); fails++; }
 		int bad = 0;
 		for(int i = 0; i < M; i++)
 			for(int j = 0; j < M; j++) { // (whole numbers: exact)
