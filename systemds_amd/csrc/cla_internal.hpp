@@ -89,6 +89,7 @@ struct Options {
 	int sdcLanes = 1;       // SDCZeros mat-vecs on lane-major lists, one lane per group
 	int sdcRows = 1;        // SDCZeros right mat-vec on row lists, one lane per row
 	int tsmmOneKernel = 1;  // decoded Gram matrix of a whole block as the call's only kernel (0: a fill in front, k_tsmm_finish behind)
+	int chainFused = 1;     // multiply chain of single-column byte-code blocks in one pass over the codes (0: two products)
 	int ddcReorder = 1;     // finalize renumbers the tuples of large DDC dictionaries by descending count (0: the caller's numbering is kept)
 };
 
@@ -191,6 +192,7 @@ struct cla_block {
 	// of 16 groups at a time as [code][16] (maxVals codes)
 	double* dDictPad = nullptr;
 	size_t dictTOff = 0;
+	bool u8ColsDistinct = false;     // ... and no two of the groups share a column (an overlapping product's do)
 	int64_t dictPadBytes = 0;
 	// list of SDCZeros groups + prefix sums of their nVals, as the row-tile kernels read it;
 	// built on first use for all groups (sdcPlanGroup -1) or for one group (its index)
@@ -274,6 +276,7 @@ int launch_rmm_mfma(cla_block* b, const double* dB, int q, const double* dConstR
 	unsigned long long* dNnz);
 int launch_lmm_u8(cla_block* b, const double* dY, int p, double* dPre);
 int launch_lmm_u8_dot(cla_block* b, const double* dY, int p, double* dOut);
+int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz);
 int launch_lmm_u8_vec(cla_block* b, const double* dY, double* dOut);
 int launch_lmm_sdc_tiles(cla_block* b, const double* dY, int p, double* dPre, int onlyGroup, double* dOut);
 int launch_lmm_sdc_lanes(cla_block* b, const double* dY, int p, double* dOut);

@@ -399,6 +399,10 @@ __global__ __launch_bounds__(256) void k_sub_inplace(double* __restrict__ x, con
 
 int launch_mmchain(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz) {
 	const int64_t nRows = b->nRows;
+	{
+		const int r = launch_chain_u8(b, dV, dW, ctype, dOut, dNnz);
+		if(r <= 0) return r;
+	}
 	// the intermediate vector has a workspace of its own: the multiplies below may resize the shared scratch
 	const size_t need = (size_t) std::max<int64_t>(nRows, 1);
 	if(need > b->chainCap) {

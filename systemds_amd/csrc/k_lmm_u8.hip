@@ -316,6 +316,9 @@ int ensure_dict_pad(cla_block* b) {
 	CLA_HIP(hipMalloc((void**) &b->dDictPad, img.size() * sizeof(double)));
 	b->dictPadBytes = (int64_t) (img.size() * sizeof(double));
 	b->derivedBytes += b->dictPadBytes;
+	std::vector<int32_t> sorted(cols, cols + nG);
+	std::sort(sorted.begin(), sorted.end());
+	b->u8ColsDistinct = std::adjacent_find(sorted.begin(), sorted.end()) == sorted.end();
 	CLA_HIP(hipMemcpy(b->dDictPad, img.data(), img.size() * sizeof(double), hipMemcpyHostToDevice));
 	return 0;
 }

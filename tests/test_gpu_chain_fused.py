@@ -1,0 +1,95 @@
+"""The multiply chain of single-column byte-code blocks in one pass (k_chain_u8): row and column edges, weights, columns without a
+group, non-finite operands; against the exact chain, and against the two products where the exact one says nothing."""
+import numpy as np
+import pytest
+
+from parity import assert_matches_truth
+
+pytestmark = pytest.mark.gpu
+
+
+def block(cla, rng, n_rows, n_cols, n_vals, gaps=0, zeros=False):
+    from systemds_amd import synth
+    at = np.sort(rng.permutation(n_cols + gaps)[:n_cols])
+    specs = []
+    for c in at:
+        d = rng.standard_normal((n_vals, 1))
+        if zeros:
+            d[rng.integers(0, n_vals)] = 0.0
+        specs.append(synth.GroupSpec("ddc", np.array([c], np.int32), d, rng.integers(0, n_vals, n_rows).astype(np.uint8)))
+    return specs, cla.build_block(n_rows, n_cols + gaps, specs)
+
+
+def names_of(blk):
+    return [k["name"] for k in blk.stats()["kernels"]]
+
+
+@pytest.mark.parametrize("ctype", [0, 1, 2])
+@pytest.mark.parametrize("n_rows, n_cols, n_vals", [
+    (1, 1, 1), (63, 16, 2), (64, 17, 256), (65, 5, 3), (511, 33, 200), (513, 48, 256), (1025, 64, 256), (4097, 65, 100),
+    (16385, 80, 250), (33000, 96, 150), (131073, 112, 150), (262143, 20, 16), (100001, 100, 7)])
+def test_chain_in_one_pass(cla, ora, n_rows, n_cols, n_vals, ctype):
+    rng = np.random.default_rng(n_rows * 3 + ctype)
+    specs, blk = block(cla, rng, n_rows, n_cols, n_vals, gaps=ctype)
+    n_cols += ctype
+    v, w = rng.standard_normal((n_cols, 1)), rng.standard_normal((n_rows, 1))
+    for _ in range(2):  # (the second call finds the first one's tickets and workspace)
+        out, nnz = blk.mmchain(v, w if ctype else None, ctype)
+        names = names_of(blk)
+    blk.close()
+    assert names == ["k_chain_u8"], names
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    xv = D.astype(np.longdouble) @ v.astype(np.longdouble)
+    u = xv * w if ctype == 1 else xv - w if ctype == 2 else xv
+    # like terms of t(X) %*% u and the rounding of u itself (n_cols terms each) stay below 1e-12 of the sums' magnitudes
+    scale = np.abs(D).T @ (np.abs(D) @ np.abs(v) * (np.abs(w) if ctype == 1 else 1.0) + (np.abs(w) if ctype == 2 else 0.0))
+    want = D.astype(np.longdouble).T @ u
+    assert np.all(np.abs(out.reshape(-1, 1) - want) <= 1e-12 * scale + 1e-300)
+    assert nnz == np.count_nonzero(out)
+
+
+def test_blocks_it_does_not_take(cla, ora):
+    """Tables beyond LDS, more than 7 column blocks, constants, the options: two products, the same result."""
+    rng = np.random.default_rng(5)
+    from systemds_amd import synth
+    n_rows = 3001
+    for n_cols, n_vals, extra, option in [(100, 256, None, None), (113, 4, None, None), (20, 9, "const", None), (20, 9, None, ("chain_fused", 0)),
+                                          (20, 9, None, ("lmm_disable", 1)), (20, 9, None, ("rmm_disable", 2))]:
+        specs, blk = block(cla, rng, n_rows, n_cols, n_vals)
+        if extra:
+            blk.close()
+            specs = specs + [synth.GroupSpec("const", np.array([n_cols], np.int32), np.array([[0.5]]))]
+            n_cols += 1
+            blk = cla.build_block(n_rows, n_cols, specs)
+        if option:
+            blk.set_option(*option)
+        v, w = rng.standard_normal((n_cols, 1)), rng.standard_normal((n_rows, 1))
+        out, _ = blk.mmchain(v, w, 1)
+        names = names_of(blk)
+        blk.close()
+        assert "k_chain_u8" not in names, (n_cols, n_vals, extra, option)
+        D = ora.np_decompress(specs, n_rows, n_cols)
+        assert_matches_truth(out.reshape(-1, 1), D.T, (D @ v) * w, what="chain as two products")
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("where", ["v", "w"])
+def test_non_finite_operands(cla, value, where):
+    """A zero dictionary cell meets no infinity of v; everything else as the two products give it."""
+    rng = np.random.default_rng(9)
+    n_rows, n_cols = 5000, 37
+    _, blk = block(cla, rng, n_rows, n_cols, 5, zeros=True)
+    v, w = rng.standard_normal((n_cols, 1)), np.abs(rng.standard_normal((n_rows, 1))) + 0.1
+    (v if where == "v" else w)[11] = value
+    got = {}
+    for fused in (1, 0):
+        blk.set_option("chain_fused", fused)
+        got[fused], nnz = blk.mmchain(v, w, 1)
+        assert ("k_chain_u8" in names_of(blk)) == bool(fused)
+        assert nnz == np.count_nonzero(got[fused])
+    blk.close()
+    assert np.array_equal(np.isnan(got[0]), np.isnan(got[1]))
+    assert np.array_equal(got[0][~np.isfinite(got[0])], got[1][~np.isfinite(got[1])], equal_nan=True)
+    fin = np.isfinite(got[0])
+    # (sums of 5000 terms: 5000 x 2^-53 of their magnitude apart at most, and they do not cancel to less than 1e-3 of it here)
+    np.testing.assert_allclose(got[1][fin], got[0][fin], rtol=1e-9)
