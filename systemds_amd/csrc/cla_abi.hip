@@ -283,7 +283,7 @@ cla_handle cla_block_create(int64_t nRows, int32_t nCols) {
 	b->constV.assign((size_t) nCols, 0.0);
 	if(hipStreamCreate(&b->stream) != hipSuccess) { set_error("hipStreamCreate failed"); delete b; return nullptr; }
 	b->ownStream = true;
-	constexpr size_t counterBytes = NNZ_SLOTS * NNZ_BYTES + 2 * NNZ_STEP * sizeof(unsigned long long); // the counters, two ticket lines
+	constexpr size_t counterBytes = NNZ_SLOTS * NNZ_BYTES + 2 * (1 + TICKET_WAYS) * NNZ_STEP * sizeof(unsigned long long); // the counters, two tickets
 	if(hipMalloc((void**) &b->dCounters, counterBytes) != hipSuccess ||
 		hipHostMalloc((void**) &b->hCounters, NNZ_BYTES) != hipSuccess) {
 		set_error("allocating counters failed");

@@ -27,6 +27,7 @@ constexpr int UPLOAD_SLACK = 128;
 constexpr int NNZ_WAYS = 64, NNZ_STEP = 16;
 constexpr int NNZ_SLOT = NNZ_WAYS * NNZ_STEP; // words of a counter
 constexpr size_t NNZ_BYTES = (size_t) NNZ_SLOT * 8;
+constexpr int TICKET_WAYS = 8;                // a ticket is counted on this many lines and a line for these (last_block)
 constexpr int NNZ_SLOTS = 4;                  // counters of a block (cla_block::nnzSlot)
 
 // Iterator state of an offset list in front of delta entry `idx`:
@@ -226,9 +227,9 @@ struct cla_block {
 	uint32_t* dSdcPacked = nullptr;  // all listed groups' entries as (code << 16 | row inside its 4096-row tile), built on first use
 	int sdcPlanGroup = -2;
 	std::vector<int32_t> sdcList, sdcBinOff;
-	unsigned long long* dCounters = nullptr;   // NNZ_SLOTS non-zero counters, then a line each for the ticket counters below
+	unsigned long long* dCounters = nullptr;   // NNZ_SLOTS non-zero counters, then the lines of the tickets below
 	unsigned* lmm_ticket() { return (unsigned*) (dCounters + cla::NNZ_SLOTS * cla::NNZ_SLOT); }   // of the left multiply's tail
-	unsigned* gram_ticket() { return (unsigned*) (dCounters + cla::NNZ_SLOTS * cla::NNZ_SLOT + cla::NNZ_STEP); } // of the Gram kernels' tail
+	unsigned* gram_ticket() { return (unsigned*) (dCounters + cla::NNZ_SLOTS * cla::NNZ_SLOT + (1 + cla::TICKET_WAYS) * cla::NNZ_STEP); } // of the Gram kernels' tail
 	unsigned long long* nnz_counter(int slot) { return dCounters + (size_t) slot * cla::NNZ_SLOT; }
 	double* dGramAcc = nullptr;      // nCols x nCols, zero between calls: where the blocks of a one-kernel t(X) %*% X add (gram_tail)
 	unsigned long long* hCounters = nullptr;   // pinned

@@ -169,27 +169,34 @@ struct RunCursors {
 // block's LDS that nobody else uses any more (no static LDS here: the Gram kernels address theirs from offset zero).
 __device__ __forceinline__ void gram_tail(unsigned* done, unsigned nBlocks, double* acc, double* out, int nCols, unsigned long long* nnz,
 	unsigned* lds) {
-	unsigned& gramTicketS = lds[0];
+	int& lastS = (int&) lds[0];
 	int* const gramPartS = (int*) lds + 1;
 	// this thread's adds have been acknowledged before the block takes its ticket (the adds, the ticket and the reads
 	// below are all performed at device scope, past the caches that the chip's parts do not share)
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 	__syncthreads();
-	if(threadIdx.x == 0) gramTicketS = atomicAdd(done, 1u);
+	if(threadIdx.x == 0) lastS = last_block(done, nBlocks);
 	__syncthreads();
-	if(gramTicketS != nBlocks - 1) return;
+	if(!lastS) return;
 	int cnt = 0;
-	for(int idx = threadIdx.x; idx < nCols * nCols; idx += blockDim.x) {
-		const int i = idx / nCols, j = idx - i * nCols;
-		if(j < i) continue;
-		unsigned long long* cell = (unsigned long long*) acc + idx;
-		const unsigned long long bits = __hip_atomic_load(cell, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		__hip_atomic_store(cell, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		double v;
-		__builtin_memcpy(&v, &bits, 8);
-		out[idx] = v;
-		out[(size_t) j * nCols + i] = v;
-		cnt += v != 0.0 ? (i == j ? 1 : 2) : 0;
+	// eight cells per thread requested together: each is a round trip past the caches
+	const int n = nCols * nCols;
+	for(int idx0 = threadIdx.x; idx0 < n; idx0 += 8 * blockDim.x) {
+		unsigned long long bits[8];
+#pragma unroll
+		for(int k = 0; k < 8; k++)
+			bits[k] = __hip_atomic_load((const unsigned long long*) acc + min(idx0 + k * (int) blockDim.x, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+		for(int k = 0; k < 8; k++) {
+			const int idx = idx0 + k * (int) blockDim.x, i = idx / nCols, j = idx - i * nCols;
+			if(idx >= n || j < i) continue;
+			__hip_atomic_store((unsigned long long*) acc + idx, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			double v;
+			__builtin_memcpy(&v, &bits[k], 8);
+			out[idx] = v;
+			out[(size_t) j * nCols + i] = v;
+			cnt += v != 0.0 ? (i == j ? 1 : 2) : 0;
+		}
 	}
 	cnt = wave_sum_i32(cnt);
 	if((threadIdx.x & (WAVE - 1)) == 0) gramPartS[threadIdx.x >> 6] = cnt;
@@ -199,7 +206,6 @@ __device__ __forceinline__ void gram_tail(unsigned* done, unsigned nBlocks, doub
 		int s = 0;
 		for(unsigned w = 0; w < (blockDim.x + WAVE - 1) / WAVE; w++) s += gramPartS[w];
 		*nnz = (unsigned long long) s;
-		*done = 0;
 	}
 }
 

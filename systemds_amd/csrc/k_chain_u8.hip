@@ -55,7 +55,7 @@ __global__ __launch_bounds__(CH_THREADS, NCB <= 3 ? 4 : 2) void k_chain_u8(const
 	int minus, int64_t nRows, double* __restrict__ part, double* __restrict__ out, int nCols, unsigned* __restrict__ done,
 	unsigned long long* __restrict__ nnz) {
 	extern __shared__ __attribute__((aligned(16))) double smem[]; // the dictionaries; at the end the sums
-	__shared__ unsigned ticketS;
+	__shared__ int lastS;
 	__shared__ int cntS[CH_WAVES];
 	constexpr int NC = NCB * 16;
 	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -210,9 +210,9 @@ __global__ __launch_bounds__(CH_THREADS, NCB <= 3 ? 4 : 2) void k_chain_u8(const
 	}
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 	__syncthreads();
-	if(tid == 0) ticketS = atomicAdd(done, 1u);
+	if(tid == 0) lastS = last_block(done, gridDim.x);
 	__syncthreads();
-	if(ticketS != gridDim.x - 1) return;
+	if(!lastS) return;
 	// the last block: the others' sums in block order, a share of the blocks per group of NC threads
 	constexpr int NP = CH_THREADS / NC;
 	const int col = tid % NC, share = tid / NC;
@@ -250,7 +250,6 @@ __global__ __launch_bounds__(CH_THREADS, NCB <= 3 ? 4 : 2) void k_chain_u8(const
 		int n = 0;
 		for(int i = 0; i < CH_WAVES; i++) n += cntS[i];
 		*nnz = (unsigned long long) n;
-		*done = 0;
 	}
 }
 
