@@ -270,6 +270,8 @@ int reorder_ddc_by_count(cla_block* b, int group);
 int launch_sdc_build(cla_block* b, HostGroup& g);
 int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned long long* dNnz, int squares = 0,
 	double* ws = nullptr, size_t wsDoubles = 0, RowOp* op = nullptr);
+int launch_rmm_q1_u8_few(cla_block* b, const double* dB, const double* constTerm, double* dOut, unsigned long long* dNnz, unsigned long long* nnzNext,
+	const RowOp& op);
 int launch_tables(cla_block* b, const double* dB, int q); // dict x B of every group (+ constV x B) into b->dTables
 int launch_aggregate(cla_block* b, int op, int dir, double* dOut, unsigned long long* dNnz);
 int ensure_counts(cla_block* b);

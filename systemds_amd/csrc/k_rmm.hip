@@ -621,8 +621,17 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 		const int per = pad20 < pad16 ? 20 : 16;
 		const double* constTerm = constRow >= 0 ? tables + constRow : nullptr;
 		unsigned long long* nnzNext = fused ? b->nnz_counter(b->nnzRot % 3 + 1) : nullptr;
-		Prof pf(b, "k_rmm_q1_u8", grid, THREADS, per * 256 * 8, bytes);
 		const RowOp rowOp = op != nullptr ? *op : RowOp();
+		if(fused) {
+			const int r = launch_rmm_q1_u8_few(b, dB, constTerm, dOut, dNnz, nnzNext, rowOp);
+			if(r < 0) return r;
+			if(r == 0) {
+				if(op != nullptr) op->done = true;
+				b->nnzRot = b->nnzRot % 3 + 1;
+				return 0;
+			}
+		}
+		Prof pf(b, "k_rmm_q1_u8", grid, THREADS, per * 256 * 8, bytes);
 #define U8_LAUNCH_OP(PER, NBV, LB, LN, F, O)                                                                    \
 	hipLaunchKernelGGL((k_rmm_q1_u8<THREADS, PER, NBV, LB, LN, F, O>), dim3(grid), dim3(THREADS), 0, st, b->dArena, \
 		b->arenaStride, nG, F ? b->dDictPad : dTpad, constTerm, dOut, nRows, dNnz, dCol0, dB, nnzNext, rowOp)
