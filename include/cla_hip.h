@@ -124,8 +124,9 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *   lmm_joint       1 / 0: Y %*% X (16 rows of Y per pass) on a block that is not mostly offset lists in passes over the decoded
  *                   rows, on the vector unit (see tsmm_direct) or on the matrix cores; blocks of more than 64 columns, or
  *                   whose code tiles exceed LDS together, go chunk of columns by chunk (sub-blocks kept with the block);
- *                   not single-column byte-code blocks, except with bit 0 of lmm_disable (the kernel reports non-finite
- *                   values of Y and the host looks, i.e. waits for the stream once per call; such a Y takes the bin kernels)
+ *                   not single-column byte-code blocks, except with bit 0 of lmm_disable (a row of a
+ *                   non-finite Y that a group does not cover stays out of its sums: decided on the device; chunk of
+ *                   columns by chunk the host looks, i.e. waits for the stream once per call, and such a Y takes the bin kernels)
  *   tsmm_one_kernel 1 / 0: t(X) %*% X of a whole block of at most 64 columns (all-DDC: 128) on the decoded Gram kernels as the call's only
  *                   kernel (a few wide DDC groups: behind the kernel of the cells inside a group; its blocks add into an
  *                   accumulator kept with the block, nCols x nCols doubles; the last block

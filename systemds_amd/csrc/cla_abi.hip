@@ -1524,30 +1524,21 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 	if(b->nCols > 64) return launch_lmm_chunked(b, dY, p, dOut, dNnz);
 	hipStream_t st = b->stream;
 	const size_t n = (size_t) p * b->nCols;
-	int rc = ensure_stage(&b->dStageOut, &b->stageOutCap, n);
+	// the sums, room for the product anew where Y holds a non-finite value (p row sums behind it), the kernel's report of one, a count. Not
+	// in the output staging buffer, which may be the caller's dOut.
+	const size_t nWs = 2 * n + (size_t) p + 2;
+	int rc = ensure_tables(b, nWs);
 	if(rc) return rc;
-	CLA_HIP(hipMemsetAsync(b->dStageOut, 0, n * sizeof(double), st));
-	CLA_HIP(hipMemsetAsync(dNnz, 0, NNZ_BYTES, st));
+	double* const ws = b->dTables;
+	unsigned long long* const dBad = (unsigned long long*) (ws + nWs - 2);
+	CLA_HIP(hipMemsetAsync(ws, 0, nWs * sizeof(double), st));
 	for(int p0 = 0; p0 < p; p0 += 16) // 16 rows of Y per pass over the block
-		if((rc = launch_lmm_decode(b, dY + (size_t) p0 * b->nRows, std::min(16, p - p0), b->dStageOut + (size_t) p0 * b->nCols, dNnz))) {
+		if((rc = launch_lmm_decode(b, dY + (size_t) p0 * b->nRows, std::min(16, p - p0), ws + (size_t) p0 * b->nCols, dBad))) {
 			if(rc == 1 && p0 == 0) return launch_lmm_chunked(b, dY, p, dOut, dNnz); // (nothing queued yet)
 			if(p0 > 0) clear_stats(b);
 			return rc;
 		}
-	{
-		// A row that a group does not cover (outside its runs or its offset list) does not enter that group's sums in
-		// the reference, whatever Y holds there; as a decoded 0.0 it turns an infinite Y into NaN. The kernel reports a
-		// non-finite value of Y, and such a Y takes the bin kernels (the host has to look: one wait for the stream).
-		unsigned long long bad = 0;
-		CLA_HIP(hipMemcpyAsync(&bad, dNnz, sizeof(bad), hipMemcpyDeviceToHost, st));
-		CLA_HIP(hipStreamSynchronize(st));
-		if(bad) { clear_stats(b); return 1; }
-	}
-	{ // (the counter is still zero: the kernel writes nothing but that flag into it)
-		Prof pf(b, "k_take_block", ((int) n + 255) / 256, 256, 0, 0);
-		hipLaunchKernelGGL(k_take_block, dim3((unsigned) std::min(((int) n + 255) / 256, 1024)), dim3(256), 0, st, b->dStageOut, b->nCols, 0, 0, p,
-			b->nCols, dOut, dNnz);
-	}
+	if((rc = launch_lmm_take(b, dY, p, ws, dOut, dNnz))) return rc;
 	CLA_HIP(hipGetLastError());
 	return 0;
 }

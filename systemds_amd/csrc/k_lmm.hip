@@ -219,6 +219,185 @@ __global__ __launch_bounds__(256) void k_lmm_finish(double* __restrict__ out, in
 	count_add(nnz, cnt);
 }
 
+// Behind a Y %*% X on decoded rows: takes the result out of its stage and counts the non-zeros. The kernels on decoded rows give
+// a row that a group does not cover the value 0.0, which an infinite Y turns into NaN; in the reference such a row does not enter the
+// group's sums. They report a non-finite Y in *bad, and then the blocks of this kernel form the product anew, from every group's
+// own rows only, row sums times constants apart, as the bin kernels do (ColGroupRLE.java:759-796, AOffset.java:288-430). The flag stays on the
+// device: the host looking at it cost 15 - 20 us per call (wait, copy, and the launches behind it), a mixed block of 5,000,011 x 20 by 6 rows
+// 114 us per call against 93 us.
+constexpr int LT_THREADS = 512;
+constexpr int LT_P = 8;            // rows of Y per look at a group's codes
+constexpr int LT_COLS = 64;        // most columns of a block
+struct LmmTake {
+	const DGroup* groups;
+	int nGroups;
+	const double* Y;
+	int p;
+	int64_t nRows;
+	const double* stage;           // p x nCols, what the kernel in front has summed
+	double* anew;                  // p x nCols and p row sums, zero
+	const unsigned long long* bad;
+	unsigned long long* count;     // zero
+	const double* constV;          // nullptr: no constants
+	double* out;
+	int nCols;
+	unsigned* done;
+	unsigned long long* nnz;
+};
+
+__global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
+	__shared__ int lastS;
+	__shared__ int cntS[LT_THREADS / WAVE];
+	__shared__ double sumS[LT_P * (LT_COLS + 1)]; // the block's sums of some rows of Y: by column, then the row sum
+	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = A.p * A.nCols;
+	double* const rs = A.anew + n;
+	const bool anew = *A.bad != 0;
+	const int nTake = min((int) gridDim.x, (n + LT_THREADS * 4 - 1) / (LT_THREADS * 4)); // blocks that take the result out of its stage
+	if(!anew && (int) blockIdx.x >= nTake) return;
+	if(anew) {
+		auto product = [&](auto pTag) { // a few rows of Y per look at a group's codes
+			constexpr int LP = decltype(pTag)::value;
+			const int64_t r0 = A.nRows * blockIdx.x / gridDim.x, r1 = A.nRows * (blockIdx.x + 1) / gridDim.x;
+			for(int i0 = 0; i0 < A.p; i0 += LP) {
+				const double* y[LP];
+#pragma unroll
+				for(int i = 0; i < LP; i++) y[i] = A.Y + (size_t) min(i0 + i, A.p - 1) * A.nRows;
+				const int np = min(LP, A.p - i0);
+				for(int i = tid; i < LP * (LT_COLS + 1); i += LT_THREADS) sumS[i] = 0.0;
+				__syncthreads();
+				// (4096 waves' adds to a cell in memory, 11.4 ns each, were most of the time: in LDS first)
+				auto give_all = [&](const double (&s)[LP], int col) {
+#pragma unroll
+					for(int i = 0; i < LP; i++)
+						if(i < np) {
+							const double w = wave_sum_f64(s[i]);
+							if(lane == 0) unsafeAtomicAdd(&sumS[i * (LT_COLS + 1) + col], w);
+						}
+				};
+				for(int g = 0; g < A.nGroups; g++) {
+					const DGroup G = dgroup(A.groups + g);
+					for(int h = 0; h < G.nColG; h++) {
+						double s[LP] = {};
+						if(G.type == G_DDC || G.type == G_UNC) {
+#pragma unroll 2
+							for(int64_t r = r0 + tid; r < r1; r += LT_THREADS) {
+								const double x = G.type == G_DDC ? G.dict[(size_t) load_code(G.codes, G.codeWidth, r) * G.nColG + h] : G.dense[(size_t) r * G.nColG + h];
+#pragma unroll
+								for(int i = 0; i < LP; i++) s[i] += y[i][r] * x;
+							}
+						}
+						else if(G.type == G_RLE && G.nRuns > 0) {
+							int64_t r = r0 + tid;
+							int j = r < r1 ? rle_find(G.runStart, G.nRuns, (int32_t) r) : 0;
+							for(; r < r1; r += LT_THREADS) {
+								while(G.runStart[j + 1] <= r) j++; // (the last run ends at the last row)
+								const int code = G.runCode[j];
+								if(code < 0) continue;
+								const double x = G.dict[(size_t) code * G.nColG + h];
+#pragma unroll
+								for(int i = 0; i < LP; i++) s[i] += y[i][r] * x;
+							}
+						}
+						else if(G.type == G_SDCZ && G.nOffsets > 0) {
+							auto take = [&](int64_t row, int idx) {
+								const double x = G.dict[(size_t) load_code(G.codes, G.codeWidth, idx) * G.nColG + h];
+#pragma unroll
+								for(int i = 0; i < LP; i++) s[i] += y[i][row] * x;
+							};
+							if(blockIdx.x == 0 && tid == 0) take(G.first, 0);
+							if(wave < SDC_CK / 256) for(int c = blockIdx.x; c < G.nCkpt; c += gridDim.x) { // (a wave takes 256 entries of a chunk)
+								const OffState st = G.ckpt[c];
+								int32_t row = st.row, emit = st.emit, rows[4], didx[4];
+								unsigned mask;
+								const int64_t base = (int64_t) c * SDC_CK;
+								for(int w = 0; w <= wave; w++) {
+									if(G.deltaWidth == 1) sdc_decode256<1>(G.deltas, G.nDeltas, base + w * 256, row, emit, rows, didx, mask);
+									else sdc_decode256<2>(G.deltas, G.nDeltas, base + w * 256, row, emit, rows, didx, mask);
+								}
+#pragma unroll
+								for(int k = 0; k < 4; k++)
+									if(mask & (1u << k)) take(rows[k], didx[k]);
+							}
+						}
+						give_all(s, G.cols[h]);
+					}
+				}
+				if(A.constV != nullptr) {
+					double s[LP] = {};
+					for(int64_t r = r0 + tid; r < r1; r += LT_THREADS)
+#pragma unroll
+						for(int i = 0; i < LP; i++) s[i] += y[i][r];
+					give_all(s, LT_COLS);
+				}
+				__syncthreads();
+				for(int idx = tid; idx < np * (LT_COLS + 1); idx += LT_THREADS) {
+					const int i = idx / (LT_COLS + 1), c = idx % (LT_COLS + 1);
+					if(sumS[idx] != 0.0) unsafeAtomicAdd(c < LT_COLS ? A.anew + (size_t) (i0 + i) * A.nCols + c : rs + i0 + i, sumS[idx]); // (a NaN is unequal to zero)
+				}
+				__syncthreads();
+			}
+		};
+		if(A.p <= 2) product(std::integral_constant<int, 2>());
+		else product(std::integral_constant<int, LT_P>());
+		asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (see lmm_tail)
+		__syncthreads();
+		if(tid == 0) lastS = last_block(A.done, gridDim.x);
+		__syncthreads();
+		if(!lastS) return;
+	}
+	auto summed = [&](const double* at) {
+		return __longlong_as_double((long long) __hip_atomic_load((const unsigned long long*) at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+	};
+	int cnt = 0;
+	const int step = LT_THREADS * (anew ? 1 : nTake);
+	for(int idx = tid + (anew ? 0 : (int) blockIdx.x * LT_THREADS); idx < n; idx += step) {
+		double v;
+		if(anew) {
+			v = summed(A.anew + idx);
+			if(A.constV != nullptr) { // (skipped for a row sum of zero, as in k_lmm_finish)
+				const double vl = summed(rs + idx / A.nCols);
+				if(vl != 0.0) v += vl * A.constV[idx % A.nCols];
+			}
+		}
+		else v = A.stage[idx];
+		A.out[idx] = v;
+		cnt += v != 0.0;
+	}
+	cnt = wave_sum_i32(cnt);
+	if(lane == 0) cntS[wave] = cnt;
+	__syncthreads();
+	if(tid == 0) {
+		unsigned long long s = 0;
+		for(int w = 0; w < LT_THREADS / WAVE; w++) s += (unsigned) cntS[w];
+		lastS = 1;
+		if(!anew && nTake > 1) {
+			atomicAdd(A.count, s);
+			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+			lastS = last_block(A.done, nTake);
+			s = __hip_atomic_load(A.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		}
+		if(lastS) // (the way that the counter's reader adds up first; the others are cleared below)
+			A.nnz[0] = s;
+	}
+	__syncthreads();
+	if(lastS && tid > 0 && tid < NNZ_WAYS) A.nnz[tid * NNZ_STEP] = 0;
+}
+
+int launch_lmm_take(cla_block* b, const double* dY, int p, double* ws, double* dOut, unsigned long long* dNnz) {
+	const size_t n = (size_t) p * b->nCols;
+	LmmTake A;
+	A.groups = b->dGroups; A.nGroups = (int) b->groups.size();
+	A.Y = dY; A.p = p; A.nRows = b->nRows; A.nCols = b->nCols;
+	A.stage = ws; A.anew = ws + n; A.bad = (const unsigned long long*) (ws + 2 * n + p); A.count = (unsigned long long*) (ws + 2 * n + p + 1);
+	A.constV = b->hasConst ? b->dConstV : nullptr;
+	A.out = dOut; A.done = b->lmm_ticket(); A.nnz = dNnz;
+	const unsigned grid = (unsigned) std::max<int64_t>(1, std::min<int64_t>((b->nRows + 1023) / 1024, g_numCU));
+	Prof pf(b, "k_take_block", grid, LT_THREADS, 0, 0);
+	hipLaunchKernelGGL(k_take_block, dim3(grid), dim3(LT_THREADS), 0, b->stream, A);
+	CLA_HIP(hipGetLastError());
+	return 0;
+}
+
 // dOut != nullptr (whole-block calls): groups whose products can be summed directly write into dOut
 // and leave their part of dPre zero.
 static int run_preagg(cla_block* b, const double* dY, int p, double* dPre, int onlyGroup, double* dOut) {

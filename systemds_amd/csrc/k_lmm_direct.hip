@@ -16,8 +16,9 @@
 // More rows of Y than 6 (8 where at most 8 columns vary) take passes (the sums of 12 columns by 6 rows are 144 registers; two
 // waves per SIMD; what spills from two rows per lane there cost 60 of 154 us, so such shapes take one).
 // Bound: HBM (Y once, the streams once per pass; vector memory path 67 % busy, vector issue 40 %), 14 us of start and end. 5,000,011 x
-// 20 (8 run-length, 8 two-byte, 2 offset-list, 2 dense columns) by 6 rows of Y 88 us (414 MB: 4.7 TB/s). Calls, with the host's look at
-// the flag: by 6 301 -> 114 us, by 1 284 -> 77, by 16 361 -> 269; 1,250,000 rows by 6 110 -> 59.
+// 20 (8 run-length, 8 two-byte, 2 offset-list, 2 dense columns) by 6 rows of Y 88 us (414 MB: 4.7 TB/s). Calls, with the fill in
+// front and k_take_block behind (k_lmm_decode with a host's look at Y; this kernel with one): by 6 301, 114 -> 93 us, by 13 241 -> 220; 1,000,000
+// rows by 6 58 -> 34, 100,000 by 2 40 -> 16.
 #include "../../include/cla_hip.h"
 #include "cla_gdr.hpp"
 #include <algorithm>
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(LD_THREADS, 2) void k_lmm_direct(const GdrArgs A, c
 }
 
 // dOut (p x nCols, zeroed) += Y %*% D of the decoded rows, constants included; *dBad is set when Y holds a value that is not
-// finite (dOut is then not used). Returns 1 when the block is not of this kernel's shape.
+// finite (dOut is then not used, see k_take_block). Returns 1 when the block is not of this kernel's shape.
 int launch_lmm_direct(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dBad) {
 	if(!b->opt.tsmmDirect || b->crossSplit > 0 || b->crossBlocks > 0) return 1;
 	const GdrPlan* P = nullptr;
