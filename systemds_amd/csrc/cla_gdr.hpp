@@ -1,31 +1,32 @@
 // Blocks of a few "varying" columns (one value per row behind a plain stream) next to run-length columns: the plan that the
-// kernels on decoded rows with lane = row share (k_gram_direct.hip, k_lmm_direct.hip).
+// kernels without tiles share (k_gram_direct.hip, k_lmm_direct.hip).
 #pragma once
 #include "cla_runs.hpp"
 
 namespace cla {
 
-struct GdrCol {            // 24 bytes
-	int32_t ringOff;       // bytes from the start of a ring buffer: the column's code / value of the chunk's first row
-	int32_t base8;         // bytes from the LDS base: the column's values by tuple
-	int32_t stride;        // bytes per row of the stream in the ring
+// A varying column as the Gram kernel reads it.
+struct GdrCol {            // 32 bytes
+	const uint8_t* src;    // its codes; a dense column: codes 0, n, 2 n .. 7 n of eight rows in the wave's copy of its group, n columns wide
+	int32_t bpr;           // bytes per row of src (1 or 2); 0: a dense column
+	int32_t base8;         // bytes from the LDS base: the column's values by tuple; a dense column: its place in a row, in bytes
+	int32_t dense0;        // -1: behind codes; else the dense columns in front of its group's
+	int32_t width;         // a dense column: of its group
 	int32_t col;           // column of the matrix
-	int32_t pad[2];
+	int32_t pad;
 };
-struct GdrStream {         // what the ring holds per chunk: bpr * GDR_CH consecutive bytes of each stream
+struct GdrDense {          // a group of dense columns, fetched as it lies
 	const uint8_t* src;
 	int32_t bpr;           // bytes per row
-	int32_t piece0;        // first 16-byte piece of the stream in a ring buffer
+	int32_t before;        // columns of the groups in front
 };
 struct GdrArgs {
 	const GdrCol* cols;
 	const double* vals;    // values of the code columns by tuple, constants added: the head of LDS as it is
 	const RunCol* runs;
-	const GdrStream* streams;
-	int nV, n2, n12, nR, nStreams; // columns [0, n2) two-byte codes, [n2, n12) one-byte codes, [n12, nV) dense
-	int packed;            // every code column has a stream of its own and the dense columns are one uncompressed group: the ring is columns in order
+	const GdrDense* dense;
+	int nV, nR, nDense;        // varying columns, run-length columns, dense groups
 	int valDoubles;        // even
-	int ringBytes;         // one ring buffer
 	int64_t nRows;
 	double* out;
 	int nCols;
@@ -49,9 +50,10 @@ struct GdrPlan {
 	int rc = 1;            // 0 usable, 1 the block does not qualify
 	void* dImg = nullptr;
 	int64_t bytes = 0;
-	size_t lds = 0;
+	size_t lds = 0;        // of k_tsmm_direct, which these belong to as well: quads of varying columns, pieces of dense values per lane, waves per block
+	int quads = 0, densePieces = 0, waves = 0;
 	GdrArgs A;
-	int spread = -1;       // 1: a varying column next to run-length columns spans too many magnitudes for summation by parts; -1: not looked at yet
+	int spread = -1;       // 1: a varying column next to run-length columns spans too many magnitudes (GDR_SPREAD); -1: not looked at yet
 	bool codeSpread = false; // the same of the columns behind codes, from their dictionaries
 	LdCols ld;             // ldNC code columns (fillers behind the real ones), ldND dense ones; ldNC == 0: no such form
 	int ldNC = 0, ldND = 0;
