@@ -108,9 +108,15 @@ int ensure_scratch(cla_block* b, size_t bytes) {
 
 int ensure_gram_acc(cla_block* b) {
 	if(b->dGramAcc != nullptr) return 0;
-	const size_t bytes = sizeof(double) * std::max<size_t>((size_t) b->nCols * b->nCols, 1);
-	CLA_HIP(hipMalloc((void**) &b->dGramAcc, bytes));
-	CLA_HIP(hipMemset(b->dGramAcc, 0, bytes));
+	const size_t bytes = sizeof(double) * (1 + GRAM_WAYS) * std::max<size_t>((size_t) b->nCols * b->nCols, 1);
+	double* acc = nullptr;
+	CLA_HIP(hipMalloc((void**) &acc, bytes));
+	if(hipMemset(acc, 0, bytes) != hipSuccess) { // (the block's only when it holds zeros)
+		(void) hipFree(acc);
+		set_error("clearing the Gram accumulator failed");
+		return -CLA_ERR_DEVICE;
+	}
+	b->dGramAcc = acc;
 	return 0;
 }
 

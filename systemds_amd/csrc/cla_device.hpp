@@ -90,15 +90,19 @@ __device__ __forceinline__ void count_add(unsigned long long* counter, int local
 // the counters cleared for the next launch. Adds to one address are served one after the other, 11.4 ns each, so the blocks
 // count on TICKET_WAYS lines first and the last of each line on the first one: 256 blocks that end together wait 0.5 us in place of
 // 2.9 us for one more round trip.
-__device__ __forceinline__ bool last_block(unsigned* done, unsigned nBlocks) {
+__device__ __forceinline__ bool last_of_way(unsigned* done, unsigned nBlocks) {
 	const unsigned id = blockIdx.y * gridDim.x + blockIdx.x, way = id % TICKET_WAYS;
 	unsigned* const line = done + (1 + way) * (NNZ_STEP * 2);
 	if(atomicAdd(line, 1u) != (nBlocks - way + TICKET_WAYS - 1) / TICKET_WAYS - 1) return false;
 	*line = 0;
+	return true;
+}
+__device__ __forceinline__ bool last_of_ways(unsigned* done, unsigned nBlocks) {
 	if(atomicAdd(done, 1u) != min(nBlocks, (unsigned) TICKET_WAYS) - 1) return false;
 	*done = 0;
 	return true;
 }
+__device__ __forceinline__ bool last_block(unsigned* done, unsigned nBlocks) { return last_of_way(done, nBlocks) && last_of_ways(done, nBlocks); }
 
 // Tail of a left multiply whose kernel is the only one of the call: every block comes here behind its last add into
 // out; the last one to arrive counts the non-zeros of out[0 .. n) into *nnz

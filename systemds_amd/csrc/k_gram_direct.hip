@@ -250,6 +250,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_tsmm_direct(const GdrArgs A) {
 		}
 	}
 	__syncthreads();
+	double* const into = A.done != nullptr ? A.acc + gram_way(A.nCols) : A.out;
 	for(int idx = tid; idx < GDR_NP * GDR_NP; idx += THREADS) {
 		const double s = gramS[idx];
 		if(s == 0.0) continue;
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_tsmm_direct(const GdrArgs A) {
 		const int ci = i < 16 ? (i < A.nV ? A.cols[i].col : -1) : (i - 16 < nR ? A.runs[i - 16].col : -1);
 		const int cj = j < 16 ? (j < A.nV ? A.cols[j].col : -1) : (j - 16 < nR ? A.runs[j - 16].col : -1);
 		if(ci < 0 || cj < 0) continue;
-		unsafeAtomicAdd(&(A.done != nullptr ? A.acc : A.out)[(size_t) min(ci, cj) * A.nCols + max(ci, cj)], s);
+		unsafeAtomicAdd(&into[(size_t) min(ci, cj) * A.nCols + max(ci, cj)], s);
 	}
 	if(A.done != nullptr) gram_tail(A.done, gridDim.x, A.acc, A.out, A.nCols, A.nnz, (unsigned*) gramS);
 }

@@ -313,11 +313,12 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 		}
 		__syncthreads();
 	}
+	double* const into = A.acc + (A.done != nullptr ? gram_way(A.nCols) : 0);
 	auto add = [&](int ia, int ib, double d) {
 		const GtCol Ca = A.cols[ia], Cb = A.cols[ib];
 		if(A.skipOwn && (Ca.group == Cb.group || Ca.stride == 0 || Cb.stride == 0)) return;
 		const int ca = Ca.col, cb = Cb.col;
-		if(ca >= 0 && cb >= 0 && d != 0.0) unsafeAtomicAdd(&A.acc[(size_t) min(ca, cb) * A.nCols + max(ca, cb)], d);
+		if(ca >= 0 && cb >= 0 && d != 0.0) unsafeAtomicAdd(&into[(size_t) min(ca, cb) * A.nCols + max(ca, cb)], d);
 	};
 	for(int i = tid; i < T * 256; i += GT_THREADS) {
 		int t = i >> 8, p = 0;
@@ -535,10 +536,12 @@ int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz, bool
 	struct Clear {
 		cla_block* b;
 		bool on;
-		~Clear() { if(on) (void) hipMemsetAsync(b->dGramAcc, 0, (size_t) b->nCols * b->nCols * sizeof(double), b->stream); }
+		~Clear() { if(on) (void) hipMemsetAsync(b->dGramAcc, 0, (size_t) (1 + GRAM_WAYS) * b->nCols * b->nCols * sizeof(double), b->stream); }
 	} clear{b, ownByCounts && dNnz != nullptr};
 	int rc = 0;
-	if(ownByCounts && (rc = launch_tsmm_self(b, A.acc, nullptr, b->hasConst ? b->dConstV : nullptr, P.constCols, P.nConst))) return rc;
+	// (into an accumulator that gram_tail reads: see gram_ways)
+	double* const own = A.acc + (A.done != nullptr && grid > 4 * GRAM_WAYS ? (size_t) b->nCols * b->nCols : 0);
+	if(ownByCounts && (rc = launch_tsmm_self(b, own, nullptr, b->hasConst ? b->dConstV : nullptr, P.constCols, P.nConst))) return rc;
 	if((rc = gt_launch_shape(b, P, A, grid)) == 0) clear.on = false;
 	return rc;
 }

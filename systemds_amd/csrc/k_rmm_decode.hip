@@ -716,7 +716,7 @@ __device__ __forceinline__ void decode_body(const DecArgs& A) {
 			}
 		}
 		__syncthreads();
-		double* const dst = A.done != nullptr ? A.acc : A.out;
+		double* const dst = A.done != nullptr ? A.acc + gram_way(A.nCols) : A.out;
 		for(int i = tid; i < NP * NP; i += DEC_THREADS) {
 			const int r = i / NP, c = i - r * NP;
 			if(r <= c && c < A.nCols && stage[i] != 0.0) unsafeAtomicAdd(&dst[(size_t) r * A.nCols + c], stage[i]);
