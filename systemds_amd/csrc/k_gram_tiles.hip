@@ -13,10 +13,10 @@
 // Two-byte codes of column pairs (co-coded groups): a wave's 64 lanes look up one group at 64 rows (below 64 rows per tile two
 // groups), a whole tuple of 16 bytes per lane, and write it to the lane's row of the tile. Dealt like the others the gathers
 // of 8 bytes bound the kernel: 10,000,000 x 50, 4096 tuples (Zipf), 1001 us; so 934, with the gathers spread between the
-// matrix instructions 692 (matrix pipe 496, gathers 400).
+// matrix instructions 692 (matrix pipe 496, gathers 400), with the codes of two tiles per load 654.
 //
 // The stages of three tiles overlap: while a tile is multiplied, the values of the next one but one are looked up and the
-// codes behind those are on their way. One barrier per tile that waits for LDS only: loads stay in flight over it.
+// codes behind those are on their way (pairs: a lane reads the codes of two rows at a time, one for each of two tiles). One barrier per tile that waits for LDS only: loads stay in flight over it.
 //
 // Bound: the fp64 matrix pipe (70 cycles per tile and 4 rows): busy 72 % of the time at 2,000,003 x 100 byte codes (vector issue 12 %,
 // LDS 19 %, vector memory path 38 %), 69 % at 10,000,000 x 50 column pairs, where the gathers keep the vector memory path busy 64 %.
@@ -59,6 +59,10 @@ struct GtArgs {
 constexpr int GT_BYTE = 1, GT_SHORT = 2, GT_PAIR = 3;
 // 32 m rows per tile (m * ncb <= 8 where a wave decodes one part; pairs: whole waves of rows as far as LDS goes)
 __host__ __device__ constexpr int gt_m(int ncb, int kind) { return ncb == 1 ? 8 : ncb == 2 ? (kind == GT_PAIR ? 4 : 3) : ncb <= 4 ? 2 : 1; }
+// Tiles that a block takes together. Pairs: a lane's codes of two tiles are those of two neighbouring rows, one load of four bytes, requested
+// two tiles before the first is looked up. A load per tile, one tile ahead, left HBM's latency in the open where tiles are short, and
+// kept the vector memory path busy: 10,000,000 x 50 678 -> 654 us, 4,000,000 x 20 112 -> 101 (four rows and tiles: 654, 103).
+__host__ __device__ constexpr int gt_group(int kind) { return kind == GT_PAIR ? 2 : 1; }
 // doubles per row: rows 128 bytes apart in the banks; pairs, written by row with 16 bytes per lane: 144 bytes apart
 __host__ __device__ constexpr int gt_stride(int ncb, int kind) { return kind == GT_PAIR ? ncb * 16 + (ncb & 1 ? 2 : 18) : ncb * 16 + (ncb & 1 ? 0 : 16); }
 
@@ -77,7 +81,9 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 	extern __shared__ __attribute__((aligned(16))) double smem[]; // two tile buffers, the dictionaries
 	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int c = lane & 15, k = lane >> 4;
-	const int t0 = (int) ((int64_t) A.nTiles * blockIdx.x / gridDim.x), t1 = (int) ((int64_t) A.nTiles * (blockIdx.x + 1) / gridDim.x);
+	constexpr int G = gt_group(KIND);
+	const int nShares = (A.nTiles + G - 1) / G;
+	const int t0 = (int) ((int64_t) nShares * blockIdx.x / gridDim.x) * G, t1 = (int) ((int64_t) nShares * (blockIdx.x + 1) / gridDim.x) * G;
 
 	// this wave's part of the decoding: column block, 32 rows of the tile
 	const int myCb = wave % NCB, sub = wave / NCB;
@@ -109,7 +115,7 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 		constexpr int MODE = decltype(modeTag)::value, HALF = decltype(halfTag)::value;
 		constexpr int U = PAIR ? NU - MODE : 0; // units of the wave (no branch around a load: it would wait for the load)
 		auto unit_row = [&](int i) { return (wave + 8 * i) % RB * UR; };
-		uint32_t pcode[2][U > 0 ? U : 1];
+		uint32_t pcode[U > 0 ? U : 1], pnext[U > 0 ? U : 1]; // codes of the two tiles looked up next, of the two behind them
 		f64x2 pv[2][U > 0 ? U : 1];
 		const uint8_t* pstream[U > 0 ? U : 1];
 		const char* pdict[U > 0 ? U : 1];
@@ -127,23 +133,22 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 		double v[2][8];
 		auto load_codes = [&](int tile, auto parity) { // (codes and values of a tile sit in the sets of its parity)
 			constexpr int Q = decltype(parity)::value;
-			if constexpr(PAIR) {
-#pragma unroll
-				for(int i = 0; i < U; i++) {
-					const int64_t row = min((int64_t) min(tile, t1 - 1) * R + unit_row(i) + uRow, A.nRows - 1);
-					pcode[Q][i] = *(const uint16_t*) (pstream[i] + 2 * row);
-				}
-				return;
-			}
 			if(MODE == 0) return;
 			const int64_t row = min((int64_t) min(tile, t1 - 1) * R + sub * 32 + 8 * k, rowLast);
 			if constexpr(W == 1) codes[Q].raw.v = *(const u32x2*) (stream + row);
 			else codes[Q].raw.v = *(const u32x4*) (stream + 2 * row);
 		};
+		auto load_pairs = [&](uint32_t (&dst)[U > 0 ? U : 1], int tile) { // of an even tile and the next one
+#pragma unroll
+			for(int i = 0; i < U; i++) {
+				const int64_t row = min((int64_t) min(tile, t1 - 2) * R + 2 * (unit_row(i) + uRow), (A.nRows - 1) & ~(int64_t) 1);
+				dst[i] = *(const uint32_t*) (pstream[i] + 2 * row);
+			}
+		};
 		constexpr int NL = PAIR ? U : MODE == 0 ? 0 : 8; // lookups per lane and tile
 		auto look_one = [&](int i, auto parity) {
 			constexpr int Q = decltype(parity)::value;
-			if constexpr(PAIR) pv[Q][i] = *(const f64x2*) (pdict[i] + (pcode[Q][i] << 4));
+			if constexpr(PAIR) pv[Q][i] = *(const f64x2*) (pdict[i] + (((pcode[i] >> (16 * Q)) & 0xffffu) << 4));
 			else {
 				const uint32_t code = (uint32_t) codes[Q].get(i);
 				if(MODE == 1) v[Q][i] = *(const double*) (ldsDict + (code << 7));
@@ -158,7 +163,7 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 			if constexpr(PAIR) { // (tile t goes from value set to buffer of the same parity)
 #pragma unroll
 				for(int i = 0; i < U; i++) {
-					const bool in = (int64_t) tile * R + unit_row(i) + uRow < A.nRows; // zeros behind the last row of the matrix
+					const bool in = (int64_t) (tile & ~1) * R + 2 * (unit_row(i) + uRow) + (tile & 1) < A.nRows; // zeros behind the last row of the matrix
 					f64x2 x = buf == 0 ? pv[0][i] : pv[1][i];
 					x.x = in ? x.x : 0.0; x.y = in ? x.y : 0.0;
 					*(f64x2*) (pput[i] + buf * BUF) = x;
@@ -228,7 +233,8 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 				if(SPREAD && i >= done) look_one(i, parity); // (more lookups than matrix instructions)
 		};
 		using std::integral_constant;
-		load_codes(t0, integral_constant<int, 0>());
+		if constexpr(PAIR) { load_pairs(pcode, t0); load_pairs(pnext, t0 + 2); }
+		else load_codes(t0, integral_constant<int, 0>());
 		{
 			// the dictionaries of the first column blocks, 8 pieces of 16 bytes per thread requested together
 			const f64x2* src = (const f64x2*) A.img;
@@ -244,23 +250,28 @@ __global__ __launch_bounds__(GT_THREADS, 2) void k_gram_tiles(GtArgs A) {
 			}
 		}
 		lds_barrier();
-		load_codes(t0 + 1, integral_constant<int, 1>());
+		if constexpr(!PAIR) load_codes(t0 + 1, integral_constant<int, 1>());
 		look(integral_constant<int, 0>());
-		load_codes(t0 + 2, integral_constant<int, 0>());
+		if constexpr(!PAIR) load_codes(t0 + 2, integral_constant<int, 0>());
 		look(integral_constant<int, 1>());
 		write(v[0], t0, 0);
 		lds_barrier();
 		auto step = [&](int tile, auto parity) {
 			constexpr int P = decltype(parity)::value;
+			if constexpr(PAIR && P == 0) {
+#pragma unroll
+				for(int i = 0; i < U; i++) pcode[i] = pnext[i];
+				load_pairs(pnext, tile + 4);
+			}
 			if(!SPREAD) look(parity);      // of tile + 2
-			load_codes(tile + 3, integral_constant<int, P ^ 1>());
+			if constexpr(!PAIR) load_codes(tile + 3, integral_constant<int, P ^ 1>());
 			multiply(P, parity);
 			write(v[P ^ 1], min(tile + 1, t1 - 1), P ^ 1); // (behind the last tile: values nobody reads)
 			lds_barrier();
 		};
 		for(int tile = t0; tile < t1; tile += 2) {
 			step(tile, integral_constant<int, 0>());
-			if(tile + 1 < t1) step(tile + 1, integral_constant<int, 1>());
+			if(PAIR || tile + 1 < t1) step(tile + 1, integral_constant<int, 1>());
 		}
 	};
 	if(t0 < t1) {
@@ -531,7 +542,7 @@ int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz, bool
 		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
 	A.skipOwn = ownByCounts;
-	const unsigned grid = (unsigned) std::min(A.nTiles, g_numCU * P.perCU);
+	const unsigned grid = (unsigned) std::min((A.nTiles + gt_group(P.kind) - 1) / gt_group(P.kind), g_numCU * P.perCU);
 	// (where k_gram_tiles does not follow, an exception on the way included, nothing clears what the counts' kernel has added)
 	struct Clear {
 		cla_block* b;
