@@ -1528,7 +1528,6 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 	if(dotForm && !(b->opt.lmmDisable & 1)) return 1;
 	if(p == 1 && lmm_q1_short_groups(b) > 0) return 1; // k_lmm_q1_short
 	if(b->nCols > 64) return launch_lmm_chunked(b, dY, p, dOut, dNnz);
-	hipStream_t st = b->stream;
 	const size_t n = (size_t) p * b->nCols;
 	// the sums, room for the product anew where Y holds a non-finite value (p row sums behind it), the kernel's report of one, a count. Not
 	// in the output staging buffer, which may be the caller's dOut.
@@ -1537,7 +1536,7 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 	if(rc) return rc;
 	double* const ws = b->dTables;
 	unsigned long long* const dBad = (unsigned long long*) (ws + nWs - 2);
-	CLA_HIP(hipMemsetAsync(ws, 0, nWs * sizeof(double), st));
+	if((rc = launch_zero(b, ws, nWs))) return rc;
 	for(int p0 = 0; p0 < p; p0 += 16) // 16 rows of Y per pass over the block
 		if((rc = launch_lmm_decode(b, dY + (size_t) p0 * b->nRows, std::min(16, p - p0), ws + (size_t) p0 * b->nCols, dBad))) {
 			if(rc == 1 && p0 == 0) return launch_lmm_chunked(b, dY, p, dOut, dNnz); // (nothing queued yet)

@@ -313,6 +313,7 @@ void dec_plans_drop(cla_block* b);
 int tsmm_decode_fits(cla_block* b);
 int launch_lmm_decode(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dBad);
 int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dNnz);
+int launch_zero(cla_block* b, double* p, size_t n); // n > 0
 int launch_lmm_take(cla_block* b, const double* dY, int p, double* ws, double* dOut, unsigned long long* dNnz); // ws: p x nCols summed, 2 n + p + 2 in all
 int launch_lmm(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dNnz);
 int launch_preagg(cla_block* b, int group, const double* dY, int p, double* dPre);

@@ -383,6 +383,17 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 	if(lastS && tid > 0 && tid < NNZ_WAYS) A.nnz[tid * NNZ_STEP] = 0;
 }
 
+// (a kernel, not hipMemsetAsync: a memset node of a captured graph has given wrong results on its replays)
+__global__ __launch_bounds__(256) void k_zero(double* __restrict__ p, size_t n) {
+	for(size_t i = (size_t) blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t) gridDim.x * 256) p[i] = 0.0;
+}
+
+int launch_zero(cla_block* b, double* p, size_t n) {
+	hipLaunchKernelGGL(k_zero, dim3((unsigned) std::min<size_t>((n + 255) / 256, 1024)), dim3(256), 0, b->stream, p, n);
+	CLA_HIP(hipGetLastError());
+	return 0;
+}
+
 int launch_lmm_take(cla_block* b, const double* dY, int p, double* ws, double* dOut, unsigned long long* dNnz) {
 	const size_t n = (size_t) p * b->nCols;
 	LmmTake A;
