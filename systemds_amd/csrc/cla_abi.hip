@@ -1775,10 +1775,13 @@ int64_t cla_mmchain(cla_handle b, const double* v, const double* w, int32_t ctyp
 	std::lock_guard<std::recursive_mutex> lk(b->mu);
 	if((rc = ensure_stage(&b->dStageIn, &b->stageInCap, nV + nW)) || (rc = ensure_stage(&b->dStageOut, &b->stageOutCap, nV)))
 		return rc;
-	CLA_HIP(hipMemcpyAsync(b->dStageIn, v, nV * sizeof(double), hipMemcpyHostToDevice, b->stream));
+	const bool pinned = nV <= HOST_VEC_MAX;
+	if(pinned) { if((rc = launch_fetch(b, b->dStageIn, v, (int) nV))) return rc; }
+	else CLA_HIP(hipMemcpyAsync(b->dStageIn, v, nV * sizeof(double), hipMemcpyHostToDevice, b->stream));
 	if(nW) CLA_HIP(hipMemcpyAsync(b->dStageIn + nV, w, nW * sizeof(double), hipMemcpyHostToDevice, b->stream));
-	const int64_t nnz = cla_mmchain_dev(b, b->dStageIn, nW ? b->dStageIn + nV : nullptr, ctype, b->dStageOut);
+	const int64_t nnz = mmchain_dev(b, b->dStageIn, nW ? b->dStageIn + nV : nullptr, ctype, b->dStageOut, !pinned);
 	if(nnz < 0) return nnz;
+	if(pinned) return deliver(b, out, b->dStageOut, (int) nV, b->dCounters);
 	CLA_HIP(hipMemcpy(out, b->dStageOut, nV * sizeof(double), hipMemcpyDeviceToHost));
 	return nnz;
 	CLA_CATCH_CODE(int64_t)

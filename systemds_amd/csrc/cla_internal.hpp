@@ -31,6 +31,8 @@ constexpr size_t NNZ_BYTES = (size_t) NNZ_SLOT * 8;
 // from L2 to L2, and 256 blocks' adds to the cells of a 20 x 20 result took 15 us.
 constexpr int GRAM_WAYS = 8; // (as many as TICKET_WAYS, dealt alike)
 constexpr int TICKET_WAYS = 8;                // a ticket is counted on this many lines and a line for these (last_block)
+// most elements of a vector that a host-pointer call hands over through the counters' pinned buffer: a count, an operand and a result fit it
+constexpr int HOST_VEC_MAX = (NNZ_SLOT - 1) / 2;
 constexpr int NNZ_SLOTS = 4;                  // counters of a block (cla_block::nnzSlot)
 
 // Iterator state of an offset list in front of delta entry `idx`:
@@ -313,6 +315,8 @@ void dec_plans_drop(cla_block* b);
 int tsmm_decode_fits(cla_block* b);
 int launch_lmm_decode(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dBad);
 int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dNnz);
+int launch_fetch(cla_block* b, double* dst, const double* v, int n);
+int64_t deliver(cla_block* b, double* out, const double* src, int n, const unsigned long long* dNnz);
 int launch_zero(cla_block* b, double* p, size_t n); // n > 0
 int launch_lmm_take(cla_block* b, const double* dY, int p, double* ws, double* dOut, unsigned long long* dNnz); // ws: p x nCols summed, 2 n + p + 2 in all
 int launch_lmm(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dNnz);

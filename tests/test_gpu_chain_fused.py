@@ -93,3 +93,22 @@ def test_non_finite_operands(cla, value, where):
     fin = np.isfinite(got[0])
     # (sums of 5000 terms: 5000 x 2^-53 of their magnitude apart at most, and they do not cancel to less than 1e-3 of it here)
     np.testing.assert_allclose(got[1][fin], got[0][fin], rtol=1e-9)
+
+
+@pytest.mark.parametrize("ctype", [0, 1, 2])
+@pytest.mark.parametrize("n_cols, n_rows", [(1, 70), (54, 4097), (510, 65), (511, 1000), (512, 1000), (700, 129)])
+def test_chain_of_host_vectors(cla, ora, n_cols, n_rows, ctype):
+    """Vectors of up to 511 elements travel through the pinned buffer of the counters; several calls, each with other vectors."""
+    rng = np.random.default_rng(n_cols + ctype)
+    specs, blk = block(cla, rng, n_rows, n_cols, 9)
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    for _ in range(3):
+        v, w = rng.standard_normal((n_cols, 1)), rng.standard_normal((n_rows, 1))
+        out, nnz = blk.mmchain(v, w if ctype else None, ctype)
+        xv = D.astype(np.longdouble) @ v.astype(np.longdouble)
+        u = xv * w if ctype == 1 else xv - w if ctype == 2 else xv
+        # (the bound of test_chain_in_one_pass: at most n_rows + n_cols roundings of 1.1e-16 of these magnitudes)
+        scale = np.abs(D).T @ (np.abs(D) @ np.abs(v) * (np.abs(w) if ctype == 1 else 1.0) + (np.abs(w) if ctype == 2 else 0.0))
+        assert np.all(np.abs(out.reshape(-1, 1) - D.astype(np.longdouble).T @ u) <= 1e-12 * scale + 1e-300)
+        assert nnz == np.count_nonzero(out) and blk.nnz() == nnz
+    blk.close()
