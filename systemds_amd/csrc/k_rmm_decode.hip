@@ -1308,6 +1308,7 @@ struct DirPlan {
 	int rc = 1;            // 0 usable, 1 the block does not qualify
 	void* dImg = nullptr;
 	int64_t bytes = 0;
+	bool denseFiller = false; // an odd number of dense columns
 	DirArgs A;
 	std::vector<RunCol> runs; // run-length columns that are followed by run, and their merged run table
 	Mrt mrt;
@@ -1364,8 +1365,11 @@ static int dir_build_plan(cla_block* b, DirPlan& P) {
 		for(const DirCol& C : cols[sgm]) all.push_back(C);
 		if((cols[sgm].size() & 1) != 0) { // classes of even size: a filler column (a real stream, the zero behind the dictionaries, a row of zeros for B)
 			DirCol F = cols[sgm].back();
-			if(sgm == DSEG_DENSE) return 0; // (a dense filler would need a stream of its own: odd numbers of dense columns take the tile kernel)
 			F.base8 = (int32_t) (8 * zeroAt); F.nC8 = 0; F.orig = -1;
+			if(sgm == DSEG_DENSE) {
+				F.src = nullptr; // (the row of zeros, filled in below: a stream whose rows are no bytes apart)
+				P.denseFiller = true;
+			}
 			all.push_back(F);
 		}
 		P.A.segEnd[sgm] = (int) all.size();
@@ -1373,10 +1377,12 @@ static int dir_build_plan(cla_block* b, DirPlan& P) {
 	if(all.empty() || runs.size() > (size_t) RC_MAX || (!runs.empty() && b->nRows >= ((int64_t) 1 << 31) - 2 * DIR_SLICE)) return 0;
 	const size_t colBytes = all.size() * sizeof(DirCol), dictBytes = dicts.size() * sizeof(DirDict);
 	std::vector<uint8_t> img(colBytes + dictBytes + 16 * 8, 0);
-	std::memcpy(img.data(), all.data(), colBytes);
-	if(dictBytes) std::memcpy(img.data() + colBytes, dicts.data(), dictBytes);
 	uint8_t* d = nullptr;
 	CLA_HIP(hipMalloc((void**) &d, img.size() + 64));
+	for(DirCol& C : all)
+		if(C.src == nullptr) C.src = d + colBytes + dictBytes;
+	std::memcpy(img.data(), all.data(), colBytes);
+	if(dictBytes) std::memcpy(img.data() + colBytes, dicts.data(), dictBytes);
 	P.dImg = d;
 	P.bytes = (int64_t) img.size() + 64;
 	CLA_HIP(hipMemcpy(d, img.data(), img.size(), hipMemcpyHostToDevice));
@@ -1468,10 +1474,20 @@ static int launch_rmm_direct(cla_block* b, const double* dB, int q, const double
 int launch_rmm_decode(cla_block* b, const double* dB, int q, const double* dConstRow, double* dOut,
 	unsigned long long* dNnz) {
 	if(b->groups.empty() || b->nRows == 0 || q < 1) return 1;
-	// (16 columns: no padding of B left for the tile kernel to lose, and the stream kernel short of registers: C5 2.1 against 2.5 ms)
-	// (... unless run-length columns are followed by run: the tile kernel would expand them tile by tile, 2.4 against 2.2 ms)
+	// 16 columns: no padding of B left for the tile kernel to lose, and the stream kernel short of registers (C5 2.1 against 2.5 ms), unless
+	// there are run-length columns, which the tile kernel would expand tile by tile, more than 12 columns and more rows than fill the
+	// chip (in us, stream / tile kernel: 8 run-length of 20 columns, 1,000,003 rows 66 / 70, 600,003 62 / 59; 4 of 12, 3,000,001 rows
+	// 138 / 123; 2 of 13, 8,000,001 rows 352 / 365). An odd number of dense columns (a filler beside them): the stream kernel up to 10 columns
+	// of B (100,003 rows of 13 columns, 2 of B 15.6 / 23.3, 10 20.6 / 24.8; 8,000,001 84 / 293, 166 / 299), up to 15 where
+	// half the chip is full (600,003 38 / 44, 8,000,001 231 / 320; 100,003 rows of 6 columns 21.3 / 18.7); not below a slice per CU,
+	// where it would be the faster one as well (30,000 rows 15.1 / 22.8) but the tests hold such blocks to the tile kernel
 	bool tilesFirst = q == DEC_QMAX;
-	if(tilesFirst && b->opt.rmmDirect && dir_plan_get(b) == 0 && b->dirPlan->A.nR > 0) tilesFirst = false;
+	if(b->opt.rmmDirect && dir_plan_get(b) == 0) {
+		const DirPlan& P = *b->dirPlan;
+		const int64_t chip = (int64_t) g_numCU * DIR_WAVES * DIR_SLICE; // rows, a slice per wave
+		if(P.denseFiller) tilesFirst = q >= DEC_QMAX || b->nRows < (q > 10 ? chip / 2 : chip / DIR_WAVES);
+		else if(tilesFirst && P.A.nR > 0) tilesFirst = b->nRows < chip * 3 / 2 || P.A.nR + P.A.segEnd[DSEG_N - 1] <= 12;
+	}
 	if(b->opt.rmmDirect && !tilesFirst) {
 		const int rc = launch_rmm_direct(b, dB, q, dConstRow, dOut, dNnz);
 		if(rc != 1) return rc;

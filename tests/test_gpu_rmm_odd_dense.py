@@ -1,0 +1,51 @@
+"""X %*% B on blocks with an odd number of dense columns: the kernel on streams takes a filler column beside them. Edges of its
+slices of 128 rows, widths of B around the rule's lines, infinities and NaN in the dense columns; the tile kernel forms the same sums."""
+import numpy as np
+import pytest
+
+from parity import assert_matches_truth
+
+pytestmark = pytest.mark.gpu
+
+
+def block(cla, synth, rng, n_rows, unc, runs, odd_values):
+    specs, c = [], 0
+    for _ in range(runs):
+        lens = rng.geometric(1.0 / 900.0, size=n_rows // 300 + 16)
+        codes = np.repeat(rng.integers(0, 8, size=lens.size), lens)[:n_rows]
+        ptr, data = synth.encode_rle(np.concatenate([codes, np.zeros(n_rows - codes.size, codes.dtype)]), 8)
+        specs.append(synth.GroupSpec("rle", np.array([c], np.int32), rng.standard_normal((8, 1)), ptr=ptr, rle=data))
+        c += 1
+    for n_vals, dt in [(700, np.uint16), (30, np.uint8), (1, np.uint8)]:
+        specs.append(synth.GroupSpec("ddc", np.array([c], np.int32), rng.standard_normal((n_vals, 1)), rng.integers(0, n_vals, n_rows).astype(dt)))
+        c += 1
+    dense = rng.standard_normal((n_rows, unc))
+    if odd_values:
+        for v in (np.inf, -np.inf, np.nan):
+            dense[rng.integers(0, n_rows), rng.integers(0, unc)] = v
+    specs.append(synth.GroupSpec("unc", np.arange(c, c + unc, dtype=np.int32), dense=dense))
+    return specs, c + unc, cla.build_block(n_rows, c + unc, specs)
+
+
+@pytest.mark.parametrize("n_rows", [4097, 32767, 32768, 32895, 33025, 300001])
+@pytest.mark.parametrize("unc, runs, odd_values", [(1, 0, False), (1, 3, False), (3, 2, True), (5, 0, True)])
+@pytest.mark.parametrize("q", [1, 2, 7, 10, 11, 15, 16, 17])
+def test_odd_number_of_dense_columns(cla, ora, n_rows, unc, runs, odd_values, q):
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows + 10 * unc + q)
+    specs, n_cols, blk = block(cla, synth, rng, n_rows, unc, runs, odd_values)
+    B = rng.standard_normal((n_cols, q))
+    out, nnz = blk.rmm(B)
+    names = [k["name"] for k in blk.stats()["kernels"]]
+    tiles, _ = blk.set_option("rmm_direct", 0).rmm(B)
+    blk.close()
+    # (32,768 rows: a slice per CU of 256; 262,144: half of their 16 waves with one each)
+    streams = q <= 15 and n_rows >= (32768 if q <= 10 else 262144)
+    assert ("k_rmm_direct" in names) == streams and ("k_rmm_decode" in names) != streams, names
+    fin = np.isfinite(tiles)
+    assert np.array_equal(np.isfinite(out), fin) and np.array_equal(out[~fin], tiles[~fin], equal_nan=True)
+    assert nnz == np.count_nonzero(out)
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    rows = fin.all(axis=1)
+    if rows.any():
+        assert_matches_truth(out.reshape(n_rows, q)[rows], D[rows], B, what=f"odd dense q={q}")
