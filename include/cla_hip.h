@@ -129,7 +129,7 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *                   columns by chunk the host looks, i.e. waits for the stream once per call, and such a Y takes the bin kernels)
  *   tsmm_one_kernel 1 / 0: t(X) %*% X of a whole block of at most 64 columns (all-DDC: 128) on the decoded Gram kernels as the call's only
  *                   kernel (a few wide DDC groups: behind the kernel of the cells inside a group; its blocks add into an
- *                   accumulator kept with the block, nCols x nCols doubles; the last block
+ *                   accumulator per XCD kept with the block, 9 x nCols x nCols doubles; the last block
  *                   to finish writes the output, mirrored, and the count of its non-zeros and clears the accumulator)
  *                   instead of a fill of the output in front of the kernel and a mirror-and-count kernel behind it
  *   chain_fused     1 / 0: the multiply chain of single-column byte-code blocks without constants whose dictionaries fit LDS (up to
