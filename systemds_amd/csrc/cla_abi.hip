@@ -8,7 +8,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <unordered_set>
+#include <unordered_map>
 #include <new>
 #include <stdexcept>
 
@@ -82,19 +82,27 @@ int ensure_tables(cla_block* b, size_t nDoubles) {
 	return 0;
 }
 
-hipError_t allow_full_lds(const void* kernel) {
+// The dynamic LDS that a block of `kernel` may have: the device's less the kernel's static shared memory, which counts against the
+// same limit (__shared__ variables, and the scratch of __syncthreads_or). Set as the kernel's limit when it is first asked for.
+hipError_t max_dynamic_lds(const void* kernel, size_t& bytes) {
 	static std::mutex mu;
-	static std::unordered_set<const void*> said;
+	static std::unordered_map<const void*, size_t> said;
 	std::lock_guard<std::mutex> lk(mu);
-	if(said.count(kernel)) return hipSuccess;
-	// (the kernel's static shared memory counts against the same limit)
+	const auto it = said.find(kernel);
+	if(it != said.end()) { bytes = it->second; return hipSuccess; }
 	hipFuncAttributes fa;
 	hipError_t e = hipFuncGetAttributes(&fa, kernel);
 	if(e != hipSuccess) return e;
-	const int room = g_ldsPerBlock - (int) fa.sharedSizeBytes;
-	e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, room > 0 ? room : 0);
-	if(e == hipSuccess) said.insert(kernel);
-	return e;
+	const int room = std::max(g_ldsPerBlock - (int) fa.sharedSizeBytes, 0);
+	e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, room);
+	if(e != hipSuccess) return e;
+	bytes = said[kernel] = (size_t) room;
+	return hipSuccess;
+}
+
+hipError_t allow_full_lds(const void* kernel) {
+	size_t bytes;
+	return max_dynamic_lds(kernel, bytes);
 }
 
 int ensure_scratch(cla_block* b, size_t bytes) {

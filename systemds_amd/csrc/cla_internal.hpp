@@ -257,6 +257,8 @@ extern int g_ldsPerBlock;   // usable LDS bytes per workgroup
 // Lets a kernel take up to the device's LDS per workgroup as dynamic shared memory; said once per kernel (a value
 // per call could be lowered by a caller on another handle between a call's setting and its launch).
 hipError_t allow_full_lds(const void* kernel);
+// The same, and how much that is: a rule that fills LDS asks here, the kernel's static shared memory is not its own to guess.
+hipError_t max_dynamic_lds(const void* kernel, size_t& bytes);
 extern int g_numCU;
 
 #define CLA_HIP(expr)                                                                              \

@@ -30,7 +30,6 @@ namespace cla {
 using std::integral_constant;
 constexpr int CH_THREADS = 512;
 constexpr int CH_WAVES = CH_THREADS / WAVE;
-constexpr int CH_MAX_CB = 7;
 
 // x of lane T of the lane's row of 16
 template <int T>
@@ -262,9 +261,14 @@ int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype,
 		!b->opt.chainFused)
 		return 1;
 	const int nCb = (nG + 15) / 16, nV = b->maxVals;
-	if(nCb > CH_MAX_CB) return 1;
+	decltype(&k_chain_u8<1, false>) kern = nullptr;
+#define CH_CASE(N) case N: kern = ctype != 0 ? k_chain_u8<N, true> : k_chain_u8<N, false>; break;
+	switch(nCb) { CH_CASE(1) CH_CASE(2) CH_CASE(3) CH_CASE(4) CH_CASE(5) CH_CASE(6) CH_CASE(7) default: return 1; }
+#undef CH_CASE
 	const size_t lds = std::max((size_t) nCb * nV * 128, (size_t) CH_WAVES * 4 * nCb * 16 * 8);
-	if(lds > (size_t) g_ldsPerBlock - 256) return 1; // (the tail's static LDS)
+	size_t room = 0;
+	CLA_HIP(max_dynamic_lds((const void*) kern, room));
+	if(lds > room) return 1;
 	const int64_t nUnits = std::max<int64_t>(nRows / WAVE, 1);
 	const int perCU = nCb <= 3 && lds <= (size_t) 78 * 1024 ? 2 : 1;
 	const unsigned grid = (unsigned) std::min<int64_t>((nUnits + CH_WAVES - 1) / CH_WAVES, (int64_t) g_numCU * perCU);
@@ -274,16 +278,8 @@ int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype,
 	clear_stats(b);
 	const double algo = (double) nRows * nG + (dW != nullptr ? (double) nRows * 8 : 0.0);
 	Prof pf(b, "k_chain_u8", grid, CH_THREADS, (long) lds, algo);
-#define CH_LAUNCH(N, O)                                                                                                            \
-	do {                                                                                                                           \
-		CLA_HIP(allow_full_lds((const void*) k_chain_u8<N, O>));                                                                   \
-		hipLaunchKernelGGL((k_chain_u8<N, O>), dim3(grid), dim3(CH_THREADS), lds, b->stream, b->dArena, b->arenaStride, nG,        \
-			b->dDictPad + b->dictTOff, nV, dCol0, dV, dW, ctype == 2 ? 1 : 0, nRows, b->dTables, dOut, b->nCols, b->lmm_ticket(), dNnz); \
-	} while(0)
-#define CH_CASE(N) case N: if(ctype != 0) CH_LAUNCH(N, true); else CH_LAUNCH(N, false); break;
-	switch(nCb) { CH_CASE(1) CH_CASE(2) CH_CASE(3) CH_CASE(4) CH_CASE(5) CH_CASE(6) CH_CASE(7) }
-#undef CH_CASE
-#undef CH_LAUNCH
+	hipLaunchKernelGGL(kern, dim3(grid), dim3(CH_THREADS), lds, b->stream, b->dArena, b->arenaStride, nG, b->dDictPad + b->dictTOff, nV, dCol0, dV, dW,
+		ctype == 2 ? 1 : 0, nRows, b->dTables, dOut, b->nCols, b->lmm_ticket(), dNnz);
 	CLA_HIP(hipGetLastError());
 	return 0;
 }

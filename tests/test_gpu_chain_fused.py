@@ -48,6 +48,25 @@ def test_chain_in_one_pass(cla, ora, n_rows, n_cols, n_vals, ctype):
     assert nnz == np.count_nonzero(out)
 
 
+@pytest.mark.parametrize("ctype", [0, 1])
+@pytest.mark.parametrize("n_cols, n_vals, fused", [(96, 212, True), (96, 213, False), (81, 213, False), (80, 255, True), (80, 256, False), (112, 181, True), (112, 182, True),
+                                                   (112, 183, False)])
+def test_dictionaries_that_just_fit(cla, ora, n_cols, n_vals, fused, ctype):
+    """LDS holds 163840 bytes: 128 per code and 16 columns, next to 304 that the kernel has of its own; what is left is too little for
+    (80, 256), which would fill it to the byte."""
+    rng = np.random.default_rng(n_vals)
+    n_rows = 4099
+    specs, blk = block(cla, rng, n_rows, n_cols, n_vals)
+    v, w = rng.standard_normal((n_cols, 1)), rng.standard_normal((n_rows, 1))
+    out, nnz = blk.mmchain(v, w if ctype else None, ctype)
+    names = names_of(blk)
+    blk.close()
+    assert ("k_chain_u8" in names) == fused, names
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    assert_matches_truth(out.reshape(-1, 1), D.T, (D @ v) * (w if ctype else 1.0), what="chain")
+    assert nnz == np.count_nonzero(out)
+
+
 def test_blocks_it_does_not_take(cla, ora):
     """Tables beyond LDS, more than 7 column blocks, constants, the options: two products, the same result."""
     rng = np.random.default_rng(5)
