@@ -147,25 +147,20 @@ int launch_rmm_q1_u8_few(cla_block* b, const double* dB, const double* constTerm
 	const int stride = std::max((b->maxVals + 1) & ~1, 2);
 	const size_t lds = ((size_t) (nG + 1) * stride + nG) * 8;
 	const int threads = nRows <= (int64_t) g_numCU * 2048 ? 512 : 1024;
+	const int rpt = threads == 1024 ? 4 : nRows <= (int64_t) g_numCU * 512 ? 1 : nRows <= (int64_t) g_numCU * 1024 ? 2 : 4;
+	const auto kern = threads == 1024 ? k_rmm_q1_u8_few<1024, 4> : rpt == 1 ? k_rmm_q1_u8_few<512, 1> : rpt == 2 ? k_rmm_q1_u8_few<512, 2> : k_rmm_q1_u8_few<512, 4>;
 	// (1,000,003 rows, in us here and on k_rmm_q1_u8: 5 columns 10.4 / 10.3, 20 12.1 / 13.0, 54 21 / 24, 100 28 / 35; 1,500,000, two turns of blocks, 54
 	// columns 37 / 27. Blocks of 512 threads, two per CU: 600,000 x 20 11.6 against 11.0, 600,000 x 30 13.6 against 12.3)
-	if(nRows > (int64_t) g_numCU * (nG <= 8 ? 3072 : 4096) || lds > (size_t) g_ldsPerBlock - 64 || (size_t) nG * stride > (size_t) uf_tpt(threads) * threads) return 1;
-	const int rpt = nRows <= (int64_t) g_numCU * 512 ? 1 : nRows <= (int64_t) g_numCU * 1024 ? 2 : 4;
+	if(nRows > (int64_t) g_numCU * (nG <= 8 ? 3072 : 4096) || (size_t) nG * stride > (size_t) uf_tpt(threads) * threads) return 1;
+	size_t room = 0;
+	CLA_HIP(max_dynamic_lds((const void*) kern, room));
+	if(lds > room) return 1;
 	const unsigned grid = (unsigned) ((nRows + (int64_t) threads * rpt - 1) / ((int64_t) threads * rpt));
 	const uint32_t magic = (uint32_t) ((((uint64_t) 1 << 32) + stride - 1) / stride); // (f / stride = f * magic >> 32 for f < 2^32 / stride)
 	const int32_t* dCol0 = (const int32_t*) (b->dDictPad + (size_t) nG * 256);
 	Prof pf(b, "k_rmm_q1_u8_few", grid, threads, (long) lds, (double) nRows * nG + (double) nRows * 8 + (double) b->totalVals * 8);
-#define UF_LAUNCH(T, R)                                                                                                            \
-	do {                                                                                                                           \
-		CLA_HIP(allow_full_lds((const void*) k_rmm_q1_u8_few<T, R>));                                                              \
-		hipLaunchKernelGGL((k_rmm_q1_u8_few<T, R>), dim3(grid), dim3(T), lds, b->stream, b->dArena, b->arenaStride, nG, b->dDictPad, stride, magic, \
-			constTerm, dOut, nRows, dNnz, dCol0, dB, nnzNext, op);                                                                 \
-	} while(0)
-	if(threads == 1024) UF_LAUNCH(1024, 4);
-	else if(rpt == 1) UF_LAUNCH(512, 1);
-	else if(rpt == 2) UF_LAUNCH(512, 2);
-	else UF_LAUNCH(512, 4);
-#undef UF_LAUNCH
+	hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, b->stream, b->dArena, b->arenaStride, nG, b->dDictPad, stride, magic, constTerm, dOut, nRows,
+		dNnz, dCol0, dB, nnzNext, op);
 	CLA_HIP(hipGetLastError());
 	return 0;
 }
