@@ -52,6 +52,7 @@ struct GdrPlan {
 	int64_t bytes = 0;
 	size_t lds = 0;        // of k_tsmm_direct, which these belong to as well: quads of varying columns, pieces of dense values per lane, waves per block
 	int quads = 0, densePieces = 0, waves = 0;
+	bool gram = false;     // whether that kernel holds them
 	GdrArgs A;
 	int spread = -1;       // 1: a varying column next to run-length columns spans too many magnitudes (GDR_SPREAD); -1: not looked at yet
 	bool codeSpread = false; // the same of the columns behind codes, from their dictionaries

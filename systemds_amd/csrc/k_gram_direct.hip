@@ -394,12 +394,13 @@ static int gdr_build_plan(cla_block* b, GdrPlan& P) {
 	const size_t valD = vals.size();
 	P.quads = (nV + 3) / 4;
 	P.densePieces = (nD * 32 * gdr_sets(P.quads) / 2 + 63) / 64;
-	if(P.densePieces > GDR_STAGE / 1024) return 0;
 	auto lds_of = [&](int waves) { return (valD + GDR_NP * GDR_NP + (size_t) waves * GDR_WDOUBLES) * 8 + (nD ? (size_t) waves * GDR_STAGE : 0); };
 	const size_t room = (size_t) std::min(g_ldsPerBlock, 160 * 1024) - 1024;
 	P.waves = lds_of(16) <= room ? 16 : 8;
 	P.lds = lds_of(P.waves);
 	if(P.lds > room) return 0;
+	// (more dense columns than a wave stages: the Gram matrix on the tile kernel. The left multiply stages none)
+	P.gram = P.densePieces <= GDR_STAGE / 1024;
 	const size_t colBytes = all.size() * sizeof(GdrCol), dictBytes = valD * sizeof(double), runBytes = runs.size() * sizeof(RunCol);
 	const size_t denseBytes = dense.size() * sizeof(GdrDense);
 	// the same columns as the left multiply wants them: straight from their streams, filled up to a shape it exists for
@@ -482,7 +483,7 @@ int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	if(!b->opt.tsmmDirect || b->crossSplit > 0 || b->crossBlocks > 0) return 1;
 	const GdrPlan* P = nullptr;
 	if(const int rc = gdr_plan(b, P)) return rc;
-	if(P->rc) return P->rc;
+	if(P->rc || !P->gram) return 1;
 	if(P->spread < 0)
 		if(const int rc = gdr_look(b, *b->gdrPlan)) return rc;
 	if(P->spread && P->A.nR > 0) return 1;

@@ -99,6 +99,24 @@ def test_column_mixes(cla, ora, shape):
     check(cla, ora, specs, n_rows, n_cols, f"mix {shape}")
 
 
+@pytest.mark.parametrize("n_rows", [2, 127, 129, 255, 20011, 70001])
+@pytest.mark.parametrize("shape, direct", [(dict(n_u16=2, n_u8=0, n_sdc=1, n_dense=1), True),   # one quad, a set of 128 rows per unit
+                                           (dict(n_u16=0, n_u8=1, n_sdc=1, n_dense=2), True),
+                                           (dict(n_u16=3, n_u8=0, n_sdc=0, n_dense=1, n_rle=0), True),
+                                           (dict(n_u16=1, n_u8=0, n_sdc=0, n_dense=2, n_rle=8), True),
+                                           (dict(n_u16=1, n_u8=0, n_sdc=0, n_dense=3), False),   # more dense values than a wave stages
+                                           (dict(n_u16=0, n_u8=1, n_sdc=0, n_dense=3, n_rle=0), False),
+                                           (dict(n_u16=1, n_u8=2, n_sdc=0, n_dense=4), True),    # two quads, 64 rows per unit
+                                           (dict(n_u16=1, n_u8=2, n_sdc=0, n_dense=5), False),
+                                           (dict(n_u16=1, n_u8=2, n_sdc=1, n_dense=7), True),    # three quads
+                                           (dict(n_u16=1, n_u8=2, n_sdc=1, n_dense=8, n_rle=0), True)])
+def test_few_varying_columns_with_dense_ones(cla, ora, shape, direct, n_rows):
+    """The forms of one and two quads of varying columns with dense ones among them, and those whose dense values the kernel does not stage."""
+    specs, n_cols = stream_block(n_rows % 13, n_rows, **{**dict(n_rle=3), **shape})
+    # (on a handful of rows run-length groups count as ones of short runs and offset lists may be empty)
+    check(cla, ora, specs, n_rows, n_cols, f"mix {shape}, {n_rows} rows", expect_direct=direct if n_rows > 1000 else None)
+
+
 def test_short_runs_and_bursts(cla, ora):
     """Runs barely longer than a slice, with stretches of one-row runs: several run ends per slice, window refills."""
     n_rows = 60000

@@ -78,6 +78,16 @@ def test_shapes(cla, ora, shape, p):
     check(cla, ora, specs, n_cols, n_rows, p, f"{shape}, {p} rows", rng)
 
 
+@pytest.mark.parametrize("shape", [(0, 1, 0, 0, 3), (3, 1, 0, 0, 3), (8, 0, 1, 0, 3), (2, 0, 1, 0, 4), (0, 3, 0, 0, 4), (2, 0, 0, 1, 3)])
+@pytest.mark.parametrize("n_rows,p", [(129, 1), (1030, 4), (70003, 8), (300001, 3)])
+def test_more_dense_columns_than_columns_behind_codes(cla, ora, shape, n_rows, p):
+    """One code column next to three dense ones: more dense values than the Gram kernel stages per unit of rows, which is no limit here."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows + p)
+    specs, n_cols = block(synth, rng, n_rows, *shape)
+    check(cla, ora, specs, n_cols, n_rows, p, f"{shape}, {p} rows", rng)
+
+
 @pytest.mark.parametrize("p,mean_run,kernel", [(6, 8, "k_lmm_decode"), (6, 40, "k_lmm_decode"), (6, 60, "k_lmm_direct"), (1, 8, "k_lmm_decode")])
 def test_many_short_runs_take_the_tile_kernel(cla, ora, p, mean_run, kernel):
     """Eight run-length columns of short runs next to too few other bytes for one-code-per-row copies: a run end for every row
