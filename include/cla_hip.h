@@ -165,7 +165,8 @@ int cla_block_drop_derived(cla_handle h);
  * instead of inside the first multiply): each product runs once on operands of zeros in temporary device
  * buffers (for CLA_PRODUCT_RMM an output of nRows x nColB doubles) that are freed before the call returns.
  * nColB: columns of B of the right multiplies to come (which forms a right multiply uses depends on it; 1 for
- * X %*% v), nRowY: rows of Y of the left multiplies; either is ignored when its product is not named. Waits for
+ * X %*% v), nRowY: rows of Y of the left multiplies; either is ignored when its product is not named. 1 and 1 are what the
+ * multiply chain consists of: the workspace of its one-pass form (option chain_fused) is allocated with them. Waits for
  * the stream. It has no counterpart in the reference. Returns 0 or a negative error. */
 #define CLA_PRODUCT_RMM 1u
 #define CLA_PRODUCT_LMM 2u

@@ -82,6 +82,15 @@ int ensure_tables(cla_block* b, size_t nDoubles) {
 	return 0;
 }
 
+int ensure_chain(cla_block* b, size_t nDoubles) {
+	if(nDoubles <= b->chainCap) return 0;
+	if(b->dChain) CLA_HIP(hipFree(b->dChain));
+	b->dChain = nullptr; b->chainCap = 0;
+	CLA_HIP(hipMalloc((void**) &b->dChain, nDoubles * sizeof(double)));
+	b->chainCap = nDoubles;
+	return 0;
+}
+
 // The dynamic LDS that a block of `kernel` may have: the device's less the kernel's static shared memory, which counts against the
 // same limit (__shared__ variables, and the scratch of __syncthreads_or). Set as the kernel's limit when it is first asked for.
 hipError_t max_dynamic_lds(const void* kernel, size_t& bytes) {
@@ -876,6 +885,8 @@ int cla_block_prepare(cla_handle b, uint32_t products, int32_t nColB, int32_t nR
 		if((rc = out.zeros((size_t) b->nCols * b->nCols, b->stream))) r = rc;
 		else r = tsmm_dev(b, out.p, true);
 	}
+	// X %*% v and one row of Y together: the products of the multiply chain, which on some blocks is a kernel with a workspace of its own
+	if(r >= 0 && (products & CLA_PRODUCT_RMM) && (products & CLA_PRODUCT_LMM) && nColB == 1 && nRowY == 1) r = prepare_chain_u8(b);
 	b->profile = profile;
 	clear_stats(b);
 	return r < 0 ? (int) r : 0;

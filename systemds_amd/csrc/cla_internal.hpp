@@ -183,7 +183,7 @@ struct cla_block {
 	double* dStageIn = nullptr; size_t stageInCap = 0;
 	double* dStageOut = nullptr; size_t stageOutCap = 0;
 	void* dScratch = nullptr;   size_t scratchCap = 0;
-	double* dChain = nullptr;   size_t chainCap = 0;   // X %*% v inside the multiply chain
+	double* dChain = nullptr;   size_t chainCap = 0;   // the multiply chain's own: X %*% v, or the sums of the blocks of its one kernel
 	// exact code counts of all dictionary-coded groups (totalVals int32, group g at tblOff[g]),
 	// computed on the first TSMM and kept, like the reference's cached counts
 	// (CG/AColGroupValue.java getCounts)
@@ -287,6 +287,7 @@ int launch_rmm_mfma(cla_block* b, const double* dB, int q, const double* dConstR
 int launch_lmm_u8(cla_block* b, const double* dY, int p, double* dPre);
 int launch_lmm_u8_dot(cla_block* b, const double* dY, int p, double* dOut);
 int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz);
+int prepare_chain_u8(cla_block* b);
 int launch_lmm_u8_vec(cla_block* b, const double* dY, double* dOut);
 int launch_lmm_sdc_tiles(cla_block* b, const double* dY, int p, double* dPre, int onlyGroup, double* dOut);
 int launch_lmm_sdc_lanes(cla_block* b, const double* dY, int p, double* dOut);
@@ -340,6 +341,7 @@ struct Prof {
 void clear_stats(cla_block* b);
 
 int ensure_tables(cla_block* b, size_t nDoubles);
+int ensure_chain(cla_block* b, size_t nDoubles);
 int ensure_dict_pad(cla_block* b); // padded dictionary image of byte-code blocks with one column per group (no-op otherwise)
 int ensure_scratch(cla_block* b, size_t bytes);
 

@@ -252,34 +252,62 @@ __global__ __launch_bounds__(CH_THREADS, NCB <= 3 ? 4 : 2) void k_chain_u8(const
 	}
 }
 
+// What a launch on a block takes.
+struct ChainLaunch {
+	decltype(&k_chain_u8<1, false>) kern = nullptr; // nullptr: the block is not eligible
+	unsigned grid = 0;
+	size_t lds = 0, wsDoubles = 0;
+};
+
+static int chain_shape(cla_block* b, bool op, ChainLaunch& L) {
+	const int nG = (int) b->groups.size();
+	// what X %*% v and t(y) %*% X of the block would run on the byte-code kernels, with nothing to add behind them; a column per group
+	if(b->dDictPad == nullptr || !b->u8ColsDistinct || b->hasConst || b->dictNonFinite || b->nRows == 0 || (b->opt.rmmDisable & 3) || (b->opt.lmmDisable & 1) ||
+		!b->opt.chainFused)
+		return 0;
+	const int nCb = (nG + 15) / 16;
+	decltype(&k_chain_u8<1, false>) kern = nullptr;
+#define CH_CASE(N) case N: kern = op ? k_chain_u8<N, true> : k_chain_u8<N, false>; break;
+	switch(nCb) { CH_CASE(1) CH_CASE(2) CH_CASE(3) CH_CASE(4) CH_CASE(5) CH_CASE(6) CH_CASE(7) default: return 0; }
+#undef CH_CASE
+	L.lds = std::max((size_t) nCb * b->maxVals * 128, (size_t) CH_WAVES * 4 * nCb * 16 * 8);
+	size_t room = 0;
+	CLA_HIP(max_dynamic_lds((const void*) kern, room));
+	if(L.lds > room) return 0;
+	const int64_t nUnits = std::max<int64_t>(b->nRows / WAVE, 1);
+	const int perCU = nCb <= 3 && L.lds <= (size_t) 78 * 1024 ? 2 : 1;
+	L.grid = (unsigned) std::min<int64_t>((nUnits + CH_WAVES - 1) / CH_WAVES, (int64_t) g_numCU * perCU);
+	L.wsDoubles = (size_t) L.grid * nCb * 16;
+	L.kern = kern;
+	return 0;
+}
+
+// The workspace of the chains to come, where the block's run in this kernel.
+int prepare_chain_u8(cla_block* b) {
+	for(bool op : {false, true}) {
+		ChainLaunch L;
+		int rc = chain_shape(b, op, L);
+		if(rc == 0 && L.kern != nullptr) rc = ensure_chain(b, L.wsDoubles);
+		if(rc) return rc;
+	}
+	return 0;
+}
+
 // Returns 1 when the block is not eligible (the chain then runs as two products), 0 when the chain has been queued.
 int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz) {
 	const int nG = (int) b->groups.size();
 	const int64_t nRows = b->nRows;
-	// what X %*% v and t(y) %*% X of the block would run on the byte-code kernels, with nothing to add behind them; a column per group
-	if(b->dDictPad == nullptr || !b->u8ColsDistinct || b->hasConst || b->dictNonFinite || nRows == 0 || (b->opt.rmmDisable & 3) || (b->opt.lmmDisable & 1) ||
-		!b->opt.chainFused)
-		return 1;
-	const int nCb = (nG + 15) / 16, nV = b->maxVals;
-	decltype(&k_chain_u8<1, false>) kern = nullptr;
-#define CH_CASE(N) case N: kern = ctype != 0 ? k_chain_u8<N, true> : k_chain_u8<N, false>; break;
-	switch(nCb) { CH_CASE(1) CH_CASE(2) CH_CASE(3) CH_CASE(4) CH_CASE(5) CH_CASE(6) CH_CASE(7) default: return 1; }
-#undef CH_CASE
-	const size_t lds = std::max((size_t) nCb * nV * 128, (size_t) CH_WAVES * 4 * nCb * 16 * 8);
-	size_t room = 0;
-	CLA_HIP(max_dynamic_lds((const void*) kern, room));
-	if(lds > room) return 1;
-	const int64_t nUnits = std::max<int64_t>(nRows / WAVE, 1);
-	const int perCU = nCb <= 3 && lds <= (size_t) 78 * 1024 ? 2 : 1;
-	const unsigned grid = (unsigned) std::min<int64_t>((nUnits + CH_WAVES - 1) / CH_WAVES, (int64_t) g_numCU * perCU);
-	const int rc = ensure_tables(b, (size_t) grid * nCb * 16);
-	if(rc) return rc;
+	ChainLaunch L;
+	int rc = chain_shape(b, ctype != 0, L);
+	if(rc || L.kern == nullptr) return rc ? rc : 1;
+	// (not the tables of the products: those of a captured one may not move)
+	if((rc = ensure_chain(b, L.wsDoubles))) return rc;
 	const int32_t* dCol0 = (const int32_t*) (b->dDictPad + (size_t) nG * 256);
 	clear_stats(b);
 	const double algo = (double) nRows * nG + (dW != nullptr ? (double) nRows * 8 : 0.0);
-	Prof pf(b, "k_chain_u8", grid, CH_THREADS, (long) lds, algo);
-	hipLaunchKernelGGL(kern, dim3(grid), dim3(CH_THREADS), lds, b->stream, b->dArena, b->arenaStride, nG, b->dDictPad + b->dictTOff, nV, dCol0, dV, dW,
-		ctype == 2 ? 1 : 0, nRows, b->dTables, dOut, b->nCols, b->lmm_ticket(), dNnz);
+	Prof pf(b, "k_chain_u8", L.grid, CH_THREADS, (long) L.lds, algo);
+	hipLaunchKernelGGL(L.kern, dim3(L.grid), dim3(CH_THREADS), L.lds, b->stream, b->dArena, b->arenaStride, nG, b->dDictPad + b->dictTOff, b->maxVals, dCol0,
+		dV, dW, ctype == 2 ? 1 : 0, nRows, b->dChain, dOut, b->nCols, b->lmm_ticket(), dNnz);
 	CLA_HIP(hipGetLastError());
 	return 0;
 }

@@ -635,15 +635,9 @@ int launch_mmchain(cla_block* b, const double* dV, const double* dW, int ctype, 
 		if(r <= 0) return r;
 	}
 	// the intermediate vector has a workspace of its own: the multiplies below may resize the shared scratch
-	const size_t need = (size_t) std::max<int64_t>(nRows, 1);
-	if(need > b->chainCap) {
-		if(b->dChain) CLA_HIP(hipFree(b->dChain));
-		b->dChain = nullptr; b->chainCap = 0;
-		CLA_HIP(hipMalloc((void**) &b->dChain, need * sizeof(double)));
-		b->chainCap = need;
-	}
+	int rc = ensure_chain(b, (size_t) std::max<int64_t>(nRows, 1));
+	if(rc) return rc;
 	double* tmp = b->dChain;
-	int rc;
 	// (the weights are read where X %*% v writes its rows: a pass of its own over 10 M rows takes 40 us)
 	RowOp op;
 	if(ctype != 0) { op.w = dW; op.minus = ctype == 2; }

@@ -1,8 +1,11 @@
 """The multiply chain of single-column byte-code blocks in one pass (k_chain_u8): row and column edges, weights, columns without a
 group, non-finite operands; against the exact chain, and against the two products where the exact one says nothing."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from devmem import DevBuf, hip
 from parity import assert_matches_truth
 
 pytestmark = pytest.mark.gpu
@@ -131,3 +134,44 @@ def test_chain_of_host_vectors(cla, ora, n_cols, n_rows, ctype):
         assert np.all(np.abs(out.reshape(-1, 1) - D.astype(np.longdouble).T @ u) <= 1e-12 * scale + 1e-300)
         assert nnz == np.count_nonzero(out) and blk.nnz() == nnz
     blk.close()
+
+
+@pytest.mark.parametrize("n_cols, n_vals, n_rows", [(5, 16, 250007), (54, 200, 100003), (3, 2, 70)])
+def test_prepared_chain_allocates_nothing(cla, ora, n_cols, n_vals, n_rows):
+    """Behind cla_block_prepare for X %*% v and one row of Y the first chain can be captured into a graph, which refuses allocations;
+    the graph's replays, other products of the block between them, give the chain of the vectors they find."""
+    rng = np.random.default_rng(n_cols)
+    specs, blk = block(cla, rng, n_rows, n_cols, n_vals)
+    h, stream = hip(), C.c_void_p()
+    ok = lambda rc: (_ for _ in ()).throw(AssertionError(rc)) if rc else None
+    ok(h.hipStreamCreate(C.byref(stream)))
+    blk.set_stream(stream.value)
+    blk.prepare(rmm_cols=1, lmm_rows=1)
+    v, w, y = rng.standard_normal(n_cols), rng.standard_normal(n_rows), rng.standard_normal((1, n_rows))
+    dV, dW, dO = DevBuf.from_numpy(v), DevBuf.from_numpy(w), DevBuf(n_cols * 8)
+    graph, run = C.c_void_p(), C.c_void_p()
+    ok(h.hipStreamBeginCapture(stream, 0))
+    blk.mmchain_dev_async(dV.ptr, dW.ptr, 1, dO.ptr)
+    ok(h.hipStreamEndCapture(stream, C.byref(graph)))
+    names = names_of(blk)
+    ok(h.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)))
+    assert names == ["k_chain_u8"], names
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    for k in range(4):
+        v = rng.standard_normal(n_cols)
+        ok(h.hipMemcpy(dV.ptr, v.ctypes.data_as(C.c_void_p), v.nbytes, 1))
+        dO.zero()
+        ok(h.hipDeviceSynchronize())
+        ok(h.hipGraphLaunch(run, stream))
+        ok(h.hipStreamSynchronize(stream))
+        got = dO.to_numpy(n_cols)
+        assert blk.nnz() == np.count_nonzero(got)
+        want, _ = blk.mmchain(v.reshape(-1, 1), w.reshape(-1, 1), 1)
+        assert np.array_equal(got, want.reshape(-1))
+        assert_matches_truth(got.reshape(-1, 1), D.T, (D @ v.reshape(-1, 1)) * w.reshape(-1, 1), what=f"replay {k}")
+        blk.rmm(v.reshape(-1, 1))
+        blk.lmm(y)
+    ok(h.hipGraphExecDestroy(run))
+    ok(h.hipGraphDestroy(graph))
+    blk.close()
+    ok(h.hipStreamDestroy(stream))
