@@ -86,23 +86,22 @@ __device__ __forceinline__ void count_add(unsigned long long* counter, int local
 		atomicAdd(nnz_way(counter, (blockDim.x / WAVE - 1) * blockIdx.x + threadIdx.x / WAVE), (unsigned long long) s);
 }
 
-// Called by one thread of every block of a launch behind the block's last add: true for the last block to arrive, which finds
-// the counters cleared for the next launch. Adds to one address are served one after the other, 11.4 ns each, so the blocks
-// count on TICKET_WAYS lines first and the last of each line on the first one: 256 blocks that end together wait 0.5 us in place of
-// 2.9 us for one more round trip.
+// Called by one thread of every block of a launch behind the block's last add: true for the last block to arrive. It clears the
+// counters for the next launch (clear_tickets) behind its own work: a store in front of it is waited for at the next barrier, 0.5 us. Adds to
+// one address are served one after the other, 11.4 ns each, a second line takes a round trip of 0.5 us: beyond TICKET_FEW blocks they count on
+// TICKET_WAYS lines first and the last of each line on the first one.
 __device__ __forceinline__ bool last_of_way(unsigned* done, unsigned nBlocks) {
 	const unsigned id = blockIdx.y * gridDim.x + blockIdx.x, way = id % TICKET_WAYS;
-	unsigned* const line = done + (1 + way) * (NNZ_STEP * 2);
-	if(atomicAdd(line, 1u) != (nBlocks - way + TICKET_WAYS - 1) / TICKET_WAYS - 1) return false;
-	*line = 0;
-	return true;
+	return atomicAdd(done + (1 + way) * (NNZ_STEP * 2), 1u) == (nBlocks - way + TICKET_WAYS - 1) / TICKET_WAYS - 1;
 }
-__device__ __forceinline__ bool last_of_ways(unsigned* done, unsigned nBlocks) {
-	if(atomicAdd(done, 1u) != min(nBlocks, (unsigned) TICKET_WAYS) - 1) return false;
-	*done = 0;
-	return true;
+__device__ __forceinline__ bool last_of_ways(unsigned* done, unsigned nBlocks) { return atomicAdd(done, 1u) == min(nBlocks, (unsigned) TICKET_WAYS) - 1; }
+__device__ __forceinline__ bool last_block(unsigned* done, unsigned nBlocks) {
+	return nBlocks <= TICKET_FEW ? atomicAdd(done, 1u) == nBlocks - 1 : last_of_way(done, nBlocks) && last_of_ways(done, nBlocks);
 }
-__device__ __forceinline__ bool last_block(unsigned* done, unsigned nBlocks) { return last_of_way(done, nBlocks) && last_of_ways(done, nBlocks); }
+// by a wave or more of the last block
+__device__ __forceinline__ void clear_tickets(unsigned* done) {
+	if(threadIdx.x < 1 + TICKET_WAYS) done[threadIdx.x * (NNZ_STEP * 2)] = 0;
+}
 
 // Tail of a left multiply whose kernel is the only one of the call: every block comes here behind its last add into
 // out; the last one to arrive counts the non-zeros of out[0 .. n) into *nnz
@@ -134,6 +133,7 @@ __device__ __forceinline__ void lmm_tail(unsigned* done, unsigned nBlocks, const
 		for(unsigned w = 0; w < (blockDim.x + WAVE - 1) / WAVE; w++) s += partS[w];
 		*nnz = (unsigned long long) s;
 	}
+	clear_tickets(done);
 }
 
 // Largest j in [0, nRuns) with runStart[j] <= row (runStart[0] == 0).

@@ -178,16 +178,17 @@ __device__ __forceinline__ void gram_tail(unsigned* done, unsigned nBlocks, doub
 	int* const gramPartS = (int*) lds + 1;
 	// rows r and nCols - 1 - r of the upper triangle together are nCols + 1 cells
 	const int w = nCols + 1, n = (nCols + 1) / 2 * w;
+	const float perW = 1.0f / (float) w;
 	auto cell_of = [&](int idx, int& i, int& j) {
-		const int r = idx / w, k = idx - r * w;
+		const int r = (int) (((float) idx + 0.5f) * perW), k = idx - r * w; // (exact: idx < 2^14, and idx + 0.5 is at least 1 / 2 w from a multiple of w)
 		const bool first = k < nCols - r;
 		i = first ? r : nCols - 1 - r;
 		j = first ? r + k : i + k - (nCols - r);
 		return idx < n && (first || i != r); // (the middle row is on its own)
 	};
-	// the cells of an accumulator, or of WAYS added up, left at zero; eight loads per thread requested together: each is a round trip past the caches
-	auto take = [&](double* from, auto waysTag, auto f) __attribute__((always_inline)) {
-		constexpr int M = decltype(waysTag)::value, NB = 8 / M;
+	// the cells of an accumulator, or of M added up, left at zero; NB cells per thread requested together: each is a round trip past the caches
+	auto take = [&](double* from, auto waysTag, auto cellsTag, auto f) __attribute__((always_inline)) {
+		constexpr int M = decltype(waysTag)::value, NB = decltype(cellsTag)::value;
 		const size_t way = (size_t) nCols * nCols;
 		for(int idx0 = threadIdx.x; idx0 < n; idx0 += NB * blockDim.x) {
 			unsigned long long bits[NB][M];
@@ -220,23 +221,26 @@ __device__ __forceinline__ void gram_tail(unsigned* done, unsigned nBlocks, doub
 		__syncthreads();
 		return lastS != 0;
 	};
-	if(!last([&]() { return last_of_way(done, nBlocks); })) return;
+	// a cell or two per thread: the last block reads all accumulators; more: the last block of each XCD adds its accumulator to the first
+	// one before (20 columns 24 against 26 us, 100 columns of 10,000 rows 40 against 43)
+	const bool ways = gram_ways(), few = n <= 2 * (int) blockDim.x, apart = ways && !few;
+	if(!last([&]() { return apart ? last_of_way(done, nBlocks) : last_block(done, nBlocks); })) return;
 	int cnt = 0;
 	auto give = [&](int i, int j, double v) __attribute__((always_inline)) {
 		out[(size_t) i * nCols + j] = v;
 		out[(size_t) j * nCols + i] = v;
 		cnt += v != 0.0 ? (i == j ? 1 : 2) : 0;
 	};
-	// a cell or two per thread: the last block reads all accumulators; more: the last block of each XCD adds its accumulator to the first
-	// one before (20 columns 24 against 26 us, 100 columns of 10,000 rows 40 against 43)
-	const bool ways = gram_ways(), apart = ways && n > 2 * (int) blockDim.x;
-	if(apart)
-		take(acc + gram_way(nCols), std::integral_constant<int, 1>(), [&](int i, int j, double v) {
+	using std::integral_constant;
+	if(apart) {
+		take(acc + gram_way(nCols), integral_constant<int, 1>(), integral_constant<int, 8>(), [&](int i, int j, double v) {
 			if(v != 0.0) unsafeAtomicAdd(&acc[(size_t) i * nCols + j], v); // (a NaN is unequal to zero)
 		});
-	if(!last([&]() { return last_of_ways(done, nBlocks); })) return;
-	if(ways && !apart) take(acc + (size_t) nCols * nCols, std::integral_constant<int, GRAM_WAYS>(), give);
-	else take(acc, std::integral_constant<int, 1>(), give);
+		if(!last([&]() { return last_of_ways(done, nBlocks); })) return;
+	}
+	if(!few) take(acc, integral_constant<int, 1>(), integral_constant<int, 8>(), give);
+	else if(ways) take(acc + (size_t) nCols * nCols, integral_constant<int, GRAM_WAYS>(), integral_constant<int, 1>(), give);
+	else take(acc, integral_constant<int, 1>(), integral_constant<int, 1>(), give); // (code that no block has run yet comes from memory, too)
 	cnt = wave_sum_i32(cnt);
 	if((threadIdx.x & (WAVE - 1)) == 0) gramPartS[threadIdx.x >> 6] = cnt;
 	nnz_clear(nnz);
@@ -246,6 +250,7 @@ __device__ __forceinline__ void gram_tail(unsigned* done, unsigned nBlocks, doub
 		for(unsigned w = 0; w < (blockDim.x + WAVE - 1) / WAVE; w++) s += gramPartS[w];
 		*nnz = (unsigned long long) s;
 	}
+	clear_tickets(done);
 }
 
 int mrt_build(cla_block* b, const std::vector<RunCol>& runs, int sliceRows, Mrt& T);

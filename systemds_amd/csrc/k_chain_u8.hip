@@ -250,6 +250,7 @@ __global__ __launch_bounds__(CH_THREADS, NCB <= 3 ? 4 : 2) void k_chain_u8(const
 		for(int i = 0; i < CH_WAVES; i++) n += cntS[i];
 		*nnz = (unsigned long long) n;
 	}
+	clear_tickets(done);
 }
 
 // What a launch on a block takes.

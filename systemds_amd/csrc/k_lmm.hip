@@ -382,7 +382,9 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 			A.nnz[0] = s;
 	}
 	__syncthreads();
-	if(lastS && tid > 0 && tid < NNZ_WAYS) A.nnz[tid * NNZ_STEP] = 0;
+	if(!lastS) return;
+	if(tid > 0 && tid < NNZ_WAYS) A.nnz[tid * NNZ_STEP] = 0;
+	clear_tickets(A.done);
 }
 
 // (a kernel, not hipMemsetAsync: a memset node of a captured graph has given wrong results on its replays)
