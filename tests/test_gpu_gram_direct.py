@@ -124,6 +124,23 @@ def test_short_runs_and_bursts(cla, ora):
     check(cla, ora, specs, n_rows, n_cols, "short runs")
 
 
+@pytest.mark.parametrize("n_rows", [1023, 1025, 30011])
+@pytest.mark.parametrize("mean_run, n_vals", [(66, 5), (120, 300), (140, 5), (400, 300), (2500, 700)])
+def test_runs_on_the_tile_kernel(cla, ora, n_rows, mean_run, n_vals):
+    """Run-length columns of one- and two-byte codes expanded tile by tile, some rows without a run: more runs per tile than the lanes
+    write together, fewer, one over several tiles."""
+    specs, n_cols = stream_block(n_vals + n_rows, n_rows, n_rle=1, n_u16=2, n_u8=1, n_sdc=1, n_dense=1, mean_run=mean_run)
+    rng = np.random.default_rng(mean_run)
+    specs += [rle_group(rng, n_rows, [n_cols], n_vals, mean_run, uncovered=True), rle_group(rng, n_rows, [n_cols + 1], n_vals, 3 * mean_run, bursts=True)]
+    n_cols += 2
+    check(cla, ora, specs, n_rows, n_cols, f"runs of {mean_run}", expect_direct=False, options={"tsmm_direct": 0, "tsmm_route": 2})
+    blk = cla.build_block(n_rows, n_cols, specs).set_option("tsmm_direct", 0).set_option("rmm_direct", 0)
+    B, Y, D = rng.standard_normal((n_cols, 5)), rng.standard_normal((3, n_rows)), ora.np_decompress(specs, n_rows, n_cols)
+    assert_matches_truth(blk.rmm(B)[0], D, B, what="X%*%B")
+    assert_matches_truth(blk.lmm(Y)[0], Y, D, what="Y%*%X")
+    blk.close()
+
+
 def test_cocoded_groups(cla, ora):
     """Two columns per DDC group (one stream, two columns) and two columns per RLE group (one run table, two columns)."""
     n_rows = 50021
