@@ -487,6 +487,18 @@ int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	if(P->spread < 0)
 		if(const int rc = gdr_look(b, *b->gdrPlan)) return rc;
 	if(P->spread && P->A.nR > 0) return 1;
+	const int nUnits = (int) ((b->nRows + 32 * gdr_sets(P->quads) - 1) / (32 * gdr_sets(P->quads)));
+	// A wave takes the run ends of its rows one after the other, 0.4 us each: a unit per wave where there are many (100,003 rows of 9 columns, 8
+	// run-length of mean run 100: 19 us, two units 27; of 5000 12 and 12, 300,007 rows 12.9 and 12.1), else two.
+	const int share = P->waves * (P->runEnds * 400 > b->nRows ? 1 : 2);
+	const unsigned grid = (unsigned) std::max(1, std::min((nUnits + share - 1) / share, g_numCU * (P->lds <= 76 * 1024 && P->waves == 8 ? 2 : 1)));
+	// The tile kernel hardly notices run ends, but takes 35 ns more per 1000 rows. Both meet at 9 run ends per wave on 20,011 rows, 10 on
+	// 100,003, 22 on 300,007, 43 on 1,000,003 and 195 on 5,000,011 (one column behind codes, 8, 4 and 2 run-length ones; in us here / there:
+	// 20,011 rows, 8 of mean run 100 17.5 / 19.2, of 48 25 / 19; 300,007, 8 of 48 29 / 34, of 24 43 / 32; 5,000,011, 4 of 48 99 / 162, of 12 290 / 160).
+	if(P->runEnds / ((int64_t) grid * P->waves) > 8 + b->nRows / 27000) {
+		const int rc = tsmm_decode_fits(b);
+		if(rc <= 0) return rc < 0 ? rc : 1;
+	}
 	GdrArgs A = P->A;
 	A.out = dOut;
 	A.acc = nullptr; A.done = nullptr; A.nnz = nullptr;
@@ -495,8 +507,6 @@ int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz) {
 		if(rc) return rc;
 		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
-	const int nUnits = (int) ((b->nRows + 32 * gdr_sets(P->quads) - 1) / (32 * gdr_sets(P->quads)));
-	const unsigned grid = (unsigned) std::max(1, std::min((nUnits + P->waves * 2 - 1) / (P->waves * 2), g_numCU * (P->lds <= 76 * 1024 && P->waves == 8 ? 2 : 1)));
 	Prof pf(b, "k_tsmm_direct", grid, P->waves * 64, (long) P->lds, (double) b->device_bytes_cached);
 	bool launched = false;
 #define GDR_CASE(NQV, NDV, HASRV, WV)                                                                                             \

@@ -124,6 +124,14 @@ def test_short_runs_and_bursts(cla, ora):
     check(cla, ora, specs, n_rows, n_cols, "short runs")
 
 
+@pytest.mark.parametrize("n_rows, n_rle, mean_run, direct", [(3001, 8, 12, False), (3001, 8, 200, True), (20011, 8, 12, False), (20011, 8, 48, False), (20011, 4, 200, True),
+                                                             (100003, 4, 12, False), (100003, 8, 66, False), (100003, 2, 100, True), (300007, 8, 12, False), (300007, 8, 100, True)])
+def test_many_run_ends_take_the_tile_kernel(cla, ora, n_rows, n_rle, mean_run, direct):
+    """Short runs next to too few other bytes for one-code-per-row copies: a wave takes its run ends one by one, the tile kernel does not."""
+    specs, n_cols = stream_block(mean_run, n_rows, n_rle=n_rle, n_u16=1, n_u8=0, n_sdc=0, n_dense=0, mean_run=mean_run)
+    check(cla, ora, specs, n_rows, n_cols, f"{n_rle} columns of runs of {mean_run}", expect_direct=direct)
+
+
 @pytest.mark.parametrize("n_rows", [1023, 1025, 30011])
 @pytest.mark.parametrize("mean_run, n_vals", [(66, 5), (120, 300), (140, 5), (400, 300), (2500, 700)])
 def test_runs_on_the_tile_kernel(cla, ora, n_rows, mean_run, n_vals):
