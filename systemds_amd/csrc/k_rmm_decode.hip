@@ -1082,6 +1082,7 @@ struct DirArgs {
 	const double* runSums;
 	int nR;
 	int nDicts, dictDoubles;
+	int stageGap;           // 16-byte pieces behind every pair of rows in a wave's staging area: 0 or 1
 	int segEnd[DSEG_N];
 	const double* B;        // first of the QV columns of this launch
 	const double* constRow;
@@ -1111,7 +1112,12 @@ __global__ __launch_bounds__(DIR_THREADS) void k_rmm_direct(const DirArgs A) {
 	if(tid < 2) smem[A.dictDoubles - 2 + tid] = 0.0; // what a filler column looks up
 	__syncthreads();
 	const uint8_t* const ldsBytes = (const uint8_t*) smem;
-	double* const wstage = smem + A.dictDoubles + (size_t) wave * DIR_SROWS * QV;
+	// Sixteen lanes write a pair of rows each and 64 read 16 bytes each. An even number of columns puts the pairs where several start in the
+	// same banks (8 columns: eight of 16, 16 columns: all), unless a gap of 16 bytes follows each (in us without / with gaps: 100,003 rows of 4
+	// columns by 8 17.5 / 12.8, of 20 by 16 38 / 29; 8,000,001 of 20 by 12 375 / 298, by 8 211 / 200).
+	const int gap = QV & 1 ? 0 : A.stageGap;
+	double* const wstage = smem + A.dictDoubles + (size_t) wave * (DIR_SROWS * QV + DIR_SROWS * gap);
+	auto staged = [&](int i) { return (const double*) wstage + i + (QV & 1 ? 0 : i / (2 * QV) * 2 * gap); }; // value i of the staged rows
 	const dec_cdp Bc = (dec_cdp) A.B;
 	const int64_t nRows = A.nRows;
 	const int64_t nSlices = (nRows + DIR_SLICE - 1) / DIR_SLICE;
@@ -1258,7 +1264,7 @@ __global__ __launch_bounds__(DIR_THREADS) void k_rmm_direct(const DirArgs A) {
 		for(int part = 0; part < DIR_SLICE / DIR_SROWS; part++) {
 			dec_wave_sync(); // the readers of the staging area are done
 			if((lane >> 4) == part) {
-				double* w = wstage + (size_t) (lane & 15) * 2 * QV;
+				double* w = wstage + (lane & 15) * 2 * (QV + gap);
 #pragma unroll
 				for(int j = 0; j < QV; j++) { w[j] = acc[0][j]; w[QV + j] = acc[1][j]; }
 			}
@@ -1271,12 +1277,12 @@ __global__ __launch_bounds__(DIR_THREADS) void k_rmm_direct(const DirArgs A) {
 #pragma unroll
 				for(int i = 2 * lane; i < DIR_SROWS * QV; i += 128) {
 					if(i + 1 < n) {
-						const f64x2 v = *(const f64x2*) (wstage + i);
+						const f64x2 v = *(const f64x2*) staged(i);
 						cnt += (v[0] != 0.0) + (v[1] != 0.0);
 						__builtin_nontemporal_store(v, (f64x2*) (o + i));
 					}
 					else if(i < n) {
-						const double v = wstage[i];
+						const double v = *staged(i);
 						cnt += v != 0.0;
 						__builtin_nontemporal_store(v, o + i);
 					}
@@ -1290,7 +1296,7 @@ __global__ __launch_bounds__(DIR_THREADS) void k_rmm_direct(const DirArgs A) {
 					const int r0 = i / QV, c0 = i - r0 * QV;
 					if(pairs) {
 						if(i + 1 < n) {
-							const f64x2 v = *(const f64x2*) (wstage + i);
+							const f64x2 v = *(const f64x2*) staged(i);
 							cnt += (v[0] != 0.0) + (v[1] != 0.0);
 							__builtin_nontemporal_store(v, (f64x2*) (o + (size_t) r0 * A.ld + c0));
 						}
@@ -1300,7 +1306,7 @@ __global__ __launch_bounds__(DIR_THREADS) void k_rmm_direct(const DirArgs A) {
 						for(int e = 0; e < 2; e++)
 							if(i + e < n) {
 								const int r = (i + e) / QV, c = (i + e) - r * QV;
-								const double v = wstage[i + e];
+								const double v = staged(i)[e];
 								cnt += v != 0.0;
 								__builtin_nontemporal_store(v, o + (size_t) r * A.ld + c);
 							}
@@ -1438,8 +1444,10 @@ static int launch_rmm_direct(cla_block* b, const double* dB, int q, const double
 		if(rc) return rc;
 	}
 	DirArgs A = b->dirPlan->A;
-	const size_t ldsMax = ((size_t) A.dictDoubles + (size_t) DIR_WAVES * DIR_SROWS * std::min(q, 16)) * 8;
-	if(ldsMax > (size_t) std::min(g_ldsPerBlock, 160 * 1024) - 1024) return 1;
+	const size_t room = (size_t) std::min(g_ldsPerBlock, 160 * 1024) - 1024;
+	const size_t ldsMax = ((size_t) A.dictDoubles + (size_t) DIR_WAVES * DIR_SROWS * std::min(q, 16)) * 8, ldsGaps = (size_t) DIR_WAVES * DIR_SROWS * 8;
+	if(ldsMax > room) return 1;
+	A.stageGap = ldsMax + ldsGaps <= room;
 	A.nnz = dNnz; A.ld = q;
 	const int64_t nSlices = (b->nRows + DIR_SLICE - 1) / DIR_SLICE;
 	const unsigned grid = (unsigned) std::min<int64_t>((nSlices + DIR_WAVES - 1) / DIR_WAVES, g_numCU);
@@ -1448,7 +1456,7 @@ static int launch_rmm_direct(cla_block* b, const double* dB, int q, const double
 	const int chunk = 16;
 	for(int c0 = 0; c0 < q; c0 += chunk) {
 		const int qv = std::min(chunk, q - c0);
-		const size_t lds = ((size_t) A.dictDoubles + (size_t) DIR_WAVES * DIR_SROWS * qv) * 8;
+		const size_t lds = ((size_t) A.dictDoubles + (size_t) DIR_WAVES * DIR_SROWS * qv) * 8 + (A.stageGap ? ldsGaps : 0);
 		A.B = dB + c0; A.constRow = dConstRow ? dConstRow + c0 : nullptr; A.out = dOut + c0;
 		const double algo = (double) b->device_bytes_cached + (double) b->nRows * qv * 8;
 		if(A.nR > 0) {

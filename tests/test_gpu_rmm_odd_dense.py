@@ -49,3 +49,28 @@ def test_odd_number_of_dense_columns(cla, ora, n_rows, unc, runs, odd_values, q)
     rows = fin.all(axis=1)
     if rows.any():
         assert_matches_truth(out.reshape(n_rows, q)[rows], D[rows], B, what=f"odd dense q={q}")
+
+
+@pytest.mark.parametrize("n_rows", [1, 31, 33, 129, 40003])
+@pytest.mark.parametrize("n_vals", [60, 970, 1010])
+@pytest.mark.parametrize("q", [1, 4, 8, 10, 12, 15, 16, 24, 32])
+def test_staging_with_and_without_gaps(cla, ora, n_rows, n_vals, q):
+    """Rows on their way out of the kernel on streams: pairs of rows apart in LDS where 12 dictionaries leave room for it (with 16 columns of B those
+    of 970 values do, those of 1010 do not), behind one another where they do not."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_vals + q)
+    specs, n_cols = [], 12
+    for c in range(n_cols):
+        specs.append(synth.GroupSpec("ddc", np.array([c], np.int32), rng.standard_normal((n_vals, 1)), rng.integers(0, n_vals, n_rows).astype(np.uint16)))
+    if n_rows > 1:  # (run-length columns: 16 columns of B on this kernel, too)
+        codes = np.where(np.arange(n_rows) < n_rows // 2, 1, 0)
+        ptr, data = synth.encode_rle(codes, 2)
+        specs.append(synth.GroupSpec("rle", np.array([n_cols], np.int32), rng.standard_normal((2, 1)), ptr=ptr, rle=data))
+        n_cols += 1
+    B = rng.standard_normal((n_cols, q))
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, nnz = blk.rmm(B)
+    blk.close()
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    assert_matches_truth(out, D, B, what=f"{n_vals} values, q={q}")
+    assert nnz == np.count_nonzero(out)
