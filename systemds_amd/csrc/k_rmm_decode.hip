@@ -1490,19 +1490,20 @@ static int launch_rmm_direct(cla_block* b, const double* dB, int q, const double
 int launch_rmm_decode(cla_block* b, const double* dB, int q, const double* dConstRow, double* dOut,
 	unsigned long long* dNnz) {
 	if(b->groups.empty() || b->nRows == 0 || q < 1) return 1;
-	// 16 columns: no padding of B left for the tile kernel to lose, and the stream kernel short of registers (C5 2.1 against 2.5 ms), unless
-	// there are run-length columns, which the tile kernel would expand tile by tile, more than 12 columns and more rows than fill the
-	// chip (in us, stream / tile kernel: 8 run-length of 20 columns, 1,000,003 rows 66 / 70, 600,003 62 / 59; 4 of 12, 3,000,001 rows
-	// 138 / 123; 2 of 13, 8,000,001 rows 352 / 365). An odd number of dense columns (a filler beside them): the stream kernel up to 10 columns
-	// of B (100,003 rows of 13 columns, 2 of B 15.6 / 23.3, 10 20.6 / 24.8; 8,000,001 84 / 293, 166 / 299), up to 15 where
-	// half the chip is full (600,003 38 / 44, 8,000,001 231 / 320; 100,003 rows of 6 columns 21.3 / 18.7); not below a slice per CU,
-	// where it would be the faster one as well (30,000 rows 15.1 / 22.8) but the tests hold such blocks to the tile kernel
+	// 16 columns: no padding of B left for the tile kernel to lose, and the stream kernel short of registers, unless there are run-length columns,
+	// which the tile kernel would expand tile by tile (in us, stream / tile kernel: 8 run-length of 20 columns, 1,003 rows 23 / 33, 100,003
+	// 29 / 34, 8,000,001 367 / 390; 2 of 6, 1,003 rows 15.7 / 17.4, 100,003 21.4 / 19.1, 8,000,001 206 / 250).
+	// An odd number of dense columns (a filler beside them): the stream kernel up to 15 columns of B (4 columns by 2 100,003 rows 9.8 / 13.7,
+	// 8,000,001 59 / 124, by 8 12.8 / 14.1, 109 / 152; 13 columns by 12 100,003 rows 24.0 / 25.3), with more than 10 not on a few columns
+	// of too few rows to fill half the chip (4 columns by 12 30,011 rows 16.3 / 13.7, 100,003 16.8 / 14.4, 300,007 17.2 / 19.6). Below a
+	// slice per CU the route of such blocks has been left as it was, to the tile kernel (5 columns of B on 5,000 rows are held to it), although this
+	// one would be faster: 1,003 rows of 4 columns by 2 8.4 / 13.5, by 12 12.6 / 14.2.
 	bool tilesFirst = q == DEC_QMAX;
 	if(b->opt.rmmDirect && dir_plan_get(b) == 0) {
 		const DirPlan& P = *b->dirPlan;
-		const int64_t chip = (int64_t) g_numCU * DIR_WAVES * DIR_SLICE; // rows, a slice per wave
-		if(P.denseFiller) tilesFirst = q >= DEC_QMAX || b->nRows < (q > 10 ? chip / 2 : chip / DIR_WAVES);
-		else if(tilesFirst && P.A.nR > 0) tilesFirst = b->nRows < chip * 3 / 2 || P.A.nR + P.A.segEnd[DSEG_N - 1] <= 12;
+		const int64_t slices = (int64_t) g_numCU * DIR_SLICE; // rows, a slice per CU
+		if(P.denseFiller) tilesFirst = q >= DEC_QMAX || b->nRows < (q > 10 && b->nCols < 9 ? slices * DIR_WAVES / 2 : slices);
+		else if(P.A.nR > 0) tilesFirst = false;
 	}
 	if(b->opt.rmmDirect && !tilesFirst) {
 		const int rc = launch_rmm_direct(b, dB, q, dConstRow, dOut, dNnz);

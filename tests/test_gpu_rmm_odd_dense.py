@@ -51,6 +51,39 @@ def test_odd_number_of_dense_columns(cla, ora, n_rows, unc, runs, odd_values, q)
         assert_matches_truth(out.reshape(n_rows, q)[rows], D[rows], B, what=f"odd dense q={q}")
 
 
+@pytest.mark.parametrize("q", [11, 12, 15])
+def test_more_columns_on_few_rows(cla, ora, q):
+    """Nine columns and more take the kernel on streams from a slice per CU on, whatever the number of columns of B up to 15."""
+    from systemds_amd import synth
+    for n_rows in (32768, 40003):
+        rng = np.random.default_rng(n_rows + q)
+        specs, n_cols, blk = block(cla, synth, rng, n_rows, 3, 3, False)
+        B = rng.standard_normal((n_cols, q))
+        out, nnz = blk.rmm(B)
+        names = [k["name"] for k in blk.stats()["kernels"]]
+        blk.close()
+        assert n_cols == 9 and "k_rmm_direct" in names, names
+        assert_matches_truth(out, ora.np_decompress(specs, n_rows, n_cols), B, what=f"nine columns, q={q}")
+        assert nnz == np.count_nonzero(out)
+
+
+@pytest.mark.parametrize("n_rows", [257, 1003, 40003])
+@pytest.mark.parametrize("q", [15, 16])
+def test_sixteen_columns_of_b(cla, ora, n_rows, q):
+    """An even number of dense columns: as for 15 columns of B next to run-length columns, on the tile kernel without them."""
+    from systemds_amd import synth
+    for runs in (3, 0):
+        rng = np.random.default_rng(n_rows + q)
+        specs, n_cols, blk = block(cla, synth, rng, n_rows, 2, runs, False)
+        B = rng.standard_normal((n_cols, q))
+        out, nnz = blk.rmm(B)
+        names = [k["name"] for k in blk.stats()["kernels"]]
+        blk.close()
+        assert ("k_rmm_direct" in names) == (q == 15 or runs > 0), (runs, names)
+        assert_matches_truth(out, ora.np_decompress(specs, n_rows, n_cols), B, what=f"{runs} run-length columns, q={q}")
+        assert nnz == np.count_nonzero(out)
+
+
 @pytest.mark.parametrize("n_rows", [1, 31, 33, 129, 40003])
 @pytest.mark.parametrize("n_vals", [60, 970, 1010])
 @pytest.mark.parametrize("q", [1, 4, 8, 10, 12, 15, 16, 24, 32])
