@@ -9,6 +9,7 @@
 //   k_lmm_finish        + rowSum (x) constV, non-zero count
 #include "../../include/cla_hip.h"
 #include "cla_device.hpp"
+#include "cla_runs.hpp"
 #include <algorithm>
 #include <cstring>
 
@@ -241,6 +242,7 @@ struct LmmTake {
 	const unsigned long long* bad;
 	unsigned long long* count;     // zero
 	const double* constV;          // nullptr: no constants
+	unsigned long long redo;       // columns that a non-finite Y takes anew
 	double* out;
 	int nCols;
 	unsigned* done;
@@ -251,16 +253,19 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 	__shared__ int lastS;
 	__shared__ int cntS[LT_THREADS / WAVE];
 	__shared__ double sumS[LT_P * (LT_COLS + 1)]; // the block's sums of some rows of Y: by column, then the row sum
+	__shared__ int32_t runS[LT_THREADS / WAVE][2 * WAVE + 1]; // per wave: starts of 64 runs and the end of the last, their codes
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = A.p * A.nCols;
 	double* const rs = A.anew + n;
-	const bool anew = *A.bad != 0;
+	const bool anew = *A.bad != 0 && (A.redo != 0 || A.constV != nullptr);
 	const int nTake = min((int) gridDim.x, (n + LT_THREADS * 4 - 1) / (LT_THREADS * 4)); // blocks that take the result out of its stage
 	if(!anew && (int) blockIdx.x >= nTake) return;
 	if(anew) {
-		auto product = [&](auto pTag) { // a few rows of Y per look at a group's codes
+		auto product = [&](auto pTag) { // a few rows of Y per look at a group's codes; a share of the rows and those rows of Y per turn of a block
 			constexpr int LP = decltype(pTag)::value;
-			const int64_t r0 = A.nRows * blockIdx.x / gridDim.x, r1 = A.nRows * (blockIdx.x + 1) / gridDim.x;
-			for(int i0 = 0; i0 < A.p; i0 += LP) {
+			const int nY = (A.p + LP - 1) / LP, nParts = max(1, (int) gridDim.x / nY);
+			for(int turn = blockIdx.x; turn < nParts * nY; turn += gridDim.x) {
+				const int part = turn / nY, i0 = (turn - part * nY) * LP;
+				const int64_t r0 = A.nRows * part / nParts, r1 = A.nRows * (part + 1) / nParts;
 				const double* y[LP];
 #pragma unroll
 				for(int i = 0; i < LP; i++) y[i] = A.Y + (size_t) min(i0 + i, A.p - 1) * A.nRows;
@@ -279,6 +284,7 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 				for(int g = 0; g < A.nGroups; g++) {
 					const DGroup G = dgroup(A.groups + g);
 					for(int h = 0; h < G.nColG; h++) {
+						if((A.redo >> G.cols[h] & 1) == 0) continue;
 						double s[LP] = {};
 						if(G.type == G_DDC || G.type == G_UNC) {
 #pragma unroll 2
@@ -289,13 +295,30 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 							}
 						}
 						else if(G.type == G_RLE && G.nRuns > 0) {
-							int64_t r = r0 + tid;
-							int j = r < r1 ? rle_find(G.runStart, G.nRuns, (int32_t) r) : 0;
-							for(; r < r1; r += LT_THREADS) {
-								while(G.runStart[j + 1] <= r) j++; // (the last run ends at the last row)
-								const int code = G.runCode[j];
-								if(code < 0) continue;
-								const double x = G.dict[(size_t) code * G.nColG + h];
+							// Consecutive rows per wave, 64 at a time. The run table comes 64 runs at a time through LDS, where every lane finds its
+							// row's: followed in memory lane by lane it takes a gather or more per row.
+							int32_t* const start = runS[wave];
+							int32_t* const code = start + WAVE + 1;
+							const int64_t w0 = r0 + (r1 - r0) * wave / (LT_THREADS / WAVE), w1 = r0 + (r1 - r0) * (wave + 1) / (LT_THREADS / WAVE);
+							int base = 0;
+							auto window = [&](int64_t row) { // the runs from the one of `row` on
+								base = __builtin_amdgcn_readfirstlane(rle_find(G.runStart, G.nRuns, (int32_t) row));
+								wave_lds_sync();
+								start[lane] = G.runStart[min(base + lane, G.nRuns)];
+								code[lane] = G.runCode[min(base + lane, G.nRuns - 1)];
+								if(lane == 0) start[WAVE] = G.runStart[min(base + WAVE, G.nRuns)]; // (the last run ends at the last row)
+								wave_lds_sync();
+							};
+							if(w0 < w1) window(w0);
+							for(int64_t row0 = w0; row0 < w1; row0 += WAVE) {
+								if(start[WAVE] < min(row0 + WAVE, w1)) window(row0); // (a run has a row at least: 64 runs hold 64 rows)
+								const int64_t r = min(row0 + lane, w1 - 1);
+								int k = 0;
+#pragma unroll
+								for(int half = WAVE / 2; half > 0; half >>= 1) k += start[k + half] <= r ? half : 0;
+								const int c = code[k];
+								if(row0 + lane >= w1 || c < 0) continue;
+								const double x = G.dict[(size_t) c * G.nColG + h];
 #pragma unroll
 								for(int i = 0; i < LP; i++) s[i] += y[i][r] * x;
 							}
@@ -306,13 +329,15 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 #pragma unroll
 								for(int i = 0; i < LP; i++) s[i] += y[i][row] * x;
 							};
-							if(blockIdx.x == 0 && tid == 0) take(G.first, 0);
-							if(wave < SDC_CK / 256) for(int c = blockIdx.x; c < G.nCkpt; c += gridDim.x) { // (a wave takes 256 entries of a chunk)
+							constexpr int CW = SDC_CK / 256, CB = LT_THREADS / WAVE / CW; // waves per chunk, 256 entries each; chunks per block
+							static_assert(CB >= 1, "a wave per 256 entries of a chunk");
+							if(part == 0 && tid == 0) take(G.first, 0);
+							if(wave < CW * CB) for(int c = part * CB + wave / CW; c < G.nCkpt; c += nParts * CB) {
 								const OffState st = G.ckpt[c];
 								int32_t row = st.row, emit = st.emit, rows[4], didx[4];
 								unsigned mask;
 								const int64_t base = (int64_t) c * SDC_CK;
-								for(int w = 0; w <= wave; w++) {
+								for(int w = 0; w <= wave % CW; w++) {
 									if(G.deltaWidth == 1) sdc_decode256<1>(G.deltas, G.nDeltas, base + w * 256, row, emit, rows, didx, mask);
 									else sdc_decode256<2>(G.deltas, G.nDeltas, base + w * 256, row, emit, rows, didx, mask);
 								}
@@ -355,7 +380,7 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 	for(int idx = tid + (anew ? 0 : (int) blockIdx.x * LT_THREADS); idx < n; idx += step) {
 		double v;
 		if(anew) {
-			v = summed(A.anew + idx);
+			v = A.redo >> (idx % A.nCols) & 1 ? summed(A.anew + idx) : A.stage[idx];
 			if(A.constV != nullptr) { // (skipped for a row sum of zero, as in k_lmm_finish)
 				const double vl = summed(rs + idx / A.nCols);
 				if(vl != 0.0) v += vl * A.constV[idx % A.nCols];
@@ -405,8 +430,14 @@ int launch_lmm_take(cla_block* b, const double* dY, int p, double* ws, double* d
 	A.Y = dY; A.p = p; A.nRows = b->nRows; A.nCols = b->nCols;
 	A.stage = ws; A.anew = ws + n; A.bad = (const unsigned long long*) (ws + 2 * n + p); A.count = (unsigned long long*) (ws + 2 * n + p + 1);
 	A.constV = b->hasConst ? b->dConstV : nullptr;
+	A.redo = ~0ull; // (at most LT_COLS columns)
+	for(const HostGroup& H : b->groups)
+		if(H.d.type == G_DDC || H.d.type == G_UNC)
+			for(int c : H.cols)
+				if(b->constV[c] == 0.0) A.redo &= ~(1ull << c);
+	if(b->nCols < LT_COLS) A.redo &= (1ull << b->nCols) - 1;
 	A.out = dOut; A.done = b->lmm_ticket(); A.nnz = dNnz;
-	const unsigned grid = (unsigned) std::max<int64_t>(1, std::min<int64_t>((b->nRows + 1023) / 1024, g_numCU));
+	const unsigned grid = (unsigned) std::max<int64_t>(1, std::min<int64_t>((b->nRows + 1023) / 1024 * ((p + LT_P - 1) / LT_P), b->nRows < 2000000 ? g_numCU : 2 * g_numCU));
 	Prof pf(b, "k_take_block", grid, LT_THREADS, 0, 0);
 	hipLaunchKernelGGL(k_take_block, dim3(grid), dim3(LT_THREADS), 0, b->stream, A);
 	CLA_HIP(hipGetLastError());

@@ -17,10 +17,23 @@ def blocks(kind, n_rows):
         return mixed_block(13, n_rows, with_unc=True, big_dict=False)
     if kind == "mixed, no constants":
         return mixed_block(4, n_rows, with_unc=True, with_const=False, big_dict=False)
+    if kind == "constants":  # under a dictionary column, a dense one and a run-length one, and on columns that no other group covers
+        specs, n_cols = block(synth, rng, n_rows, 2, 2, 1, 1, 2)
+        cols = np.array([next(s for s in specs if s.type == t).cols[0] for t in ("ddc", "unc", "rle")] + [n_cols, n_cols + 1], np.int32)
+        return specs + [synth.GroupSpec("const", cols, np.array([[-0.75, 1.5, 2.0, 0.0, -3.0]]))], n_cols + 2
+    if kind == "short runs":
+        return block(synth, rng, n_rows, 8, 1, 0, 0, 0, mean_run=7)
+    if kind == "wide groups":
+        specs, n_cols = block(synth, rng, n_rows, 1, 0, 1, 1, 0)
+        specs.append(synth.GroupSpec("ddc", np.arange(n_cols, n_cols + 7, dtype=np.int32), rng.standard_normal((300, 7)), rng.integers(0, 300, n_rows).astype(np.uint16)))
+        codes = np.repeat(rng.integers(-1, 5, n_rows // 9 + 1), 9)[:n_rows]
+        ptr, rle = synth.encode_rle(codes, 5)
+        specs.append(synth.GroupSpec("rle", np.arange(n_cols + 7, n_cols + 10, dtype=np.int32), rng.standard_normal((5, 3)), ptr=ptr, rle=rle))
+        return specs, n_cols + 10
     return block(synth, rng, n_rows, *{"runs": (8, 4, 2, 1, 2), "streams": (0, 5, 3, 0, 0), "dense": (2, 0, 1, 1, 4)}[kind])
 
 
-@pytest.mark.parametrize("kind", ["mixed", "mixed, no constants", "runs", "streams", "dense"])
+@pytest.mark.parametrize("kind", ["mixed", "mixed, no constants", "runs", "streams", "dense", "constants", "short runs", "wide groups"])
 @pytest.mark.parametrize("n_rows,p", [(1, 1), (257, 3), (1025, 17), (40001, 2), (40001, 9), (300007, 70)])
 @pytest.mark.parametrize("direct", [1, 0])
 def test_non_finite_y(cla, ora, kind, n_rows, p, direct):
