@@ -108,8 +108,8 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  * the decompressing right multiply, CG/ColGroupDDC.java:647-692). The defaults are the tuned dispatch.
  *   tsmm_route      0 cost model, 1 one pass per pair of groups, 2 decoded Gram matrix
  *   tsmm_chunks     1 / 0: more than 64 columns decoded: all-DDC blocks of up to 128 at once, others as pairs of column chunks
- *   tsmm_direct     1 / 0: blocks of a few streamed columns next to run-length columns on the vector unit, both t(X) %*% X and
- *                   Y %*% X (0: both on the decoded tiles)
+ *   tsmm_direct     1 / 0: blocks of a few streamed columns next to run-length columns without code tiles, both t(X) %*% X (on the
+ *                   4x4x4 matrix instruction) and Y %*% X (on the vector unit) (0: both on the decoded tiles)
  *   tsmm_wide_dense 0 / 1, tsmm_mfma 1 / 0, tsmm_pair_dot 1 / 0
  *   tsmm_narrow     1 / 0: decoded Gram matrix with a last column block of at most 4 columns on the 4x4x4 matrix instruction
  *   expand_streams  1 / 0: one code per row for small RLE / SDCZeros groups (set before the first multiply)
@@ -296,7 +296,8 @@ int cla_preagg(cla_handle h, int32_t group, const double* Y, int32_t nRowY, doub
 /* enable != 0: bracket every kernel of this block with HIP events on its stream. */
 int cla_block_profile(cla_handle h, int enable);
 /* JSON with the kernels launched by the last driver call on this block: launch
- * geometry, algorithmic bytes and (when profiling) milliseconds. */
+ * geometry, algorithmic bytes and (when profiling) milliseconds. Copies and fills are not among them, whether the runtime makes
+ * them or a kernel does (a workspace cleared, a host vector fetched or delivered: 1 - 4 us each). */
 int cla_stats(cla_handle h, char* json, size_t cap);
 
 /* Diagnostic: throws inside the library (kind 0 std::bad_alloc, 1 std::length_error, 2 a non-standard

@@ -87,7 +87,7 @@ struct Options {
 	int tsmmNarrow = 1;     // decoded Gram matrix: a last column block of at most 4 columns on the 4 x 4 x 4 matrix instruction
 	int tsmmPairDot = 1;    // DDC x DDC pairs in dot form (0: pre-aggregate form with LDS bins)
 	int expandStreams = 1;  // one code per row for small RLE / SDCZeros groups in the decode kernels
-	int tsmmDirect = 1;     // decoded Gram matrix of blocks with few columns besides run-length columns on the vector unit, run-length columns by run (0: the tile kernel on the matrix cores)
+	int tsmmDirect = 1;     // t(X) %*% X and Y %*% X of blocks with few columns besides run-length columns without code tiles, run-length columns by run (0: the tile kernels)
 	int rmmDirect = 1;      // X %*% B for narrow B on blocks of plain streams: codes straight from global memory, sums on the vector unit (0: the tile kernel on the matrix cores)
 	int rmmDisable = 0;     // bit 0 byte-code mat-vec, 1 fused tables of the byte-code mat-vec, 2 matrix-core kernel, 3 decode kernel
 	int lmmDisable = 0;     // bit 0 dot form on byte codes, 1 byte-code bin kernel

@@ -43,12 +43,6 @@ __device__ __forceinline__ void wave_lds_sync() {
 	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The cursors' state in LDS (one per wave), for kernels that are short of registers between two run ends.
-struct RunPark {
-	double val[RC_MAX];
-	int32_t j[RC_MAX], jw[RC_MAX], end[RC_MAX];
-};
-
 struct RunCursors {
 	int32_t j;     // cursor lanes: run the column is in
 	int32_t jw;    // cursor lanes: run in slot 0 of the column's window
@@ -118,19 +112,6 @@ struct RunCursors {
 			refill(lane);
 			read_window(lane);
 		}
-	}
-
-	__device__ __forceinline__ void park(RunPark* p, int lane) const {
-		const int a = lane - RC_LANE0;
-		wave_lds_sync();
-		if(a >= 0 && a < RC_MAX) { p->val[a] = val; p->j[a] = j; p->jw[a] = jw; p->end[a] = end; }
-		wave_lds_sync();
-	}
-	__device__ __forceinline__ void unpark(const RunPark* p, const RunCol* c, int n, int32_t* we, double* wv, int lane) {
-		cols = c; nR = n; winEnd = we; winVal = wv;
-		const int a = lane - RC_LANE0;
-		j = 0; jw = 0; end = RC_NEVER; val = 0.0;
-		if(a >= 0 && a < RC_MAX) { val = p->val[a]; j = p->j[a]; jw = p->jw[a]; end = p->end[a]; }
 	}
 
 	// First row at which some column's run ends (RC_NEVER: none does any more).

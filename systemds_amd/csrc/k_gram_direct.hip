@@ -10,7 +10,7 @@
 // 8 k .. 8 k + 7 of a unit of 32 rows, straight from the column's stream (16 bytes of codes per lane, a unit ahead by two) and the values
 // by tuple in LDS. The looked-up values are both operands of v_mfma_f64_4x4x4, four products of 4 x 4 columns over 4 rows:
 //   V x V   x times itself and x times x rotated by four lanes: all pairs of three groups of four columns (quads) in two
-//           instructions per 4 rows, in two registers per lane (four quads take a third instruction; one or two quads fill the
+//           instructions per 4 rows, in two registers per lane (one or two quads fill the
 //           slots with 4 or 2 sets of rows). The sums of 78 products per row on the vector unit, lane = row, took 156 registers: one
 //           wave per SIMD, and every wait of it a wait of the SIMD;
 //   R x V   a run-length column is never looked up per row. The rows between two run ends (of any column) are a stretch on
@@ -69,7 +69,7 @@ template <int NQ, int ND, bool HASR, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void k_tsmm_direct(const GdrArgs A) {
 	extern __shared__ __align__(16) double smem[];
 	constexpr int THREADS = WAVES * 64, SETS = gdr_sets(NQ), UR = 32 * SETS;
-	constexpr int NM = NQ == 1 ? 1 : NQ == 4 ? 3 : 2; // matrix instructions per 4 rows
+	constexpr int NM = NQ == 1 ? 1 : 2; // matrix instructions per 4 rows
 	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int k = lane >> 4, c = lane & 15, b = c >> 2;
 	double* const gramS = smem + A.valDoubles;
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_tsmm_direct(const GdrArgs A) {
 	const int nR = HASR ? A.nR : 0;
 
 	// the lane's column: quad by slot, set of rows where quads are fewer than slots
-	auto quad_of = [](int bb) { return NQ == 1 ? 0 : NQ == 2 ? bb & 1 : NQ == 3 ? (bb == 3 ? 0 : bb) : bb; };
+	auto quad_of = [](int bb) { return NQ == 1 ? 0 : NQ == 2 ? bb & 1 : bb == 3 ? 0 : bb; };
 	const int rowIn = 8 * (k + 4 * (NQ == 1 ? b : NQ == 2 ? b >> 1 : 0));
 	const GdrCol C = A.cols[min(4 * quad_of(b) + (c & 3), A.nV - 1)];
 	const bool pad = C.col < 0 || 4 * quad_of(b) + (c & 3) >= A.nV;
@@ -184,11 +184,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_tsmm_direct(const GdrArgs A) {
 #pragma unroll
 			for(int t = 0; t < 8; t++) {
 				acc[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[t], x[t], acc[0], 0, 0, 0);
-				if(NQ > 1) {
-					const double y = gdr_next_quad(x[t]);
-					acc[NQ > 1 ? 1 : 0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[t], y, acc[NQ > 1 ? 1 : 0], 0, 0, 0);
-					if(NQ == 4) acc[NQ == 4 ? 2 : 0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[t], gdr_next_quad(y), acc[NQ == 4 ? 2 : 0], 0, 0, 0);
-				}
+				if(NQ > 1) acc[NQ > 1 ? 1 : 0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x[t], gdr_next_quad(x[t]), acc[NQ > 1 ? 1 : 0], 0, 0, 0);
 			}
 			if(HASR) {
 				const int32_t uEnd = TAIL ? nRows : (u + 1) * UR;
@@ -237,7 +233,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_tsmm_direct(const GdrArgs A) {
 #pragma unroll
 		for(int m = 0; m < NM; m++) {
 			const int qa = quad_of(b), qb = quad_of((b + m) & 3), i = 4 * qa + k, j = 4 * qb + (c & 3);
-			const bool mine = m == 0 ? (NQ == 3 ? b < 3 : true) && k <= (c & 3) : m == 2 ? b < 2 : NQ == 2 ? (b & 1) == 0 : NQ == 3 ? b < 3 : true;
+			const bool mine = m == 0 ? (NQ == 3 ? b < 3 : true) && k <= (c & 3) : NQ == 2 ? (b & 1) == 0 : b < 3;
 			if(mine && tot[m] != 0.0) unsafeAtomicAdd(&gramS[min(i, j) * GDR_NP + max(i, j)], tot[m]);
 		}
 		if(HASR) {
@@ -491,7 +487,7 @@ int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	// A wave takes the run ends of its rows one after the other, 0.4 us each: a unit per wave where there are many (100,003 rows of 9 columns, 8
 	// run-length of mean run 100: 19 us, two units 27; of 5000 12 and 12, 300,007 rows 12.9 and 12.1), else two.
 	const int share = P->waves * (P->runEnds * 400 > b->nRows ? 1 : 2);
-	const unsigned grid = (unsigned) std::max(1, std::min((nUnits + share - 1) / share, g_numCU * (P->lds <= 76 * 1024 && P->waves == 8 ? 2 : 1)));
+	const unsigned grid = (unsigned) std::max(1, std::min((nUnits + share - 1) / share, g_numCU));
 	// The tile kernel hardly notices run ends, but takes 35 ns more per 1000 rows. Both meet at 9 run ends per wave on 20,011 rows, 10 on
 	// 100,003, 22 on 300,007, 43 on 1,000,003 and 195 on 5,000,011 (one column behind codes, 8, 4 and 2 run-length ones; in us here / there:
 	// 20,011 rows, 8 of mean run 100 17.5 / 19.2, of 48 25 / 19; 300,007, 8 of 48 29 / 34, of 24 43 / 32; 5,000,011, 4 of 48 99 / 162, of 12 290 / 160).

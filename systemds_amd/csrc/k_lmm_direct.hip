@@ -246,9 +246,10 @@ int launch_lmm_direct(cla_block* b, const double* dY, int p, double* dOut, unsig
 	// 100,003 x 20 by 6 29 against 20; 5,000,011 x 20 by 16 332 against 247).
 	if(passes > 1 && b->nRows <= (int64_t) 500000 * (passes - 1)) return 1;
 	// A run end takes 0.24 - 0.32 ns of a pass (by 1 and 6 rows of Y, all waves together), the tile kernel hardly notices it. One to six rows
-	// and a pass is where they meet, whatever the number of run-length columns and of rows: 3,000,017 rows by 6 of Y, 8 run-length
-	// columns of mean run 24 381 against 279 us, 48 235 against 334; 4 of 16 284 against 233, of 24 216 against 256; 2 of 8 296 against
-	// 209, of 12 217 against 219; 300,007 rows, 4 of 16 76 against 69, of 24 66 against 75.
+	// and a pass is where they met when that kernel tested the code width on every row; it has become faster since and they meet at
+	// one to ten by 6 rows of Y, one to eight by 1 (in us here / there: 3,000,017 rows by 6, 8 run-length columns of mean run 48 228 / 145,
+	// 66 178 / 148, 100 130 / 150; 4 of 24 200 / 135, of 48 122 / 137; 2 of 12 211 / 133, of 24 122 / 131; by 1, 8 of 66 132 / 134; 300,007 rows
+	// by 6, 4 of 24 42 / 37, of 48 30 / 38). The line has been left.
 	if(P->runEnds * passes * 6 > b->nRows) return 1;
 	const size_t lds = ((size_t) P->A.valDoubles + LD_PMAX * (nc + nd + RC_MAX) + (size_t) LD_WAVES * LD_WDOUBLES) * 8;
 	if(lds > (size_t) std::min(g_ldsPerBlock, 160 * 1024)) return 1;

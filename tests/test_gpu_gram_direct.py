@@ -1,5 +1,5 @@
-"""GPU parity of t(X) %*% X on blocks of a few stream columns next to run-length columns: the Gram kernel on the
-vector unit that follows the run-length columns by run (k_tsmm_direct) against the CPU oracle and the exact
+"""GPU parity of t(X) %*% X on blocks of a few stream columns next to run-length columns: the Gram kernel without tiles
+that follows the run-length columns by run (k_tsmm_direct) against the CPU oracle and the exact
 product, through the C ABI. Every case also checks which kernel ran."""
 import numpy as np
 import pytest
@@ -78,16 +78,16 @@ def check(cla, ora, specs, n_rows, n_cols, what, expect_direct=True, options=Non
 
 @pytest.mark.parametrize("n_rows", [1, 63, 64, 65, 127, 128, 129, 1000, 20011, 150001])
 def test_row_counts_around_the_slices(cla, ora, n_rows):
-    """Slices of 64 rows, chunks of 128: full, ragged and single-row blocks (a run-length group of a block of a few rows
+    """Units of 32 to 128 rows: full, ragged and single-row blocks (a run-length group of a block of a few rows
     counts as one of short runs and is read from its one-code-per-row copy: twelve stream columns then)."""
     specs, n_cols = stream_block(10 + n_rows % 7, n_rows, n_u16=3)
     # (a single row: an offset list may be empty, and a column without row data is not this kernel's)
     check(cla, ora, specs, n_rows, n_cols, f"{n_rows} rows", expect_direct=True if n_rows > 1 else None)
 
 
-@pytest.mark.parametrize("shape", [dict(n_u16=8, n_u8=0, n_sdc=2, n_dense=2),   # the widths known at compile time
+@pytest.mark.parametrize("shape", [dict(n_u16=8, n_u8=0, n_sdc=2, n_dense=2),   # three quads, one piece of dense values per lane
                                    dict(n_u16=8, n_u8=0, n_sdc=2, n_dense=2, n_rle=0),
-                                   dict(n_u16=3, n_u8=2, n_sdc=0, n_dense=0),   # odd number of code columns: a filler
+                                   dict(n_u16=3, n_u8=2, n_sdc=0, n_dense=0),   # two quads, three columns short
                                    dict(n_u16=0, n_u8=5, n_sdc=1, n_dense=1),
                                    dict(n_u16=2, n_u8=2, n_sdc=2, n_dense=4),
                                    dict(n_u16=6, n_u8=4, n_sdc=2, n_dense=0),   # twelve code columns
@@ -118,7 +118,7 @@ def test_few_varying_columns_with_dense_ones(cla, ora, shape, direct, n_rows):
 
 
 def test_short_runs_and_bursts(cla, ora):
-    """Runs barely longer than a slice, with stretches of one-row runs: several run ends per slice, window refills."""
+    """Runs of a few units, with stretches of one-row runs: several run ends per unit, window refills."""
     n_rows = 60000
     specs, n_cols = stream_block(5, n_rows, n_rle=4, mean_run=80, bursts=True)
     check(cla, ora, specs, n_rows, n_cols, "short runs")
@@ -171,8 +171,8 @@ def test_blocks_outside_the_kernels_shape(cla, ora):
 
 
 def test_non_finite_run_length_values_take_the_tile_kernel(cla, ora):
-    """The run-following kernel handles run-length columns by summation by parts (sums of earlier rows times the step
-    of a run-length value), which is the rows' own products only for finite values: a block with an infinite or NaN
+    """The run-following kernel multiplies a run-length value by the sum of a column over the rows it holds on, which is the rows' own
+    products only for finite values: a block with an infinite or NaN
     dictionary value next to run-length columns takes the tile kernel, whose cells are the per-row products
     (infinite and NaN cells where the decompressed product has them)."""
     n_rows = 20011
@@ -199,9 +199,8 @@ def test_non_finite_run_length_values_take_the_tile_kernel(cla, ora):
 
 @pytest.mark.parametrize("kind", ["infinity", "dense", "dictionary", "zeros"])
 def test_values_of_many_magnitudes_next_to_run_length_columns(cla, ora, kind):
-    """Summation by parts takes every row of a varying column into its sums, also those on which a run-length column is zero: a
-    column with values far above the others (a marker of 1e14 on uncovered rows, an infinity) goes to the tile kernel, which
-    forms every row's cells; many zeros among ordinary values do not count as a wide span."""
+    """A column with values far above the others (a marker of 1e14 on rows where a run-length column is zero, an infinity) goes to the
+    tile kernel, which forms every row's cells; many zeros among ordinary values do not count as a wide span."""
     n_rows = 70003
     specs, n_cols = stream_block(41, n_rows, n_rle=3, n_u16=2, n_u8=1, n_sdc=1, n_dense=2)
     D = ora.np_decompress(specs, n_rows, n_cols)
