@@ -88,15 +88,18 @@ __device__ __forceinline__ void count_add(unsigned long long* counter, int local
 
 // Called by one thread of every block of a launch behind the block's last add: true for the last block to arrive. It clears the
 // counters for the next launch (clear_tickets) behind its own work: a store in front of it is waited for at the next barrier, 0.5 us. Adds to
-// one address are served one after the other, 11.4 ns each, a second line takes a round trip of 0.5 us: beyond TICKET_FEW blocks they count on
-// TICKET_WAYS lines first and the last of each line on the first one.
+// one address are served one after the other, 11.4 ns each, a second line takes a round trip of 0.5 us: beyond `few` blocks they count on
+// TICKET_WAYS lines first and the last of each line on the first one. TICKET_FEW is where both meet for blocks that end together (on one
+// line / on eight, in us: chain of 54 byte-code columns 32 blocks 9.0 / 9.4, 64 9.6 / 9.8, 128 11.0 / 10.5, 256 15.4 / 13.7, 512 of 10 columns 12.1 / 8.5;
+// t(X) %*% X of 100,000 x 20 12.4 / 10.7). Blocks that all add to the same cells come from a queue of that kind and never end
+// together: TICKET_QUEUED (Y %*% X of 131,072 x 54 by 1 row 15.0 / 15.4, by 8 20.6 / 20.9, 400,000 rows of 60 offset lists 27.5 / 27.8).
 __device__ __forceinline__ bool last_of_way(unsigned* done, unsigned nBlocks) {
 	const unsigned id = blockIdx.y * gridDim.x + blockIdx.x, way = id % TICKET_WAYS;
 	return atomicAdd(done + (1 + way) * (NNZ_STEP * 2), 1u) == (nBlocks - way + TICKET_WAYS - 1) / TICKET_WAYS - 1;
 }
 __device__ __forceinline__ bool last_of_ways(unsigned* done, unsigned nBlocks) { return atomicAdd(done, 1u) == min(nBlocks, (unsigned) TICKET_WAYS) - 1; }
-__device__ __forceinline__ bool last_block(unsigned* done, unsigned nBlocks) {
-	return nBlocks <= TICKET_FEW ? atomicAdd(done, 1u) == nBlocks - 1 : last_of_way(done, nBlocks) && last_of_ways(done, nBlocks);
+__device__ __forceinline__ bool last_block(unsigned* done, unsigned nBlocks, unsigned few = TICKET_FEW) {
+	return nBlocks <= few ? atomicAdd(done, 1u) == nBlocks - 1 : last_of_way(done, nBlocks) && last_of_ways(done, nBlocks);
 }
 // by a wave or more of the last block
 __device__ __forceinline__ void clear_tickets(unsigned* done) {
@@ -106,7 +109,7 @@ __device__ __forceinline__ void clear_tickets(unsigned* done) {
 // Tail of a left multiply whose kernel is the only one of the call: every block comes here behind its last add into
 // out; the last one to arrive counts the non-zeros of out[0 .. n) into *nnz
 // (the same is what a kernel of its own behind this one would do; done == nullptr: no tail).
-__device__ __forceinline__ void lmm_tail(unsigned* done, unsigned nBlocks, const double* out, int n, unsigned long long* nnz) {
+__device__ __forceinline__ void lmm_tail(unsigned* done, unsigned nBlocks, const double* out, int n, unsigned long long* nnz, unsigned few = TICKET_QUEUED) {
 	if(done == nullptr) return;
 	__shared__ int lastS;
 	__shared__ int partS[16];
@@ -115,7 +118,7 @@ __device__ __forceinline__ void lmm_tail(unsigned* done, unsigned nBlocks, const
 	// written back or invalidated, which a fence would do)
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 	__syncthreads();
-	if(threadIdx.x == 0) lastS = last_block(done, nBlocks);
+	if(threadIdx.x == 0) lastS = last_block(done, nBlocks, few);
 	__syncthreads();
 	if(!lastS) return;
 	int cnt = 0;

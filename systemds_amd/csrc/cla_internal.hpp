@@ -31,7 +31,7 @@ constexpr size_t NNZ_BYTES = (size_t) NNZ_SLOT * 8;
 // from L2 to L2, and 256 blocks' adds to the cells of a 20 x 20 result took 15 us.
 constexpr int GRAM_WAYS = 8; // (as many as TICKET_WAYS, dealt alike)
 constexpr int TICKET_WAYS = 8;                // a ticket is counted on this many lines and a line for these (last_block)
-constexpr unsigned TICKET_FEW = 512;          // ... of more blocks than these
+constexpr unsigned TICKET_FEW = 64, TICKET_QUEUED = 512; // ... of more blocks than these, the second where the blocks do not end together
 // most elements of a vector that a host-pointer call hands over through the counters' pinned buffer: a count, an operand and a result fit it
 constexpr int HOST_VEC_MAX = (NNZ_SLOT - 1) / 2;
 constexpr int NNZ_SLOTS = 4;                  // counters of a block (cla_block::nnzSlot)

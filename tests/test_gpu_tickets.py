@@ -46,3 +46,24 @@ def test_offset_lists_in_turn(cla, ora, n_rows):
         assert_matches_truth(out, Y, D, what=f"{p} rows of Y")
         assert nnz == np.count_nonzero(out)
     blk.close()
+
+
+@pytest.mark.parametrize("n_cols", [6, 16, 24, 50])  # (one slab of groups, two, three, seven)
+@pytest.mark.parametrize("n_rows", [5000, 150001])
+def test_column_pairs_in_turn(cla, ora, n_rows, n_cols):
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows + n_cols)
+    specs = [synth.GroupSpec("ddc", np.array([c, c + 1], np.int32), rng.standard_normal((1000, 2)), rng.integers(0, 1000, n_rows).astype(np.uint16))
+             for c in range(0, n_cols, 2)]
+    blk = cla.build_block(n_rows, n_cols, specs)
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    v = rng.standard_normal((n_cols, 1))
+    for k in range(4):
+        Y = rng.standard_normal((1, n_rows))
+        out, nnz = blk.lmm(Y)
+        assert_matches_truth(out, Y, D, what="a row of Y")
+        assert nnz == np.count_nonzero(out)
+        out, nnz = blk.mmchain(v)
+        assert_matches_truth(out.reshape(-1, 1), D.T, D @ v, what="chain")
+        assert nnz == np.count_nonzero(out)
+    blk.close()
