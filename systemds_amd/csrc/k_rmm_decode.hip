@@ -1082,7 +1082,6 @@ struct DirArgs {
 	const double* runSums;
 	int nR;
 	int nDicts, dictDoubles;
-	int stageGap;           // 16-byte pieces behind every pair of rows in a wave's staging area: 0 or 1
 	int segEnd[DSEG_N];
 	const double* B;        // first of the QV columns of this launch
 	const double* constRow;
@@ -1090,6 +1089,7 @@ struct DirArgs {
 	int ld;                 // columns of B and of the output (>= QV: wide B goes in chunks of 16 columns)
 	int64_t nRows;
 	unsigned long long* nnz;
+	int stageGap;           // 8 or 16 columns of B: 16-byte pieces behind every pair of rows in a wave's staging area, 0 or 1
 };
 typedef const __attribute__((address_space(4))) DirCol* dir_ccp;
 typedef unsigned long long dir_u64x4 __attribute__((ext_vector_type(4)));
@@ -1112,12 +1112,13 @@ __global__ __launch_bounds__(DIR_THREADS) void k_rmm_direct(const DirArgs A) {
 	if(tid < 2) smem[A.dictDoubles - 2 + tid] = 0.0; // what a filler column looks up
 	__syncthreads();
 	const uint8_t* const ldsBytes = (const uint8_t*) smem;
-	// Sixteen lanes write a pair of rows each and 64 read 16 bytes each. An even number of columns puts the pairs where several start in the
-	// same banks (8 columns: eight of 16, 16 columns: all), unless a gap of 16 bytes follows each (in us without / with gaps: 100,003 rows of 4
-	// columns by 8 17.5 / 12.8, of 20 by 16 38 / 29; 8,000,001 of 20 by 12 375 / 298, by 8 211 / 200).
-	const int gap = QV & 1 ? 0 : A.stageGap;
+	// Sixteen lanes write a pair of rows each and 64 read 16 bytes each. 8 columns put eight of the 16 pairs in the same banks, 16 columns all
+	// of them, unless a gap of 16 bytes follows each (in us without / with gaps: 100,003 rows of 4 columns by 8 17.5 / 12.8, 20,000,003 of 13 by 8
+	// 474 / 398; 100,003 of 20 by 16 38 / 29, 20,000,000 of 20 by 16 900 / 820). With 12 columns, four in the same banks, gaps win up to 8 M rows and
+	// lose beyond (3,000,003 of 13 84 / 79, 20,000,003 637 / 707: stores that leave faster reach HBM in a worse order): none.
+	const int gap = QV % 8 ? 0 : A.stageGap;
 	double* const wstage = smem + A.dictDoubles + (size_t) wave * (DIR_SROWS * QV + DIR_SROWS * gap);
-	auto staged = [&](int i) { return (const double*) wstage + i + (QV & 1 ? 0 : i / (2 * QV) * 2 * gap); }; // value i of the staged rows
+	auto staged = [&](int i) { return (const double*) wstage + i + (QV % 8 ? 0 : i / (2 * QV) * 2 * gap); }; // value i of the staged rows
 	const dec_cdp Bc = (dec_cdp) A.B;
 	const int64_t nRows = A.nRows;
 	const int64_t nSlices = (nRows + DIR_SLICE - 1) / DIR_SLICE;
@@ -1456,7 +1457,7 @@ static int launch_rmm_direct(cla_block* b, const double* dB, int q, const double
 	const int chunk = 16;
 	for(int c0 = 0; c0 < q; c0 += chunk) {
 		const int qv = std::min(chunk, q - c0);
-		const size_t lds = ((size_t) A.dictDoubles + (size_t) DIR_WAVES * DIR_SROWS * qv) * 8 + (A.stageGap ? ldsGaps : 0);
+		const size_t lds = ((size_t) A.dictDoubles + (size_t) DIR_WAVES * DIR_SROWS * qv) * 8 + (A.stageGap && qv % 8 == 0 ? ldsGaps : 0);
 		A.B = dB + c0; A.constRow = dConstRow ? dConstRow + c0 : nullptr; A.out = dOut + c0;
 		const double algo = (double) b->device_bytes_cached + (double) b->nRows * qv * 8;
 		if(A.nR > 0) {
