@@ -1324,6 +1324,8 @@ struct DirPlan {
 	void* dImg = nullptr;
 	int64_t bytes = 0;
 	bool denseFiller = false; // an odd number of dense columns
+	int codeCols = 0;      // columns behind codes
+	int64_t rowBytes = 0;  // of all streams together
 	DirArgs A;
 	std::vector<RunCol> runs; // run-length columns that are followed by run, and their merged run table
 	Mrt mrt;
@@ -1347,6 +1349,7 @@ static int dir_build_plan(cla_block* b, DirPlan& P) {
 		if(G.type == G_UNC) {
 			if(((uintptr_t) G.dense & 7) != 0) return 0;
 			for(int h = 0; h < G.nColG; h++) cols[DSEG_DENSE].push_back(DirCol{(const uint8_t*) (G.dense + h), 0, G.nColG * 8, hc[h], 0, 0, 0});
+			P.rowBytes += G.nColG * 8;
 			continue;
 		}
 		if(G.type != G_DDC && G.type != G_RLE && !(G.type == G_SDCZ && G.nOffsets > 0)) continue; // no row data
@@ -1367,6 +1370,8 @@ static int dir_build_plan(cla_block* b, DirPlan& P) {
 			src = b->expCodes[g];
 			cls = DSEG_GAP1;
 		}
+		P.codeCols += G.nColG;
+		P.rowBytes += cls == DSEG_DDC2 ? 2 : 1;
 		dicts.push_back(DirDict{G.dict, G.nVals * G.nColG, (int32_t) valD});
 		for(int h = 0; h < G.nColG; h++) cols[cls].push_back(DirCol{src, (int32_t) (8 * (valD + h)), G.nColG * 8, hc[h], 0, 0, 0});
 		valD += (size_t) G.nVals * G.nColG;
@@ -1499,12 +1504,18 @@ int launch_rmm_decode(cla_block* b, const double* dB, int q, const double* dCons
 	// of too few rows to fill half the chip (4 columns by 12 30,011 rows 16.3 / 13.7, 100,003 16.8 / 14.4, 300,007 17.2 / 19.6). Below a
 	// slice per CU the route of such blocks has been left as it was, to the tile kernel (5 columns of B on 5,000 rows are held to it), although this
 	// one would be faster: 1,003 rows of 4 columns by 2 8.4 / 13.5, by 12 12.6 / 14.2.
+	// Streams of more bytes than the 256 MB cache in front of HBM keeps from call to call: the stream kernel's reads, 128 bytes to 1 KB per wave and
+	// column, then go to HBM among its stores, and with 15 and 16 columns of B the tile kernel is the faster one up to 16 columns, unless it has
+	// more than 8 to look up, and not for an even number of dense columns alone (run-length, behind codes, dense columns: 2, 5, 1 by 15
+	// 14,000,003 rows, 238 MB, 408 / 432, 18,000,003 709 / 551; 1, 3, 11 by 15 2,150,537 rows, 200 MB, 132 / 157, 3,225,806 246 / 214; 2, 3, 2 by 16
+	// 8,000,003 211 / 255, 14,000,003 540 / 431; 6, 6, 1 by 15 24,000,003 980 / 841; 5, 10, 1 1003 / 1014; 8, 8, 1, 17 columns, 1018 / 1087; 0, 8, 2 767 / 796).
 	bool tilesFirst = q == DEC_QMAX;
 	if(b->opt.rmmDirect && dir_plan_get(b) == 0) {
 		const DirPlan& P = *b->dirPlan;
 		const int64_t slices = (int64_t) g_numCU * DIR_SLICE; // rows, a slice per CU
 		if(P.denseFiller) tilesFirst = q >= DEC_QMAX || b->nRows < (q > 10 && b->nCols < 9 ? slices * DIR_WAVES / 2 : slices);
 		else if(P.A.nR > 0) tilesFirst = false;
+		tilesFirst |= (q == DEC_QMAX - 1 || q == DEC_QMAX) && (P.denseFiller || P.A.nR > 0) && b->nCols <= 16 && P.codeCols <= 8 && P.rowBytes * b->nRows > 250000000;
 	}
 	if(b->opt.rmmDirect && !tilesFirst) {
 		const int rc = launch_rmm_direct(b, dB, q, dConstRow, dOut, dNnz);

@@ -107,3 +107,22 @@ def test_staging_with_and_without_gaps(cla, ora, n_rows, n_vals, q):
     D = ora.np_decompress(specs, n_rows, n_cols)
     assert_matches_truth(out, D, B, what=f"{n_vals} values, q={q}")
     assert nnz == np.count_nonzero(out)
+
+
+@pytest.mark.parametrize("unc, row_bytes, q, n_rows, direct", [(11, 92, 15, 2717391, True), (11, 92, 15, 2717392, False), (11, 92, 14, 2717392, True), (12, 100, 16, 2500000, True),
+                                                               (12, 100, 16, 2500001, False), (13, 108, 15, 2400000, True)])
+def test_streams_beyond_the_cache(cla, ora, unc, row_bytes, q, n_rows, direct):
+    """Streams of 250 MB together and a row more, 15 and 16 columns of B: the kernel on streams, the tile kernel (up to 16 columns)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(q)
+    specs, n_cols, blk = block(cla, synth, rng, n_rows, unc, 1, False)
+    assert n_cols == unc + 4 and row_bytes == 8 * unc + 4
+    B = rng.standard_normal((n_cols, q))
+    out, nnz = blk.rmm(B)
+    names = [k["name"] for k in blk.stats()["kernels"]]
+    blk.close()
+    assert ("k_rmm_direct" in names) == direct and ("k_rmm_decode" in names) != direct, names
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    # (two fp64 sums of at most 17 terms, each within 17 * 2^-53 of the sum of magnitudes)
+    assert np.all(np.abs(out - D @ B) <= 34 * 2.0 ** -53 * (np.abs(D) @ np.abs(B)))
+    assert nnz == np.count_nonzero(out)
