@@ -152,7 +152,7 @@ __device__ __forceinline__ size_t gram_way(int nCols) { return (size_t) (gram_wa
 // of an XCD to arrive may add that XCD's accumulator to the first; the last of all copies the sum
 // to out, mirrored, counts out's non-zeros into *nnz and leaves everything at zero for the next
 // launch: what a fill of out in front of the kernel and a kernel of its own behind it would do. `lds`: 17 words of the
-// block's LDS that nobody else uses any more (no static LDS here: the Gram kernels address theirs from offset zero).
+// block's LDS that nobody else uses any more (no static LDS here: k_gram_tiles fills LDS to the device's limit).
 __device__ __forceinline__ void gram_tail(unsigned* done, unsigned nBlocks, double* acc, double* out, int nCols, unsigned long long* nnz,
 	unsigned* lds) {
 	int& lastS = (int&) lds[0];

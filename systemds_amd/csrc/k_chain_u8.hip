@@ -16,11 +16,12 @@
 // output and counts its non-zeros: the call is this one launch, without a fill in front of it.
 //
 // Bound: vector issue (about 410 instructions of 4 cycles per 64 rows at 4 column blocks; the fold over the lanes costs the same
-// whatever the number of columns), on large blocks next to HBM (8,000,001 x 100: 3.6 TB/s); on small ones the start, the copy of the
-// dictionaries and the hand-over. Why not rows per thread as in k_rmm_q1_u8: the second product would add a value per thread, group
+// whatever the number of columns): 81 % of the CUs' busy cycles on 8,000,001 x 54, LDS 50 (half of it bank conflicts), the vector memory address
+// unit 40, next to HBM (8,000,001 x 100: 3.7 TB/s). On small blocks the start, the copy of the dictionaries and the hand-over: vector issue 34 % on
+// 250,007 x 54, nothing else above. Why not rows per thread as in k_rmm_q1_u8: the second product would add a value per thread, group
 // and pass through LDS, and sums over 100 columns do not fit a thread's registers. Measured (before: k_rmm_q1_u8, k_lmm_u8_dot or
-// k_lmm_u8_vec and a fill): 1,000 x 5 5.7 us (16.5), 250,007 x 54 16.0 (36), 1,000,003 x 80 31 (62), 8,000,001 x 48 122 (202), 8,000,001 x
-// 100 223 (334), 8,000,001 x 10 56 (82); nowhere slower, so every block that fits takes it.
+// k_lmm_u8_vec and a fill): 1,000 x 5 5.8 us (16.5), 250,007 x 54 13.8 (36), 1,000,003 x 80 29 (62), 8,000,001 x 48 108 (202), 8,000,001 x
+// 100 216 (334), 8,000,001 x 10 49 (82); nowhere slower, so every block that fits takes it.
 #include "../../include/cla_hip.h"
 #include "cla_device.hpp"
 #include <algorithm>

@@ -22,9 +22,9 @@
 // Dense columns go through a wave's LDS (16 bytes per lane and unit, as they lie), from where they are "looked up" by row.
 //
 // Bound: matrix and vector issue, which do not overlap on a SIMD (per 32 rows of 9 - 12 columns 16 matrix instructions of 17 - 19 cycles and 54
-// vector instructions, 140 more where a run ends; four waves per SIMD), next to HBM. Measured (lane = row on the vector unit before,
-// one wave per SIMD): 50,000,000 rows, 8 run-length, 8 two-byte, 2 offset-list, 2 dense columns 802 -> 488 us (3.5 TB/s), 5,000,000 113 -> 74,
-// 1,000,000 56 -> 38; 40,000,000 of 2 / 2 / 1 / 1 176 -> 111, 300,000 of 4 / 3 / 1 / 1 45 -> 22.
+// vector instructions, 140 more where a run ends; four waves per SIMD: vector 50 %, matrix 37 % of the CUs' busy cycles), next to HBM. Measured
+// (lane = row on the vector unit before, one wave per SIMD): 50,000,000 rows, 8 run-length, 8 two-byte, 2 offset-list, 2 dense columns 802 ->
+// 478 us (3.5 TB/s), 5,000,000 113 -> 58, 1,000,000 56 -> 23; 40,000,000 of 2 / 2 / 1 / 1 176 -> 103, 300,000 of 4 / 3 / 1 / 1 45 -> 13.
 #include "../../include/cla_hip.h"
 #include "cla_gdr.hpp"
 #include <algorithm>

@@ -19,7 +19,7 @@
 // codes behind those are on their way (pairs: a lane reads the codes of two rows at a time, one for each of two tiles). One barrier per tile that waits for LDS only: loads stay in flight over it.
 //
 // Bound: the fp64 matrix pipe (70 cycles per tile and 4 rows): busy 72 % of the time at 2,000,003 x 100 byte codes (vector issue 12 %,
-// LDS 19 %, vector memory path 38 %), 69 % at 10,000,000 x 50 column pairs, where the gathers keep the vector memory path busy 46 % (64 with a code load per tile).
+// LDS 19 %, vector memory path 38 %), 73 % at 10,000,000 x 50 column pairs, where the gathers keep the vector memory path busy 55 % (64 with a code load per tile).
 #include "../../include/cla_hip.h"
 #include "cla_device.hpp"
 #include "cla_runs.hpp"

@@ -224,10 +224,11 @@ __global__ __launch_bounds__(256) void k_lmm_finish(double* __restrict__ out, in
 
 // Behind a Y %*% X on decoded rows: takes the result out of its stage and counts the non-zeros. The kernels on decoded rows give
 // a row that a group does not cover the value 0.0, which an infinite Y turns into NaN; in the reference such a row does not enter the
-// group's sums. They report a non-finite Y in *bad, and then the blocks of this kernel form the product anew, from every group's
-// own rows only, row sums times constants apart, as the bin kernels do (ColGroupRLE.java:759-796, AOffset.java:288-430). The flag stays on the
+// group's sums. They report a non-finite Y in *bad, and then the blocks of this kernel form anew, from a group's own rows only, the
+// columns whose group leaves rows out or that a constant is added to, row sums times constants apart, as the bin kernels do
+// (ColGroupRLE.java:759-796, AOffset.java:288-430); the others have the same sums either way. The flag stays on the
 // device: the host looking at it cost 15 - 20 us per call (wait, copy, and the launches behind it), a mixed block of 5,000,011 x 20 by 6 rows
-// 114 us per call against 93 us.
+// 114 us per call against 91 us (with an infinity in Y 611, on the bin kernels 1502).
 constexpr int LT_THREADS = 512;
 constexpr int LT_P = 8;            // rows of Y per look at a group's codes
 constexpr int LT_COLS = 64;        // most columns of a block

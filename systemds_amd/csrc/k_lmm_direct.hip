@@ -17,8 +17,8 @@
 // waves per SIMD; what spills from two rows per lane there cost 60 of 154 us, so such shapes take one).
 // Bound: HBM (Y once, the streams once per pass; vector memory path 67 % busy, vector issue 40 %), 14 us of start and end. 5,000,011 x
 // 20 (8 run-length, 8 two-byte, 2 offset-list, 2 dense columns) by 6 rows of Y 88 us (414 MB: 4.7 TB/s). Calls, with the fill in
-// front and k_take_block behind (k_lmm_decode with a host's look at Y; this kernel with one): by 6 301, 114 -> 93 us, by 13 241 -> 220; 1,000,000
-// rows by 6 58 -> 34, 100,000 by 2 40 -> 16.
+// front and k_take_block behind (k_lmm_decode with a host's look at Y; this kernel with one): by 6 301, 114 -> 91 us, by 13 241 -> 215; 1,000,000
+// rows by 6 58 -> 32, 100,000 by 2 40 -> 15.
 #include "../../include/cla_hip.h"
 #include "cla_gdr.hpp"
 #include <algorithm>
