@@ -268,11 +268,12 @@ static int chain_shape(cla_block* b, bool op, ChainLaunch& L) {
 		!b->opt.chainFused)
 		return 0;
 	const int nCb = (nG + 15) / 16;
+	L.lds = std::max((size_t) nCb * b->maxVals * 128, (size_t) CH_WAVES * 4 * nCb * 16 * 8);
+	if(L.lds > (size_t) g_ldsPerBlock) return 0; // (before the kernel is asked: the first question of a process loads its code, 1.1 ms)
 	decltype(&k_chain_u8<1, false>) kern = nullptr;
 #define CH_CASE(N) case N: kern = op ? k_chain_u8<N, true> : k_chain_u8<N, false>; break;
 	switch(nCb) { CH_CASE(1) CH_CASE(2) CH_CASE(3) CH_CASE(4) CH_CASE(5) CH_CASE(6) CH_CASE(7) default: return 0; }
 #undef CH_CASE
-	L.lds = std::max((size_t) nCb * b->maxVals * 128, (size_t) CH_WAVES * 4 * nCb * 16 * 8);
 	size_t room = 0;
 	CLA_HIP(max_dynamic_lds((const void*) kern, room));
 	if(L.lds > room) return 0;

@@ -151,7 +151,7 @@ int launch_rmm_q1_u8_few(cla_block* b, const double* dB, const double* constTerm
 	const auto kern = threads == 1024 ? k_rmm_q1_u8_few<1024, 4> : rpt == 1 ? k_rmm_q1_u8_few<512, 1> : rpt == 2 ? k_rmm_q1_u8_few<512, 2> : k_rmm_q1_u8_few<512, 4>;
 	// (1,000,003 rows, in us here and on k_rmm_q1_u8: 5 columns 10.4 / 10.3, 20 12.1 / 13.0, 54 21 / 24, 100 28 / 35; 1,500,000, two turns of blocks, 54
 	// columns 37 / 27. Blocks of 512 threads, two per CU: 600,000 x 20 11.6 against 11.0, 600,000 x 30 13.6 against 12.3)
-	if(nRows > (int64_t) g_numCU * (nG <= 8 ? 3072 : 4096) || (size_t) nG * stride > (size_t) uf_tpt(threads) * threads) return 1;
+	if(nRows > (int64_t) g_numCU * (nG <= 8 ? 3072 : 4096) || (size_t) nG * stride > (size_t) uf_tpt(threads) * threads || lds > (size_t) g_ldsPerBlock) return 1;
 	size_t room = 0;
 	CLA_HIP(max_dynamic_lds((const void*) kern, room));
 	if(lds > room) return 1;
