@@ -1537,7 +1537,18 @@ int launch_rmm_decode(cla_block* b, const double* dB, int q, const double* dCons
 		int rpl = 4; // rows per lane and pass: the smaller output staging area when LDS is short
 		int rc = dec_prepare(b, false, qv, rpl, L);
 		if(rc == 1) rc = dec_prepare(b, false, qv, rpl = 2, L);
-		if(rc == 1 && c0 == 0 && tilesFirst && b->opt.rmmDirect) return launch_rmm_direct(b, dB, q, dConstRow, dOut, dNnz);
+		if(rc == 1 && c0 == 0 && tilesFirst && b->opt.rmmDirect) {
+			// More than 16 columns of B with an odd number of dense columns: decompressed rows times B (k_dense_rmm), which takes all columns of B
+			// at once and does not mind rows of an odd number of doubles (stream kernel / that one, in us, 18 - 21 columns: 150,000 rows by 24 45 / 46, by
+			// 32 52 / 47, by 64 102 / 56; 300,000 by 18 63 / 65, by 40 78 / 74; 700,000 by 64 205 / 205, by 21 214 / 126, by 63 598 / 248; 2,000,000 by 24
+			// 147 / 459, by 64 348 / 565, by 17 357 / 434, by 21 541 / 453, by 63 1536 / 658).
+			const int64_t from = q & 1 ? 900000 : (int64_t) 250000 * ((q - 1) / DEC_QMAX);
+			if(q > DEC_QMAX && (b->nRows < from || ((q & 1) && q > DEC_QMAX + 1))) {
+				const int r = launch_rmm_decompressed(b, dB, q, dOut, dNnz); // (1: few rows, on which it is not worth its start)
+				if(r <= 0) return r;
+			}
+			return launch_rmm_direct(b, dB, q, dConstRow, dOut, dNnz);
+		}
 		if(rc) return rc;
 		L.A.B = dB + c0; L.A.ld = q; L.A.constRow = dConstRow ? dConstRow + c0 : nullptr; L.A.out = dOut + c0; L.A.nnz = dNnz;
 		double algo = (double) b->device_bytes_cached + (double) b->nRows * qv * 8;

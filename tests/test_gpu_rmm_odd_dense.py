@@ -126,3 +126,33 @@ def test_streams_beyond_the_cache(cla, ora, unc, row_bytes, q, n_rows, direct):
     # (two fp64 sums of at most 17 terms, each within 17 * 2^-53 of the sum of magnitudes)
     assert np.all(np.abs(out - D @ B) <= 34 * 2.0 ** -53 * (np.abs(D) @ np.abs(B)))
     assert nnz == np.count_nonzero(out)
+
+
+@pytest.mark.parametrize("n_rows, q, direct", [(1003, 17, True), (899999, 17, False), (900000, 17, True), (900001, 19, False), (249999, 24, False), (250000, 24, True),
+                                               (250001, 18, True), (499999, 40, False), (500000, 40, True), (500003, 33, False), (20011, 16, True)])
+def test_wide_b_beside_dictionaries_that_fill_lds(cla, ora, n_rows, q, direct):
+    """Dictionaries that leave the tile kernel no room: more than 16 columns of B on decompressed rows below the lines (but for very
+    few rows), on streams above."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows + q)
+    specs, c = [], 0
+    for _ in range(3):
+        codes = np.repeat(rng.integers(0, 8, n_rows // 500 + 1), 500)[:n_rows]
+        ptr, data = synth.encode_rle(codes, 8)
+        specs.append(synth.GroupSpec("rle", np.array([c], np.int32), rng.standard_normal((8, 1)), ptr=ptr, rle=data))
+        c += 1
+    for _ in range(8):
+        specs.append(synth.GroupSpec("ddc", np.array([c], np.int32), rng.standard_normal((1024, 1)), rng.integers(0, 1024, n_rows).astype(np.uint16)))
+        c += 1
+    specs.append(synth.GroupSpec("unc", np.arange(c, c + 5, dtype=np.int32), dense=rng.standard_normal((n_rows, 5))))
+    c += 5
+    B = rng.standard_normal((c, q))
+    blk = cla.build_block(n_rows, c, specs)
+    out, nnz = blk.rmm(B)
+    names = [k["name"] for k in blk.stats()["kernels"]]
+    blk.close()
+    assert ("k_rmm_direct" in names) == direct and ("k_dense_rmm" in names) != direct, names
+    D = ora.np_decompress(specs, n_rows, c)
+    # (two fp64 sums of at most 17 terms, each within 17 * 2^-53 of the sum of magnitudes)
+    assert np.all(np.abs(out - D @ B) <= 34 * 2.0 ** -53 * (np.abs(D) @ np.abs(B)))
+    assert nnz == np.count_nonzero(out)
