@@ -95,6 +95,7 @@ struct Options {
 	int sdcPacked = 1;      // packed SDCZeros lists for the mat-vecs
 	int sdcLanes = 1;       // SDCZeros mat-vecs on lane-major lists, one lane per group
 	int sdcRows = 1;        // SDCZeros right mat-vec on row lists, one lane per row
+	int tsmmDigits = 1;     // t(X) %*% X of byte-code blocks on digits and the integer matrix cores (0: fp64; 2: short blocks, too)
 	int tsmmOneKernel = 1;  // decoded Gram matrix of a whole block as the call's only kernel (0: a fill in front, k_tsmm_finish behind)
 	int chainFused = 1;     // multiply chain of single-column byte-code blocks in one pass over the codes (0: two products)
 	int ddcReorder = 1;     // finalize renumbers the tuples of large DDC dictionaries by descending count (0: the caller's numbering is kept)
@@ -119,6 +120,7 @@ struct DecPlanCache;
 struct DirPlan;
 struct GdrPlan;
 struct GtPlan;
+struct GdPlan;
 
 } // namespace cla
 
@@ -215,6 +217,7 @@ struct cla_block {
 	cla::DirPlan* dirPlan = nullptr;     // plan of k_rmm_direct (dropped with the decode plans)
 	cla::GdrPlan* gdrPlan = nullptr;     // plan of k_tsmm_direct (likewise)
 	cla::GtPlan* gtPlan = nullptr;       // plan of k_gram_tiles (likewise)
+	cla::GdPlan* gdPlan = nullptr;       // plan of k_gram_tiles_i8 (likewise)
 	void* dMfPlan = nullptr;         // matrix-core right multiply (k_rmm_mfma.hip): slab descriptors, column info, code streams, B row list
 	int mfState = 0;                 // 0 not planned yet, 1 ready, -1 not eligible
 	int mfNSlabs = 0, mfNColsAll = 0, mfWidth = 1, mfMaxKc = 0, mfNRowCol = 0, mfMaxDict = 0;
@@ -307,6 +310,9 @@ int launch_tsmm_self(cla_block* b, double* out, double* colSum, const double* co
 int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr, bool ownByCounts = false);
 int gram_tiles_behind_decode(const cla_block* b);
 void gt_plan_drop(cla_block* b);
+int gram_digits_plan(cla_block* b);
+int launch_gram_digits(cla_block* b, double* acc, double* dOut, unsigned long long* dNnz, int skipOwn, int clearAcc);
+void gd_plan_drop(cla_block* b);
 int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);
 int ensure_gram_acc(cla_block* b); // the zeroed accumulators (1 + GRAM_WAYS of nCols x nCols) of the one-kernel t(X) %*% X (a workspace kept with the block)
 int ensure_expanded(cla_block* b);

@@ -542,6 +542,9 @@ int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz, bool
 		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
 	A.skipOwn = ownByCounts;
+	int rc = P.kind == GT_BYTE ? gram_digits_plan(b) : 1;
+	if(rc < 0) return rc;
+	const bool digits = rc == 0;
 	const unsigned grid = (unsigned) std::min((A.nTiles + gt_group(P.kind) - 1) / gt_group(P.kind), g_numCU * P.perCU);
 	// (where k_gram_tiles does not follow, an exception on the way included, nothing clears what the counts' kernel has added)
 	struct Clear {
@@ -549,11 +552,11 @@ int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz, bool
 		bool on;
 		~Clear() { if(on) (void) hipMemsetAsync(b->dGramAcc, 0, (size_t) (1 + GRAM_WAYS) * b->nCols * b->nCols * sizeof(double), b->stream); }
 	} clear{b, ownByCounts && dNnz != nullptr};
-	int rc = 0;
 	// (into an accumulator that gram_tail reads: see gram_ways)
-	double* const own = A.acc + (A.done != nullptr && grid > 4 * GRAM_WAYS ? (size_t) b->nCols * b->nCols : 0);
+	double* const own = A.acc + (A.done != nullptr && !digits && grid > 4 * GRAM_WAYS ? (size_t) b->nCols * b->nCols : 0);
 	if(ownByCounts && (rc = launch_tsmm_self(b, own, nullptr, b->hasConst ? b->dConstV : nullptr, P.constCols, P.nConst))) return rc;
-	if((rc = gt_launch_shape(b, P, A, grid)) == 0) clear.on = false;
+	rc = digits ? launch_gram_digits(b, A.acc, A.out, A.nnz, A.skipOwn, dNnz != nullptr) : gt_launch_shape(b, P, A, grid);
+	if(rc == 0) clear.on = false;
 	return rc;
 }
 
