@@ -127,6 +127,9 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *                   not single-column byte-code blocks, except with bit 0 of lmm_disable (a row of a
  *                   non-finite Y that a group does not cover stays out of its sums: decided on the device; chunk of
  *                   columns by chunk the host looks, i.e. waits for the stream once per call, and such a Y takes the bin kernels)
+ *   rmm_digits      X %*% B of all-DDC byte-code blocks of 64 to 100 columns as exact sums of products of 8-bit digits of the values on the
+ *                   integer matrix cores (rows whose outputs' terms are far below their columns' largest in fp64): 0 never (fp64), 1 where
+ *                   it is the faster way, 2 at any number of rows and columns of B
  *   tsmm_digits     t(X) %*% X of all-DDC byte-code blocks of 17 to 112 columns as exact sums of products of 8-bit digits of the values on the
  *                   integer matrix cores: 0 never (fp64), 1 where it is the faster way, 2 wherever its errors suit the block
  *   tsmm_one_kernel 1 / 0: t(X) %*% X of a whole block of at most 64 columns (all-DDC: 128) on the decoded Gram kernels as the call's only

@@ -752,6 +752,7 @@ int cla_block_set_option(cla_handle b, const char* key, int32_t value) {
 		{"ddc_reorder", &Options::ddcReorder, 0, 1},
 		{"chain_fused", &Options::chainFused, 0, 1},
 		{"tsmm_one_kernel", &Options::tsmmOneKernel, 0, 1}, {"tsmm_digits", &Options::tsmmDigits, 0, 2},
+		{"rmm_digits", &Options::rmmDigits, 0, 2},
 	};
 	for(const Entry& e : table)
 		if(strcmp(e.name, key) == 0) {

@@ -95,6 +95,7 @@ struct Options {
 	int sdcPacked = 1;      // packed SDCZeros lists for the mat-vecs
 	int sdcLanes = 1;       // SDCZeros mat-vecs on lane-major lists, one lane per group
 	int sdcRows = 1;        // SDCZeros right mat-vec on row lists, one lane per row
+	int rmmDigits = 1;      // X %*% B of byte-code blocks on digits and the integer matrix cores (0: fp64; 2: short blocks and narrow B, too)
 	int tsmmDigits = 1;     // t(X) %*% X of byte-code blocks on digits and the integer matrix cores (0: fp64; 2: short blocks, too)
 	int tsmmOneKernel = 1;  // decoded Gram matrix of a whole block as the call's only kernel (0: a fill in front, k_tsmm_finish behind)
 	int chainFused = 1;     // multiply chain of single-column byte-code blocks in one pass over the codes (0: two products)
@@ -121,6 +122,7 @@ struct DirPlan;
 struct GdrPlan;
 struct GtPlan;
 struct GdPlan;
+struct RdPlan;
 
 } // namespace cla
 
@@ -218,6 +220,7 @@ struct cla_block {
 	cla::GdrPlan* gdrPlan = nullptr;     // plan of k_tsmm_direct (likewise)
 	cla::GtPlan* gtPlan = nullptr;       // plan of k_gram_tiles (likewise)
 	cla::GdPlan* gdPlan = nullptr;       // plan of k_gram_tiles_i8 (likewise)
+	cla::RdPlan* rdPlan = nullptr;       // plan of k_rmm_mfma_i8 (likewise)
 	void* dMfPlan = nullptr;         // matrix-core right multiply (k_rmm_mfma.hip): slab descriptors, column info, code streams, B row list
 	int mfState = 0;                 // 0 not planned yet, 1 ready, -1 not eligible
 	int mfNSlabs = 0, mfNColsAll = 0, mfWidth = 1, mfMaxKc = 0, mfNRowCol = 0, mfMaxDict = 0;
@@ -313,6 +316,9 @@ void gt_plan_drop(cla_block* b);
 int gram_digits_plan(cla_block* b);
 int launch_gram_digits(cla_block* b, double* acc, double* dOut, unsigned long long* dNnz, int skipOwn, int clearAcc);
 void gd_plan_drop(cla_block* b);
+int rmm_digits_plan(cla_block* b, int q, int n0);
+int launch_rmm_digits(cla_block* b, const double* dB, int q, int n0, const double* dConstRow, double* dOut, unsigned long long* dNnz, const uint8_t** marks);
+void rd_plan_drop(cla_block* b);
 int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);
 int ensure_gram_acc(cla_block* b); // the zeroed accumulators (1 + GRAM_WAYS of nCols x nCols) of the one-kernel t(X) %*% X (a workspace kept with the block)
 int ensure_expanded(cla_block* b);

@@ -114,9 +114,21 @@ template <int WAVES, int W, int NQ = 4>
 __global__ __launch_bounds__(WAVES * 64) void k_rmm_mfma(const MfSlab* __restrict__ slabs, int nSlabs,
 	const uint32_t* __restrict__ infoG, const MfSrc* __restrict__ colSrc, int nColsAll, const double* __restrict__ Bl, int q, int n0,
 	const double* __restrict__ constRow, double* __restrict__ out, int64_t nRows, int ldsDictDoubles, int ldsKc, int bufBytes,
-	unsigned long long* __restrict__ nnz) {
+	const uint8_t* __restrict__ marks, unsigned long long* __restrict__ nnz) {
 	constexpr int THREADS = WAVES * 64;
 	constexpr int ROWS = WAVES * MF_MT * 16; // rows per tile
+	// marks (may be null): only 32 rows whose byte is not zero are wanted. Usually none is, which a block finds out before anything else.
+	static_assert(ROWS == 512, "16 marks per tile");
+	auto wanted = [&](int tile) {
+		const u32x4 w = *(const u32x4*) (marks + (size_t) tile * 16);
+		return (w.x | w.y | w.z | w.w) != 0;
+	};
+	if(marks != nullptr) {
+		int any = 0;
+		const int n = (int) ((nRows + ROWS - 1) / ROWS);
+		for(int t = blockIdx.x + (int) threadIdx.x * gridDim.x; t < n; t += THREADS * gridDim.x) any |= wanted(t);
+		if(!__syncthreads_or(any)) return;
+	}
 	extern __shared__ __align__(16) double smem[];
 	uint8_t* const lds = (uint8_t*) smem;
 	// offsets inside a slab buffer
@@ -183,8 +195,14 @@ __global__ __launch_bounds__(WAVES * 64) void k_rmm_mfma(const MfSlab* __restric
 
 	// persistent block: row tiles blockIdx.x, + gridDim.x, ...
 	int buf = 0;
-	if((int) blockIdx.x < nTiles) fill(blockIdx.x, 0, 0);
-	for(int tile = blockIdx.x; tile < nTiles; tile += gridDim.x) {
+	auto from = [&](int tile) {
+		while(marks != nullptr && tile < nTiles && !wanted(tile)) tile += gridDim.x;
+		return tile;
+	};
+	int tile = from(blockIdx.x);
+	if(tile < nTiles) fill(tile, 0, 0);
+	for(int next; tile < nTiles; tile = next) {
+		next = from(tile + gridDim.x);
 		const int64_t blockRow0 = (int64_t) tile * ROWS;
 		double acc[MF_MT][4 * NQ];
 #pragma unroll
@@ -199,7 +217,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_rmm_mfma(const MfSlab* __restric
 			__builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0)
 			__syncthreads();
 			if(s + 1 < nSlabs) fill(tile, s + 1, buf ^ 1);
-			else if(tile + (int) gridDim.x < nTiles) fill(tile + gridDim.x, 0, buf ^ 1);
+			else if(next < nTiles) fill(next, 0, buf ^ 1);
 
 			const uint8_t* const base = lds + (size_t) buf * bufBytes;
 			const double* dictS = (const double*) base;
@@ -305,6 +323,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_rmm_mfma(const MfSlab* __restric
 #pragma unroll
 			for(int m = 0; m < MF_MT; m++) {
 				const int64_t row = rowBase + 16 * m;
+				if(marks != nullptr && marks[(blockRow0 >> 5) + wave * 2 + m / 2] == 0) continue;
 #pragma unroll
 				for(int L = 0; L < NQ; L++) {
 					const int col = n0 + 16 * L + 8 * odd + 2 * lj;
@@ -461,6 +480,9 @@ int launch_rmm_mfma(cla_block* b, const double* dB, int q, const double* dConstR
 	for(auto& gr : b->groups) codeBytes += (double) b->nRows * gr.d.codeWidth;
 	for(int n0 = 0; n0 < q; n0 += 64) {
 		const int qq = std::min(64, q - n0);
+		const uint8_t* marks = nullptr; // digits: the rows that are left to fp64
+		if((rc = rmm_digits_plan(b, q, n0)) < 0) return rc;
+		if(rc == 0 && (rc = launch_rmm_digits(b, dB, q, n0, dConstRow, dOut, dNnz, &marks))) return rc;
 		{
 			Prof pf(b, "k_mfma_blayout", (long) b->mfNRowCol, 128, 0, 0);
 			hipLaunchKernelGGL(k_mfma_blayout, dim3((unsigned) b->mfNRowCol), dim3(128), 0, st, dB, q, n0, dRowCol, dBl);
@@ -471,7 +493,7 @@ int launch_rmm_mfma(cla_block* b, const double* dB, int q, const double* dConstR
 	do {                                                                                                                       \
 		CLA_HIP(allow_full_lds((const void*) k_rmm_mfma<MF_WAVES, CW, NQV>));                                                  \
 		hipLaunchKernelGGL((k_rmm_mfma<MF_WAVES, CW, NQV>), dim3(grid), dim3(MF_WAVES * 64), lds, st, dSlabs, b->mfNSlabs, dInfo, dSrc, \
-			b->mfNColsAll, dBl, q, n0, dConstRow, dOut, b->nRows, b->mfMaxDict, b->mfMaxKc, (int) b->mfBufBytes, dNnz);               \
+			b->mfNColsAll, dBl, q, n0, dConstRow, dOut, b->nRows, b->mfMaxDict, b->mfMaxKc, (int) b->mfBufBytes, marks, dNnz);        \
 	} while(0)
 #define MF_WIDTH(NQV)                                                   \
 	do {                                                                \

@@ -1,0 +1,117 @@
+"""X %*% B of byte-code blocks on the integer matrix cores (k_rmm_mfma_i8, option rmm_digits): the edges of its tiles, steps and passes, and the
+rows and right-hand sides that its digits do not suit, which the fp64 kernel computes."""
+import numpy as np
+import pytest
+
+from test_gpu_gram_tiles import columns
+
+pytestmark = pytest.mark.gpu
+
+
+def product(cla, specs, n_rows, n_cols, B, digits=2):
+    blk = cla.build_block(n_rows, n_cols, specs)
+    blk.set_option("rmm_digits", digits)
+    out, nnz = blk.rmm(B)
+    names = [k["name"] for k in blk.stats()["kernels"]]
+    again, _ = blk.rmm(B)  # (the marks are the call's)
+    blk.close()
+    assert np.array_equal(out, again, equal_nan=True)
+    return out, nnz, names
+
+
+def check(out, D, B, rows=slice(None)):
+    """Outputs against 80-bit products. Digits lose 6 products of weight 7 a column (each of standard deviation 2^-70 74^2 of the largest possible
+    term), which is 1.1e-16 sqrt(K / 100) of it together, and an output's terms come to 2^-2 sqrt(K / 100) of it at least: 4.5e-16 of their
+    sum. 8e-15 is 17 times that, and more than 100 rounded additions in fp64 come to."""
+    D = D[rows].astype(np.longdouble)
+    err = np.abs(out[rows] - D @ B.astype(np.longdouble))
+    assert np.all(err <= 8e-15 * (np.abs(D) @ np.abs(B).astype(np.longdouble)))
+
+
+@pytest.mark.parametrize("n_cols", [64, 65, 68, 69, 80, 95, 96, 97, 100])
+@pytest.mark.parametrize("n_rows,n_vals,q", [(1, 3, 64), (31, 256, 33), (257, 7, 9), (511, 256, 128), (33 * 512 + 5, 256, 32), (256 * 257 + 33, 60, 81), (256 * 300, 256, 61)])
+def test_edges(cla, ora, n_cols, n_rows, n_vals, q):
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_cols * q + n_rows)
+    specs = columns(synth, rng, n_rows, n_cols, n_vals, np.uint8, 1)
+    B = rng.standard_normal((n_cols, q))
+    out, nnz, names = product(cla, specs, n_rows, n_cols, B)
+    assert "k_rmm_mfma_i8" in names, names
+    check(out, ora.np_decompress(specs, n_rows, n_cols), B, np.r_[0:min(n_rows, 1200), max(0, n_rows - 1200):n_rows])
+    assert nnz == np.count_nonzero(out)
+
+
+def test_wide_groups_and_constants(cla, ora):
+    from systemds_amd import synth
+    rng = np.random.default_rng(5)
+    n_rows, n_cols, q = 9001, 90, 50
+    specs = columns(synth, rng, n_rows, n_cols - 4, 30, np.uint8, 8)
+    specs[1].dict[:, 0] = 0.0
+    specs.append(synth.GroupSpec("const", np.array([n_cols - 3, n_cols - 1], np.int32), np.array([[2.5, -1.0]])))
+    specs.append(synth.GroupSpec("const", np.array([0, 7], np.int32), np.array([[1.5, 0.25]])))
+    B = rng.standard_normal((n_cols, q))
+    B[:, 3] = 0.0
+    out, nnz, names = product(cla, specs, n_rows, n_cols, B)
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    check(out, D, B)
+    assert nnz == np.count_nonzero(out) and not out[:, 3].any()
+
+
+def test_whole_numbers_are_exact(cla):
+    """Products below 2^53 together have no digits at weights above 6, whatever their factors' sizes."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(3)
+    n_rows, n_cols, q = 70_001, 99, 40
+    codes = rng.integers(0, 200, (n_cols, n_rows)).astype(np.uint8)
+    bits = rng.integers(1, 36, n_cols)
+    dicts = np.stack([rng.integers(-2 ** int(b), 2 ** int(b) + 1, 200) for b in bits])
+    B = np.stack([rng.integers(-2 ** int(45 - b), 2 ** int(45 - b) + 1, q) for b in bits])
+    specs = [synth.GroupSpec("ddc", np.array([c], np.int32), dicts[c].astype(np.float64)[:, None], codes[c]) for c in range(n_cols)]
+    out, nnz, names = product(cla, specs, n_rows, n_cols, B.astype(np.float64))
+    D = np.stack([dicts[c][codes[c]] for c in range(n_cols)], 1)
+    assert np.array_equal(out, (D @ B).astype(np.float64)) and nnz == np.count_nonzero(out)
+
+
+@pytest.mark.parametrize("kind", ["some rows", "most rows", "one-hot", "far apart", "infinite B", "nan B", "tiny B", "huge B", "infinite", "far columns"])
+@pytest.mark.parametrize("q", [20, 64])
+def test_values_that_digits_do_not_suit(cla, ora, kind, q):
+    """Outputs whose terms are far below their columns' largest values keep fp64's accuracy, and what is not finite in B comes out as in fp64."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(4)
+    n_rows, n_cols = 140_011, 66
+    specs = columns(synth, rng, n_rows, n_cols, 40, np.uint8, 1)
+    B = rng.standard_normal((n_cols, q))
+    small = {"some rows": np.arange(n_rows) % 9973 == 17, "most rows": np.arange(n_rows) % 50 < 40}.get(kind)
+    for s in specs:
+        if small is not None:
+            s.dict[:20, 0] *= 1e-9
+            s.codes[:] = np.where(small, s.codes % 20, 20 + s.codes % 20)
+        elif kind == "one-hot":
+            s.dict[:, 0] = np.arange(40) == 3
+        elif kind == "far apart":
+            s.dict[0, 0] = 1e12
+    if kind == "infinite B":
+        B[7, 5] = np.inf
+    elif kind == "nan B":
+        B[7, 5] = np.nan
+    elif kind == "tiny B":
+        B *= 1e-290
+    elif kind == "huge B":
+        B *= 1e290
+        specs[0].dict *= 1e17
+    elif kind == "infinite":
+        specs[5].dict[3, 0] = np.inf
+    elif kind == "far columns":  # (only the last columns' terms count: the first step's magnitudes are not enough)
+        B[:40] *= 1e-12
+    out, nnz, names = product(cla, specs, n_rows, n_cols, B)
+    want, want_nnz, _ = product(cla, specs, n_rows, n_cols, B, 0)
+    assert ("k_rmm_mfma_i8" in names) == (kind != "infinite")
+    if kind in ("infinite B", "nan B", "infinite", "tiny B", "huge B"):
+        assert np.array_equal(np.isfinite(out), np.isfinite(want)) and np.array_equal(np.isnan(out), np.isnan(want))
+        if kind not in ("tiny B", "huge B"):
+            assert np.array_equal(out, want, equal_nan=True) and nnz == want_nnz
+            return
+    assert nnz == np.count_nonzero(out)
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    rows = np.r_[0:3000] if small is None else np.r_[0:1000, np.flatnonzero(small)[:1000]]
+    check(out, D, B, rows)
