@@ -366,8 +366,9 @@ struct GtPlan {
 // rms relative error 20 columns 1.2e-14 -> 7.4e-15 (k_tsmm_decode 7.1e-15), 38 1.3e-14 -> 7.6e-15 (7.6e-15), 100 2.3e-14 -> 1.2e-14
 // (1.0e-14); column pairs of 300 tuples, 20 columns 4.1e-15 -> 2.0e-15 (2.1e-15). A second block costs 8 - 23 us where it starts behind the first
 // (2,000,003 rows of 256 values: 20 columns 73 -> 81 us, 100 columns 438 -> 461; 10,000,000 x 20 of 7 values, side by side: 280 -> 239).
-static int gt_blocks_per_cu(int nf, int nn, int kind, int nTiles) {
-	if(nTiles < 16 * g_numCU) return 1; // (short chains: below 1e-15 with one block)
+static int gt_blocks_per_cu(int nf, int nn, int kind, int nTiles, int nCols) {
+	// (below 1e-15 with one block; pairs below 13 columns ran in shorter chains before: diagonal cells of 1,000,003 x 10 4.0e-16, 1.0e-15 with one block, 3.8e-16 with two)
+	if(nTiles < (nCols < 13 ? 2 : 16) * g_numCU) return 1;
 	if(nf > 5) return 2;
 	const int ncb = nf + (nn ? 1 : 0);
 	return kind == GT_PAIR ? (nf == 1 && nn < 2) || ncb == 3 ? 2 : 1 : ncb <= 3 ? 2 : 1;
@@ -376,7 +377,7 @@ static int gt_blocks_per_cu(int nf, int nn, int kind, int nTiles) {
 static int gt_build_plan(cla_block* b, GtPlan& P) {
 	P.rc = 1;
 	const int n = b->nCols;
-	if(b->dArena == nullptr || b->arenaWidth > 2 || n < 13 || n > 128 || b->nRows == 0 || b->crossSplit > 0 || b->crossBlocks > 0) return 0;
+	if(b->dArena == nullptr || b->arenaWidth > 2 || n < 4 || n > 128 || b->nRows == 0 || b->crossSplit > 0 || b->crossBlocks > 0) return 0;
 	std::vector<int> groupOf((size_t) n, -1);
 	for(size_t g = 0; g < b->groups.size(); g++)
 		for(int col : b->groups[g].cols) {
@@ -385,10 +386,11 @@ static int gt_build_plan(cla_block* b, GtPlan& P) {
 		}
 	// columns in the groups' order, then those that only carry a constant
 	const int last = n - n / 16 * 16;
-	P.nn = last >= 1 && last <= 4 ? 1 : last >= 5 && last <= 8 ? 2 : 0;
-	P.nf = n / 16 + (last > 8 ? 1 : 0);
+	P.nn = n < 16 ? 0 : last >= 1 && last <= 4 ? 1 : last >= 5 && last <= 8 ? 2 : 0;
+	P.nf = n < 16 ? 1 : n / 16 + (last > 8 ? 1 : 0);
 	bool pairs = b->arenaWidth == 2 && n == 2 * (int) b->groups.size();
 	for(const HostGroup& H : b->groups) pairs &= H.d.nColG == 2;
+	if(n < 13 && !pairs) return 0;
 	// Column pairs whose dictionaries LDS cannot hold: a unit's lanes all look up one group, 16 bytes at a time. The lanes
 	// share the lines of the frequent tuples, and each lookup gives two columns: 62.9 M tuples of 24 dictionaries of 4096
 	// (Zipf) take 99 us of gathers like this, 170 us as 8 bytes per column with 8 groups per instruction.
@@ -461,7 +463,7 @@ static int gt_build_plan(cla_block* b, GtPlan& P) {
 	P.nConst = (int) constCols.size();
 	A.nRows = b->nRows;
 	A.nTiles = (int) ((b->nRows + 32 * gt_m(ncb, P.kind) - 1) / (32 * gt_m(ncb, P.kind)));
-	P.perCU = gt_blocks_per_cu(P.nf, P.nn, P.kind, A.nTiles);
+	P.perCU = gt_blocks_per_cu(P.nf, P.nn, P.kind, A.nTiles, n);
 	A.nLds = nLds; A.imgV = imgV; A.nCols = n; A.nGroups = (int) b->groups.size();
 	P.rc = 0;
 	return 0;

@@ -683,7 +683,12 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz) {
 	// the code counts, one small kernel in front (rms relative error on 4,000,003 rows of like terms, 5 groups of 4 columns of 16 tuples
 	// 5.0e-15 decoded, 7.5e-17 by counts, 99 -> 100 us; 2 of 50 columns 2.1e-15, 1.0e-16, 851 -> 859; 300,007 rows, 3 of 8 25 -> 27).
 	const bool ownByCounts = !dense && !(nCols > 64 && chunkCheaper);
-	if(nPairs > 0 && !forcePairs && split == 0 && b->crossBlocks == 0 && nRows > 0 && b->opt.tsmmMfma && (nCols <= 64 || b->opt.tsmmChunks)) {
+	// Blocks of column pairs below 13 columns are of that kernel, too (its time hardly depends on their number), but those that went by pairs of groups
+	// only up to 2,500,000 rows: a pass per pair adds up by tuple, in shorter chains (cells across groups, rms relative error by pairs / decoded 1,000,003 x 8
+	// of 257 tuples 4.3e-16 / 4.0e-16, 2,000,003 3.9e-16 / 3.0e-16, 4,000,000 3.8e-16 / 7.2e-16). By pairs of groups / decoded in us, 257 tuples: 2 groups 1,000 rows 38 / 11,
+	// 2,000,000 54 / 32; 3 groups 20,000 53 / 11, 2,000,000 62 / 32; 4 groups 20,000 67 / 11, 2,000,000 83 / 32, 5000 tuples 1,000,000 83 / 27.
+	const bool fewPairs = ownByCounts && nRows > 2500000 && nCols < 13;
+	if(nPairs > 0 && !forcePairs && !fewPairs && split == 0 && b->crossBlocks == 0 && nRows > 0 && b->opt.tsmmMfma && (nCols <= 64 || b->opt.tsmmChunks)) {
 		if(!b->opt.tsmmOneKernel && (rc = clear())) return rc;
 		rc = nCols <= 64 && dense ? 1 : launch_gram_tiles(b, dOut, b->opt.tsmmOneKernel ? dNnz : nullptr, ownByCounts);
 		if(rc < 0) return rc;
