@@ -289,7 +289,7 @@ int launch_rmm_q1_u8_few(cla_block* b, const double* dB, const double* constTerm
 int launch_tables(cla_block* b, const double* dB, int q); // dict x B of every group (+ constV x B) into b->dTables
 int launch_aggregate(cla_block* b, int op, int dir, double* dOut, unsigned long long* dNnz);
 int ensure_counts(cla_block* b);
-int launch_rmm_mfma(cla_block* b, const double* dB, int q, const double* dConstRow, double* dOut,
+int launch_rmm_mfma(cla_block* b, const double* dB, int q, double* dConstRow, double* dOut,
 	unsigned long long* dNnz);
 int launch_lmm_u8(cla_block* b, const double* dY, int p, double* dPre);
 int launch_lmm_u8_dot(cla_block* b, const double* dY, int p, double* dOut);
@@ -317,7 +317,8 @@ int gram_digits_plan(cla_block* b);
 int launch_gram_digits(cla_block* b, double* acc, double* dOut, unsigned long long* dNnz, int skipOwn, int clearAcc);
 void gd_plan_drop(cla_block* b);
 int rmm_digits_plan(cla_block* b, int q, int n0);
-int launch_rmm_digits(cla_block* b, const double* dB, int q, int n0, const double* dConstRow, double* dOut, unsigned long long* dNnz, const uint8_t** marks);
+struct MfPrep;
+int launch_rmm_digits(cla_block* b, const MfPrep& prep, double* dOut, unsigned long long* dNnz, const uint8_t** marks);
 void rd_plan_drop(cla_block* b);
 int launch_tsmm_direct(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr);
 int ensure_gram_acc(cla_block* b); // the zeroed accumulators (1 + GRAM_WAYS of nCols x nCols) of the one-kernel t(X) %*% X (a workspace kept with the block)

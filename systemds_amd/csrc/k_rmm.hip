@@ -597,15 +597,18 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 		}
 		b->nnzSlot = 0;
 	}
-	// K1 (also clears the non-zero counter)
-	if(!fused || b->hasConst) {
+	// K1 (also clears the non-zero counter). Wide B: only where the matrix-core kernel, which makes what it needs itself, does not take the block. (The decoding
+	// kernels read the constants' row alone, but the tables take no longer than it and bring the dictionaries into the caches: 8,000,000 mixed rows 216 us behind the tables, 218.)
+	auto preagg = [&]() {
 		const int nK1 = fused ? 0 : nG; // fused: the constants' row only
 		const int maxWork = (u8Path && !fused ? 256 : (b->maxVals > 1 ? b->maxVals : 1)) * q;
 		dim3 grid(fused ? 1 : ((maxWork + 255) / 256 > (q + 255) / 256 ? (maxWork + 255) / 256 : (q + 255) / 256), nK1 + 1);
 		Prof pf(b, "k_preagg", (long) grid.x * grid.y, 256, 0, 0);
 		hipLaunchKernelGGL(k_preagg, grid, dim3(256), 0, st, b->dGroups, nK1, dB, q, b->nCols,
 			b->hasConst ? b->dConstV : nullptr, tables, b->totalVals, dNnz, fused ? nullptr : dTpad, squares);
-	}
+	};
+	const bool wide = q >= 8 && !noAlloc && nRows > 0 && !(b->opt.rmmDisable & 4);
+	if(!wide && (!fused || b->hasConst)) preagg();
 	const int constRow = b->hasConst ? b->totalVals : -1;
 	if(nRows == 0) return 0;
 
@@ -680,10 +683,11 @@ int launch_rmm(cla_block* b, const double* dB, int q, double* dOut, unsigned lon
 		return 0;
 	}
 
-	// wide B on an all-DDC block: fused decode + fp64 MFMA (K1 above still supplies constV x B)
-	if(q >= 8 && !noAlloc && !(b->opt.rmmDisable & 4)) {
+	// wide B on an all-DDC block: fused decode + fp64 MFMA (its first launch makes constV x B)
+	if(wide) {
 		const int r = launch_rmm_mfma(b, dB, q, constRow >= 0 ? tables + (size_t) constRow * q : nullptr, dOut, dNnz);
 		if(r <= 0) return r;
+		preagg();
 	}
 
 	// narrow B on any group mix: decode rows from LDS dictionaries, B rows as scalars. A single column as well

@@ -25,7 +25,7 @@
 // next tables ordered between the products (3.0), products of a step between the look-ups of the next (2.28: LDS and matrix cores still take turns), two columns a
 // lane for 16-byte stores (2.29).
 #include "../../include/cla_hip.h"
-#include "cla_device.hpp"
+#include "k_rmm_prep.hpp"
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -353,10 +353,18 @@ __global__ __launch_bounds__(RD_THREADS, 2) void k_rmm_mfma_i8(RdArgs A) {
 
 // ---- B's operands
 
-constexpr int RB_THREADS = 256, RB_PIECES = 32; // (3 steps of 8, and 8)
+static_assert(MF_BL_THREADS == 256, "blocks of k_rmm_digits_b");
+constexpr int RB_THREADS = MF_BL_THREADS, RB_PIECES = 32; // (3 steps of 8, and 8)
 // Block c: 32 columns of B of the pass into their operands, scales and least sums.
-__global__ __launch_bounds__(RB_THREADS) void k_rmm_digits_b(const double* __restrict__ B, int q, int n0, int K, int S, int T, const int32_t* __restrict__ rowCol,
+// The blocks behind those make what the fp64 kernel reads (mf_prep).
+__global__ __launch_bounds__(RB_THREADS) void k_rmm_digits_b(const MfPrep P, int blocks, int K, int S, int T, const int32_t* __restrict__ rowCol,
 	const double* __restrict__ up, uint8_t* __restrict__ bImg, double* __restrict__ scale, int32_t* __restrict__ least, int32_t* __restrict__ bad, int leastSum) {
+	if((int) blockIdx.x >= blocks) {
+		mf_prep(P, (int) blockIdx.x - blocks);
+		return;
+	}
+	const double* __restrict__ const B = P.B;
+	const int q = P.q, n0 = P.n0;
 	__shared__ __attribute__((aligned(16))) uint8_t img[RB_PIECES * 1024];
 	__shared__ double most[RB_THREADS / 32][32];
 	__shared__ int badS;
@@ -550,18 +558,20 @@ static int rd_launch(cla_block* b, const RdArgs& A) {
 }
 
 // Up to 64 columns of B from n0 on; the rows that are left (*marks: per 32 rows) are the caller's.
-int launch_rmm_digits(cla_block* b, const double* dB, int q, int n0, const double* dConstRow, double* dOut, unsigned long long* dNnz, const uint8_t** marks) {
+int launch_rmm_digits(cla_block* b, const MfPrep& prep, double* dOut, unsigned long long* dNnz, const uint8_t** marks) {
+	const int q = prep.q, n0 = prep.n0;
 	const RdPlan& P = *b->rdPlan;
 	const int cols = std::min(64, q - n0), c32 = (cols + 31) / 32;
 	// 2^-2 sqrt(K / 100) of the largest possible term, in squares of 1 / 128
 	const int leastSum = (int) (16384.0 / 4 * std::sqrt(P.K / 100.0));
 	{
-		Prof pf(b, "k_rmm_digits_b", c32, RB_THREADS, 0, 0);
-		hipLaunchKernelGGL(k_rmm_digits_b, dim3((unsigned) c32), dim3(RB_THREADS), 0, b->stream, dB, q, n0, P.K, P.S, P.T, P.rowCol, P.up, P.bImg, P.scale, P.least,
+		const int blocks = c32 + prep.blocks();
+		Prof pf(b, "k_rmm_digits_b", blocks, RB_THREADS, 0, 0);
+		hipLaunchKernelGGL(k_rmm_digits_b, dim3((unsigned) blocks), dim3(RB_THREADS), 0, b->stream, prep, c32, P.K, P.S, P.T, P.rowCol, P.up, P.bImg, P.scale, P.least,
 			P.bad, leastSum);
 	}
 	RdArgs A = P.A;
-	A.constRow = dConstRow; A.out = dOut; A.nnz = dNnz; A.q = q; A.n0 = n0;
+	A.constRow = prep.constRow; A.out = dOut; A.nnz = dNnz; A.q = q; A.n0 = n0;
 	*marks = A.marks;
 #define RD_CASE(SV, TV) case SV * 2 + TV: return c32 == 1 ? rd_launch<SV, TV, 1>(b, A) : rd_launch<SV, TV, 2>(b, A);
 	switch(P.S * 2 + P.T) { RD_CASE(2, 0) RD_CASE(2, 1) RD_CASE(3, 0) RD_CASE(3, 1) }

@@ -18,7 +18,7 @@
 // lane's 16 accumulators, so that the four lanes of a row hold eight consecutive output columns in each pair of
 // accumulators: 64 contiguous bytes per row and store instruction.
 #include "../../include/cla_hip.h"
-#include "cla_device.hpp"
+#include "k_rmm_prep.hpp"
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -27,11 +27,6 @@ namespace cla {
 
 constexpr int MF_WAVES = 8;                  // waves per block (two per SIMD): 512-row tiles
 constexpr int MF_MT = 4;                     // 16-row tiles per wave
-// B slab in LDS: row k at k * MF_BK, inside it the 16 values of lane column j (accumulators jg = 0..15)
-// at j * MF_BJ: the 16 distinct 16-byte pieces of a wave's read fall on 16 distinct
-// bank quads (row stride 16 banks, j stride 36 banks)
-constexpr int MF_BJ = 18;
-constexpr int MF_BK = 4 * MF_BJ;
 // code stream of a decoded column (device array: at row 0; LDS copy: at the block's first row)
 struct MfSrc {
 	const uint8_t* codes;
@@ -48,15 +43,7 @@ struct MfSlab {
 	const double* dictSrc; // the slab's dictionaries, back to back
 };
 
-// B in the slab layout: row r of the list (decoded column rowCol[r], -1 = padding) at r * MF_BK,
-// output column n0 + 8 (jg / 2) + 2 j + jg % 2 at j * MF_BJ + jg
-__global__ __launch_bounds__(128) void k_mfma_blayout(const double* __restrict__ B, int q, int n0, const int32_t* __restrict__ rowCol,
-	double* __restrict__ Bl) {
-	const int r = blockIdx.x, t = threadIdx.x;
-	if(t >= MF_BK) return;
-	const int j = t / MF_BJ, jg = t - j * MF_BJ, col = n0 + 8 * (jg >> 1) + 2 * j + (jg & 1), gc = rowCol[r];
-	Bl[(size_t) r * MF_BK + t] = (jg < 16 && gc >= 0 && col < q) ? B[(size_t) gc * q + col] : 0.0;
-}
+__global__ __launch_bounds__(MF_BL_THREADS) void k_mfma_blayout(const MfPrep P) { mf_prep(P, (int) blockIdx.x); }
 
 // LDS layout: two slab buffers, then the code streams of all decoded columns (srcS) and the slab
 // descriptors (slabS), read once per block. A slab buffer holds
@@ -459,7 +446,7 @@ static int mf_plan(cla_block* b) {
 
 // Plan (once per block) + launch. Returns 1 when the block/shape is not eligible (caller
 // uses the gather path), 0 on success, negative on error.
-int launch_rmm_mfma(cla_block* b, const double* dB, int q, const double* dConstRow, double* dOut,
+int launch_rmm_mfma(cla_block* b, const double* dB, int q, double* dConstRow, double* dOut,
 	unsigned long long* dNnz) {
 	int rc = mf_plan(b);
 	if(rc) return rc;
@@ -480,12 +467,15 @@ int launch_rmm_mfma(cla_block* b, const double* dB, int q, const double* dConstR
 	for(auto& gr : b->groups) codeBytes += (double) b->nRows * gr.d.codeWidth;
 	for(int n0 = 0; n0 < q; n0 += 64) {
 		const int qq = std::min(64, q - n0);
+		const MfPrep prep{dB, dRowCol, dBl, dConstRow != nullptr ? b->dConstV : nullptr, dConstRow, n0 == 0 ? dNnz : nullptr, q, n0, b->mfNRowCol, b->nCols};
 		const uint8_t* marks = nullptr; // digits: the rows that are left to fp64
 		if((rc = rmm_digits_plan(b, q, n0)) < 0) return rc;
-		if(rc == 0 && (rc = launch_rmm_digits(b, dB, q, n0, dConstRow, dOut, dNnz, &marks))) return rc;
-		{
-			Prof pf(b, "k_mfma_blayout", (long) b->mfNRowCol, 128, 0, 0);
-			hipLaunchKernelGGL(k_mfma_blayout, dim3((unsigned) b->mfNRowCol), dim3(128), 0, st, dB, q, n0, dRowCol, dBl);
+		if(rc == 0) {
+			if((rc = launch_rmm_digits(b, prep, dOut, dNnz, &marks))) return rc;
+		}
+		else {
+			Prof pf(b, "k_mfma_blayout", prep.blocks(), MF_BL_THREADS, 0, 0);
+			hipLaunchKernelGGL(k_mfma_blayout, dim3((unsigned) prep.blocks()), dim3(MF_BL_THREADS), 0, st, prep);
 		}
 		Prof pf(b, "k_rmm_mfma", grid, MF_WAVES * 64, (long) lds, codeBytes + (double) b->nRows * qq * 8);
 		const int nq = (qq + 15) / 16; // quarters of the pass's 64 columns that B has

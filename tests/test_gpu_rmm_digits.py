@@ -41,17 +41,21 @@ def test_edges(cla, ora, n_cols, n_rows, n_vals, q):
     assert nnz == np.count_nonzero(out)
 
 
-def test_wide_groups_and_constants(cla, ora):
+@pytest.mark.parametrize("q", [9, 50, 130])
+@pytest.mark.parametrize("digits", [0, 2])
+def test_wide_groups_and_constants(cla, ora, q, digits):
+    """Constants come with the layout of B, 64 columns of B at a time, not from a kernel of their own; the counter is cleared once."""
     from systemds_amd import synth
     rng = np.random.default_rng(5)
-    n_rows, n_cols, q = 9001, 90, 50
+    n_rows, n_cols = 9001, 90
     specs = columns(synth, rng, n_rows, n_cols - 4, 30, np.uint8, 8)
     specs[1].dict[:, 0] = 0.0
     specs.append(synth.GroupSpec("const", np.array([n_cols - 3, n_cols - 1], np.int32), np.array([[2.5, -1.0]])))
     specs.append(synth.GroupSpec("const", np.array([0, 7], np.int32), np.array([[1.5, 0.25]])))
     B = rng.standard_normal((n_cols, q))
     B[:, 3] = 0.0
-    out, nnz, names = product(cla, specs, n_rows, n_cols, B)
+    out, nnz, names = product(cla, specs, n_rows, n_cols, B, digits)
+    assert ("k_rmm_mfma_i8" in names) == (digits == 2) and "k_preagg" not in names
     D = ora.np_decompress(specs, n_rows, n_cols)
     check(out, D, B)
     assert nnz == np.count_nonzero(out) and not out[:, 3].any()
