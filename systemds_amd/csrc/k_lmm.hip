@@ -665,7 +665,8 @@ int64_t deliver(cla_block* b, double* out, const double* src, int n, const unsig
 int launch_mmchain(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz) {
 	const int64_t nRows = b->nRows;
 	{
-		const int r = launch_chain_u8(b, dV, dW, ctype, dOut, dNnz);
+		int r = launch_chain_u8(b, dV, dW, ctype, dOut, dNnz);
+		if(r == 1) r = launch_chain_sdc(b, dV, dW, ctype, dOut, dNnz);
 		if(r <= 0) return r;
 	}
 	// the intermediate vector has a workspace of its own: the multiplies below may resize the shared scratch

@@ -2,6 +2,7 @@
 //
 //   k_rows_build      one-time transposition of the listed groups' offset and code lists into row lists
 //   k_rmm_sdc_rows    out[row] = init + sum over the row's entries of T[entry]               (X %*% u)
+//   k_chain_sdc       out[col] = sum over the col's entries of (w *) (X %*% u)[row] * value (the multiply chain)
 //
 // An SDCZeros group lists the rows that differ from the default; X %*% u needs, for every row, the sum of the
 // table values of the groups that list it. Scattering the lists into an output tile in LDS costs one LDS add of
@@ -36,6 +37,8 @@ constexpr int RW_WAVES = 8;        // waves per block (C4: 0.110 / 0.095 / 0.086
 constexpr int RW_THREADS = RW_WAVES * 64;
 constexpr int RW_PF = 24;          // groups of a quarter that a lane requests a quarter ahead
 constexpr int RW_TBL_MAX = 16000;  // table entries of all listed groups in LDS (125 KB, next to 2 KB per wave)
+constexpr int CS_WAVES = 12, CS_THREADS = CS_WAVES * 64; // the multiply chain's kernel
+constexpr int CS_TBL_MAX = 8448;   // its table entries (two tables of them: 132 KB)
 constexpr uint32_t RW_LAST = 0x8000u; // a row's last group
 static_assert(RW_WIN == 1024 && RW_Q == 256 && RW_F == 4 && RW_TBL_MAX < (int) RW_LAST,
 	"a conversion block sorts the four quarters of a window; a row's place in its quarter is a byte; bit 15 of a position is free");
@@ -276,6 +279,215 @@ __global__ __launch_bounds__(RW_THREADS) void k_rmm_sdc_rows(const int32_t* __re
 	count_add(nnz, cntNz);
 }
 
+// The multiply chain t(X) %*% (w * (X %*% v)) on blocks of single-column lists only, in one pass over the row lists: a row's sum, with its weight, is
+// added to its entries' places in a second table in LDS; at the end that table times the dictionary values is the block's share of every column. The
+// blocks hand their shares over in a workspace and the last one adds them up in block order (as in k_chain_u8): the call is this one launch.
+// Bound: below a few million entries the start (dictionaries, headers, lists: three round trips to memory) and the hand-over, then the LDS accesses, a look-up and
+// an add per entry, beside HBM (10,000,000 x 60 of 5 %: 3.3 TB/s). Two launches before (k_rmm_sdc_rows, k_lmm_sdc_lanes), which read two forms of the lists and carry
+// X %*% v through memory: 100,000 x 20 22.6 -> 13.2 us, 200,000 x 60 26.2 -> 16.3, 1,320,173 x 35 33.7 -> 20.8, 2,606,481 x 82 of 8 % 51 -> 39, 9,128,715 x
+// 32 88 -> 51, 10,000,000 x 60 107 -> 70, x 130 of 10 % 196 -> 161; nowhere slower, so every block whose two tables fit takes it. (8 waves a block: 9,128,715 x 32 55.) Larger
+// dictionaries with one table after the other in LDS and the rows' values through memory: 10,000,000 x 200 160 -> 169, taken back.
+template <bool OP>
+__global__ __launch_bounds__(CS_THREADS) void k_chain_sdc(const int32_t* __restrict__ tblIndex, int nTbl, const int32_t* __restrict__ gBase, int nL,
+	const uint2* __restrict__ hdr, const uint32_t* __restrict__ perm, const uint32_t* __restrict__ data, const double* __restrict__ D,
+	const int32_t* __restrict__ tblCol, const double* __restrict__ v, const double* __restrict__ w, int minus, int64_t nRows, int nQuarters,
+	double* __restrict__ part, double* __restrict__ out, int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz) {
+	extern __shared__ double smemD[];
+	__shared__ int lastS;
+	__shared__ int cntS[CS_WAVES];
+	const int nPad = (nTbl + 2) / 2 * 2;
+	double* tbl = smemD;            // dictionary value x v of the column, and a 0.0
+	double* hist = smemD + nPad;    // sums of the rows' values by entry
+	const int tid = threadIdx.x, lane = tid & 63;
+	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	double* back = smemD + 2 * nPad + wave * RW_Q; // this wave's sums in row order
+	struct Ahead {
+		uint32_t v[RW_PF];
+		uint2 h;
+		uint32_t p;
+		double w[OP ? RW_F : 1];
+	};
+	int vzero = 0;
+	asm volatile("" : "+v"(vzero));
+	auto header = [&](int qt) { return hdr[min(qt, nQuarters - 1) + vzero]; };
+	auto request = [&](Ahead& A, int qt, const uint2 h) { // qt < nQuarters
+		A.h = make_uint2((uint32_t) __builtin_amdgcn_readfirstlane((int) h.x), (uint32_t) __builtin_amdgcn_readfirstlane((int) h.y));
+		const uint32_t* src = data + (size_t) A.h.x * 64 + lane;
+		const int kq = (int) A.h.y;
+#pragma unroll
+		for(int q = 0; q < RW_PF; q++) A.v[q] = __builtin_nontemporal_load(src + (size_t) min(q, kq - 1) * 64);
+		A.p = perm[(size_t) qt * 64 + lane];
+		if(OP) {
+#pragma unroll
+			for(int j = 0; j < RW_F; j++) A.w[j] = __builtin_nontemporal_load(w + min((int64_t) qt * RW_Q + j * 64 + lane, nRows - 1));
+		}
+	};
+	const int step = gridDim.x * CS_WAVES, q0 = blockIdx.x * CS_WAVES + wave;
+	const uint2 h0 = header(q0), h1 = header(q0 + step); // (on their way beside the tables)
+	constexpr int TPT = (CS_TBL_MAX + CS_THREADS - 1) / CS_THREADS;
+	auto dict = [&](double (&d)[TPT]) {
+		int32_t ti[TPT];
+#pragma unroll
+		for(int j = 0; j < TPT; j++) ti[j] = tblIndex[min(j * CS_THREADS + tid, nTbl - 1)];
+#pragma unroll
+		for(int j = 0; j < TPT; j++) d[j] = D[ti[j]];
+	};
+	{
+		double d[TPT], x[TPT];
+		int32_t tc[TPT];
+#pragma unroll
+		for(int j = 0; j < TPT; j++) tc[j] = tblCol[min(j * CS_THREADS + tid, nTbl - 1)];
+		dict(d);
+#pragma unroll
+		for(int j = 0; j < TPT; j++) x[j] = v[tc[j]];
+#pragma unroll
+		for(int j = 0; j < TPT; j++)
+			if(j * CS_THREADS + tid < nTbl) {
+				tbl[j * CS_THREADS + tid] = __dmul_rn(d[j], x[j]);
+				hist[j * CS_THREADS + tid] = 0.0;
+			}
+	}
+	if(tid == 0) tbl[nTbl] = 0.0;
+	__syncthreads();
+	const uint32_t zero = (uint32_t) nTbl, none = zero * 0x00010001u; // the place of the 0.0; a group of two of it
+	auto work = [&](Ahead& A, Ahead& B, int qt, uint2& hNext) { // A holds the requests of `qt`, hNext the header of qt + step
+		request(B, min(qt + step, nQuarters - 1), hNext);
+		hNext = header(qt + 2 * step);
+		const int kq = (int) A.h.y;
+		const uint32_t* src = data + (size_t) A.h.x * 64 + lane;
+		uint32_t pw = A.p;
+		double acc = 0.0;
+		auto close = [&](uint32_t e) { // a group with bit 15 set ends the row at hand
+			if(e & RW_LAST) {
+				back[pw & 0xffu] = acc;
+				acc = 0.0;
+				pw >>= 8;
+			}
+		};
+#pragma unroll
+		for(int qq = 0; qq < RW_PF; qq += 4) {
+			if(qq < kq) {
+				uint32_t e[4];
+				double a[4], b2[4];
+#pragma unroll
+				for(int j = 0; j < 4; j++) {
+					e[j] = qq + j < kq ? A.v[qq + j] : none;
+					a[j] = tbl[e[j] & (RW_LAST - 1)];
+					b2[j] = tbl[e[j] >> 16];
+				}
+#pragma unroll
+				for(int j = 0; j < 4; j++) {
+					acc = (acc + a[j]) + b2[j];
+					close(e[j]);
+				}
+			}
+		}
+		for(int q = RW_PF; q < kq; q++) {
+			const uint32_t e = src[(size_t) q * 64];
+			acc = (acc + tbl[e & (RW_LAST - 1)]) + tbl[e >> 16];
+			close(e);
+		}
+		__builtin_amdgcn_wave_barrier(); // LDS serves a wave's accesses in order: the reads below see the sums
+		if(OP) {
+#pragma unroll
+			for(int j = 0; j < RW_F; j++) back[j * 64 + lane] = row_op(back[j * 64 + lane], A.w[j], minus);
+			__builtin_amdgcn_wave_barrier();
+		}
+		double y[RW_F];
+#pragma unroll
+		for(int j = 0; j < RW_F; j++) y[j] = back[(A.p >> (8 * j)) & 0xffu];
+		auto add = [&](uint32_t e) {
+			const uint32_t lo = e & (RW_LAST - 1), hi = e >> 16;
+			if(lo != zero) unsafeAtomicAdd(&hist[lo], y[0]);
+			if(hi != zero) unsafeAtomicAdd(&hist[hi], y[0]);
+			const bool last = (e & RW_LAST) != 0;
+#pragma unroll
+			for(int j = 0; j + 1 < RW_F; j++) y[j] = last ? y[j + 1] : y[j];
+		};
+#pragma unroll
+		for(int qq = 0; qq < RW_PF; qq += 4) {
+			if(qq < kq) {
+#pragma unroll
+				for(int j = 0; j < 4; j++) add(qq + j < kq ? A.v[qq + j] : none);
+			}
+		}
+		for(int q = RW_PF; q < kq; q++) add(src[(size_t) q * 64]);
+		__builtin_amdgcn_wave_barrier();
+	};
+	if(q0 < nQuarters) {
+		Ahead A, B;
+		request(A, q0, h0);
+		uint2 hNext = h1;
+		for(int qt = q0; qt < nQuarters; qt += 2 * step) {
+			work(A, B, qt, hNext);
+			if(qt + step < nQuarters) work(B, A, qt + step, hNext);
+		}
+	}
+	double d[TPT];
+	dict(d);
+	__syncthreads();
+#pragma unroll
+	for(int j = 0; j < TPT; j++)
+		if(j * CS_THREADS + tid < nTbl) hist[j * CS_THREADS + tid] *= d[j];
+	__syncthreads();
+	// the block's share of every column: 8 lanes a group
+	for(int l0 = 0; l0 < nL; l0 += CS_THREADS / 8) {
+		const int l = l0 + tid / 8;
+		double s = 0.0;
+		if(l < nL) {
+			const int e1 = l + 1 < nL ? gBase[l + 1] : nTbl;
+			for(int e = gBase[l] + (tid & 7); e < e1; e += 8) s += hist[e];
+		}
+		s += __shfl_xor(s, 1); s += __shfl_xor(s, 2); s += __shfl_xor(s, 4);
+		// (exchanged, not stored: performed at device scope, see k_chain_u8)
+		if(l < nL && (tid & 7) == 0)
+			(void) __hip_atomic_exchange((unsigned long long*) part + (size_t) blockIdx.x * nL + l, (unsigned long long) __double_as_longlong(s), __ATOMIC_RELAXED,
+				__HIP_MEMORY_SCOPE_AGENT);
+	}
+	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+	__syncthreads();
+	if(tid == 0) lastS = last_block(done, gridDim.x);
+	__syncthreads();
+	if(!lastS) return;
+	// the last block: the others' shares in block order, a part of the blocks per nL threads
+	const int nP = CS_THREADS / nL, l = tid % nL, share = tid / nL;
+	double s = 0.0;
+	if(share < nP) {
+		for(int b0 = share; b0 < (int) gridDim.x; b0 += 8 * nP) {
+			unsigned long long r[8];
+#pragma unroll
+			for(int j = 0; j < 8; j++) {
+				const int bj = b0 + j * nP;
+				r[j] = bj < (int) gridDim.x
+					? __hip_atomic_load((const unsigned long long*) part + (size_t) bj * nL + l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+			}
+#pragma unroll
+			for(int j = 0; j < 8; j++) s += __longlong_as_double((long long) r[j]);
+		}
+		smemD[share * nL + l] = s;
+	}
+	if(nCols > nL) // columns that no list covers
+		for(int i = tid; i < nCols; i += CS_THREADS) out[i] = 0.0;
+	nnz_clear(nnz);
+	__syncthreads();
+	int nz = 0;
+	if(tid < nL) {
+		s = smemD[tid];
+		for(int i = 1; i < nP; i++) s += smemD[i * nL + tid];
+		out[tblCol[gBase[tid]]] = s;
+		nz = s != 0.0; // (a NaN counts, a negative zero does not)
+	}
+	nz = wave_sum_i32(nz);
+	if(lane == 0) cntS[wave] = nz;
+	__syncthreads();
+	if(tid == 0) {
+		int n = 0;
+		for(int i = 0; i < CS_WAVES; i++) n += cntS[i];
+		*nnz = (unsigned long long) n;
+	}
+	clear_tickets(done);
+}
+
 // The row lists of the block's listed groups (whole-block plan), built once.
 static int rows_plan(cla_block* b) {
 	if(b->rowsState != 0) return 0;
@@ -406,6 +618,55 @@ bool rows_fusable(cla_block* b) {
 		if(g.d.type != G_SDCZ || g.d.nOffsets <= 0 || g.d.nColG != 1) return false;
 	if(sdc_plan_all(b) != 0 || rows_plan(b) != 0) return false;
 	return b->rowsState == 1 && b->rowsFusable;
+}
+
+// The multiply chain of a block of single-column lists in one kernel.
+static int chain_sdc_shape(cla_block* b, unsigned& grid, size_t& lds) { // 1: not of its shape
+	const int nL = (int) b->groups.size();
+	if(!b->opt.chainFused || !b->opt.sdcRows || !b->opt.sdcLanes || b->dictNonFinite || nL == 0 || nL > CS_THREADS || b->nRows == 0) return 1;
+	std::vector<char> seen((size_t) b->nCols, 0);
+	for(const HostGroup& H : b->groups) {
+		if(H.d.type != G_SDCZ || H.d.nColG != 1 || seen[H.cols[0]]) return 1;
+		seen[H.cols[0]] = 1;
+	}
+	if(!rows_fusable(b) || b->rowsTbl > CS_TBL_MAX) return 1;
+	const int nQuarters = (int) ((b->nRows + RW_Q - 1) / RW_Q);
+	grid = (unsigned) std::min((nQuarters + CS_WAVES - 1) / CS_WAVES, g_numCU);
+	lds = sizeof(double) * ((size_t) (b->rowsTbl + 2) / 2 * 4 + (size_t) CS_WAVES * RW_Q);
+	return lds + 256 > (size_t) std::min(g_ldsPerBlock, 160 * 1024);
+}
+
+// The workspace of the chains to come, where the block's run in this kernel.
+int prepare_chain_sdc(cla_block* b) {
+	unsigned grid = 0;
+	size_t lds = 0;
+	return chain_sdc_shape(b, grid, lds) ? 0 : ensure_chain(b, (size_t) grid * b->groups.size());
+}
+
+// Returns 1 when the block is not eligible (the chain then runs as two products), 0 when the chain has been queued.
+int launch_chain_sdc(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz) {
+	unsigned grid = 0;
+	size_t lds = 0;
+	if(chain_sdc_shape(b, grid, lds)) return 1;
+	const int nL = (int) b->groups.size();
+	int rc = ensure_chain(b, (size_t) grid * nL);
+	if(rc) return rc;
+	char* meta = (char*) b->dRowsMeta;
+	const int32_t* dBase = (const int32_t*) (meta + 2 * b->rowsColOff) + nL;
+	clear_stats(b);
+	double algo = ctype != 0 ? (double) b->nRows * 8 : 0.0;
+	for(const HostGroup& H : b->groups) algo += (double) H.d.nDeltas * H.d.deltaWidth + (double) H.d.nOffsets * H.d.codeWidth;
+	Prof pf(b, "k_chain_sdc", (long) grid, CS_THREADS, (long) lds, algo);
+	auto go = [&](auto kernel) {
+		CLA_HIP(allow_full_lds((const void*) kernel));
+		hipLaunchKernelGGL(kernel, dim3(grid), dim3(CS_THREADS), lds, b->stream, (const int32_t*) meta, b->rowsTbl, dBase, nL, (const uint2*) (meta + b->rowsOff[0]),
+			(const uint32_t*) (meta + b->rowsOff[1]), (const uint32_t*) b->dRowsData, (const double*) b->dAllDict, (const int32_t*) (meta + b->rowsColOff), dV, dW,
+			ctype == 2 ? 1 : 0, b->nRows, (int) ((b->nRows + RW_Q - 1) / RW_Q), b->dChain, dOut, b->nCols, b->lmm_ticket(), dNnz);
+		return 0;
+	};
+	if((rc = ctype != 0 ? go(k_chain_sdc<true>) : go(k_chain_sdc<false>))) return rc;
+	CLA_HIP(hipGetLastError());
+	return 0;
 }
 
 } // namespace cla
