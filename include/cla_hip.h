@@ -138,7 +138,8 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *                   to finish writes the output, mirrored, and the count of its non-zeros and clears the accumulator)
  *                   instead of a fill of the output in front of the kernel and a mirror-and-count kernel behind it
  *   chain_fused     1 / 0: the multiply chain of single-column byte-code blocks without constants whose dictionaries fit LDS (up to
- *                   112 columns), and of blocks of single-column SDCZeros lists of up to 8,448 values together (with sdc_rows and sdc_lanes), in one
+ *                   112 columns), of up to 25 column pairs with two-byte codes without constants (dictionaries in LDS, or not too many rows), and of
+ *                   blocks of single-column SDCZeros lists of up to 8,448 values together (with sdc_rows and sdc_lanes), in one
  *                   pass over the codes or row lists, as the call's only kernel (0: two products)
  *   ddc_reorder     1 / 0 (read by cla_block_finalize): the block's copy of a DDC group with two- or four-byte codes and a
  *                   dictionary of 16 KiB or more is renumbered by descending count of the tuples (codes in place, dictionary

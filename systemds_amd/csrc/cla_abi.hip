@@ -887,7 +887,7 @@ int cla_block_prepare(cla_handle b, uint32_t products, int32_t nColB, int32_t nR
 		else r = tsmm_dev(b, out.p, true);
 	}
 	// X %*% v and one row of Y together: the products of the multiply chain, which on some blocks is a kernel with a workspace of its own
-	if(r >= 0 && (products & CLA_PRODUCT_RMM) && (products & CLA_PRODUCT_LMM) && nColB == 1 && nRowY == 1 && (r = prepare_chain_u8(b)) >= 0) r = prepare_chain_sdc(b);
+	if(r >= 0 && (products & CLA_PRODUCT_RMM) && (products & CLA_PRODUCT_LMM) && nColB == 1 && nRowY == 1 && (r = prepare_chain_u8(b)) >= 0 && (r = prepare_chain_sdc(b)) >= 0) r = prepare_chain_pairs(b);
 	b->profile = profile;
 	clear_stats(b);
 	return r < 0 ? (int) r : 0;

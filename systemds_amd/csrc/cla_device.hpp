@@ -106,6 +106,63 @@ __device__ __forceinline__ void clear_tickets(unsigned* done) {
 	if(threadIdx.x < 1 + TICKET_WAYS) done[threadIdx.x * (NNZ_STEP * 2)] = 0;
 }
 
+// End of a multiply chain's only kernel: sums[0 .. n) of every block in LDS (n <= THREADS, behind a barrier) through the workspace `part`, a row
+// per block; the last block to arrive adds them up in block order, writes out[column(i)] (0.0 to the columns without a sum) and the count of its
+// non-zeros. `room` is LDS for THREADS doubles beside the sums, which no one reads any more.
+template <int THREADS, typename Column>
+__device__ __forceinline__ void chain_hand_over(const double* sums, int n, double* __restrict__ part, double* room, const Column& column, double* __restrict__ out,
+	int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz) {
+	__shared__ int lastS;
+	__shared__ int cntS[THREADS / WAVE];
+	const int tid = threadIdx.x;
+	// (exchanged, not stored: performed at device scope, past the caches that the chip's parts do not share, see lmm_tail)
+	if(tid < n)
+		(void) __hip_atomic_exchange((unsigned long long*) part + (size_t) blockIdx.x * n + tid, (unsigned long long) __double_as_longlong(sums[tid]), __ATOMIC_RELAXED,
+			__HIP_MEMORY_SCOPE_AGENT);
+	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+	__syncthreads();
+	if(tid == 0) lastS = last_block(done, gridDim.x);
+	__syncthreads();
+	if(!lastS) return;
+	// a share of the blocks per n threads
+	const int nP = THREADS / n, i = tid % n, share = tid / n;
+	double s = 0.0;
+	if(share < nP) {
+		for(int b0 = share; b0 < (int) gridDim.x; b0 += 8 * nP) {
+			unsigned long long r[8];
+#pragma unroll
+			for(int j = 0; j < 8; j++) {
+				const int bj = b0 + j * nP;
+				r[j] = bj < (int) gridDim.x
+					? __hip_atomic_load((const unsigned long long*) part + (size_t) bj * n + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+			}
+#pragma unroll
+			for(int j = 0; j < 8; j++) s += __longlong_as_double((long long) r[j]);
+		}
+		room[share * n + i] = s;
+	}
+	if(nCols > n)
+		for(int c = tid; c < nCols; c += THREADS) out[c] = 0.0;
+	nnz_clear(nnz);
+	__syncthreads();
+	int nz = 0;
+	if(tid < n) {
+		s = room[tid];
+		for(int j = 1; j < nP; j++) s += room[j * n + tid];
+		out[column(tid)] = s;
+		nz = s != 0.0; // (a NaN counts, a negative zero does not)
+	}
+	nz = wave_sum_i32(nz);
+	if((tid & (WAVE - 1)) == 0) cntS[tid / WAVE] = nz;
+	__syncthreads();
+	if(tid == 0) {
+		int total = 0;
+		for(int j = 0; j < THREADS / WAVE; j++) total += cntS[j];
+		*nnz = (unsigned long long) total;
+	}
+	clear_tickets(done);
+}
+
 // Tail of a left multiply whose kernel is the only one of the call: every block comes here behind its last add into
 // out; the last one to arrive counts the non-zeros of out[0 .. n) into *nnz
 // (the same is what a kernel of its own behind this one would do; done == nullptr: no tail).

@@ -98,7 +98,7 @@ struct Options {
 	int rmmDigits = 1;      // X %*% B of byte-code blocks on digits and the integer matrix cores (0: fp64; 2: short blocks and narrow B, too)
 	int tsmmDigits = 1;     // t(X) %*% X of byte-code blocks on digits and the integer matrix cores (0: fp64; 2: short blocks, too)
 	int tsmmOneKernel = 1;  // decoded Gram matrix of a whole block as the call's only kernel (0: a fill in front, k_tsmm_finish behind)
-	int chainFused = 1;     // multiply chain of single-column byte-code blocks or lists in one pass over the codes or row lists (0: two products)
+	int chainFused = 1;     // multiply chain of single-column byte-code blocks, of two-byte column pairs or of lists in one pass over the codes or row lists (0: two products)
 	int ddcReorder = 1;     // finalize renumbers the tuples of large DDC dictionaries by descending count (0: the caller's numbering is kept)
 };
 
@@ -297,6 +297,8 @@ int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype,
 int prepare_chain_u8(cla_block* b);
 int launch_chain_sdc(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz);
 int prepare_chain_sdc(cla_block* b);
+int launch_chain_pairs(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz);
+int prepare_chain_pairs(cla_block* b);
 int launch_lmm_u8_vec(cla_block* b, const double* dY, double* dOut);
 int launch_lmm_sdc_tiles(cla_block* b, const double* dY, int p, double* dPre, int onlyGroup, double* dOut);
 int launch_lmm_sdc_lanes(cla_block* b, const double* dY, int p, double* dOut);

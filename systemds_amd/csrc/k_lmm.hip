@@ -667,6 +667,7 @@ int launch_mmchain(cla_block* b, const double* dV, const double* dW, int ctype, 
 	{
 		int r = launch_chain_u8(b, dV, dW, ctype, dOut, dNnz);
 		if(r == 1) r = launch_chain_sdc(b, dV, dW, ctype, dOut, dNnz);
+		if(r == 1) r = launch_chain_pairs(b, dV, dW, ctype, dOut, dNnz);
 		if(r <= 0) return r;
 	}
 	// the intermediate vector has a workspace of its own: the multiplies below may resize the shared scratch

@@ -293,8 +293,6 @@ __global__ __launch_bounds__(CS_THREADS) void k_chain_sdc(const int32_t* __restr
 	const int32_t* __restrict__ tblCol, const double* __restrict__ v, const double* __restrict__ w, int minus, int64_t nRows, int nQuarters,
 	double* __restrict__ part, double* __restrict__ out, int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz) {
 	extern __shared__ double smemD[];
-	__shared__ int lastS;
-	__shared__ int cntS[CS_WAVES];
 	const int nPad = (nTbl + 2) / 2 * 2;
 	double* tbl = smemD;            // dictionary value x v of the column, and a 0.0
 	double* hist = smemD + nPad;    // sums of the rows' values by entry
@@ -431,6 +429,7 @@ __global__ __launch_bounds__(CS_THREADS) void k_chain_sdc(const int32_t* __restr
 		if(j * CS_THREADS + tid < nTbl) hist[j * CS_THREADS + tid] *= d[j];
 	__syncthreads();
 	// the block's share of every column: 8 lanes a group
+	double* const sums = smemD + 2 * nPad; // (in place of the rows' sums)
 	for(int l0 = 0; l0 < nL; l0 += CS_THREADS / 8) {
 		const int l = l0 + tid / 8;
 		double s = 0.0;
@@ -439,53 +438,10 @@ __global__ __launch_bounds__(CS_THREADS) void k_chain_sdc(const int32_t* __restr
 			for(int e = gBase[l] + (tid & 7); e < e1; e += 8) s += hist[e];
 		}
 		s += __shfl_xor(s, 1); s += __shfl_xor(s, 2); s += __shfl_xor(s, 4);
-		// (exchanged, not stored: performed at device scope, see k_chain_u8)
-		if(l < nL && (tid & 7) == 0)
-			(void) __hip_atomic_exchange((unsigned long long*) part + (size_t) blockIdx.x * nL + l, (unsigned long long) __double_as_longlong(s), __ATOMIC_RELAXED,
-				__HIP_MEMORY_SCOPE_AGENT);
+		if(l < nL && (tid & 7) == 0) sums[l] = s;
 	}
-	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 	__syncthreads();
-	if(tid == 0) lastS = last_block(done, gridDim.x);
-	__syncthreads();
-	if(!lastS) return;
-	// the last block: the others' shares in block order, a part of the blocks per nL threads
-	const int nP = CS_THREADS / nL, l = tid % nL, share = tid / nL;
-	double s = 0.0;
-	if(share < nP) {
-		for(int b0 = share; b0 < (int) gridDim.x; b0 += 8 * nP) {
-			unsigned long long r[8];
-#pragma unroll
-			for(int j = 0; j < 8; j++) {
-				const int bj = b0 + j * nP;
-				r[j] = bj < (int) gridDim.x
-					? __hip_atomic_load((const unsigned long long*) part + (size_t) bj * nL + l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
-			}
-#pragma unroll
-			for(int j = 0; j < 8; j++) s += __longlong_as_double((long long) r[j]);
-		}
-		smemD[share * nL + l] = s;
-	}
-	if(nCols > nL) // columns that no list covers
-		for(int i = tid; i < nCols; i += CS_THREADS) out[i] = 0.0;
-	nnz_clear(nnz);
-	__syncthreads();
-	int nz = 0;
-	if(tid < nL) {
-		s = smemD[tid];
-		for(int i = 1; i < nP; i++) s += smemD[i * nL + tid];
-		out[tblCol[gBase[tid]]] = s;
-		nz = s != 0.0; // (a NaN counts, a negative zero does not)
-	}
-	nz = wave_sum_i32(nz);
-	if(lane == 0) cntS[wave] = nz;
-	__syncthreads();
-	if(tid == 0) {
-		int n = 0;
-		for(int i = 0; i < CS_WAVES; i++) n += cntS[i];
-		*nnz = (unsigned long long) n;
-	}
-	clear_tickets(done);
+	chain_hand_over<CS_THREADS>(sums, nL, part, smemD, [&](int l) { return tblCol[gBase[l]]; }, out, nCols, done, nnz);
 }
 
 // The row lists of the block's listed groups (whole-block plan), built once.
@@ -632,7 +588,7 @@ static int chain_sdc_shape(cla_block* b, unsigned& grid, size_t& lds) { // 1: no
 	if(!rows_fusable(b) || b->rowsTbl > CS_TBL_MAX) return 1;
 	const int nQuarters = (int) ((b->nRows + RW_Q - 1) / RW_Q);
 	grid = (unsigned) std::min((nQuarters + CS_WAVES - 1) / CS_WAVES, g_numCU);
-	lds = sizeof(double) * ((size_t) (b->rowsTbl + 2) / 2 * 4 + (size_t) CS_WAVES * RW_Q);
+	lds = sizeof(double) * (std::max<size_t>((size_t) (b->rowsTbl + 2) / 2 * 4, CS_THREADS) + (size_t) CS_WAVES * RW_Q);
 	return lds + 256 > (size_t) std::min(g_ldsPerBlock, 160 * 1024);
 }
 
