@@ -238,9 +238,9 @@ struct LmmTake {
 	const double* Y;
 	int p;
 	int64_t nRows;
-	const double* stage;           // p x nCols, what the kernel in front has summed
+	double* stage;                 // p x nCols, what the kernel in front has summed; left at zero, like the next three
 	double* anew;                  // p x nCols and p row sums, zero
-	const unsigned long long* bad;
+	unsigned long long* bad;
 	unsigned long long* count;     // zero
 	const double* constV;          // nullptr: no constants
 	unsigned long long redo;       // columns that a non-finite Y takes anew
@@ -388,6 +388,7 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 			}
 		}
 		else v = A.stage[idx];
+		A.stage[idx] = 0.0; // (nobody else reads it)
 		A.out[idx] = v;
 		cnt += v != 0.0;
 	}
@@ -411,6 +412,11 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 	if(!lastS) return;
 	if(tid > 0 && tid < NNZ_WAYS) A.nnz[tid * NNZ_STEP] = 0;
 	clear_tickets(A.done);
+	if(anew) { // (all blocks have taken a ticket: nobody reads these any more)
+		for(int i = tid; i < n + A.p; i += LT_THREADS) A.anew[i] = 0.0;
+		if(tid == 0) *A.bad = 0;
+	}
+	if(tid == 0) *A.count = 0;
 }
 
 // (a kernel, not hipMemsetAsync: a memset node of a captured graph has given wrong results on its replays)
@@ -429,7 +435,7 @@ int launch_lmm_take(cla_block* b, const double* dY, int p, double* ws, double* d
 	LmmTake A;
 	A.groups = b->dGroups; A.nGroups = (int) b->groups.size();
 	A.Y = dY; A.p = p; A.nRows = b->nRows; A.nCols = b->nCols;
-	A.stage = ws; A.anew = ws + n; A.bad = (const unsigned long long*) (ws + 2 * n + p); A.count = (unsigned long long*) (ws + 2 * n + p + 1);
+	A.stage = ws; A.anew = ws + n; A.bad = (unsigned long long*) (ws + 2 * n + p); A.count = (unsigned long long*) (ws + 2 * n + p + 1);
 	A.constV = b->hasConst ? b->dConstV : nullptr;
 	A.redo = ~0ull; // (at most LT_COLS columns)
 	for(const HostGroup& H : b->groups)
