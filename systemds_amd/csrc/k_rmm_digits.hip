@@ -21,7 +21,7 @@
 //
 // Bound: a tile of 256 x 100 rows and 64 columns of B takes 27,000 cycles, 14,000 of them the matrix cores' (380 products per SIMD); decoding (5,600) is LDS reads with barriers
 // between, the outputs (128 KB) wait for their turn with the tables behind the products; the clock is 2.0 GHz under this load. 10,000,000 x 100 of 256 values times 64 columns 2.57 ms in fp64, 2.27 here;
-// 400,000 rows 182 / 120 us, 50,000 67 / 43; 400,000 x 64 128 / 88. Taken back: outputs kept until the next tile's products (64 registers more: 3.6 ms), the
+// 400,000 rows 182 / 120 us, 150,000 100 / 55, 500 64 / 25; 400,000 x 64 128 / 88. Taken back: outputs kept until the next tile's products (64 registers more: 3.6 ms), the
 // next tables ordered between the products (3.0), products of a step between the look-ups of the next (2.28: LDS and matrix cores still take turns), two columns a
 // lane for 16-byte stores (2.29).
 #include "../../include/cla_hip.h"
@@ -35,6 +35,7 @@
 namespace cla {
 
 constexpr int RD_THREADS = 512, RD_WAVES = 8, RD_ROWS = 256;
+constexpr int RD_COLS = 100;                      // most columns of X
 constexpr int RD_TABLE = 2048;                    // bytes of a column's table in LDS and in the image
 constexpr int RD_CODES = 2 * 1024 + 128;          // a wave's codes: two steps' 32 columns x 32 rows, 4 x 32 behind them
 typedef int i32x4_rd __attribute__((ext_vector_type(4)));
@@ -370,17 +371,27 @@ __global__ __launch_bounds__(RB_THREADS) void k_rmm_digits_b(const MfPrep P, int
 	__shared__ int badS;
 	const int c = blockIdx.x, tid = threadIdx.x, r = tid & 31, slice = tid >> 5, col = n0 + 32 * c + r;
 	const int pieces = S * 8 + 8 * T;
+	// all of a thread's values requested at once, in two round trips (walked twice, one after the other, they took 14.5 us of a call, 7.0 now). up[k]: 2^(exponent
+	// of X's column k)
+	constexpr int VALS = (RD_COLS + RB_THREADS / 32 - 1) / (RB_THREADS / 32);
+	double v[VALS];
+	{
+		int32_t at[VALS];
+#pragma unroll
+		for(int i = 0; i < VALS; i++) at[i] = rowCol[min(slice + i * (RB_THREADS / 32), K - 1)];
+#pragma unroll
+		for(int i = 0; i < VALS; i++) v[i] = B[(size_t) at[i] * q + min(col, q - 1)] * up[min(slice + i * (RB_THREADS / 32), K - 1)];
+	}
 	if(tid == 0) badS = 0;
 	for(int i = tid; i < pieces * 256; i += RB_THREADS) ((uint32_t*) img)[i] = 0;
-	// up[k]: 2^(exponent of X's column k)
 	double m = 0.0;
 	bool odd = false;
-	if(col < q)
-		for(int k = slice; k < K; k += RB_THREADS / 32) {
-			const double v = fabs(B[(size_t) rowCol[k] * q + col] * up[k]);
-			odd |= !(v <= 1e300); // (a NaN, an infinity or close to it)
-			m = v > m ? v : m;
-		}
+#pragma unroll
+	for(int i = 0; i < VALS; i++) {
+		if(col >= q || slice + i * (RB_THREADS / 32) >= K) v[i] = 0.0;
+		odd |= !(fabs(v[i]) <= 1e300); // (a NaN, an infinity or close to it)
+		m = fabs(v[i]) > m ? fabs(v[i]) : m;
+	}
 	most[slice][r] = m;
 	__syncthreads();
 	for(int i = 0; i < RB_THREADS / 32; i++) m = most[i][r] > m ? most[i][r] : m;
@@ -396,8 +407,11 @@ __global__ __launch_bounds__(RB_THREADS) void k_rmm_digits_b(const MfPrep P, int
 		least[32 * c + r] = m > 0.0 ? leastSum : 0;
 	}
 	if(col < q)
-		for(int k = slice; k < K; k += RB_THREADS / 32) {
-			const double x = ldexp(B[(size_t) rowCol[k] * q + col] * up[k], -e);
+#pragma unroll
+		for(int j = 0; j < VALS; j++) {
+			const int k = slice + j * (RB_THREADS / 32);
+			if(k >= K) break;
+			const double x = ldexp(v[j], -e);
 			int64_t X = odd ? 0 : (int64_t) rint(x * (double) ((int64_t) 1 << 55));
 			const int mag = odd ? 0 : min(127, (int) (fabs(x) * 128.0));
 			int d[7];
@@ -455,7 +469,7 @@ static int rd_build_plan(cla_block* b, RdPlan& P) {
 	int K = 0;
 	for(const HostGroup& H : b->groups) K += H.d.nColG;
 	const int rest = K % 32, T = rest >= 1 && rest <= 4 ? 1 : 0, S = T ? K / 32 : (K + 31) / 32;
-	if(K < 64 || S > 3) return 0;
+	if(K < 64 || K > RD_COLS) return 0;
 	P.K = K; P.S = S; P.T = T;
 	const int places = S * 32 + 4 * T;
 	std::vector<int32_t> streams((size_t) places, 0), rowCol((size_t) places, 0);

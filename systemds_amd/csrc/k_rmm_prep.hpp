@@ -27,7 +27,7 @@ struct MfPrep {
 // B in the slab layout: row r of the list (decoded column rowCol[r], -1 = padding) at r * MF_BK,
 // output column n0 + 8 (jg / 2) + 2 j + jg % 2 at j * MF_BJ + jg. The block behind the last row makes the constants' row of the pass, rounded
 // and skipped like the tables' (k_preagg), and clears the counter. Bound: one launch; before, k_preagg made tables in front that nobody read and k_mfma_blayout was a
-// launch of its own beside k_rmm_digits_b: 2,914 x 10 by 31 14.3 -> 12.1 us, 500 x 100 by 64 38 -> 29, 150,000 x 100 by 64 69 -> 59, two-byte codes 50,000 x 50 of 4000 tuples by 16 71 -> 63.
+// launch of its own beside k_rmm_digits_b: 2,914 x 10 by 31 14.3 -> 12.1 us, 500 x 100 by 64 38 -> 25, 150,000 x 100 by 64 69 -> 55, two-byte codes 50,000 x 50 of 4000 tuples by 16 71 -> 63.
 __device__ __forceinline__ void mf_prep(const MfPrep& P, int block) {
 	const int t = threadIdx.x & 127, r = block * MF_BL_ROWS + (threadIdx.x >> 7);
 	if(block * MF_BL_ROWS < P.nRowCol) {

@@ -579,7 +579,7 @@ bool rows_fusable(cla_block* b) {
 // The multiply chain of a block of single-column lists in one kernel.
 static int chain_sdc_shape(cla_block* b, unsigned& grid, size_t& lds) { // 1: not of its shape
 	const int nL = (int) b->groups.size();
-	if(!b->opt.chainFused || !b->opt.sdcRows || !b->opt.sdcLanes || b->dictNonFinite || nL == 0 || nL > CS_THREADS || b->nRows == 0) return 1;
+	if(!b->opt.chainFused || !b->opt.sdcRows || !b->opt.sdcLanes || b->rowsTbl > CS_TBL_MAX || b->dictNonFinite || nL == 0 || nL > CS_THREADS || b->nRows == 0) return 1;
 	std::vector<char> seen((size_t) b->nCols, 0);
 	for(const HostGroup& H : b->groups) {
 		if(H.d.type != G_SDCZ || H.d.nColG != 1 || seen[H.cols[0]]) return 1;
