@@ -1776,7 +1776,7 @@ int64_t cla_aggregate(cla_handle b, int32_t op, int32_t dir, double* out) {
 	CLA_CATCH_CODE(int64_t)
 }
 
-static int64_t mmchain_dev(cla_handle b, const double* dV, const double* dW, int32_t ctype, double* dOut, bool sync) {
+static int64_t mmchain_dev(cla_handle b, const double* dV, const double* dW, int32_t ctype, double* dOut, bool sync, ChainHost* host = nullptr) {
 	int rc = check_final(b);
 	if(rc) return rc;
 	if(!dV || !dOut) { set_error("mmchain: null vector"); return -CLA_ERR_INVALID; }
@@ -1784,7 +1784,7 @@ static int64_t mmchain_dev(cla_handle b, const double* dV, const double* dW, int
 	if(ctype != 0 && !dW) { set_error("mmchain: XtwXv and XtXvy need w"); return -CLA_ERR_INVALID; }
 	std::lock_guard<std::recursive_mutex> lk(b->mu);
 	b->nnzSlot = 0;
-	if((rc = launch_mmchain(b, dV, dW, ctype, dOut, b->dCounters))) return rc;
+	if((rc = launch_mmchain(b, dV, dW, ctype, dOut, b->dCounters, host))) return rc;
 	return finish_nnz(b, sync);
 }
 
@@ -1814,9 +1814,11 @@ int64_t cla_mmchain(cla_handle b, const double* v, const double* w, int32_t ctyp
 	if(pinned) { if((rc = launch_fetch(b, b->dStageIn, v, (int) nV))) return rc; }
 	else CLA_HIP(hipMemcpyAsync(b->dStageIn, v, nV * sizeof(double), hipMemcpyHostToDevice, b->stream));
 	if(nW) CLA_HIP(hipMemcpyAsync(b->dStageIn + nV, w, nW * sizeof(double), hipMemcpyHostToDevice, b->stream));
-	const int64_t nnz = mmchain_dev(b, b->dStageIn, nW ? b->dStageIn + nV : nullptr, ctype, b->dStageOut, !pinned);
+	ChainHost host;
+	if(pinned) host = chain_host(b);
+	const int64_t nnz = mmchain_dev(b, b->dStageIn, nW ? b->dStageIn + nV : nullptr, ctype, b->dStageOut, !pinned, pinned ? &host : nullptr);
 	if(nnz < 0) return nnz;
-	if(pinned) return deliver(b, out, b->dStageOut, (int) nV, b->dCounters);
+	if(pinned) return deliver(b, out, b->dStageOut, (int) nV, b->dCounters, host.done);
 	CLA_HIP(hipMemcpy(out, b->dStageOut, nV * sizeof(double), hipMemcpyDeviceToHost));
 	return nnz;
 	CLA_CATCH_CODE(int64_t)

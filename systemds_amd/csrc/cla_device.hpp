@@ -108,10 +108,10 @@ __device__ __forceinline__ void clear_tickets(unsigned* done) {
 
 // End of a multiply chain's only kernel: sums[0 .. n) of every block in LDS (n <= THREADS, behind a barrier) through the workspace `part`, a row
 // per block; the last block to arrive adds them up in block order, writes out[column(i)] (0.0 to the columns without a sum) and the count of its
-// non-zeros. `room` is LDS for THREADS doubles beside the sums, which no one reads any more.
+// non-zeros, both also to hostOut and hostCount unless null. `room` is LDS for THREADS doubles beside the sums, which no one reads any more.
 template <int THREADS, typename Column>
 __device__ __forceinline__ void chain_hand_over(const double* sums, int n, double* __restrict__ part, double* room, const Column& column, double* __restrict__ out,
-	int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz) {
+	int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz, double* __restrict__ hostOut, unsigned long long* __restrict__ hostCount) {
 	__shared__ int lastS;
 	__shared__ int cntS[THREADS / WAVE];
 	const int tid = threadIdx.x;
@@ -142,14 +142,19 @@ __device__ __forceinline__ void chain_hand_over(const double* sums, int n, doubl
 		room[share * n + i] = s;
 	}
 	if(nCols > n)
-		for(int c = tid; c < nCols; c += THREADS) out[c] = 0.0;
+		for(int c = tid; c < nCols; c += THREADS) {
+			out[c] = 0.0;
+			if(hostOut != nullptr) hostOut[c] = 0.0;
+		}
 	nnz_clear(nnz);
 	__syncthreads();
 	int nz = 0;
 	if(tid < n) {
 		s = room[tid];
 		for(int j = 1; j < nP; j++) s += room[j * n + tid];
-		out[column(tid)] = s;
+		const int c = column(tid);
+		out[c] = s;
+		if(hostOut != nullptr) hostOut[c] = s;
 		nz = s != 0.0; // (a NaN counts, a negative zero does not)
 	}
 	nz = wave_sum_i32(nz);
@@ -159,6 +164,7 @@ __device__ __forceinline__ void chain_hand_over(const double* sums, int n, doubl
 		int total = 0;
 		for(int j = 0; j < THREADS / WAVE; j++) total += cntS[j];
 		*nnz = (unsigned long long) total;
+		if(hostCount != nullptr) *hostCount = (unsigned long long) total;
 	}
 	clear_tickets(done);
 }

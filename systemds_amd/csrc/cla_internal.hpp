@@ -294,11 +294,17 @@ int launch_rmm_mfma(cla_block* b, const double* dB, int q, double* dConstRow, do
 	unsigned long long* dNnz);
 int launch_lmm_u8(cla_block* b, const double* dY, int p, double* dPre);
 int launch_lmm_u8_dot(cla_block* b, const double* dY, int p, double* dOut);
-int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz);
+// Where a chain's only kernel also writes its result and the count (pinned host memory; null: nowhere). done: it has been queued to.
+struct ChainHost {
+	double* out = nullptr;
+	unsigned long long* count = nullptr;
+	bool done = false;
+};
+int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz, ChainHost& host);
 int prepare_chain_u8(cla_block* b);
-int launch_chain_sdc(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz);
+int launch_chain_sdc(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz, ChainHost& host);
 int prepare_chain_sdc(cla_block* b);
-int launch_chain_pairs(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz);
+int launch_chain_pairs(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz, ChainHost& host);
 int prepare_chain_pairs(cla_block* b);
 int launch_lmm_u8_vec(cla_block* b, const double* dY, double* dOut);
 int launch_lmm_sdc_tiles(cla_block* b, const double* dY, int p, double* dPre, int onlyGroup, double* dOut);
@@ -338,7 +344,8 @@ int tsmm_decode_fits(cla_block* b);
 int launch_lmm_decode(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dBad);
 int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dNnz);
 int launch_fetch(cla_block* b, double* dst, const double* v, int n);
-int64_t deliver(cla_block* b, double* out, const double* src, int n, const unsigned long long* dNnz);
+ChainHost chain_host(cla_block* b);
+int64_t deliver(cla_block* b, double* out, const double* src, int n, const unsigned long long* dNnz, bool there = false);
 int launch_zero(cla_block* b, double* p, size_t n); // n > 0
 int launch_lmm_take(cla_block* b, const double* dY, int p, double* ws, double* dOut, unsigned long long* dNnz); // ws: p x nCols summed, 2 n + p + 2 in all
 int launch_lmm(cla_block* b, const double* dY, int p, double* dOut, unsigned long long* dNnz);
@@ -347,7 +354,8 @@ int launch_tsmm(cla_block* b, double* dOut, unsigned long long* dNnz);
 int launch_tsmm_chunked(cla_block* b, double* dOut);
 int launch_cooc(cla_block* b, int gA, int gB, unsigned long long* dOut);
 int launch_mmchain(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut,
-	unsigned long long* dNnz);
+	unsigned long long* dNnz,
+	ChainHost* host = nullptr);
 
 // Scope around one kernel launch: records launch geometry and, when the block is
 // in profiling mode, HIP events on the block's stream in front of and behind it.

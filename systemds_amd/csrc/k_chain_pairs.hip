@@ -33,7 +33,8 @@ static constexpr int cp_groups(int nG) { return nG <= 4 ? 4 : nG <= 8 ? 8 : nG <
 template <int NG, bool LDS, bool OP>
 __global__ __launch_bounds__(CP_THREADS, NG <= 8 ? 4 : 2) void k_chain_pairs(const uint8_t* __restrict__ arena, size_t arenaStride, int nG, const CpGroups P,
 	const f64x2* __restrict__ dict, int nTuples, const double* __restrict__ v, const double* __restrict__ w, int minus, int64_t nRows,
-	double* __restrict__ part, double* __restrict__ out, int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz) {
+	double* __restrict__ part, double* __restrict__ out, int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz, double* __restrict__ hostOut,
+	unsigned long long* __restrict__ hostCount) {
 	extern __shared__ __attribute__((aligned(16))) double smem[]; // the dictionaries; at the end the sums
 	constexpr int N2 = 2 * NG, FOLD = N2 <= 8 ? 8 : N2 <= 16 ? 16 : N2 <= 32 ? 32 : 64;
 	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -126,7 +127,7 @@ __global__ __launch_bounds__(CP_THREADS, NG <= 8 ? 4 : 2) void k_chain_pairs(con
 		sums[tid] = s;
 	}
 	__syncthreads();
-	chain_hand_over<CP_THREADS>(sums, 2 * nG, part, smem, [&](int i) { return i & 1 ? P.c1[i / 2] : P.c0[i / 2]; }, out, nCols, done, nnz);
+	chain_hand_over<CP_THREADS>(sums, 2 * nG, part, smem, [&](int i) { return i & 1 ? P.c1[i / 2] : P.c0[i / 2]; }, out, nCols, done, nnz, hostOut, hostCount);
 }
 
 struct CpLaunch {
@@ -170,7 +171,7 @@ int prepare_chain_pairs(cla_block* b) {
 }
 
 // Returns 1 when the block is not eligible (the chain then runs as two products), 0 when the chain has been queued.
-int launch_chain_pairs(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz) {
+int launch_chain_pairs(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz, ChainHost& host) {
 	CpLaunch L;
 	if(cp_shape(b, L)) return 1;
 	const int nG = (int) b->groups.size();
@@ -187,7 +188,7 @@ int launch_chain_pairs(cla_block* b, const double* dV, const double* dW, int cty
 	auto go = [&](auto kern) {
 		CLA_HIP(allow_full_lds((const void*) kern));
 		hipLaunchKernelGGL(kern, dim3(L.grid), dim3(CP_THREADS), L.lds, b->stream, b->dArena, b->arenaStride, nG, P, (const f64x2*) b->dAllDict, b->totalVals, dV, dW,
-			ctype == 2 ? 1 : 0, b->nRows, b->dChain, dOut, b->nCols, b->lmm_ticket(), dNnz);
+			ctype == 2 ? 1 : 0, b->nRows, b->dChain, dOut, b->nCols, b->lmm_ticket(), dNnz, host.out, host.count);
 		return 0;
 	};
 #define CP_CASE(N)                                                                                                                \

@@ -53,7 +53,7 @@ template <int NCB, bool OP>
 __global__ __launch_bounds__(CH_THREADS, NCB <= 3 ? 4 : 2) void k_chain_u8(const uint8_t* __restrict__ arena, size_t arenaStride, int nGroups,
 	const double* __restrict__ dictT, int nVals, const int32_t* __restrict__ col0, const double* __restrict__ v, const double* __restrict__ w,
 	int minus, int64_t nRows, double* __restrict__ part, double* __restrict__ out, int nCols, unsigned* __restrict__ done,
-	unsigned long long* __restrict__ nnz) {
+	unsigned long long* __restrict__ nnz, double* __restrict__ hostOut, unsigned long long* __restrict__ hostCount) {
 	extern __shared__ __attribute__((aligned(16))) double smem[]; // the dictionaries; at the end the sums
 	__shared__ int lastS;
 	__shared__ int cntS[CH_WAVES];
@@ -232,7 +232,10 @@ __global__ __launch_bounds__(CH_THREADS, NCB <= 3 ? 4 : 2) void k_chain_u8(const
 		smem[share * NC + col] = s;
 	}
 	if(nCols > nGroups) // columns that no group covers
-		for(int i = tid; i < nCols; i += CH_THREADS) out[i] = 0.0;
+		for(int i = tid; i < nCols; i += CH_THREADS) {
+			out[i] = 0.0;
+			if(hostOut != nullptr) hostOut[i] = 0.0;
+		}
 	nnz_clear(nnz);
 	__syncthreads();
 	int nz = 0;
@@ -241,6 +244,7 @@ __global__ __launch_bounds__(CH_THREADS, NCB <= 3 ? 4 : 2) void k_chain_u8(const
 #pragma unroll
 		for(int i = 1; i < NP; i++) s += smem[i * NC + tid];
 		out[col0[tid]] = s;
+		if(hostOut != nullptr) hostOut[col0[tid]] = s;
 		nz = s != 0.0; // (a NaN counts, a negative zero does not)
 	}
 	nz = wave_sum_i32(nz);
@@ -250,6 +254,7 @@ __global__ __launch_bounds__(CH_THREADS, NCB <= 3 ? 4 : 2) void k_chain_u8(const
 		int n = 0;
 		for(int i = 0; i < CH_WAVES; i++) n += cntS[i];
 		*nnz = (unsigned long long) n;
+		if(hostCount != nullptr) *hostCount = (unsigned long long) n;
 	}
 	clear_tickets(done);
 }
@@ -297,7 +302,7 @@ int prepare_chain_u8(cla_block* b) {
 }
 
 // Returns 1 when the block is not eligible (the chain then runs as two products), 0 when the chain has been queued.
-int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz) {
+int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz, ChainHost& host) {
 	const int nG = (int) b->groups.size();
 	const int64_t nRows = b->nRows;
 	ChainLaunch L;
@@ -310,7 +315,7 @@ int launch_chain_u8(cla_block* b, const double* dV, const double* dW, int ctype,
 	const double algo = (double) nRows * nG + (dW != nullptr ? (double) nRows * 8 : 0.0);
 	Prof pf(b, "k_chain_u8", L.grid, CH_THREADS, (long) L.lds, algo);
 	hipLaunchKernelGGL(L.kern, dim3(L.grid), dim3(CH_THREADS), L.lds, b->stream, b->dArena, b->arenaStride, nG, b->dDictPad + b->dictTOff, b->maxVals, dCol0,
-		dV, dW, ctype == 2 ? 1 : 0, nRows, b->dChain, dOut, b->nCols, b->lmm_ticket(), dNnz);
+		dV, dW, ctype == 2 ? 1 : 0, nRows, b->dChain, dOut, b->nCols, b->lmm_ticket(), dNnz, host.out, host.count);
 	CLA_HIP(hipGetLastError());
 	return 0;
 }

@@ -658,22 +658,33 @@ int launch_fetch(cla_block* b, double* dst, const double* v, int n) {
 	return 0;
 }
 
-// src (n <= HOST_VEC_MAX) into out (host); waits for the stream and returns the count in dNnz
-int64_t deliver(cla_block* b, double* out, const double* src, int n, const unsigned long long* dNnz) {
+// Where a chain's only kernel writes for deliver(): a launch less (250,007 x 54 34.6 -> 33.2 us, 3,085 x 23 26.8 -> 24.4).
+ChainHost chain_host(cla_block* b) {
+	ChainHost h;
+	h.out = (double*) b->hCounters + 1 + HOST_VEC_MAX;
+	h.count = b->hCounters;
+	return h;
+}
+
+// src (n <= HOST_VEC_MAX) into out (host); waits for the stream and returns the count in dNnz. there: both are on their way to chain_host(b) already.
+int64_t deliver(cla_block* b, double* out, const double* src, int n, const unsigned long long* dNnz, bool there) {
 	double* const host = (double*) b->hCounters + 1 + HOST_VEC_MAX;
-	hipLaunchKernelGGL(k_deliver, dim3(1), dim3(512), 0, b->stream, host, src, n, b->hCounters, dNnz);
+	if(!there) hipLaunchKernelGGL(k_deliver, dim3(1), dim3(512), 0, b->stream, host, src, n, b->hCounters, dNnz);
 	CLA_HIP(hipGetLastError());
 	CLA_HIP(hipStreamSynchronize(b->stream));
 	memcpy(out, host, (size_t) n * sizeof(double));
 	return (int64_t) b->hCounters[0];
 }
 
-int launch_mmchain(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz) {
+int launch_mmchain(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz, ChainHost* host) {
 	const int64_t nRows = b->nRows;
 	{
-		int r = launch_chain_u8(b, dV, dW, ctype, dOut, dNnz);
-		if(r == 1) r = launch_chain_sdc(b, dV, dW, ctype, dOut, dNnz);
-		if(r == 1) r = launch_chain_pairs(b, dV, dW, ctype, dOut, dNnz);
+		ChainHost none;
+		ChainHost& to = host != nullptr ? *host : none;
+		int r = launch_chain_u8(b, dV, dW, ctype, dOut, dNnz, to);
+		if(r == 1) r = launch_chain_sdc(b, dV, dW, ctype, dOut, dNnz, to);
+		if(r == 1) r = launch_chain_pairs(b, dV, dW, ctype, dOut, dNnz, to);
+		to.done = r == 0;
 		if(r <= 0) return r;
 	}
 	// the intermediate vector has a workspace of its own: the multiplies below may resize the shared scratch

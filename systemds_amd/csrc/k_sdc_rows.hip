@@ -291,7 +291,8 @@ template <bool OP>
 __global__ __launch_bounds__(CS_THREADS) void k_chain_sdc(const int32_t* __restrict__ tblIndex, int nTbl, const int32_t* __restrict__ gBase, int nL,
 	const uint2* __restrict__ hdr, const uint32_t* __restrict__ perm, const uint32_t* __restrict__ data, const double* __restrict__ D,
 	const int32_t* __restrict__ tblCol, const double* __restrict__ v, const double* __restrict__ w, int minus, int64_t nRows, int nQuarters,
-	double* __restrict__ part, double* __restrict__ out, int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz) {
+	double* __restrict__ part, double* __restrict__ out, int nCols, unsigned* __restrict__ done, unsigned long long* __restrict__ nnz, double* __restrict__ hostOut,
+	unsigned long long* __restrict__ hostCount) {
 	extern __shared__ double smemD[];
 	const int nPad = (nTbl + 2) / 2 * 2;
 	double* tbl = smemD;            // dictionary value x v of the column, and a 0.0
@@ -441,7 +442,7 @@ __global__ __launch_bounds__(CS_THREADS) void k_chain_sdc(const int32_t* __restr
 		if(l < nL && (tid & 7) == 0) sums[l] = s;
 	}
 	__syncthreads();
-	chain_hand_over<CS_THREADS>(sums, nL, part, smemD, [&](int l) { return tblCol[gBase[l]]; }, out, nCols, done, nnz);
+	chain_hand_over<CS_THREADS>(sums, nL, part, smemD, [&](int l) { return tblCol[gBase[l]]; }, out, nCols, done, nnz, hostOut, hostCount);
 }
 
 // The row lists of the block's listed groups (whole-block plan), built once.
@@ -600,7 +601,7 @@ int prepare_chain_sdc(cla_block* b) {
 }
 
 // Returns 1 when the block is not eligible (the chain then runs as two products), 0 when the chain has been queued.
-int launch_chain_sdc(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz) {
+int launch_chain_sdc(cla_block* b, const double* dV, const double* dW, int ctype, double* dOut, unsigned long long* dNnz, ChainHost& host) {
 	unsigned grid = 0;
 	size_t lds = 0;
 	if(chain_sdc_shape(b, grid, lds)) return 1;
@@ -617,7 +618,7 @@ int launch_chain_sdc(cla_block* b, const double* dV, const double* dW, int ctype
 		CLA_HIP(allow_full_lds((const void*) kernel));
 		hipLaunchKernelGGL(kernel, dim3(grid), dim3(CS_THREADS), lds, b->stream, (const int32_t*) meta, b->rowsTbl, dBase, nL, (const uint2*) (meta + b->rowsOff[0]),
 			(const uint32_t*) (meta + b->rowsOff[1]), (const uint32_t*) b->dRowsData, (const double*) b->dAllDict, (const int32_t*) (meta + b->rowsColOff), dV, dW,
-			ctype == 2 ? 1 : 0, b->nRows, (int) ((b->nRows + RW_Q - 1) / RW_Q), b->dChain, dOut, b->nCols, b->lmm_ticket(), dNnz);
+			ctype == 2 ? 1 : 0, b->nRows, (int) ((b->nRows + RW_Q - 1) / RW_Q), b->dChain, dOut, b->nCols, b->lmm_ticket(), dNnz, host.out, host.count);
 		return 0;
 	};
 	if((rc = ctype != 0 ? go(k_chain_sdc<true>) : go(k_chain_sdc<false>))) return rc;
