@@ -548,6 +548,10 @@ int rmm_digits_plan(cla_block* b, int q, int n0) {
 	for(const HostGroup& H : b->groups) K += H.d.nColG;
 	if(b->opt.rmmDigits == 1 && !rd_pays(b, K, std::min(64, q - n0))) return 1;
 	if(b->rdPlan == nullptr) {
+		// (a block prepared for other widths, which the rule may leave to fp64: a capture refuses the plan's allocation)
+		hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+		CLA_HIP(hipStreamIsCapturing(b->stream, &capturing));
+		if(capturing != hipStreamCaptureStatusNone) return 1;
 		std::unique_ptr<RdPlan> plan(new RdPlan()); // (the block's only when it is complete)
 		const int rc = rd_build_plan(b, *plan);
 		if(rc < 0) {

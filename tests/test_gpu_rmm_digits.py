@@ -1,8 +1,11 @@
 """X %*% B of byte-code blocks on the integer matrix cores (k_rmm_mfma_i8, option rmm_digits): the edges of its tiles, steps and passes, and the
 rows and right-hand sides that its digits do not suit, which the fp64 kernel computes."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from devmem import DevBuf, hip
 from test_gpu_gram_tiles import columns
 
 pytestmark = pytest.mark.gpu
@@ -119,3 +122,46 @@ def test_values_that_digits_do_not_suit(cla, ora, kind, q):
     D = ora.np_decompress(specs, n_rows, n_cols)
     rows = np.r_[0:3000] if small is None else np.r_[0:1000, np.flatnonzero(small)[:1000]]
     check(out, D, B, rows)
+
+
+def test_capture_without_a_plan(cla, ora):
+    """A block prepared without the digits' plan can be captured all the same (in fp64: a capture refuses the plan's allocation); eager calls
+    between the replays take the digits."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(11)
+    n_rows, n_cols, q = 1500, 80, 32
+    specs = columns(synth, rng, n_rows, n_cols, 30, np.uint8, 1)
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    blk = cla.build_block(n_rows, n_cols, specs)
+    h, stream = hip(), C.c_void_p()
+    ok = lambda rc: (_ for _ in ()).throw(AssertionError(rc)) if rc else None
+    ok(h.hipStreamCreate(C.byref(stream)))
+    blk.set_stream(stream.value)
+    blk.set_option("rmm_digits", 0)
+    blk.prepare(rmm_cols=q)
+    blk.set_option("rmm_digits", 2)
+    dB, dO = DevBuf.from_numpy(np.zeros((n_cols, q))), DevBuf(n_rows * q * 8)
+    graph, run = C.c_void_p(), C.c_void_p()
+    ok(h.hipStreamBeginCapture(stream, 0))
+    blk.rmm_dev_async(dB.ptr, q, dO.ptr)
+    ok(h.hipStreamEndCapture(stream, C.byref(graph)))
+    names = [k["name"] for k in blk.stats()["kernels"]]
+    assert "k_rmm_mfma" in names and "k_rmm_mfma_i8" not in names, names
+    ok(h.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)))
+    for _ in range(3):
+        B = rng.standard_normal((n_cols, q))
+        ok(h.hipMemcpy(dB.ptr, B.ctypes.data_as(C.c_void_p), B.nbytes, 1))
+        dO.zero()
+        ok(h.hipDeviceSynchronize())
+        ok(h.hipGraphLaunch(run, stream))
+        ok(h.hipStreamSynchronize(stream))
+        got = dO.to_numpy(n_rows * q).reshape(n_rows, q)
+        assert blk.nnz() == np.count_nonzero(got)
+        check(got, D, B)
+        out, _ = blk.rmm(B)
+        assert "k_rmm_mfma_i8" in [k["name"] for k in blk.stats()["kernels"]]
+        check(out, D, B)
+    ok(h.hipGraphExecDestroy(run))
+    ok(h.hipGraphDestroy(graph))
+    blk.close()
+    ok(h.hipStreamDestroy(stream))
