@@ -412,11 +412,9 @@ __global__ __launch_bounds__(LT_THREADS) void k_take_block(const LmmTake A) {
 	if(!lastS) return;
 	if(tid > 0 && tid < NNZ_WAYS) A.nnz[tid * NNZ_STEP] = 0;
 	clear_tickets(A.done);
-	if(anew) { // (all blocks have taken a ticket: nobody reads these any more)
+	if(anew) // (all blocks have taken a ticket: nobody reads these any more)
 		for(int i = tid; i < n + A.p; i += LT_THREADS) A.anew[i] = 0.0;
-		if(tid == 0) *A.bad = 0;
-	}
-	if(tid == 0) *A.count = 0;
+	if(tid == 0) *A.bad = *A.count = 0; // (a report that no column or constant of this block heeds, too: the word is a sum of a call of more rows)
 }
 
 // (a kernel, not hipMemsetAsync: a memset node of a captured graph has given wrong results on its replays)
