@@ -1563,13 +1563,16 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 	double* const ws = b->dLmmWs;
 	unsigned long long* const dBad = (unsigned long long*) (ws + nWs - 2);
 	// Zeros: k_take_block leaves the workspace as it has found it (a fill in front of every call: mixed rows by 4, 294,957 19.2 -> 17.7 us, by 6 5,000,011 94 -> 92).
-	const bool dirty = !b->lmmWsClean;
-	if(dirty && (rc = launch_zero(b, ws, b->lmmWsCap))) return rc;
+	// A captured call has its fill all the same: what the workspace holds when it is replayed, behind a call that failed between its kernels, is not known now.
+	hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+	CLA_HIP(hipStreamIsCapturing(b->stream, &capturing));
+	const bool recorded = capturing != hipStreamCaptureStatusNone, clean = b->lmmWsClean;
+	if((recorded || !clean) && (rc = launch_zero(b, ws, b->lmmWsCap))) return rc;
 	b->lmmWsClean = false; // (until what clears it is queued)
 	for(int p0 = 0; p0 < p; p0 += 16) // 16 rows of Y per pass over the block
 		if((rc = launch_lmm_decode(b, dY + (size_t) p0 * b->nRows, std::min(16, p - p0), ws + (size_t) p0 * b->nCols, dBad))) {
 			if(rc == 1 && p0 == 0) { // (nothing queued yet)
-				b->lmmWsClean = !dirty;
+				b->lmmWsClean = clean;
 				return launch_lmm_chunked(b, dY, p, dOut, dNnz);
 			}
 			if(p0 > 0) clear_stats(b);
@@ -1577,9 +1580,7 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 		}
 	if((rc = launch_lmm_take(b, dY, p, ws, dOut, dNnz))) return rc;
 	CLA_HIP(hipGetLastError());
-	hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone; // (a fill that is only recorded has cleared nothing yet)
-	if(dirty) CLA_HIP(hipStreamIsCapturing(b->stream, &capturing));
-	b->lmmWsClean = capturing == hipStreamCaptureStatusNone;
+	b->lmmWsClean = recorded ? clean : true; // (what is only recorded has cleared nothing yet)
 	return 0;
 }
 

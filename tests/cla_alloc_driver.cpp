@@ -5,6 +5,9 @@
  * of the failed chain must not show in it). The same for cla_tsmm of a block of two wide groups, whose kernels add into an
  * accumulator that the block keeps: the next t(X) %*% X must hold nothing of the failed one.
  *
+ * Its own hipLaunchKernel fails the k-th launch of a Y %*% X on decoded rows, whose workspace is left at zero by a call: neither a
+ * replay of a call captured before nor the next call may hold anything of the failed one.
+ *
  * Prints "ALLOC-DRIVER OK" at the end; exit code 0 only then.
  */
 #include <dlfcn.h>
@@ -35,6 +38,34 @@ __attribute__((noinline)) void* operator new(size_t n) {
 }
 __attribute__((noinline)) void operator delete(void* p) noexcept { free(p); }
 __attribute__((noinline)) void operator delete(void* p, size_t) noexcept { free(p); }
+
+static thread_local long launchLeft = -1; // launches of the library until one fails; -1: none does
+static thread_local int launchError = 0;
+static thread_local bool launchFailed = false;
+struct Dim3 { uint32_t x, y, z; };
+
+extern "C" int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args, size_t lds, void* stream) {
+	static const auto next = (int (*)(const void*, Dim3, Dim3, void**, size_t, void*)) dlsym(RTLD_NEXT, "hipLaunchKernel");
+	if(launchLeft >= 0 && launchLeft-- == 0) {
+		launchFailed = true;
+		return launchError = 2;
+	}
+	return next(f, grid, block, args, lds, stream);
+}
+extern "C" int hipGetLastError() {
+	static const auto next = (int (*)()) dlsym(RTLD_NEXT, "hipGetLastError");
+	const int injected = launchError;
+	launchError = 0;
+	return injected ? injected : next();
+}
+
+// The rest of the HIP runtime that libclahip.so has loaded
+template <typename... A> static int hip(const char* name, A... a) {
+	const auto f = (int (*)(A...)) dlsym(RTLD_DEFAULT, name);
+	const int rc = f ? f(a...) : -1;
+	if(rc) printf("%s: error %d\n", name, rc);
+	return rc;
+}
 
 static const int64_t N = 1031;
 enum { COLS = 3 };
@@ -117,6 +148,65 @@ static int gram_failures(int& thrown) {
 	}
 }
 
+// Y %*% X on decoded rows with each launch of the library failing in turn, a replay of a captured call and a plain call behind each.
+static int left_failures(int& thrown) {
+	enum { M = 4, P = 2 };
+	std::vector<double> X((size_t) N * M), Y((size_t) P * N), want(P * M, 0.0), got(P * M);
+	std::vector<double> dict(2 * 300), dense((size_t) N * 2);
+	std::vector<uint16_t> codes((size_t) N);
+	for(int i = 0; i < 300; i++) { dict[2 * i] = i % 7; dict[2 * i + 1] = 3 - i % 5; }
+	for(int64_t r = 0; r < N; r++) {
+		codes[(size_t) r] = (uint16_t) (r * 7 % 300);
+		for(int c = 0; c < 2; c++) {
+			X[(size_t) r * M + c] = dict[2 * codes[(size_t) r] + c];
+			X[(size_t) r * M + 2 + c] = dense[(size_t) r * 2 + c] = (double) ((r + c) % 9);
+		}
+		for(int i = 0; i < P; i++) Y[(size_t) i * N + r] = (double) ((r + 3 * i) % 11) - 4;
+		for(int i = 0; i < P; i++)
+			for(int c = 0; c < M; c++) want[(size_t) i * M + c] += Y[(size_t) i * N + r] * X[(size_t) r * M + c];
+	}
+	const int32_t c01[2] = {0, 1}, c23[2] = {2, 3};
+	cla_handle h = cla_block_create(N, M);
+	void *dY = nullptr, *dOut = nullptr, *stream = nullptr, *graph = nullptr, *exec = nullptr;
+	const size_t outBytes = sizeof(double) * P * M;
+	if(!h || cla_block_add_ddc(h, c01, 2, dict.data(), 300, codes.data(), 2) < 0 || cla_block_add_uncompressed(h, c23, 2, dense.data()) < 0 || cla_block_finalize(h) < 0 ||
+		hip("hipMalloc", &dY, Y.size() * 8) || hip("hipMalloc", &dOut, outBytes) || hip("hipMemcpy", dY, (const void*) Y.data(), Y.size() * 8, 1) || hip("hipStreamCreate", &stream) ||
+		cla_block_set_stream(h, stream) < 0 || cla_block_prepare(h, CLA_PRODUCT_LMM, 0, P) < 0 || hip("hipStreamBeginCapture", stream, 0) ||
+		cla_lmm_dev_async(h, (const double*) dY, P, (double*) dOut) < 0 || hip("hipStreamEndCapture", stream, &graph) ||
+		hip("hipGraphInstantiate", &exec, graph, (void*) nullptr, (char*) nullptr, (size_t) 0)) {
+		printf("left: %s\n", cla_last_error());
+		return 1;
+	}
+	char stats[2048] = "";
+	(void) cla_stats(h, stats, sizeof(stats));
+	if(!strstr(stats, "k_take_block")) { printf("left: another kernel: %s\n", stats); return 1; }
+	int fails = 0;
+	auto right = [&](const char* what, long k) { // (whole numbers: exact)
+		if(hip("hipStreamSynchronize", stream) || hip("hipMemcpy", (void*) got.data(), (const void*) dOut, outBytes, 2) || got != want) {
+			printf("left, launch %ld: %s is wrong\n", k, what);
+			fails++;
+		}
+	};
+	for(long k = 0;; k++) {
+		launchFailed = false;
+		launchLeft = k;
+		const int64_t rc = cla_lmm_dev(h, (const double*) dY, P, (double*) dOut);
+		launchLeft = -1;
+		if(launchFailed == (rc >= 0)) { printf("left, launch %ld: %s\n", k, rc < 0 ? cla_last_error() : "no error"); fails++; }
+		if(launchFailed) thrown++;
+		for(int i = 0; i < 2; i++) {
+			if(hip("hipGraphLaunch", exec, stream)) return fails + 1;
+			right("a replay", k);
+		}
+		if(cla_lmm_dev(h, (const double*) dY, P, (double*) dOut) < 0) { printf("left: %s\n", cla_last_error()); fails++; }
+		right("the next call", k);
+		if(!launchFailed) break;
+	}
+	cla_block_free(h);
+	if(hip("hipGraphExecDestroy", exec) || hip("hipGraphDestroy", graph) || hip("hipStreamDestroy", stream) || hip("hipFree", dY) || hip("hipFree", dOut)) fails++;
+	return fails;
+}
+
 int main() {
 	if(cla_init(0) < 0) { fprintf(stderr, "cla_init: %s\n", cla_last_error()); return 2; }
 	int fails = 0, thrown = 0;
@@ -150,8 +240,10 @@ int main() {
 			}
 	int gramThrown = 0;
 	fails += gram_failures(gramThrown);
-	printf("%d + %d failed allocations\n", thrown, gramThrown);
-	if(fails || thrown < 4 || gramThrown < 2) { printf("FAIL\n"); return 1; }
+	int leftThrown = 0;
+	fails += left_failures(leftThrown);
+	printf("%d + %d failed allocations, %d failed launches\n", thrown, gramThrown, leftThrown);
+	if(fails || thrown < 4 || gramThrown < 2 || leftThrown < 2) { printf("FAIL\n"); return 1; }
 	printf("ALLOC-DRIVER OK\n");
 	return 0;
 }
