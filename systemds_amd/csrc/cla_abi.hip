@@ -342,6 +342,7 @@ void cla_block_free(cla_handle b) {
 	if(b->dTblOff) (void) hipFree(b->dTblOff);
 	if(b->dTables) (void) hipFree(b->dTables);
 	if(b->dLmmWs) (void) hipFree(b->dLmmWs);
+	for(double* p : b->lmmWsOld) (void) hipFree(p);
 	if(b->dStageIn) (void) hipFree(b->dStageIn);
 	if(b->dStageOut) (void) hipFree(b->dStageOut);
 	if(b->dScratch) (void) hipFree(b->dScratch);
@@ -1554,20 +1555,28 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 	// in the output staging buffer, which may be the caller's dOut.
 	const size_t nWs = 2 * n + (size_t) p + 2;
 	int rc = 0;
-	if(nWs > b->lmmWsCap) {
-		if(b->dLmmWs) CLA_HIP(hipFree(b->dLmmWs));
-		b->dLmmWs = nullptr; b->lmmWsCap = 0; b->lmmWsClean = false;
-		CLA_HIP(hipMalloc((void**) &b->dLmmWs, nWs * sizeof(double)));
-		b->lmmWsCap = nWs;
+	hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+	CLA_HIP(hipStreamIsCapturing(b->stream, &capturing));
+	const bool recorded = capturing != hipStreamCaptureStatusNone;
+	// (a workspace that is too small stays until the block goes: calls captured with it may be replayed, and each is at least twice the one before)
+	const bool room = nWs <= b->lmmWsCap, grow = !room && !recorded;
+	if(grow) {
+		const size_t cap = std::max(nWs, 2 * b->lmmWsCap);
+		double* p2 = nullptr;
+		b->lmmWsOld.reserve(b->lmmWsOld.size() + 1);
+		CLA_HIP(hipMalloc((void**) &p2, cap * sizeof(double)));
+		if(b->dLmmWs) b->lmmWsOld.push_back(b->dLmmWs);
+		b->dLmmWs = p2; b->lmmWsCap = cap; b->lmmWsClean = false;
 	}
-	double* const ws = b->dLmmWs;
+	// Captured with more rows of Y than any call before: a capture refuses an allocation, the tables of earlier products may have the room.
+	const bool own = room || grow;
+	if(!own && (rc = ensure_tables(b, nWs))) return rc;
+	double* const ws = own ? b->dLmmWs : b->dTables;
 	unsigned long long* const dBad = (unsigned long long*) (ws + nWs - 2);
 	// Zeros: k_take_block leaves the workspace as it has found it (a fill in front of every call: mixed rows by 4, 294,957 19.2 -> 17.7 us, by 6 5,000,011 94 -> 92).
 	// A captured call has its fill all the same: what the workspace holds when it is replayed, behind a call that failed between its kernels, is not known now.
-	hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-	CLA_HIP(hipStreamIsCapturing(b->stream, &capturing));
-	const bool recorded = capturing != hipStreamCaptureStatusNone, clean = b->lmmWsClean;
-	if((recorded || !clean) && (rc = launch_zero(b, ws, b->lmmWsCap))) return rc;
+	const bool clean = b->lmmWsClean;
+	if((recorded || !clean) && (rc = launch_zero(b, ws, own ? b->lmmWsCap : nWs))) return rc;
 	b->lmmWsClean = false; // (until what clears it is queued)
 	for(int p0 = 0; p0 < p; p0 += 16) // 16 rows of Y per pass over the block
 		if((rc = launch_lmm_decode(b, dY + (size_t) p0 * b->nRows, std::min(16, p - p0), ws + (size_t) p0 * b->nCols, dBad))) {
