@@ -355,6 +355,8 @@ void cla_block_free(cla_handle b) {
 	if(b->dRowsMeta) (void) hipFree(b->dRowsMeta);
 	if(b->dMfPlan) (void) hipFree(b->dMfPlan);
 	dec_plans_drop(b);
+	gd_plan_drop(b);
+	rd_plan_drop(b);
 	if(b->dRowsData) (void) hipFree(b->dRowsData);
 	if(b->dDictPad) (void) hipFree(b->dDictPad);
 	if(b->dCountsAll) (void) hipFree(b->dCountsAll);
@@ -760,7 +762,7 @@ int cla_block_set_option(cla_handle b, const char* key, int32_t value) {
 		if(strcmp(e.name, key) == 0) {
 			if(value < e.lo || value > e.hi) { set_error("set_option: %s takes %d..%d (got %d)", key, e.lo, e.hi, value); return -CLA_ERR_INVALID; }
 			b->opt.*(e.field) = value;
-			dec_plans_drop(b); // plans kept with the block were made under the old options
+			dec_plans_drop(b); // plans kept with the block were made under the old options (those of digits depend on none)
 			return 0;
 		}
 	set_error("set_option: unknown option '%s'", key);
@@ -819,6 +821,8 @@ static int drop_derived(cla_block* b) {
 	free_lmm_subs(b);
 	b->lmmSubWidth = 0;
 	dec_plans_drop(b);
+	gd_plan_drop(b);
+	rd_plan_drop(b);
 	auto drop = [](auto*& p) { if(p) { (void) hipFree((void*) p); p = nullptr; } };
 	drop(b->dSdcPlan); drop(b->dSdcDesc); drop(b->dSdcPacked);
 	b->sdcPlanGroup = -2; b->sdcPackFailed = false;

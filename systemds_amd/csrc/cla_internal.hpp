@@ -221,8 +221,8 @@ struct cla_block {
 	cla::DirPlan* dirPlan = nullptr;     // plan of k_rmm_direct (dropped with the decode plans)
 	cla::GdrPlan* gdrPlan = nullptr;     // plan of k_tsmm_direct (likewise)
 	cla::GtPlan* gtPlan = nullptr;       // plan of k_gram_tiles (likewise)
-	cla::GdPlan* gdPlan = nullptr;       // plan of k_gram_tiles_i8 (likewise)
-	cla::RdPlan* rdPlan = nullptr;       // plan of k_rmm_mfma_i8 (likewise)
+	cla::GdPlan* gdPlan = nullptr;       // plan of k_gram_tiles_i8 (kept until drop_derived: captured calls read it, whatever options are set since)
+	cla::RdPlan* rdPlan = nullptr;       // plan of k_rmm_mfma_i8 (likewise kept)
 	void* dMfPlan = nullptr;         // matrix-core right multiply (k_rmm_mfma.hip): slab descriptors, column info, code streams, B row list
 	int mfState = 0;                 // 0 not planned yet, 1 ready, -1 not eligible
 	int mfNSlabs = 0, mfNColsAll = 0, mfWidth = 1, mfMaxKc = 0, mfNRowCol = 0, mfMaxDict = 0;

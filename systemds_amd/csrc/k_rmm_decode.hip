@@ -990,8 +990,6 @@ void dec_plans_drop(cla_block* b) {
 	dir_plan_drop(b);
 	gdr_plan_drop(b);
 	gt_plan_drop(b);
-	gd_plan_drop(b);
-	rd_plan_drop(b);
 	if(b->decPlans == nullptr) return;
 	for(auto& e : b->decPlans->entries)
 		if(e.dImg) { (void) hipFree(e.dImg); b->derivedBytes -= e.bytes; }

@@ -165,3 +165,62 @@ def test_capture_without_a_plan(cla, ora):
     ok(h.hipGraphDestroy(graph))
     blk.close()
     ok(h.hipStreamDestroy(stream))
+
+
+def test_replays_behind_an_option(cla, ora):
+    """Captured products on digits, replayed behind options set since (unrelated ones, and those that send the eager calls between the
+    replays elsewhere): what they read and write stays with the block."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(12)
+    n_rows, n_cols, q = 21_000, 80, 32
+    specs = columns(synth, rng, n_rows, n_cols, 200, np.uint8, 1)
+    for s in specs:
+        s.dict = rng.uniform(-1, 1, s.dict.shape)
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    h, stream = hip(), C.c_void_p()
+    ok = lambda rc: (_ for _ in ()).throw(AssertionError(rc)) if rc else None
+    ok(h.hipStreamCreate(C.byref(stream)))
+    blk = cla.build_block(n_rows, n_cols, specs)
+    blk.set_stream(stream.value)
+    for key in ("rmm_digits", "tsmm_digits"):
+        blk.set_option(key, 2)
+    blk.prepare(rmm_cols=q, tsmm=True)
+    dB, dO, dG = DevBuf.from_numpy(np.zeros((n_cols, q))), DevBuf(n_rows * q * 8), DevBuf(n_cols * n_cols * 8)
+    runs = []
+    for call in (lambda: blk.rmm_dev_async(dB.ptr, q, dO.ptr), lambda: blk.tsmm_dev_async(dG.ptr)):
+        graph, run = C.c_void_p(), C.c_void_p()
+        ok(h.hipStreamBeginCapture(stream, 0))
+        call()
+        ok(h.hipStreamEndCapture(stream, C.byref(graph)))
+        ok(h.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)))
+        runs.append((graph, run, {k["name"]: k["lds"] for k in blk.stats()["kernels"]}))
+    assert "k_rmm_mfma_i8" in runs[0][2]
+    gram = blk.tsmm()[0]
+    for options in ((("sdc_rows", 1),), (("rmm_digits", 0), ("tsmm_digits", 0)), (("rmm_digits", 2), ("tsmm_digits", 1))):
+        for key, value in options:
+            blk.set_option(key, value)
+        others = [DevBuf(1 << 20) for _ in range(8)]  # (freed memory would be given out again)
+        for o in others:
+            o.zero()
+        B = rng.standard_normal((n_cols, q))
+        eager, _ = blk.rmm(B)
+        out, _ = blk.tsmm()
+        if options[-1] == ("tsmm_digits", 0):
+            assert blk.stats()["kernels"][0]["lds"] != runs[1][2]["k_gram_tiles"]  # (the captured one is the digits' kernel)
+        ok(h.hipMemcpy(dB.ptr, B.ctypes.data_as(C.c_void_p), B.nbytes, 1))
+        dO.zero()
+        dG.zero()
+        ok(h.hipDeviceSynchronize())
+        for _, run, _ in runs:
+            ok(h.hipGraphLaunch(run, stream))
+        ok(h.hipStreamSynchronize(stream))
+        got = dO.to_numpy(n_rows * q).reshape(n_rows, q)
+        check(got, D, B)
+        check(eager, D, B)
+        assert np.array_equal(dG.to_numpy(n_cols * n_cols).reshape(n_cols, n_cols), gram)  # (the same sums in every call)
+        assert np.allclose(out, gram, rtol=0, atol=2 * n_rows ** 2 * 2.0 ** -53)  # (as many roundings of sums below n_rows)
+    for graph, run, _ in runs:
+        ok(h.hipGraphExecDestroy(run))
+        ok(h.hipGraphDestroy(graph))
+    blk.close()
+    ok(h.hipStreamDestroy(stream))
