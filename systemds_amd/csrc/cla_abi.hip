@@ -82,6 +82,13 @@ int ensure_tables(cla_block* b, size_t nDoubles) {
 	return 0;
 }
 
+bool no_room(void** p, size_t bytes) {
+	if(hipMalloc(p, bytes) == hipSuccess) return false;
+	*p = nullptr;
+	(void) hipGetLastError();
+	return true;
+}
+
 int ensure_chain(cla_block* b, size_t nDoubles) {
 	if(nDoubles <= b->chainCap) return 0;
 	if(b->dChain) CLA_HIP(hipFree(b->dChain));

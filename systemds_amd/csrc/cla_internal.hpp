@@ -369,6 +369,7 @@ struct Prof {
 void clear_stats(cla_block* b);
 
 int ensure_tables(cla_block* b, size_t nDoubles);
+bool no_room(void** p, size_t bytes); // true: the device memory for a form that a product can do without was not to be had
 int ensure_chain(cla_block* b, size_t nDoubles);
 int ensure_dict_pad(cla_block* b); // padded dictionary image of byte-code blocks with one column per group (no-op otherwise)
 int ensure_scratch(cla_block* b, size_t bytes);

@@ -583,11 +583,12 @@ struct GdPlan {
 	const GdTile* tiles = nullptr;
 	int nCellTiles = 0, grid = 0;
 	size_t lds = 0;
+	~GdPlan() { if(dImg) (void) hipFree(dImg); }
 };
 
 void gd_plan_drop(cla_block* b) {
 	if(b->gdPlan == nullptr) return;
-	if(b->gdPlan->dImg) { (void) hipFree(b->gdPlan->dImg); b->derivedBytes -= b->gdPlan->bytes; }
+	b->derivedBytes -= b->gdPlan->bytes;
 	delete b->gdPlan;
 	b->gdPlan = nullptr;
 }
@@ -604,6 +605,7 @@ static bool gd_digits(double x, int8_t (&d)[GD_DIGITS]) {
 	return whole == scaled;
 }
 
+// 1: no room on the device for the plan
 static int gd_build_plan(cla_block* b, GdPlan& P) {
 	P.rc = 1;
 	const int n = b->nCols;
@@ -712,7 +714,7 @@ static int gd_build_plan(cla_block* b, GdPlan& P) {
 	std::memcpy(all.data() + oTiles, tiles.data(), tiles.size() * sizeof(GdTile));
 	std::memcpy(all.data() + oTabs, tabs.data(), tabs.size());
 	uint8_t* d = nullptr;
-	CLA_HIP(hipMalloc((void**) &d, oParts + partBytes * (chunks ? 1 + gd_sets(nf) : 1)));
+	if(no_room((void**) &d, oParts + partBytes * (chunks ? 1 + gd_sets(nf) : 1))) return 1;
 	P.dImg = d;
 	P.bytes = (int64_t) (oParts + partBytes * (chunks ? 1 + gd_sets(nf) : 1));
 	CLA_HIP(hipMemcpy(d, all.data(), all.size(), hipMemcpyHostToDevice));
@@ -728,7 +730,7 @@ static int gd_build_plan(cla_block* b, GdPlan& P) {
 	// sign would leave 2^-44 of the terms' sum; they are of either sign and differ from tuple to tuple.)
 	struct Tmp { void* p = nullptr; ~Tmp() { if(p) (void) hipFree(p); } } tmp;
 	const size_t magBytes = nMag * sizeof(unsigned long long);
-	CLA_HIP(hipMalloc(&tmp.p, magBytes + magTabs.size()));
+	if(no_room(&tmp.p, magBytes + magTabs.size())) return 1;
 	unsigned long long* dMag = (unsigned long long*) tmp.p;
 	uint8_t* dMagTabs = (uint8_t*) tmp.p + magBytes;
 	CLA_HIP(hipMemsetAsync(dMag, 0, magBytes, b->stream));
@@ -776,10 +778,14 @@ static bool gd_pays(const cla_block* b) {
 int gram_digits_plan(cla_block* b) {
 	if(b->opt.tsmmDigits == 0 || (b->opt.tsmmDigits == 1 && !gd_pays(b))) return 1;
 	if(b->gdPlan == nullptr) {
+		// (a capture refuses the plan's allocations and its wait: the fp64 kernel)
+		hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+		CLA_HIP(hipStreamIsCapturing(b->stream, &capturing));
+		if(capturing != hipStreamCaptureStatusNone) return 1;
 		std::unique_ptr<GdPlan> plan(new GdPlan()); // (the block's only when it is complete)
 		const int rc = gd_build_plan(b, *plan);
-		if(plan->dImg && (rc < 0 || plan->rc)) { (void) hipFree(plan->dImg); plan->dImg = nullptr; plan->bytes = 0; }
-		if(rc < 0) return rc;
+		if(rc) return rc;
+		if(plan->dImg && plan->rc) { (void) hipFree(plan->dImg); plan->dImg = nullptr; plan->bytes = 0; }
 		b->derivedBytes += plan->bytes;
 		b->gdPlan = plan.release();
 	}

@@ -454,15 +454,17 @@ struct RdPlan {
 	double* scale = nullptr;
 	int32_t *least = nullptr, *bad = nullptr;
 	int K = 0, S = 0, T = 0;
+	~RdPlan() { if(dImg) (void) hipFree(dImg); }
 };
 
 void rd_plan_drop(cla_block* b) {
 	if(b->rdPlan == nullptr) return;
-	if(b->rdPlan->dImg) { (void) hipFree(b->rdPlan->dImg); b->derivedBytes -= b->rdPlan->bytes; }
+	b->derivedBytes -= b->rdPlan->bytes;
 	delete b->rdPlan;
 	b->rdPlan = nullptr;
 }
 
+// 1: no room on the device for the plan
 static int rd_build_plan(cla_block* b, RdPlan& P) {
 	P.rc = 1;
 	if(b->dArena == nullptr || b->arenaWidth != 1 || b->dictNonFinite || b->nRows == 0) return 0;
@@ -513,7 +515,7 @@ static int rd_build_plan(cla_block* b, RdPlan& P) {
 	std::memcpy(all.data() + oUp, up.data(), up.size() * 8);
 	std::memcpy(all.data() + oTabs, tabs.data(), tabs.size());
 	uint8_t* d = nullptr;
-	CLA_HIP(hipMalloc((void**) &d, total));
+	if(no_room((void**) &d, total)) return 1;
 	P.dImg = d;
 	P.bytes = (int64_t) total;
 	CLA_HIP(hipMemcpy(d, all.data(), all.size(), hipMemcpyHostToDevice));
@@ -554,10 +556,7 @@ int rmm_digits_plan(cla_block* b, int q, int n0) {
 		if(capturing != hipStreamCaptureStatusNone) return 1;
 		std::unique_ptr<RdPlan> plan(new RdPlan()); // (the block's only when it is complete)
 		const int rc = rd_build_plan(b, *plan);
-		if(rc < 0) {
-			if(plan->dImg) (void) hipFree(plan->dImg);
-			return rc;
-		}
+		if(rc) return rc;
 		b->derivedBytes += plan->bytes;
 		b->rdPlan = plan.release();
 	}

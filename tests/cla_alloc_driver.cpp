@@ -8,6 +8,9 @@
  * Its own hipLaunchKernel fails the k-th launch of a Y %*% X on decoded rows, whose workspace is left at zero by a call: neither a
  * replay of a call captured before nor the next call may hold anything of the failed one.
  *
+ * Its own hipMalloc fails the k-th device allocation of a first X %*% B and t(X) %*% X of a byte-code block: the plans of the forms on digits
+ * are none that a call fails for.
+ *
  * Prints "ALLOC-DRIVER OK" at the end; exit code 0 only then.
  */
 #include <dlfcn.h>
@@ -42,6 +45,8 @@ __attribute__((noinline)) void operator delete(void* p, size_t) noexcept { free(
 static thread_local long launchLeft = -1; // launches of the library until one fails; -1: none does
 static thread_local int launchError = 0;
 static thread_local bool launchFailed = false;
+static thread_local long roomLeft = -1; // device allocations of the library until one fails; -1: none does
+static thread_local bool roomFailed = false;
 struct Dim3 { uint32_t x, y, z; };
 
 extern "C" int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args, size_t lds, void* stream) {
@@ -51,6 +56,14 @@ extern "C" int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args
 		return launchError = 2;
 	}
 	return next(f, grid, block, args, lds, stream);
+}
+extern "C" int hipMalloc(void** p, size_t bytes) {
+	static const auto next = (int (*)(void**, size_t)) dlsym(RTLD_NEXT, "hipMalloc");
+	if(roomLeft >= 0 && roomLeft-- == 0) {
+		roomFailed = true;
+		return 2;
+	}
+	return next(p, bytes);
 }
 extern "C" int hipGetLastError() {
 	static const auto next = (int (*)()) dlsym(RTLD_NEXT, "hipGetLastError");
@@ -207,6 +220,54 @@ static int left_failures(int& thrown) {
 	return fails;
 }
 
+// X %*% B and t(X) %*% X of 64 byte-code columns with each device allocation of the first call failing in turn: with digits as many calls fail as
+// without, and the results and the next call are right.
+static int room_failures(int& thrown) {
+	enum { M = 64, Q = 16, V = 5 };
+	std::vector<uint8_t> codes((size_t) N * M);
+	std::vector<double> dict(V), B((size_t) M * Q), X((size_t) N * M), want[2], got;
+	for(int i = 0; i < V; i++) dict[(size_t) i] = i - 2 + (i == 2 ? 3 : 0);
+	for(int64_t r = 0; r < N; r++)
+		for(int c = 0; c < M; c++) X[(size_t) r * M + c] = dict[codes[(size_t) c * N + r] = (uint8_t) ((r * (c + 3) + c) % V)];
+	for(int i = 0; i < M * Q; i++) B[(size_t) i] = i % 7 - 3;
+	want[0].assign((size_t) N * Q, 0.0);
+	want[1].assign(M * M, 0.0);
+	for(int64_t r = 0; r < N; r++)
+		for(int c = 0; c < M; c++) {
+			for(int j = 0; j < Q; j++) want[0][(size_t) r * Q + j] += X[(size_t) r * M + c] * B[(size_t) c * Q + j];
+			for(int j = 0; j < M; j++) want[1][(size_t) c * M + j] += X[(size_t) r * M + c] * X[(size_t) r * M + j];
+		}
+	int fails = 0;
+	for(int gram = 0; gram < 2; gram++) {
+		int failed[2] = {0, 0};
+		for(int digits = 0; digits < 2; digits++)
+			for(long k = 0;; k++) {
+				cla_handle h = cla_block_create(N, M);
+				bool ok = h != nullptr;
+				for(int32_t c = 0; c < M && ok; c++) ok = cla_block_add_ddc(h, &c, 1, dict.data(), V, codes.data() + (size_t) c * N, 1) >= 0;
+				if(!ok || cla_block_finalize(h) < 0 || cla_block_set_option(h, gram ? "tsmm_digits" : "rmm_digits", 2 * digits) < 0) { printf("room: %s\n", cla_last_error()); return fails + 1; }
+				got.assign(want[gram].size(), -1.0);
+				auto call = [&]() { return gram ? cla_tsmm(h, got.data()) : cla_rmm(h, B.data(), Q, got.data()); };
+				roomFailed = false;
+				roomLeft = k;
+				const int64_t rc = call();
+				roomLeft = -1;
+				if(roomFailed) thrown++;
+				failed[digits] += rc < 0;
+				if(rc >= 0 && got != want[gram]) { printf("room, allocation %ld, gram %d, digits %d: the result is wrong\n", k, gram, digits); fails++; }
+				got.assign(want[gram].size(), -1.0);
+				if(call() < 0 || got != want[gram]) { printf("room, allocation %ld, gram %d, digits %d: the next call is wrong\n", k, gram, digits); fails++; }
+				char stats[2048] = "";
+				(void) cla_stats(h, stats, sizeof(stats));
+				if(!gram && rc >= 0 && digits != (strstr(stats, "k_rmm_mfma_i8") != nullptr)) { printf("room, allocation %ld: the next call took another kernel: %s\n", k, stats); fails++; }
+				cla_block_free(h);
+				if(!roomFailed) break;
+			}
+		if(failed[0] != failed[1]) { printf("room, gram %d: %d failed calls without digits, %d with\n", gram, failed[0], failed[1]); fails++; }
+	}
+	return fails;
+}
+
 int main() {
 	if(cla_init(0) < 0) { fprintf(stderr, "cla_init: %s\n", cla_last_error()); return 2; }
 	int fails = 0, thrown = 0;
@@ -242,8 +303,10 @@ int main() {
 	fails += gram_failures(gramThrown);
 	int leftThrown = 0;
 	fails += left_failures(leftThrown);
-	printf("%d + %d failed allocations, %d failed launches\n", thrown, gramThrown, leftThrown);
-	if(fails || thrown < 4 || gramThrown < 2 || leftThrown < 2) { printf("FAIL\n"); return 1; }
+	int roomThrown = 0;
+	fails += room_failures(roomThrown);
+	printf("%d + %d failed allocations, %d failed launches, %d failed device allocations\n", thrown, gramThrown, leftThrown, roomThrown);
+	if(fails || thrown < 4 || gramThrown < 2 || leftThrown < 2 || roomThrown < 8) { printf("FAIL\n"); return 1; }
 	printf("ALLOC-DRIVER OK\n");
 	return 0;
 }
