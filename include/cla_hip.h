@@ -131,7 +131,9 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *                   integer matrix cores (rows whose outputs' terms are far below their columns' largest in fp64): 0 never (fp64), 1 where
  *                   it is the faster way, 2 at any number of rows and columns of B
  *   tsmm_digits     t(X) %*% X of all-DDC byte-code blocks of 17 to 112 columns as exact sums of products of 8-bit digits of the values on the
- *                   integer matrix cores: 0 never (fp64), 1 where it is the faster way, 2 wherever its errors suit the block
+ *                   integer matrix cores: 0 never (fp64), 1 where it is the faster way and its error no larger than fp64's on this block (decided once per
+ *                   block, from both results), 2 at any number of rows, wherever every cell's terms reach 2^-10 of the product of its columns'
+ *                   largest values on average (errors up to 2^-43 of their sum)
  *   tsmm_one_kernel 1 / 0: t(X) %*% X of a whole block of at most 64 columns (all-DDC: 128) on the decoded Gram kernels as the call's only
  *                   kernel (a few wide DDC groups: behind the kernel of the cells inside a group; its blocks add into an
  *                   accumulator per XCD kept with the block, 9 x nCols x nCols doubles; the last block

@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <mutex>
 #include <atomic>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -325,7 +326,7 @@ int launch_tsmm_self(cla_block* b, double* out, double* colSum, const double* co
 int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz = nullptr, bool ownByCounts = false);
 int gram_tiles_behind_decode(const cla_block* b);
 void gt_plan_drop(cla_block* b);
-int gram_digits_plan(cla_block* b);
+int gram_digits_plan(cla_block* b, bool across, const std::function<int(double*)>& fp64);
 int launch_gram_digits(cla_block* b, double* acc, double* dOut, unsigned long long* dNnz, int skipOwn, int clearAcc);
 void gd_plan_drop(cla_block* b);
 int rmm_digits_plan(cla_block* b, int q, int n0);

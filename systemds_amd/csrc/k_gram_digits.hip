@@ -3,11 +3,10 @@
 // A column's values (dictionary + constant) are scaled by a power of two to |x| < 1 and rounded to X = x 2^55, a whole number of seven signed
 // base-256 digits. A row's lookup brings all seven (8 bytes, like the fp64 value), the products of digits i + j <= 6 are
 // summed as 32-bit integers, exactly, one sum per weight i + j, and at the end or every 18,688 rows the seven sums are joined in fp64. So
-// a cell's error is that of the rounded values (2^-56 of the column's largest) and of the products left out (2^-56 of both
-// columns' largest), not that of chains of fp64 additions. Rms over cells of the error divided by the sum of the terms' magnitudes, against exact
-// counts times products in long double, 256 normal values (k_gram_tiles): 2,000,003 x 100 5.3e-17 (1.5e-15), 200,003 x 100 3.9e-17 (1.7e-16),
-// 10,007 x 100 4.0e-17 (4.8e-17), 10,000,001 x 50 of 40 values 6.8e-17 (1.2e-14). It is absolute, in parts of the columns' largest
-// values; gd_build_plan says which blocks that suits. The same sums in every call: no atomic adds.
+// a cell's error is that of the rounded values (2^-56 of the column's largest) and of the products left out (six of up to 2^-56 of both columns'
+// largest), not that of chains of fp64 additions. It is absolute, in parts of the columns' largest values; gd_build_plan and gd_judge say which blocks
+// that suits. Rms over cells of the error divided by the sum of the terms' magnitudes, against exact counts times products in long double, 256 normal
+// values, Zipf(1.1) codes (k_gram_tiles): 2,000,003 x 100 3.5e-17 (1.2e-15); more beside gd_judge. The same sums in every call: no atomic adds.
 //
 // A workgroup of 8 waves, one per CU, takes a contiguous share of the rows in tiles of 64 rows per set of waves. Decoding is dealt by (16 columns, 64
 // rows): lane (k, c) looks up 16 consecutive codes of column c (in LDS where the column block's tables fit beside the tile, else in global
@@ -16,8 +15,8 @@
 // dealt to the waves so that a wave's pairs share few blocks (its reads) and the four SIMDs have the same work (gd_role).
 //
 // Why integers: 28 products of 16 cycles per 64 rows and pair of column blocks stand against 16 fp64 steps of 64 (v_mfma_f64_16x16x4), and,
-// unlike those, leave the SIMD's vector unit to the other wave. 2,000,003 x 100 435 -> 272 us (of 40 values, all tables in LDS, 235), 200,003 x 100
-// 97 -> 52, 10,007 x 100 40 -> 25, 2,000,003 x 64 209 -> 119, x 40 121 -> 90, x 20 65 -> 53.
+// unlike those, leave the SIMD's vector unit to the other wave. 2,000,003 x 100 441 -> 289 us (of 40 values, all tables in LDS, 235 without the join), 200,003 x 100
+// 97 -> 52, 2,000,003 x 64 209 -> 119, x 40 121 -> 90, x 20 65 -> 53.
 // Bound: the integer matrix pipe (2,400 cycles per 64 rows of 100 columns at 8.5 ns per 16: the clock drops under it; two buffers for the tile, or the lookups
 // elsewhere in it, change nothing) and, where tables are in global memory, the vector memory path: a lookup of 64 lanes takes it 57 cycles.
 #include "../../include/cla_hip.h"
@@ -26,6 +25,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <memory>
 
 namespace cla {
@@ -33,7 +33,7 @@ namespace cla {
 constexpr int GD_THREADS = 512, GD_DIGITS = 7;
 constexpr int GD_BITS = 55;             // X = x 2^GD_BITS, |x| < 127.5 / 128: the first digit fits
 constexpr int GD_CHUNK = 18688;         // rows between two joins: a weight's sum grows by at most 7 2^14 a row
-constexpr int GD_MAG = 128;             // magnitudes of the rule below in 1 / GD_MAG
+constexpr int GD_MAG = 128;             // magnitudes of the rules below in 1 / GD_MAG
 typedef int i32x4_gd __attribute__((ext_vector_type(4)));
 
 // a decoded column
@@ -523,55 +523,71 @@ __global__ __launch_bounds__(GJ_THREADS) void k_gram_join(const GdTile* __restri
 
 // ---- which blocks
 
-// mags[16 NCB x 16 NCB] += sums over the rows of the products of the columns' magnitudes (whole 1 / GD_MAG of the largest), for
-// the pairs of column blocks p <= q. A wave takes 64 rows at a time, all column blocks of them.
-template <int NCB>
-__global__ __launch_bounds__(GD_THREADS, 2) void k_gram_magnitudes(const uint8_t* __restrict__ arena, size_t arenaStride, const GdCol* __restrict__ cols,
-	int places, const uint8_t* __restrict__ magTabs, int64_t nRows, unsigned long long* __restrict__ mags) {
-	__shared__ uint8_t tab[NCB * 16 * 256];
-	constexpr int T = NCB * (NCB + 1) / 2;
+// For pairs of column blocks p <= q: left += the sums over the rows of the digit products of weight 7, the largest that the kernel above leaves out (the rounding of the
+// values is among them, as an eighth digit), mags += those of the products of the magnitudes (of the first digits, 1 / GD_MAG of the largest value). 16 NCB cells a
+// row of either. A workgroup takes a pair of column blocks, a wave 64 rows at a time. (Once per block: 2,000,003 x 100 1.3 ms, and where gd_judge needs it a call of either kernel.)
+constexpr int GC_UNITS = 240; // 64 rows each, between two flushes: a sum grows by at most 8 2^14 a row
+constexpr int GC_TAB = 16 * 256 * 8, GC_LDS = 2 * GC_TAB;
+__global__ __launch_bounds__(GD_THREADS, 2) void k_gram_left(const uint8_t* __restrict__ arena, size_t arenaStride, const GdCol* __restrict__ cols, int places, int ncb,
+	const uint8_t* __restrict__ digitTabs, int64_t nRows, unsigned long long* __restrict__ left, unsigned long long* __restrict__ mags) {
+	extern __shared__ __attribute__((aligned(16))) uint8_t gd_smem[]; // digits of block p, of q
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, k = lane >> 4;
-	for(int i = tid; i < NCB * 16 * 256 / 4; i += GD_THREADS) ((uint32_t*) tab)[i] = ((const uint32_t*) magTabs)[i];
-	__syncthreads();
-	i32x4_gd acc[T];
-#pragma unroll
-	for(int t = 0; t < T; t++) acc[t] = i32x4_gd{0, 0, 0, 0};
-	const int64_t nUnits = (nRows + 63) / 64;
-	for(int64_t u = (int64_t) blockIdx.x * 8 + wave; u < nUnits; u += (int64_t) gridDim.x * 8) {
-		i32x4_gd x[NCB];
-		const int64_t row = u * 64 + 16 * k;
-#pragma unroll
-		for(int b = 0; b < NCB; b++) {
-			const u32x4 codes = *(const u32x4*) (arena + (size_t) cols[min(b * 16 + c, places - 1)].stream * arenaStride + row); // (behind them: zeros, whatever the code)
-			const uint8_t* t = tab + (b * 16 + c) * 256;
-#pragma unroll
-			for(int w = 0; w < 4; w++) {
-				uint32_t v = 0;
-#pragma unroll
-				for(int i = 0; i < 4; i++) {
-					const uint32_t m = t[(codes[w] >> (8 * i)) & 0xffu];
-					v |= (row + 4 * w + i < nRows ? m : 0u) << (8 * i);
-				}
-				x[b][w] = (int) v;
-			}
-			__builtin_amdgcn_sched_barrier(0); // (a column block's lookups at a time: all of them together do not fit the registers)
-		}
-		int t = 0;
-#pragma unroll
-		for(int p = 0; p < NCB; p++)
-#pragma unroll
-			for(int q = p; q < NCB; q++, t++) acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[p], x[q], acc[t], 0, 0, 0);
+	int p = 0, q = blockIdx.y;
+	while(q >= ncb - p) { q -= ncb - p; p++; }
+	q += p;
+	for(int i = tid; i < 2 * GC_TAB / 16; i += GD_THREADS) {
+		const int side = i / (GC_TAB / 16);
+		((u32x4*) gd_smem)[i] = ((const u32x4*) (digitTabs + (size_t) (side ? q : p) * GC_TAB))[i % (GC_TAB / 16)];
 	}
-	int t = 0;
+	__syncthreads();
+	i32x4_gd l{0, 0, 0, 0}, m{0, 0, 0, 0};
+	auto flush = [&]() {
 #pragma unroll
-	for(int p = 0; p < NCB; p++)
+		for(int i = 0; i < 4; i++) {
+			const size_t at = (size_t) (16 * p + 4 * k + i) * (16 * ncb) + 16 * q + c;
+			atomicAdd(&left[at], (unsigned long long) (int64_t) l[i]);
+			atomicAdd(&mags[at], (unsigned long long) (int64_t) m[i]);
+		}
+		l = m = i32x4_gd{0, 0, 0, 0};
+	};
+	const int64_t nUnits = (nRows + 63) / 64;
+	int since = 0;
+	for(int64_t u = (int64_t) blockIdx.x * 8 + wave; u < nUnits; u += (int64_t) gridDim.x * 8) {
+		const int64_t row = u * 64 + 16 * k;
+		i32x4_gd x[2][8], xm[2];
 #pragma unroll
-		for(int q = p; q < NCB; q++, t++)
+		for(int side = 0; side < 2; side++) {
+			const u32x4 codes = *(const u32x4*) (arena + (size_t) cols[min((side ? q : p) * 16 + c, places - 1)].stream * arenaStride + row); // (behind them: zeros, whatever the code)
+			const uint8_t* const digits = gd_smem + side * GC_TAB + c * 2048;
 #pragma unroll
-			for(int i = 0; i < 4; i++) {
-				const int r = 16 * p + 4 * k + i, cc = 16 * q + c;
-				if(r <= cc) atomicAdd(&mags[r * (16 * NCB) + cc], (unsigned long long) (uint32_t) acc[t][i]);
+			for(int g = 0; g < 4; g++) {
+				u32x2 raw[4];
+#pragma unroll
+				for(int t = 0; t < 4; t++) raw[t] = *(const u32x2*) (digits + (((codes[g] >> (8 * t)) & 0xffu) << 3));
+				if((u + 1) * 64 > nRows) {
+#pragma unroll
+					for(int t = 0; t < 4; t++) raw[t] = row + 4 * g + t < nRows ? raw[t] : u32x2{0, 0};
+				}
+				uint32_t o[4];
+				gd_transpose(raw[0].x, raw[1].x, raw[2].x, raw[3].x, o);
+#pragma unroll
+				for(int d = 0; d < 4; d++) x[side][d][g] = (int) o[d];
+				const uint32_t sign = (o[0] >> 7) & 0x01010101u;
+				xm[side][g] = (int) ((o[0] ^ (sign * 255u)) + sign); // the first digit's magnitude, byte by byte (at most 127)
+				gd_transpose(raw[0].y, raw[1].y, raw[2].y, raw[3].y, o);
+#pragma unroll
+				for(int d = 0; d < 4; d++) x[side][4 + d][g] = (int) o[d];
 			}
+		}
+#pragma unroll
+		for(int i = 0; i < 8; i++) l = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[0][i], x[1][7 - i], l, 0, 0, 0);
+		m = __builtin_amdgcn_mfma_i32_16x16x64_i8(xm[0], xm[1], m, 0, 0, 0);
+		if(++since == GC_UNITS) {
+			flush();
+			since = 0;
+		}
+	}
+	if(since > 0) flush();
 }
 
 struct GdPlan {
@@ -583,6 +599,11 @@ struct GdPlan {
 	const GdTile* tiles = nullptr;
 	int nCellTiles = 0, grid = 0;
 	size_t lds = 0;
+	// Until the block has been judged: per column its place's group and column, per cell i <= j what is left out and the terms' magnitudes (NaN: exact or zero)
+	std::vector<GdCol> cols;
+	std::vector<double> left, mags;
+	bool judged = false;
+	bool suits[2] = {false, false}; // all cells / those across groups: no further from the exact sums than the fp64 kernel's
 	~GdPlan() { if(dImg) (void) hipFree(dImg); }
 };
 
@@ -593,8 +614,8 @@ void gd_plan_drop(cla_block* b) {
 	b->gdPlan = nullptr;
 }
 
-// The digits of x 2^GD_BITS rounded to a whole number; true if nothing was rounded
-static bool gd_digits(double x, int8_t (&d)[GD_DIGITS]) {
+// The digits of x 2^GD_BITS rounded to a whole number, and of what that lost; true if nothing was rounded
+static bool gd_digits(double x, int8_t (&d)[GD_DIGITS + 1]) {
 	const double scaled = x * (double) ((int64_t) 1 << GD_BITS), whole = std::nearbyint(scaled);
 	int64_t X = (int64_t) whole;
 	for(int i = GD_DIGITS - 1; i > 0; i--) {
@@ -602,6 +623,7 @@ static bool gd_digits(double x, int8_t (&d)[GD_DIGITS]) {
 		X = (X - d[i]) >> 8;
 	}
 	d[0] = (int8_t) X;
+	d[GD_DIGITS] = (int8_t) std::min(127.0, std::nearbyint((scaled - whole) * 256.0));
 	return whole == scaled;
 }
 
@@ -610,7 +632,7 @@ static int gd_build_plan(cla_block* b, GdPlan& P) {
 	P.rc = 1;
 	const int n = b->nCols;
 	if(b->dArena == nullptr || b->arenaWidth != 1 || n < 17 || n > 112 || b->nRows == 0 || b->dictNonFinite || b->crossSplit > 0 || b->crossBlocks > 0) return 0;
-	if(b->nRows > (int64_t) 131072 * 8 * 64) return 0; // (the magnitudes' sums of a wave, on few CUs too)
+	if(b->nRows > (int64_t) 131072 * 8 * 64) return 0; // (longer ones have not been measured)
 	std::vector<int> groupOf((size_t) n, -1);
 	for(size_t g = 0; g < b->groups.size(); g++)
 		for(int col : b->groups[g].cols) {
@@ -623,7 +645,7 @@ static int gd_build_plan(cla_block* b, GdPlan& P) {
 	const int places = narrow ? nf * 16 + 4 : nf * 16;
 	std::vector<GdCol> cols((size_t) places);
 	std::vector<uint8_t> tabs;
-	std::vector<uint8_t> magTabs((size_t) ncb * 16 * 256, 0);
+	std::vector<uint8_t> digitTabs((size_t) ncb * GC_TAB, 0);
 	std::vector<char> exact((size_t) n), zero((size_t) n); // few digits and nothing rounded; only zeros
 	struct Src { int col, group, h; };
 	std::vector<Src> src; // columns in the groups' order, then those that only carry a constant
@@ -652,10 +674,10 @@ static int gd_build_plan(cla_block* b, GdPlan& P) {
 		bool ex = true;
 		for(int i = 0; i < entries; i++) {
 			const double x = val[std::min(i, nV - 1)] * down; // (exact: what is lost of values 2^-700 of the largest is below every digit)
-			int8_t d[GD_DIGITS];
+			int8_t d[GD_DIGITS + 1];
 			ex &= gd_digits(x, d) && d[4] == 0 && d[5] == 0 && d[6] == 0;
 			std::memcpy(tabs.data() + C.tab + (size_t) i * 8, d, GD_DIGITS);
-			magTabs[(size_t) place * 256 + i] = (uint8_t) std::min(GD_MAG - 1, (int) (std::fabs(x) * GD_MAG));
+			std::memcpy(digitTabs.data() + ((size_t) place * 256 + i) * 8, d, GD_DIGITS + 1);
 		}
 		exact[place] = ex; zero[place] = most == 0.0;
 		return true;
@@ -726,27 +748,38 @@ static int gd_build_plan(cla_block* b, GdPlan& P) {
 	A.nLds = nLds; A.ldsTab = (int) ldsTab;
 
 	// The errors are parts of the columns' largest values, a cell's terms need not be: every cell whose columns are not both free of
-	// rounding has to reach, on average over the rows, 2^-10 of the product of their largest values. (2^-10: rounding errors of 2^-55 all of one
-	// sign would leave 2^-44 of the terms' sum; they are of either sign and differ from tuple to tuple.)
+	// rounding has to reach, on average over the rows, 2^-10 of the product of their largest values, whoever asks.
+	// (Six products left out of up to 2^14 2^-70 and two roundings of up to 2^-56: 2^-53.0 a row, all of one sign where a tuple has nearly all rows: up to 2^-43 of the
+	// terms' sum. Unasked a block comes here only if gd_judge finds less than in fp64.)
 	struct Tmp { void* p = nullptr; ~Tmp() { if(p) (void) hipFree(p); } } tmp;
-	const size_t magBytes = nMag * sizeof(unsigned long long);
-	if(no_room(&tmp.p, magBytes + magTabs.size())) return 1;
-	unsigned long long* dMag = (unsigned long long*) tmp.p;
-	uint8_t* dMagTabs = (uint8_t*) tmp.p + magBytes;
-	CLA_HIP(hipMemsetAsync(dMag, 0, magBytes, b->stream));
-	CLA_HIP(hipMemcpyAsync(dMagTabs, magTabs.data(), magTabs.size(), hipMemcpyHostToDevice, b->stream));
-	const unsigned grid = (unsigned) std::min<int64_t>((b->nRows + 511) / 512, g_numCU);
-#define GD_MAGS(N) case N: hipLaunchKernelGGL(k_gram_magnitudes<N>, dim3(grid), dim3(GD_THREADS), 0, b->stream, A.arena, A.arenaStride, A.cols, places, dMagTabs, A.nRows, dMag); break;
-	switch(ncb) { GD_MAGS(2) GD_MAGS(3) GD_MAGS(4) GD_MAGS(5) GD_MAGS(6) GD_MAGS(7) }
-#undef GD_MAGS
+	const size_t sumBytes = nMag * sizeof(unsigned long long);
+	if(no_room(&tmp.p, 2 * sumBytes + digitTabs.size())) return 1;
+	unsigned long long* const dLeft = (unsigned long long*) tmp.p;
+	uint8_t* const dDigits = (uint8_t*) tmp.p + 2 * sumBytes;
+	CLA_HIP(hipMemsetAsync(dLeft, 0, 2 * sumBytes, b->stream));
+	CLA_HIP(hipMemcpyAsync(dDigits, digitTabs.data(), digitTabs.size(), hipMemcpyHostToDevice, b->stream));
+	const int pairs = ncb * (ncb + 1) / 2;
+	const unsigned gx = (unsigned) std::min<int64_t>((b->nRows + 511) / 512, (2 * g_numCU + pairs - 1) / pairs);
+	CLA_HIP(allow_full_lds((const void*) k_gram_left));
+	hipLaunchKernelGGL(k_gram_left, dim3(gx, (unsigned) pairs), dim3(GD_THREADS), GC_LDS, b->stream, A.arena, A.arenaStride, A.cols, places, ncb, dDigits, A.nRows,
+		dLeft, dLeft + nMag);
 	CLA_HIP(hipGetLastError());
-	std::vector<unsigned long long> mags(nMag);
-	CLA_HIP(hipMemcpyAsync(mags.data(), dMag, magBytes, hipMemcpyDeviceToHost, b->stream));
+	std::vector<unsigned long long> sums(2 * nMag);
+	CLA_HIP(hipMemcpyAsync(sums.data(), dLeft, 2 * sumBytes, hipMemcpyDeviceToHost, b->stream));
 	CLA_HIP(hipStreamSynchronize(b->stream));
+	P.cols = std::move(cols);
+	P.left.assign((size_t) n * n, NAN);
+	P.mags.assign((size_t) n * n, NAN);
 	const double least = (double) b->nRows * GD_MAG * GD_MAG / 1024.0;
 	for(int i = 0; i < n; i++)
-		for(int j = i; j < n; j++)
-			if(!zero[i] && !zero[j] && !(exact[i] && exact[j]) && (double) mags[(size_t) i * ncb * 16 + j] < least) return 0;
+		for(int j = i; j < n; j++) {
+			if(zero[i] || zero[j] || (exact[i] && exact[j])) continue;
+			const size_t at = (size_t) i * ncb * 16 + j;
+			if((double) sums[nMag + at] < least) return 0;
+			const double largest = P.cols[i].scale * P.cols[j].scale * (GD_MAG * GD_MAG); // product of the columns' scales
+			P.left[(size_t) i * n + j] = (double) (int64_t) sums[at] * std::ldexp(largest, -70);
+			P.mags[(size_t) i * n + j] = (double) sums[nMag + at] * largest / (GD_MAG * GD_MAG);
+		}
 	P.rc = 0;
 	return 0;
 }
@@ -774,8 +807,60 @@ static bool gd_pays(const cla_block* b) {
 	return rows >= (v > 48 ? 500000 : n >= 24 ? 1000000 : 3000000);
 }
 
-// 0: the block goes this way (its plan is made), 1: it does not, negative: an error.
-int gram_digits_plan(cla_block* b) {
+// Is the block's result on digits no further from the exact sums than the fp64 kernel's, which `fp64` writes to a zeroed matrix (its upper triangle at least)? Both
+// are formed once and compared: what the digits leave out of a cell is known (k_gram_left), so the exact sums are, but for what is left out at weight 8. Neither the rms over the cells of the
+// error divided by the sum of the terms' magnitudes nor the largest of them may exceed fp64's. (That depends on how the codes are distributed, more than on the values:
+// where few tuples have most rows, the same rounding is added again and again, in fp64 in the long chains of many rows, on digits at any number. Rms fp64 / digits, diagonal
+// and other cells, Zipf(1.1) codes of 256 normal values, 100 columns: 2,000 rows 8.0e-17 / 7.9e-17 and 8.8e-18 / 2.0e-17, which stay in fp64 as up to some 20,000 rows do, 50,000 1.7e-16 / 1.1e-16 and
+// 1.0e-17 / 2.4e-17, 200,003 3.5e-16 / 8.9e-17 and 1.6e-17 / 2.3e-17, 2,000,003 2.4e-15 / 1.0e-16 and 7.5e-17 / 3.0e-17; uniform codes 10,007 rows 1.0e-16 / 5.2e-17 and
+// 4.3e-18 / 3.4e-18. One value at 5 among them stays in fp64 at 200,003 rows, three decades of values, or a tuple with 99 % of the rows far below the largest, at any number measured.)
+static int gd_judge(cla_block* b, GdPlan& P, const std::function<int(double*)>& fp64) {
+	const int n = b->nCols;
+	auto relative = [&](size_t at) { return P.left[at] / P.mags[at]; };
+	double sum = 0.0, most = 0.0;
+	int cells = 0;
+	for(size_t at = 0; at < P.left.size(); at++)
+		if(!std::isnan(P.left[at])) {
+			sum += relative(at) * relative(at);
+			most = std::max(most, std::fabs(relative(at)));
+			cells++;
+		}
+	if(sum <= 1e-34 * cells && most <= 0x1p-55) P.suits[0] = P.suits[1] = true; // (fp64 1.5e-17 and more on any block that is not exact)
+	else {
+		struct Tmp { void* p = nullptr; ~Tmp() { if(p) (void) hipFree(p); } } tmp;
+		const size_t nn = (size_t) n * n;
+		if(no_room(&tmp.p, 2 * nn * sizeof(double))) return 1;
+		double* const d = (double*) tmp.p;
+		int rc = launch_zero(b, d, nn);
+		if(rc || (rc = fp64(d)) || (rc = launch_gram_digits(b, nullptr, d + nn, nullptr, 0, 0))) return rc;
+		std::vector<double> out(2 * nn);
+		CLA_HIP(hipMemcpyAsync(out.data(), d, 2 * nn * sizeof(double), hipMemcpyDeviceToHost, b->stream));
+		CLA_HIP(hipStreamSynchronize(b->stream));
+		struct { double ours = 0.0, theirs = 0.0, oursMost = 0.0, theirsMost = 0.0; } of[2]; // all cells, those across groups
+		for(int i = 0; i < n; i++)
+			for(int j = i; j < n; j++) {
+				const size_t at = (size_t) i * n + j;
+				if(std::isnan(P.left[at])) continue;
+				const GdCol &a = P.cols[i], &c = P.cols[j];
+				const size_t cell = (size_t) std::min(a.col, c.col) * n + std::max(a.col, c.col);
+				const double e = relative(at), f = (out[cell] - out[nn + cell] - P.left[at]) / P.mags[at];
+				const double r = 0.58 * 0x1p-54 * out[cell] / P.mags[at]; // both results are rounded, and f has the rounding of either
+				for(int s = 0; s < (a.group != c.group && a.group >= 0 && c.group >= 0 ? 2 : 1); s++) {
+					of[s].ours += e * e + 2.0 * r * r;
+					of[s].theirs += f * f;
+					of[s].oursMost = std::max(of[s].oursMost, std::fabs(e));
+					of[s].theirsMost = std::max(of[s].theirsMost, std::fabs(f));
+				}
+			}
+		for(int s = 0; s < 2; s++) P.suits[s] = of[s].ours <= of[s].theirs && of[s].oursMost <= of[s].theirsMost;
+	}
+	P.judged = true;
+	P.cols = {}; P.left = {}; P.mags = {};
+	return 0;
+}
+
+// 0: the block goes this way (its plan is made), 1: it does not, negative: an error. across: only cells across groups are wanted of it. fp64: see gd_judge.
+int gram_digits_plan(cla_block* b, bool across, const std::function<int(double*)>& fp64) {
 	if(b->opt.tsmmDigits == 0 || (b->opt.tsmmDigits == 1 && !gd_pays(b))) return 1;
 	if(b->gdPlan == nullptr) {
 		// (a capture refuses the plan's allocations and its wait: the fp64 kernel)
@@ -789,7 +874,22 @@ int gram_digits_plan(cla_block* b) {
 		b->derivedBytes += plan->bytes;
 		b->gdPlan = plan.release();
 	}
-	return b->gdPlan->rc;
+	GdPlan& P = *b->gdPlan;
+	if(P.rc || b->opt.tsmmDigits == 2) return P.rc;
+	if(!P.judged) {
+		hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+		CLA_HIP(hipStreamIsCapturing(b->stream, &capturing));
+		if(capturing != hipStreamCaptureStatusNone) return 1;
+		// (its launches are not the call's)
+		const size_t stats = b->lastStats.size();
+		const bool profile = b->profile;
+		b->profile = false;
+		const int rc = gd_judge(b, P, fp64);
+		b->lastStats.resize(stats);
+		b->profile = profile;
+		if(rc) return rc;
+	}
+	return P.suits[across] ? 0 : 1;
 }
 
 // dOut = t(X) %*% X, both triangles; dNnz (may be null): its non-zeros. skipOwn: cells inside a group and of columns without one

@@ -544,10 +544,16 @@ int launch_gram_tiles(cla_block* b, double* dOut, unsigned long long* dNnz, bool
 		A.acc = b->dGramAcc; A.done = b->gram_ticket(); A.nnz = dNnz;
 	}
 	A.skipOwn = ownByCounts;
-	int rc = P.kind == GT_BYTE ? gram_digits_plan(b) : 1;
+	const unsigned grid = (unsigned) std::min((A.nTiles + gt_group(P.kind) - 1) / gt_group(P.kind), g_numCU * P.perCU);
+	auto fp64 = [&](double* out) { // the upper triangle into a zeroed matrix, as the call would have it
+		GtArgs F = A;
+		F.out = out; F.skipOwn = 0;
+		if(F.done == nullptr) F.acc = out;
+		return gt_launch_shape(b, P, F, grid);
+	};
+	int rc = P.kind == GT_BYTE ? gram_digits_plan(b, ownByCounts, fp64) : 1;
 	if(rc < 0) return rc;
 	const bool digits = rc == 0;
-	const unsigned grid = (unsigned) std::min((A.nTiles + gt_group(P.kind) - 1) / gt_group(P.kind), g_numCU * P.perCU);
 	// (where k_gram_tiles does not follow, an exception on the way included, nothing clears what the counts' kernel has added)
 	struct Clear {
 		cla_block* b;

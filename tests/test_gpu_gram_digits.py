@@ -107,3 +107,47 @@ def test_values_that_digits_do_not_suit(cla, ora, kind):
         assert np.array_equal(out, want * 1e200 * 1e200)
         return
     assert_matches_truth(out, D.T, D, what=kind)
+
+
+def errors(specs, out, n_cols):
+    """|error| / sum of the terms' magnitudes per cell, against exact counts of pairs of values in long double."""
+    err = []
+    for i in range(n_cols):
+        for j in range(i, n_cols):
+            x, y = (specs[c].dict[:, 0].astype(np.longdouble) for c in (i, j))
+            count = np.bincount(specs[i].codes.astype(np.int64) * len(y) + specs[j].codes, minlength=len(x) * len(y)).reshape(len(x), len(y))
+            terms = x[:, None] * y[None] * count
+            err.append(abs(float(out[i, j] - terms.sum())) / float(abs(terms).sum()))
+    return np.array(err)
+
+
+@pytest.mark.parametrize("kind,n_rows,n_cols,n_vals,digits", [
+    ("one tuple", 500, 100, 256, False), ("one tuple", 60_011, 100, 40, False), ("one at 5", 10_007, 100, 256, False), ("one at 10", 10_007, 100, 256, False),
+    ("three decades", 500, 100, 256, False), ("normal", 2_000, 100, 256, False), ("normal", 600_007, 50, 40, True), ("uniform", 10_007, 60, 40, True)])
+def test_no_less_precise_than_fp64(cla, kind, n_rows, n_cols, n_vals, digits):
+    """Unasked a block goes to digits only where their error does not exceed the fp64 kernel's, also where the values' magnitudes alone would let
+    it in: one tuple with nearly all rows, whose rounding is added again and again, a rare value that takes the others' digits, short blocks."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_rows + n_cols)
+    share = np.cumsum(1 / np.arange(1, n_vals + 1) ** 1.1)
+    specs = []
+    for c in range(n_cols):
+        d = rng.standard_normal(n_vals)
+        codes = np.searchsorted(share / share[-1], rng.random(n_rows)).clip(max=n_vals - 1)
+        if kind == "one tuple":  # 0.135 and 1.1 / 128 of the largest value
+            d = rng.permutation([0.135, 1.1 / 128])[0] * (1 + 0.01 * d)
+            d[0] = 1.0
+            codes = np.where(rng.random(n_rows) < 0.99, 1, np.where(rng.random(n_rows) < 0.5, 0, codes))
+        elif kind.startswith("one at"):
+            d[200] = float(kind.split()[-1])
+        elif kind == "three decades":
+            d *= 10 ** rng.uniform(-3, 0, n_vals)
+        elif kind == "uniform":
+            codes = rng.integers(0, n_vals, n_rows)
+        specs.append(synth.GroupSpec("ddc", np.array([c], np.int32), d[:, None], codes.astype(np.uint8)))
+    out, _, lds = product(cla, specs, n_rows, n_cols, 1)
+    want, _, fp64 = product(cla, specs, n_rows, n_cols, 0)
+    assert (lds != fp64) == digits
+    if digits:
+        got, ref = (errors(specs, o, n_cols) for o in (out, want))
+        assert np.sqrt((got ** 2).mean()) <= np.sqrt((ref ** 2).mean()) and got.max() <= ref.max()
