@@ -128,8 +128,9 @@ int cla_block_set_stream(cla_handle h, void* hipStream);
  *                   non-finite Y that a group does not cover stays out of its sums: decided on the device; chunk of
  *                   columns by chunk the host looks, i.e. waits for the stream once per call, and such a Y takes the bin kernels)
  *   rmm_digits      X %*% B of all-DDC byte-code blocks of 64 to 100 columns as exact sums of products of 8-bit digits of the values on the
- *                   integer matrix cores (rows whose outputs' terms are far below their columns' largest in fp64): 0 never (fp64), 1 where
- *                   it is the faster way, 2 at any number of rows and columns of B
+ *                   integer matrix cores: 0 never (fp64), 1 where it is the faster way and leaves no larger error than fp64 (64 columns of B at a time, decided on
+ *                   the device from their values and X's mean magnitudes; rows whose outputs' terms are a fifth of their column's mean in fp64),
+ *                   2 at any number of rows and columns of B (rows whose outputs' terms are far below their columns' largest in fp64)
  *   tsmm_digits     t(X) %*% X of all-DDC byte-code blocks of 17 to 112 columns as exact sums of products of 8-bit digits of the values on the
  *                   integer matrix cores: 0 never (fp64), 1 where it is the faster way and its error no larger than fp64's on this block (decided once per
  *                   block, from both results), 2 at any number of rows, wherever every cell's terms reach 2^-10 of the product of its columns'

@@ -7,9 +7,9 @@
 // (rms; fp64 kernel / here): 64 columns 5.2e-17 / 3.7e-17 - 4.7e-17, 80 5.3e-17 / 3.5e-17 - 4.6e-17, 100 5.2e-17 / 3.0e-17 - 4.2e-17; of few distinct values less.
 // From fewer than 64 columns the fp64 kernel loses less (32: 5.2e-17 / 5.1e-17 - 6.5e-17, 16: 5.1e-17 / 6.3e-17): they do not come here.
 //
-// That error is absolute, an output's terms need not reach their columns' largest values. An eighth byte holds a value's magnitude in 1 / 128
-// of the largest (rounded down), and one more product sums those of an output's terms (of the first 32 columns: nearly always enough). 32 rows that have an output below 2^-2
-// sqrt(K / 100) of the largest possible term (random values: 4 K / 100) are marked and left to the fp64 kernel, which follows
+// That error is absolute, an output's terms need not reach their columns' largest values. Columns of B whose outputs do not reach enough of it on average are fp64's
+// (k_rmm_digits_b, which says how much is enough). An eighth byte holds a value's magnitude in 1 / 128 of the largest (rounded down), and one more product sums
+// those of an output's terms. 32 rows that have an output far below the column's average are marked and left to the fp64 kernel, which follows
 // and otherwise finds nothing to do; so are all rows if B holds an infinity or a NaN, and a workgroup's further rows if most of its first ones are.
 //
 // v_mfma_i32_32x32x32_i8, lane l: A row l % 32, columns 16 (l / 32) .. + 15; B column l % 32, rows alike; D column l % 32, place r row 8 (r / 4) + 4 (l / 32) + r % 4.
@@ -50,7 +50,8 @@ struct RdArgs {
 	const uint8_t* bImg;      // B's operands: per 32 columns S * 8 + 8 T pieces of 1 KB
 	const double* scale;      // per column of the pass: 2^(exponent - 22)
 	const int32_t* least;     // ... sum of magnitudes from which its outputs stand
-	const int32_t* bad;       // per 32 columns: B not finite or out of range
+	const int32_t* bad;       // per 32 columns: B not finite or out of range, or a column that digits do not suit
+	const float* over;        // ... above zero over the pass: its columns together
 	const double* constRow;
 	double* out;
 	uint8_t* marks;           // per 32 rows: 1: left to the fp64 kernel
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(RD_THREADS, 2) void k_rmm_mfma_i8(RdArgs A) {
 		const int64_t at = (int64_t) tile * RD_WAVES + wave;
 		if(lane_now() == 0 && at * 32 < A.nRows) A.marks[at] = (uint8_t) m;
 	};
-	bool give = A.bad[0] != 0 || (C > 1 && A.bad[C - 1] != 0);
+	bool give = A.bad[0] != 0 || (C > 1 && A.bad[C - 1] != 0) || A.over[0] + (C > 1 ? A.over[C - 1] : 0.0f) > 0.0f;
 	if(give || tile0 >= A.nTiles) { // (uniform)
 		for(int tile = tile0; tile < A.nTiles; tile += gridDim.x) mark(tile, 1);
 		return;
@@ -284,8 +285,8 @@ __global__ __launch_bounds__(RD_THREADS, 2) void k_rmm_mfma_i8(RdArgs A) {
 			}
 			return __ballot(low) != 0;
 		};
-		bool marked = magnitudes(0, 1); // (the first step's sums are nearly always enough)
-		if(marked && S + T > 1) marked = magnitudes(1, S + T);
+		bool marked = magnitudes(0, 2); // (64 columns' sums are nearly always enough)
+		if(marked && S + T > 2) marked = magnitudes(2, S + T);
 		__builtin_amdgcn_sched_barrier(0);
 		mark(tile, marked);
 #pragma unroll
@@ -356,10 +357,18 @@ __global__ __launch_bounds__(RD_THREADS, 2) void k_rmm_mfma_i8(RdArgs A) {
 
 static_assert(MF_BL_THREADS == 256, "blocks of k_rmm_digits_b");
 constexpr int RB_THREADS = MF_BL_THREADS, RB_PIECES = 32; // (3 steps of 8, and 8)
-// Block c: 32 columns of B of the pass into their operands, scales and least sums.
+constexpr double RD_LOST = 1.2e-16, RD_FP64 = 4.5e-17;    // (1.1e-16 for the products of weight 7, the rest for the values' rounding)
+// Block c: 32 columns of B of the pass into their operands, scales and least sums. What the digits leave out of an output is RD_LOST sqrt(K / 100) (rms) of the largest possible
+// term, whatever the values, and how far an output's terms come on average is known from X's mean magnitudes: a column's mean error is the quotient. The pass goes
+// to fp64 if the rms of that over its columns exceeds RD_FP64, the least that fp64 leaves of values that are not short, or one column's 2^-53; rows are left to
+// fp64 where an output's terms come to a fifth of the column's mean only. (Rms error over the sum of the terms' magnitudes, fp64 / digits, expected: normal values 64 columns
+// 5.3e-17 / 3.9e-17, 3.6e-17, 100 5.1e-17 / 3.2e-17, 3.0e-17, uniform 4.5e-17 / 1.6e-17, 1.5e-17; in fp64 then: B of Student's t, 3 degrees 5.8e-17 / 6.9e-17,
+// X of it 6.0e-17 / 1.6e-16, X lognormal 6.6e-17 / 1.5e-16, X normal with one value at 8 5.5e-17 / 1.1e-16.)
+// leastSum > 0: rows whose outputs' terms come to that are enough, whatever the columns'.
 // The blocks behind those make what the fp64 kernel reads (mf_prep).
 __global__ __launch_bounds__(RB_THREADS) void k_rmm_digits_b(const MfPrep P, int blocks, int K, int S, int T, const int32_t* __restrict__ rowCol,
-	const double* __restrict__ up, uint8_t* __restrict__ bImg, double* __restrict__ scale, int32_t* __restrict__ least, int32_t* __restrict__ bad, int leastSum) {
+	const double* __restrict__ up, const double* __restrict__ mean, uint8_t* __restrict__ bImg, double* __restrict__ scale, int32_t* __restrict__ least, int32_t* __restrict__ bad,
+	float* __restrict__ over, int leastSum) {
 	if((int) blockIdx.x >= blocks) {
 		mf_prep(P, (int) blockIdx.x - blocks);
 		return;
@@ -374,11 +383,13 @@ __global__ __launch_bounds__(RB_THREADS) void k_rmm_digits_b(const MfPrep P, int
 	// all of a thread's values requested at once, in two round trips (walked twice, one after the other, they took 14.5 us of a call, 7.0 now). up[k]: 2^(exponent
 	// of X's column k)
 	constexpr int VALS = (RD_COLS + RB_THREADS / 32 - 1) / (RB_THREADS / 32);
-	double v[VALS];
+	double v[VALS], xm[VALS];
 	{
 		int32_t at[VALS];
 #pragma unroll
 		for(int i = 0; i < VALS; i++) at[i] = rowCol[min(slice + i * (RB_THREADS / 32), K - 1)];
+#pragma unroll
+		for(int i = 0; i < VALS; i++) xm[i] = mean[min(slice + i * (RB_THREADS / 32), K - 1)];
 #pragma unroll
 		for(int i = 0; i < VALS; i++) v[i] = B[(size_t) at[i] * q + min(col, q - 1)] * up[min(slice + i * (RB_THREADS / 32), K - 1)];
 	}
@@ -401,11 +412,25 @@ __global__ __launch_bounds__(RB_THREADS) void k_rmm_digits_b(const MfPrep P, int
 		if(f >= 0.99) e++;
 	}
 	odd |= m > 0.0 && e < -900;
-	if(odd) badS = 1;
+	double terms = 0.0;
+#pragma unroll
+	for(int i = 0; i < VALS; i++) terms += xm[i] * fabs(ldexp(v[i], -e)); // (zeros from K on)
+	__syncthreads();
+	most[slice][r] = terms;
+	__syncthreads();
 	if(slice == 0) {
+		for(int i = 1; i < RB_THREADS / 32; i++) terms += most[i][r];
+		const double lost = RD_LOST * sqrt(K * 0.01) / terms; // (a column of zeros: nothing)
+		const bool any = m > 0.0 && leastSum == 0;
+		odd |= any && !(lost <= 0x1p-53);
 		scale[32 * c + r] = ldexp(1.0, e - 22);
-		least[32 * c + r] = m > 0.0 ? leastSum : 0;
+		least[32 * c + r] = any ? (int) fmin(16384.0 / 5 * terms, 1e9) : m > 0.0 ? leastSum : 0;
+		float o = any ? (float) (lost * lost / (RD_FP64 * RD_FP64)) - 1.0f : 0.0f;
+#pragma unroll
+		for(int d = 1; d < 32; d *= 2) o += __shfl_xor(o, d);
+		if(r == 0) over[c] = o;
 	}
+	if(odd) badS = 1;
 	if(col < q)
 #pragma unroll
 		for(int j = 0; j < VALS; j++) {
@@ -443,17 +468,41 @@ __global__ __launch_bounds__(RB_THREADS) void k_rmm_digits_b(const MfPrep P, int
 	if(tid == 0) bad[c] = badS;
 }
 
+constexpr int RM_THREADS = 256, RM_ONE = 1 << 20;
+// sums[place] += the sum over the rows of column `place`'s magnitudes, in 1 / RM_ONE of its scale (mags, 256 codes a place). (Once per block: 10,000,000 x 100 0.30 ms.)
+__global__ __launch_bounds__(RM_THREADS) void k_rmm_digits_means(const uint8_t* __restrict__ arena, size_t arenaStride, const int32_t* __restrict__ streams,
+	const uint32_t* __restrict__ mags, int64_t nRows, unsigned long long* __restrict__ sums) {
+	__shared__ uint32_t tab[256];
+	const int place = blockIdx.y, tid = threadIdx.x;
+	tab[tid] = mags[place * 256 + tid];
+	__syncthreads();
+	const uint8_t* const stream = arena + (size_t) (uint32_t) streams[place] * arenaStride;
+	unsigned long long sum = 0;
+	for(int64_t row = ((int64_t) blockIdx.x * RM_THREADS + tid) * 16; row < nRows; row += (int64_t) gridDim.x * RM_THREADS * 16) {
+		const u32x4 codes = *(const u32x4*) (stream + row);
+		uint32_t s = 0;
+#pragma unroll
+		for(int i = 0; i < 16; i++) s += row + i < nRows ? tab[(codes[i >> 2] >> (8 * (i & 3))) & 0xffu] : 0u;
+		sum += s;
+	}
+#pragma unroll
+	for(int d = 1; d < WAVE; d *= 2) sum += __shfl_xor(sum, d, WAVE);
+	if((tid & (WAVE - 1)) == 0) atomicAdd(&sums[place], sum);
+}
+
 struct RdPlan {
 	int rc = 0; // 1: not of this kernel's shape
 	RdArgs A;
 	void* dImg = nullptr;
 	int64_t bytes = 0;
 	const int32_t* rowCol = nullptr;
-	const double* up = nullptr;
+	const double *up = nullptr, *mean = nullptr;
 	uint8_t* bImg = nullptr;
 	double* scale = nullptr;
 	int32_t *least = nullptr, *bad = nullptr;
+	float* over = nullptr;
 	int K = 0, S = 0, T = 0;
+	bool suits = true; // a B of even magnitudes could come to what fp64 leaves
 	~RdPlan() { if(dImg) (void) hipFree(dImg); }
 };
 
@@ -475,7 +524,8 @@ static int rd_build_plan(cla_block* b, RdPlan& P) {
 	P.K = K; P.S = S; P.T = T;
 	const int places = S * 32 + 4 * T;
 	std::vector<int32_t> streams((size_t) places, 0), rowCol((size_t) places, 0);
-	std::vector<double> up((size_t) places, 1.0);
+	std::vector<double> up((size_t) places, 1.0), mean((size_t) places, 0.0); // (mean: of a column's magnitudes, in parts of its scale)
+	std::vector<uint32_t> mags((size_t) places * 256, 0);
 	std::vector<uint8_t> tabs((size_t) places * RD_TABLE, 0);
 	int place = 0;
 	for(size_t g = 0; g < b->groups.size(); g++) {
@@ -502,11 +552,13 @@ static int rd_build_plan(cla_block* b, RdPlan& P) {
 				}
 				d[0] = (uint8_t) X;
 				d[7] = (uint8_t) std::min(127, (int) (std::fabs(x) * 128.0));
+				mags[(size_t) place * 256 + i] = (uint32_t) (std::fabs(x) * RM_ONE);
 			}
 		}
 	}
 	auto up256 = [](size_t n) { return (n + 255) & ~(size_t) 255; };
-	const size_t oRow = up256((size_t) places * 4), oUp = oRow + up256((size_t) places * 4), oTabs = oUp + up256((size_t) places * 8), oB = oTabs + tabs.size();
+	const size_t oRow = up256((size_t) places * 4), oUp = oRow + up256((size_t) places * 4), oMean = oUp + up256((size_t) places * 8);
+	const size_t oTabs = oMean + up256((size_t) places * 8), oB = oTabs + tabs.size();
 	const size_t oScale = oB + (size_t) 2 * RB_PIECES * 1024, oLeast = oScale + 512, oBad = oLeast + 256, oMarks = oBad + 256;
 	const size_t total = oMarks + up256((size_t) (b->nRows + 511) / 512 * 16);
 	std::vector<uint8_t> all(oB, 0);
@@ -520,12 +572,30 @@ static int rd_build_plan(cla_block* b, RdPlan& P) {
 	P.bytes = (int64_t) total;
 	CLA_HIP(hipMemcpy(d, all.data(), all.size(), hipMemcpyHostToDevice));
 	CLA_HIP(hipMemset(d + oMarks, 0, total - oMarks)); // (behind the last row)
-	P.rowCol = (const int32_t*) (d + oRow); P.up = (const double*) (d + oUp);
-	P.bImg = d + oB; P.scale = (double*) (d + oScale); P.least = (int32_t*) (d + oLeast); P.bad = (int32_t*) (d + oBad);
+	{
+		struct Tmp { void* p = nullptr; ~Tmp() { if(p) (void) hipFree(p); } } tmp;
+		const size_t sumBytes = up256((size_t) places * 8);
+		if(no_room(&tmp.p, sumBytes + mags.size() * 4)) return 1;
+		CLA_HIP(hipMemsetAsync(tmp.p, 0, sumBytes, b->stream));
+		CLA_HIP(hipMemcpyAsync((char*) tmp.p + sumBytes, mags.data(), mags.size() * 4, hipMemcpyHostToDevice, b->stream));
+		const unsigned gx = (unsigned) std::min<int64_t>((b->nRows + RM_THREADS * 16 - 1) / (RM_THREADS * 16), (8 * g_numCU + K - 1) / K);
+		hipLaunchKernelGGL(k_rmm_digits_means, dim3(gx, (unsigned) K), dim3(RM_THREADS), 0, b->stream, b->dArena, b->arenaStride, (const int32_t*) d,
+			(const uint32_t*) ((char*) tmp.p + sumBytes), b->nRows, (unsigned long long*) tmp.p);
+		CLA_HIP(hipGetLastError());
+		std::vector<unsigned long long> sums((size_t) K);
+		CLA_HIP(hipMemcpyAsync(sums.data(), tmp.p, (size_t) K * 8, hipMemcpyDeviceToHost, b->stream));
+		CLA_HIP(hipStreamSynchronize(b->stream));
+		double all = 0.0;
+		for(int k = 0; k < K; k++) all += mean[k] = (double) sums[k] / RM_ONE / (double) b->nRows;
+		P.suits = 0.5 * all >= RD_LOST / RD_FP64 * std::sqrt(K / 100.0);
+		CLA_HIP(hipMemcpy(d + oMean, mean.data(), mean.size() * 8, hipMemcpyHostToDevice));
+	}
+	P.rowCol = (const int32_t*) (d + oRow); P.up = (const double*) (d + oUp); P.mean = (const double*) (d + oMean);
+	P.bImg = d + oB; P.scale = (double*) (d + oScale); P.least = (int32_t*) (d + oLeast); P.bad = (int32_t*) (d + oBad); P.over = (float*) (d + oBad + 128);
 	RdArgs& A = P.A;
 	A.arena = b->dArena; A.arenaStride = b->arenaStride;
 	A.streams = (const int32_t*) d; A.tabs = d + oTabs; A.bImg = P.bImg;
-	A.scale = P.scale; A.least = P.least; A.bad = P.bad; A.marks = d + oMarks;
+	A.scale = P.scale; A.least = P.least; A.bad = P.bad; A.over = P.over; A.marks = d + oMarks;
 	A.nRows = b->nRows; A.nTiles = (int) ((b->nRows + RD_ROWS - 1) / RD_ROWS);
 	P.rc = 0;
 	return 0;
@@ -560,7 +630,7 @@ int rmm_digits_plan(cla_block* b, int q, int n0) {
 		b->derivedBytes += plan->bytes;
 		b->rdPlan = plan.release();
 	}
-	return b->rdPlan->rc;
+	return b->rdPlan->rc || (b->opt.rmmDigits == 1 && !b->rdPlan->suits);
 }
 
 template <int S, int T, int C>
@@ -579,13 +649,13 @@ int launch_rmm_digits(cla_block* b, const MfPrep& prep, double* dOut, unsigned l
 	const int q = prep.q, n0 = prep.n0;
 	const RdPlan& P = *b->rdPlan;
 	const int cols = std::min(64, q - n0), c32 = (cols + 31) / 32;
-	// 2^-2 sqrt(K / 100) of the largest possible term, in squares of 1 / 128
-	const int leastSum = (int) (16384.0 / 4 * std::sqrt(P.K / 100.0));
+	// asked for by option: 2^-2 sqrt(K / 100) of the largest possible term, in squares of 1 / 128
+	const int leastSum = b->opt.rmmDigits == 2 ? (int) (16384.0 / 4 * std::sqrt(P.K / 100.0)) : 0;
 	{
 		const int blocks = c32 + prep.blocks();
 		Prof pf(b, "k_rmm_digits_b", blocks, RB_THREADS, 0, 0);
-		hipLaunchKernelGGL(k_rmm_digits_b, dim3((unsigned) blocks), dim3(RB_THREADS), 0, b->stream, prep, c32, P.K, P.S, P.T, P.rowCol, P.up, P.bImg, P.scale, P.least,
-			P.bad, leastSum);
+		hipLaunchKernelGGL(k_rmm_digits_b, dim3((unsigned) blocks), dim3(RB_THREADS), 0, b->stream, prep, c32, P.K, P.S, P.T, P.rowCol, P.up, P.mean, P.bImg, P.scale,
+			P.least, P.bad, P.over, leastSum);
 	}
 	RdArgs A = P.A;
 	A.constRow = prep.constRow; A.out = dOut; A.nnz = dNnz; A.q = q; A.n0 = n0;

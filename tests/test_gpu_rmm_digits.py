@@ -224,3 +224,46 @@ def test_replays_behind_an_option(cla, ora):
         ok(h.hipGraphDestroy(graph))
     blk.close()
     ok(h.hipStreamDestroy(stream))
+
+
+@pytest.mark.parametrize("kind,digits", [("normal", True), ("uniform", True), ("X t", False), ("B t", False), ("X one at 8", False), ("B one at 20", False), ("X lognormal", False),
+                                         ("X mostly zeros", False), ("B three decades", False), ("B one column", False)])
+@pytest.mark.parametrize("n_cols", [64, 100])
+def test_no_less_precise_than_fp64(cla, ora, kind, digits, n_cols):
+    """Unasked, columns of B go to digits only where the error that is to be expected does not exceed the fp64 kernel's."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_cols)
+    n_rows, n_vals, q = 3001, 256, 64
+    specs = columns(synth, rng, n_rows, n_cols, n_vals, np.uint8, 1)
+    B = rng.standard_normal((n_cols, q))
+    for s in specs:
+        if kind == "uniform":
+            s.dict = rng.uniform(-1, 1, s.dict.shape)
+        elif kind == "X t":
+            s.dict = rng.standard_t(3, s.dict.shape)
+        elif kind == "X one at 8":
+            s.dict[200] = 8.0
+        elif kind == "X lognormal":
+            s.dict = np.exp(s.dict)
+        elif kind == "X mostly zeros":
+            s.dict[rng.random(s.dict.shape) < 0.9] = 0.0
+    if kind == "B t":
+        B = rng.standard_t(2, B.shape)
+    elif kind == "B one at 20":
+        B[33] = 20.0
+    elif kind == "B three decades":
+        B *= 10 ** rng.uniform(-3, 0, B.shape)
+    elif kind == "B one column":  # (one of the second half whose values but one are far below that)
+        B[:, 40] *= 1e-4
+        B[5, 40] = 1.0
+    out, nnz, names = product(cla, specs, n_rows, n_cols, B, 1)
+    want, want_nnz, _ = product(cla, specs, n_rows, n_cols, B, 0)
+    assert nnz == want_nnz == np.count_nonzero(out)
+    if not digits:
+        assert np.array_equal(out, want)  # (the fp64 kernel's sums have one order)
+        return
+    assert "k_rmm_mfma_i8" in names
+    D = ora.np_decompress(specs, n_rows, n_cols).astype(np.longdouble)
+    scale = np.abs(D) @ np.abs(B)
+    got, ref = (np.abs(o - D @ B.astype(np.longdouble)) / scale for o in (out, want))
+    assert not np.array_equal(out, want) and np.sqrt((got ** 2).mean()) <= np.sqrt((ref ** 2).mean()) and got.max() <= ref.max()
