@@ -490,6 +490,39 @@ __global__ __launch_bounds__(RM_THREADS) void k_rmm_digits_means(const uint8_t* 
 	if((tid & (WAVE - 1)) == 0) atomicAdd(&sums[place], sum);
 }
 
+constexpr int RL_THREADS = 512, RL_TILES = RL_THREADS * 4 / 512; // 4 rows a thread; 512 rows are a tile of the fp64 kernel
+// low += the tiles of 512 rows with a row whose magnitudes (mags, 256 codes a place, in any unit) sum to less than `least`. (Once per block: 10,000,000 x 100 0.19 ms.)
+__global__ __launch_bounds__(RL_THREADS) void k_rmm_digits_low(const uint8_t* __restrict__ arena, size_t arenaStride, const int32_t* __restrict__ streams,
+	const uint16_t* __restrict__ mags, int K, int64_t nRows, uint32_t least, int* __restrict__ low) {
+	extern __shared__ __attribute__((aligned(16))) uint16_t rl_smem[];
+	__shared__ int lowS[RL_TILES];
+	const int tid = threadIdx.x;
+	for(int i = tid; i < K * 256; i += RL_THREADS) rl_smem[i] = mags[i];
+	int n = 0;
+	for(int64_t row0 = (int64_t) blockIdx.x * RL_THREADS * 4; row0 < nRows; row0 += (int64_t) gridDim.x * RL_THREADS * 4) {
+		if(tid < RL_TILES) lowS[tid] = 0;
+		__syncthreads();
+		const int64_t row = row0 + tid * 4;
+		uint32_t s[4] = {0, 0, 0, 0};
+		if(row < nRows) { // (the streams are padded to more than 4 rows)
+#pragma unroll 8
+			for(int k = 0; k < K; k++) {
+				const uint32_t codes = *(const uint32_t*) (arena + (size_t) (uint32_t) streams[k] * arenaStride + row);
+#pragma unroll
+				for(int i = 0; i < 4; i++) s[i] += rl_smem[k * 256 + ((codes >> (8 * i)) & 0xffu)];
+			}
+#pragma unroll
+			for(int i = 0; i < 4; i++)
+				if(row + i < nRows && s[i] < least) lowS[tid / 128] = 1;
+		}
+		__syncthreads();
+		if(tid == 0)
+			for(int t = 0; t < RL_TILES; t++) n += lowS[t];
+		__syncthreads();
+	}
+	if(tid == 0 && n > 0) atomicAdd(low, n);
+}
+
 struct RdPlan {
 	int rc = 0; // 1: not of this kernel's shape
 	RdArgs A;
@@ -502,7 +535,7 @@ struct RdPlan {
 	int32_t *least = nullptr, *bad = nullptr;
 	float* over = nullptr;
 	int K = 0, S = 0, T = 0;
-	bool suits = true; // a B of even magnitudes could come to what fp64 leaves
+	bool suits = true; // a B of even magnitudes could come to what fp64 leaves, and would leave it few rows
 	~RdPlan() { if(dImg) (void) hipFree(dImg); }
 };
 
@@ -588,6 +621,28 @@ static int rd_build_plan(cla_block* b, RdPlan& P) {
 		double all = 0.0;
 		for(int k = 0; k < K; k++) all += mean[k] = (double) sums[k] / RM_ONE / (double) b->nRows;
 		P.suits = 0.5 * all >= RD_LOST / RD_FP64 * std::sqrt(K / 100.0);
+		// Rows whose magnitudes are below a quarter of the mean would be marked whatever B, and 512 rows with one of them go through both kernels (us, fp64 / here: 2,000,000 x 100 by
+		// 64 with no such tile 570 / 437 - 462, 10 % 570 / 547 - 616, 22 % 570 / 665 - 747, all 570 / 933; 60,000 rows, whose one round of tiles is all or nothing, none 56 / 28, one and more 56 / 60 - 79).
+		if(P.suits) {
+			double largest = 0.0, sum = 0.0;
+			for(int k = 0; k < K; k++) {
+				largest = std::max(largest, up[k]);
+				sum += mean[k] * up[k];
+			}
+			std::vector<uint16_t> share((size_t) K * 256);
+			for(size_t i = 0; i < share.size(); i++) share[i] = (uint16_t) (mags[i] * (65535.0 / RM_ONE) * (up[i / 256] / largest));
+			int low = 0;
+			CLA_HIP(hipMemcpyAsync((char*) tmp.p + sumBytes, share.data(), share.size() * 2, hipMemcpyHostToDevice, b->stream));
+			CLA_HIP(hipMemsetAsync(tmp.p, 0, sizeof(int), b->stream));
+			const int64_t tiles = (b->nRows + 511) / 512;
+			const unsigned blocks = (unsigned) std::min<int64_t>((tiles + RL_TILES - 1) / RL_TILES, 3 * g_numCU);
+			hipLaunchKernelGGL(k_rmm_digits_low, dim3(blocks), dim3(RL_THREADS), (size_t) K * 512, b->stream, b->dArena, b->arenaStride, (const int32_t*) d,
+				(const uint16_t*) ((char*) tmp.p + sumBytes), K, b->nRows, (uint32_t) (sum / largest * 65535.0 / 4), (int*) tmp.p);
+			CLA_HIP(hipGetLastError());
+			CLA_HIP(hipMemcpyAsync(&low, tmp.p, sizeof(int), hipMemcpyDeviceToHost, b->stream));
+			CLA_HIP(hipStreamSynchronize(b->stream));
+			P.suits = low == 0 || (tiles > 2 * g_numCU && low * 20 <= tiles);
+		}
 		CLA_HIP(hipMemcpy(d + oMean, mean.data(), mean.size() * 8, hipMemcpyHostToDevice));
 	}
 	P.rowCol = (const int32_t*) (d + oRow); P.up = (const double*) (d + oUp); P.mean = (const double*) (d + oMean);

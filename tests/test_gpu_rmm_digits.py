@@ -267,3 +267,22 @@ def test_no_less_precise_than_fp64(cla, ora, kind, digits, n_cols):
     scale = np.abs(D) @ np.abs(B)
     got, ref = (np.abs(o - D @ B.astype(np.longdouble)) / scale for o in (out, want))
     assert not np.array_equal(out, want) and np.sqrt((got ** 2).mean()) <= np.sqrt((ref ** 2).mean()) and got.max() <= ref.max()
+
+
+@pytest.mark.parametrize("n_rows,low,digits", [(60_000, 0, True), (60_000, 1, False), (300_001, 0, True), (300_001, 20, True), (300_001, 60, False)])
+def test_rows_far_below_the_others(cla, ora, n_rows, low, digits):
+    """512 rows with one that digits do not suit go through both kernels: a block with many such rows is not sent to digits at all, nor is a
+    short one with any (117 and 586 times 512 rows)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(low)
+    n_cols, q = 80, 40
+    specs = columns(synth, rng, n_rows, n_cols, 200, np.uint8, 1)
+    at = np.arange(low) * 512 * (n_rows // 512 // max(low, 1)) + 3
+    for s in specs:
+        s.dict[:20] *= 1e-9
+        s.codes[:] = 20 + s.codes % 180
+        s.codes[at] %= 20
+    B = rng.standard_normal((n_cols, q))
+    out, nnz, names = product(cla, specs, n_rows, n_cols, B, 1)
+    assert ("k_rmm_mfma_i8" in names) == digits and nnz == np.count_nonzero(out)
+    check(out, ora.np_decompress(specs, n_rows, n_cols), B, np.r_[0:1000, at.astype(int), n_rows - 1000:n_rows])
