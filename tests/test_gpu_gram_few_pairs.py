@@ -32,3 +32,20 @@ def test_few_pairs(cla, ora, n_cols, n_rows, n_vals, one_kernel):
         assert_matches_truth(got, D.T, D, what=f"{n_rows} x {n_cols} of {n_vals}")
         assert np.array_equal(got, got.T)
     assert nnz == np.count_nonzero(out)
+
+
+@pytest.mark.parametrize("n_rows,by_pairs", [(2_500_000, False), (2_500_001, True)])
+def test_many_rows_go_by_pairs_of_groups(cla, ora, n_rows, by_pairs):
+    """Two or three groups go by pairs of groups from there on (shorter chains of additions)."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(1)
+    n_cols = 6
+    specs = columns(synth, rng, n_rows, n_cols, 300, np.uint16, 2)
+    blk = cla.build_block(n_rows, n_cols, specs)
+    out, nnz = blk.tsmm()
+    names = [k["name"] for k in blk.stats()["kernels"]]
+    blk.close()
+    assert ("k_gram_tiles" not in names) == by_pairs, names
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    assert_matches_truth(out, D.T, D, what=str(names))
+    assert np.array_equal(out, out.T) and nnz == np.count_nonzero(out)
