@@ -23,6 +23,8 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0     # MI355X published HBM3E bandwidth
 MFMA_F64_PEAK_TF = 78.6   # MI355X published dense fp64 matrix rate
+MFMA_I8_PEAK_TOPS = 5033.0 # MI355X dense 8-bit matrix rate (65,536 operations in 32 cycles per SIMD at 2.4 GHz)
+I8_KERNELS = {"k_rmm_mfma_i8": 28}  # products of 8-bit digits per product of two fp64 values
 
 # Sources whose text decides what the headline kernel does; a traffic figure measured with rocprofv3 is only
 # reported while their hash matches the one recorded next to the figure.
@@ -119,7 +121,8 @@ def time_async(blk, launch, reps, warm=2):
 def extra_row(blk, launch, n_rows, algo_bytes, flops=0.0, reps=10, prepare=None):
     """One row of `extra`: first-call time (includes derived formats built on first use), steady-state wall
     time per call, the dominant kernel with its HIP-event time, and the fraction of the bound that limits the
-    call (the larger of the HBM floor and the fp64 matrix floor) over the summed HIP-event times of all its
+    call (the larger of the HBM floor and the matrix floor, fp64 or of the digit products where the dominant kernel
+    forms those) over the summed HIP-event times of all its
     kernels. With `prepare` (a call of cla_block_prepare for this product) the row starts from a block without
     derived formats, so that `derived_bytes_built` is this product's alone, and also gives the time of the prepare
     call and of the first product call behind it."""
@@ -147,7 +150,9 @@ def extra_row(blk, launch, n_rows, algo_bytes, flops=0.0, reps=10, prepare=None)
     kms = ks[kname]["ms"]
     ksum = sum(v["ms"] for v in ks.values())
     hbm_floor_ms = algo_bytes / (HBM_PEAK_GBS * 1e9) * 1e3
-    mfma_floor_ms = flops / (MFMA_F64_PEAK_TF * 1e12) * 1e3
+    digits = I8_KERNELS.get(kname)
+    mfma, ops, peak = ("mfma_i8", flops * digits, MFMA_I8_PEAK_TOPS) if digits else ("mfma_f64", flops, MFMA_F64_PEAK_TF)
+    mfma_floor_ms = ops / (peak * 1e12) * 1e3
     row = {"ms": round(ms, 5), "cold_ms": round(cold_ms, 5), "first_call_ms": round(first_ms, 3), "rows_per_s": n_rows / (ms * 1e-3),
            "kernel": kname, "kernel_ms": round(kms, 5), "kernels": {k: round(v["ms"], 5) for k, v in ks.items()},
            "kernels_ms": round(ksum, 5), "algo_bytes": algo_bytes, "algo_GBs": algo_bytes / (ksum * 1e-3) / 1e9,
@@ -155,9 +160,9 @@ def extra_row(blk, launch, n_rows, algo_bytes, flops=0.0, reps=10, prepare=None)
            "derived_bytes_built": int(blk.derived_bytes() - d0), **prep}
     if flops:
         row["flops"] = flops
-        row["frac_mfma_f64"] = flops / (ksum * 1e-3) / 1e12 / MFMA_F64_PEAK_TF
+        row["frac_" + mfma] = ops / (ksum * 1e-3) / 1e12 / peak
     if mfma_floor_ms > hbm_floor_ms:
-        row["bound"], row["frac"] = "mfma_f64", row["frac_mfma_f64"]
+        row["bound"], row["frac"] = mfma, row["frac_" + mfma]
     else:
         row["bound"], row["frac"] = "hbm", row["frac_hbm"]
     return row

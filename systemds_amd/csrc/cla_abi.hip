@@ -1584,7 +1584,7 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 	if(!own && (rc = ensure_tables(b, nWs))) return rc;
 	double* const ws = own ? b->dLmmWs : b->dTables;
 	unsigned long long* const dBad = (unsigned long long*) (ws + nWs - 2);
-	// Zeros: k_take_block leaves the workspace as it has found it (a fill in front of every call: mixed rows by 4, 294,957 19.2 -> 17.7 us, by 6 5,000,011 94 -> 92).
+	// Zeros: k_take_block leaves the workspace as it has found it (a fill in front of every call: mixed rows by 4, 294,957 19.2 -> 17.7 us; of 5,000,011 rows no more than noise).
 	// A captured call has its fill all the same: what the workspace holds when it is replayed, behind a call that failed between its kernels, is not known now.
 	const bool clean = b->lmmWsClean;
 	if((recorded || !clean) && (rc = launch_zero(b, ws, own ? b->lmmWsCap : nWs))) return rc;

@@ -20,8 +20,8 @@
 // table, B's operand of weight w holds digit w - i there: 7 products instead of 28.
 //
 // Bound: a tile of 256 x 100 rows and 64 columns of B takes 27,000 cycles, 14,000 of them the matrix cores' (380 products per SIMD); decoding (5,600) is LDS reads with barriers
-// between, the outputs (128 KB) wait for their turn with the tables behind the products; the clock is 2.0 GHz under this load. 10,000,000 x 100 of 256 values times 64 columns 2.57 ms in fp64, 2.27 here;
-// 400,000 rows 182 / 120 us, 150,000 100 / 55, 500 64 / 25; 400,000 x 64 128 / 88. Taken back: outputs kept until the next tile's products (64 registers more: 3.6 ms), the
+// between, the outputs (128 KB) wait for their turn with the tables behind the products; the clock is 2.0 GHz under this load. 10,000,000 x 100 of 256 values times 64 columns 2.57 ms in fp64, 2.28 - 2.32 here;
+// 400,000 rows 171 / 114 us, 150,000 92 / 56, 500 56 / 26; 400,000 x 64 120 / 98 (both in their present form). Taken back: outputs kept until the next tile's products (64 registers more: 3.6 ms), the
 // next tables ordered between the products (3.0), products of a step between the look-ups of the next (2.28: LDS and matrix cores still take turns), two columns a
 // lane for 16-byte stores (2.29).
 #include "../../include/cla_hip.h"
@@ -656,11 +656,12 @@ static int rd_build_plan(cla_block* b, RdPlan& P) {
 	return 0;
 }
 
-// Where this pays, p columns of B in the pass (us, fp64 / here): a step that is nearly full (64 - 68 and 80 - 100 columns) and not many rows always, 500 x 64 of 8
-// columns of B 28 / 24, 500 x 100 of 64 64 / 38, 150,000 x 64 of 8 38 / 38, 400,000 x 80 of 32 102 / 82, 1,000,000 x 80 of 40 228 / 221. 16 columns of B at most (half of
-// the products are for nothing) 150,000 x 96 of 16 53 / 48, 400,000 x 80 77 / 81, 3,000,000 x 100 393 / 416; 33 - 48 columns (the fp64 kernel is
-// at its best) 1,500,000 x 80 of 40 320 / 314, of 48 325 / 328, 6,000,000 1026 / 1145; 17 - 32 and 49 - 64 at any number of rows, 3,000,000 x 80 of 32 458 / 408, 6,000,000 x 80
-// of 64 1303 / 1273, x 100 1578 / 1366. 69 - 79 columns (the last step a fifth or a half full) 150,000 x 72 of 48 63 / 62, 400,000 112 / 112, 6,000,000 920 / 1159.
+// Where this pays, p columns of B in the pass (us, fp64 / here, 256 values): up to 200,000 rows always, 500 x 64 of 8 columns of B 25 / 17, 500 x 100 of 64 56 / 26, 150,000 x 64
+// of 8 34 / 30, x 72 of 8 36 / 36, of 64 67 / 55, x 100 of 64 92 / 56. Past that, 16 columns of B at most (half of the products are for nothing) 250,000 x 64 of 8 34 / 36, x 100 of
+// 16 52 / 49, 400,000 x 80 71 / 72, 1,000,000 x 80 119 / 146, 3,000,000 x 100 368 / 436; 33 - 48 columns (the fp64 kernel is at its best) 250,000 x 80 of 40 66 / 67, 400,000
+// 121 / 106, 1,000,000 x 80 of 48 220 / 230, x 100 250 / 231, 3,000,000 x 100 631 / 669; 17 - 32 and 49 - 64 at any number of rows, 3,000,000 x 64 of 32 350 / 317, x 80
+// 428 / 407, of 64 665 / 645, x 100 805 / 697. 69 - 79 columns (the last step a fifth or a half full), of 32 and of 64 columns of B, 250,000 x 72 45 / 48 and 66 / 70, x 78 54 / 48 and
+// 76 / 71, 400,000 x 72 84 / 74 and 129 / 109, 1,000,000 147 / 151 and 233 / 228, 3,000,000 378 / 399 and 599 / 634: left to fp64, with what some 400,000 rows of them would give.
 static bool rd_pays(const cla_block* b, int K, int p) {
 	if(p < 8) return false;
 	if(b->nRows <= 200000) return true;
