@@ -91,9 +91,13 @@ bool no_room(void** p, size_t bytes) {
 
 int ensure_chain(cla_block* b, size_t nDoubles) {
 	if(nDoubles <= b->chainCap) return 0;
-	if(b->dChain) CLA_HIP(hipFree(b->dChain));
-	b->dChain = nullptr; b->chainCap = 0;
-	CLA_HIP(hipMalloc((void**) &b->dChain, nDoubles * sizeof(double)));
+	// (one that is too small stays until the block goes: the one-kernel chains need far less than X %*% v does, and calls captured with one may be replayed behind a chain
+	// of two products, or of another kernel)
+	double* p = nullptr;
+	b->wsOld.reserve(b->wsOld.size() + 1);
+	CLA_HIP(hipMalloc((void**) &p, nDoubles * sizeof(double)));
+	if(b->dChain) b->wsOld.push_back(b->dChain);
+	b->dChain = p;
 	b->chainCap = nDoubles;
 	return 0;
 }
@@ -349,7 +353,7 @@ void cla_block_free(cla_handle b) {
 	if(b->dTblOff) (void) hipFree(b->dTblOff);
 	if(b->dTables) (void) hipFree(b->dTables);
 	if(b->dLmmWs) (void) hipFree(b->dLmmWs);
-	for(double* p : b->lmmWsOld) (void) hipFree(p);
+	for(double* p : b->wsOld) (void) hipFree(p);
 	if(b->dStageIn) (void) hipFree(b->dStageIn);
 	if(b->dStageOut) (void) hipFree(b->dStageOut);
 	if(b->dScratch) (void) hipFree(b->dScratch);
@@ -1574,9 +1578,9 @@ int launch_lmm_joint(cla_block* b, const double* dY, int p, double* dOut, unsign
 	if(grow) {
 		const size_t cap = std::max(nWs, 2 * b->lmmWsCap);
 		double* p2 = nullptr;
-		b->lmmWsOld.reserve(b->lmmWsOld.size() + 1);
+		b->wsOld.reserve(b->wsOld.size() + 1);
 		CLA_HIP(hipMalloc((void**) &p2, cap * sizeof(double)));
-		if(b->dLmmWs) b->lmmWsOld.push_back(b->dLmmWs);
+		if(b->dLmmWs) b->wsOld.push_back(b->dLmmWs);
 		b->dLmmWs = p2; b->lmmWsCap = cap; b->lmmWsClean = false;
 	}
 	// Captured with more rows of Y than any call before: a capture refuses an allocation, the tables of earlier products may have the room.

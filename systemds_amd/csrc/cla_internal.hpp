@@ -190,8 +190,8 @@ struct cla_block {
 	double* dStageOut = nullptr; size_t stageOutCap = 0;
 	void* dScratch = nullptr;   size_t scratchCap = 0;
 	double* dLmmWs = nullptr;   size_t lmmWsCap = 0; bool lmmWsClean = false; // launch_lmm_joint: zeros between calls (k_take_block clears what a call has used)
-	std::vector<double*> lmmWsOld;      // smaller ones of earlier calls
 	double* dChain = nullptr;   size_t chainCap = 0;   // the multiply chain's own: X %*% v, or the sums of the blocks of its one kernel
+	std::vector<double*> wsOld;         // smaller ones of either of earlier calls
 	// exact code counts of all dictionary-coded groups (totalVals int32, group g at tblOff[g]),
 	// computed on the first TSMM and kept, like the reference's cached counts
 	// (CG/AColGroupValue.java getCounts)

@@ -83,3 +83,53 @@ def test_blocks_of_another_shape(cla, ora, kind):
     if kind != "infinite":
         D = ora.np_decompress(specs, n_rows, n_cols)
         np.testing.assert_allclose(out, (D.T @ (D @ v)).ravel(), rtol=1e-9, atol=1e-7)
+
+
+@pytest.mark.parametrize("kind", ["pairs", "byte codes", "lists"])
+def test_replays_behind_a_chain_of_two_products(cla, ora, kind):
+    """A captured chain, replayed behind one that runs as two products and needs a larger workspace: its own stays with the block."""
+    import ctypes as C
+    from devmem import DevBuf, hip
+    from systemds_amd import synth
+    rng = np.random.default_rng(13)
+    n_rows, n_cols = 30_011, 12
+    if kind == "pairs":
+        specs, blk = block(cla, rng, n_rows, n_cols, 300)
+    else:
+        specs = [synth.sdc_group(rng, n_rows, [c], 16, 0.05, None) if kind == "lists" else
+                 synth.GroupSpec("ddc", np.array([c], np.int32), rng.standard_normal((30, 1)), rng.integers(0, 30, n_rows).astype(np.uint8)) for c in range(n_cols)]
+        blk = cla.build_block(n_rows, n_cols, specs)
+    D = ora.np_decompress(specs, n_rows, n_cols)
+    h, stream = hip(), C.c_void_p()
+    ok = lambda rc: (_ for _ in ()).throw(AssertionError(rc)) if rc else None
+    ok(h.hipStreamCreate(C.byref(stream)))
+    blk.set_stream(stream.value)
+    blk.prepare(rmm_cols=1, lmm_rows=1)
+    dV, dO = DevBuf.from_numpy(np.zeros(n_cols)), DevBuf(n_cols * 8)
+    graph, run = C.c_void_p(), C.c_void_p()
+    ok(h.hipStreamBeginCapture(stream, 0))
+    blk.mmchain_dev_async(dV.ptr, None, 0, dO.ptr)
+    ok(h.hipStreamEndCapture(stream, C.byref(graph)))
+    assert len(blk.stats()["kernels"]) == 1
+    ok(h.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)))
+    for fused in (0, 1, 0):
+        v = rng.standard_normal((n_cols, 1))
+        blk.set_option("chain_fused", fused)
+        eager, _, names = chain(blk, v, None, 0)
+        assert (len(names) == 1) == bool(fused)
+        others = [DevBuf(1 << 16) for _ in range(16)]  # (freed memory would be given out again)
+        for o in others:
+            o.zero()
+        ok(h.hipMemcpy(dV.ptr, v.ctypes.data_as(C.c_void_p), v.nbytes, 1))
+        dO.zero()
+        ok(h.hipDeviceSynchronize())
+        ok(h.hipGraphLaunch(run, stream))
+        ok(h.hipStreamSynchronize(stream))
+        scale = np.abs(D).T @ (np.abs(D) @ np.abs(v))
+        want = D.T.astype(np.longdouble) @ (D @ v.astype(np.longdouble))
+        for got in (dO.to_numpy(n_cols), eager):  # (3000 roundings as above)
+            assert np.all(np.abs(got.reshape(-1, 1) - want) <= 3000 * 2.0 ** -53 * scale)
+    ok(h.hipGraphExecDestroy(run))
+    ok(h.hipGraphDestroy(graph))
+    blk.close()
+    ok(h.hipStreamDestroy(stream))
