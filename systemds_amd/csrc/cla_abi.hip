@@ -885,8 +885,7 @@ int cla_block_prepare(cla_handle b, uint32_t products, int32_t nColB, int32_t nR
 			return 0;
 		}
 	};
-	const bool profile = b->profile;
-	b->profile = false;
+	const NoProfile quiet(b);
 	int64_t r = 0;
 	if(r >= 0 && (products & CLA_PRODUCT_RMM)) {
 		Tmp in, out;
@@ -905,7 +904,6 @@ int cla_block_prepare(cla_handle b, uint32_t products, int32_t nColB, int32_t nR
 	}
 	// X %*% v and one row of Y together: the products of the multiply chain, which on some blocks is a kernel with a workspace of its own
 	if(r >= 0 && (products & CLA_PRODUCT_RMM) && (products & CLA_PRODUCT_LMM) && nColB == 1 && nRowY == 1 && (r = prepare_chain_u8(b)) >= 0 && (r = prepare_chain_sdc(b)) >= 0) r = prepare_chain_pairs(b);
-	b->profile = profile;
 	clear_stats(b);
 	return r < 0 ? (int) r : 0;
 	CLA_CATCH_CODE(int)
@@ -963,10 +961,8 @@ int64_t cla_rmm_dev_noalloc(cla_handle b, const double* dB, int32_t nColB, doubl
 	// the counter and the tables live in the static workspace (the pre-aggregation kernel clears the counter
 	// and rewrites every table entry that is read); event pairs of the profiling mode would be allocations
 	unsigned long long* dNnz = (unsigned long long*) ws;
-	const bool profile = b->profile;
-	b->profile = false;
+	const NoProfile quiet(b);
 	rc = launch_rmm(b, dB, nColB, dOut, dNnz, 0, (double*) (ws + NNZ_BYTES), CLA_SCRATCH_TABLES / sizeof(double));
-	b->profile = profile;
 	if(rc) return rc;
 	return read_nnz(b, dNnz);
 	CLA_CATCH_CODE(int64_t)

@@ -367,6 +367,13 @@ struct Prof {
 	Prof(cla_block* b, const char* name, long grid, long block, long lds, double algoBytes);
 	~Prof();
 };
+// No events for the launches of its scope, which are not the caller's (the mode is back however the scope ends).
+struct NoProfile {
+	cla_block* b;
+	const bool was;
+	explicit NoProfile(cla_block* blk) : b(blk), was(blk->profile) { b->profile = false; }
+	~NoProfile() { b->profile = was; }
+};
 void clear_stats(cla_block* b);
 
 int ensure_tables(cla_block* b, size_t nDoubles);

@@ -882,11 +882,9 @@ int gram_digits_plan(cla_block* b, bool across, const std::function<int(double*)
 		if(capturing != hipStreamCaptureStatusNone) return 1;
 		// (its launches are not the call's)
 		const size_t stats = b->lastStats.size();
-		const bool profile = b->profile;
-		b->profile = false;
+		const NoProfile quiet(b);
 		const int rc = gd_judge(b, P, fp64);
 		b->lastStats.resize(stats);
-		b->profile = profile;
 		if(rc) return rc;
 	}
 	return P.suits[across] ? 0 : 1;

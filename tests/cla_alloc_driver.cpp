@@ -11,6 +11,8 @@
  * Its own hipMalloc fails the k-th device allocation of a first X %*% B and t(X) %*% X of a byte-code block: the plans of the forms on digits
  * are none that a call fails for.
  *
+ * Host memory running out inside a first t(X) %*% X of a byte-code block, or inside cla_block_prepare, leaves the profiling mode as it was set.
+ *
  * Prints "ALLOC-DRIVER OK" at the end; exit code 0 only then.
  */
 #include <dlfcn.h>
@@ -268,6 +270,38 @@ static int room_failures(int& thrown) {
 	return fails;
 }
 
+// t(X) %*% X of 64 byte-code columns, called or prepared, with each allocation of the library failing in turn while profiling is on: the next call's
+// kernels have their times. (Values that digits round: the block is judged by both kernels, whose launches are not the call's.)
+static int profile_failures(int& thrown) {
+	enum { M = 64, V = 5 };
+	std::vector<uint8_t> codes((size_t) N);
+	std::vector<double> dict(V), out(M * M);
+	for(int i = 0; i < V; i++) dict[(size_t) i] = 1.0 / (3 + i);
+	int fails = 0;
+	for(int prepare = 0; prepare < 2; prepare++)
+		for(long k = 0;; k++) {
+			cla_handle h = cla_block_create(N, M);
+			bool ok = h != nullptr;
+			for(int32_t c = 0; c < M && ok; c++) {
+				for(int64_t r = 0; r < N; r++) codes[(size_t) r] = (uint8_t) ((r * (c + 3) + c) % V);
+				ok = cla_block_add_ddc(h, &c, 1, dict.data(), V, codes.data(), 1) >= 0;
+			}
+			if(!ok || cla_block_finalize(h) < 0 || cla_block_profile(h, 1) < 0) { printf("profile: %s\n", cla_last_error()); return fails + 1; }
+			allocFailed = false;
+			allocLeft = k;
+			const int64_t rc = prepare ? cla_block_prepare(h, CLA_PRODUCT_TSMM, 0, 0) : cla_tsmm(h, out.data());
+			allocLeft = -1;
+			if(allocFailed) thrown++;
+			if(allocFailed == (rc >= 0)) { printf("profile, allocation %ld: %s\n", k, rc < 0 ? cla_last_error() : "no error"); fails++; }
+			char stats[2048] = "";
+			if(cla_tsmm(h, out.data()) < 0 || cla_stats(h, stats, sizeof(stats)) < 0) { printf("profile: %s\n", cla_last_error()); fails++; }
+			if(!strstr(stats, "k_gram_tiles") || strstr(stats, "\"ms\":-")) { printf("profile, allocation %ld, prepare %d: the next call's times: %s\n", k, prepare, stats); fails++; }
+			cla_block_free(h);
+			if(!allocFailed) break;
+		}
+	return fails;
+}
+
 int main() {
 	if(cla_init(0) < 0) { fprintf(stderr, "cla_init: %s\n", cla_last_error()); return 2; }
 	int fails = 0, thrown = 0;
@@ -305,8 +339,10 @@ int main() {
 	fails += left_failures(leftThrown);
 	int roomThrown = 0;
 	fails += room_failures(roomThrown);
-	printf("%d + %d failed allocations, %d failed launches, %d failed device allocations\n", thrown, gramThrown, leftThrown, roomThrown);
-	if(fails || thrown < 4 || gramThrown < 2 || leftThrown < 2 || roomThrown < 8) { printf("FAIL\n"); return 1; }
+	int profileThrown = 0;
+	fails += profile_failures(profileThrown);
+	printf("%d + %d + %d failed allocations, %d failed launches, %d failed device allocations\n", thrown, gramThrown, profileThrown, leftThrown, roomThrown);
+	if(fails || thrown < 4 || gramThrown < 2 || leftThrown < 2 || roomThrown < 8 || profileThrown < 8) { printf("FAIL\n"); return 1; }
 	printf("ALLOC-DRIVER OK\n");
 	return 0;
 }

@@ -27,7 +27,8 @@ def test_allocation_failures_leave_no_state():
     """Host memory runs out at every place inside cla_mmchain in turn: an error code each time, and no trace of the chain's
     weights in the next X %*% v of the block; likewise inside cla_tsmm of two wide groups, and no trace of the failed call's
     sums in the next t(X) %*% X. A launch fails at every place inside a Y %*% X on decoded rows: no trace in a replay or the next call.
-    A device allocation fails at every place inside a first product of a byte-code block: none of the digits' plans makes it fail."""
+    A device allocation fails at every place inside a first product of a byte-code block: none of the digits' plans makes it fail.
+    Profiling that was on before a failed call or prepare is on behind it."""
     assert os.path.exists(ALLOC_DRIVER), "tests/cla_alloc_driver not built: run __graft_entry__.build()"
     r = subprocess.run([ALLOC_DRIVER], capture_output=True, text=True, timeout=110)
     print(r.stdout)
