@@ -4,9 +4,9 @@
 // base-256 digits. A row's lookup brings all seven (8 bytes, like the fp64 value), the products of digits i + j <= 6 are
 // summed as 32-bit integers, exactly, one sum per weight i + j, and at the end or every 18,688 rows the seven sums are joined in fp64. So
 // a cell's error is that of the rounded values (2^-56 of the column's largest) and of the products left out (six of up to 2^-56 of both columns'
-// largest), not that of chains of fp64 additions. It is absolute, in parts of the columns' largest values; gd_build_plan and gd_judge say which blocks
+// largest), not that of chains of fp64 additions. It is absolute, in parts of the columns' largest values; gd_build_plan and gd_compare say which blocks
 // that suits. Rms over cells of the error divided by the sum of the terms' magnitudes, against exact counts times products in long double, 256 normal
-// values, Zipf(1.1) codes (k_gram_tiles): 2,000,003 x 100 3.5e-17 (1.2e-15); more beside gd_judge. The same sums in every call: no atomic adds.
+// values, Zipf(1.1) codes (k_gram_tiles): 2,000,003 x 100 3.5e-17 (1.2e-15); more beside gd_compare. The same sums in every call: no atomic adds.
 //
 // A workgroup of 8 waves, one per CU, takes a contiguous share of the rows in tiles of 64 rows per set of waves. Decoding is dealt by (16 columns, 64
 // rows): lane (k, c) looks up 16 consecutive codes of column c (in LDS where the column block's tables fit beside the tile, else in global
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(GJ_THREADS) void k_gram_join(const GdTile* __restri
 
 // For pairs of column blocks p <= q: left += the sums over the rows of the digit products of weight 7, the largest that the kernel above leaves out (the rounding of the
 // values is among them, as an eighth digit), mags += those of the products of the magnitudes (of the first digits, 1 / GD_MAG of the largest value). 16 NCB cells a
-// row of either. A workgroup takes a pair of column blocks, a wave 64 rows at a time. (Once per block: 2,000,003 x 100 1.3 ms, and where gd_judge needs it a call of either kernel.)
+// row of either. A workgroup takes a pair of column blocks, a wave 64 rows at a time. (Once per block: 2,000,003 x 100 1.3 ms, and where gd_compare needs it a call of either kernel.)
 constexpr int GC_UNITS = 240; // 64 rows each, between two flushes: a sum grows by at most 8 2^14 a row
 constexpr int GC_TAB = 16 * 256 * 8, GC_LDS = 2 * GC_TAB;
 __global__ __launch_bounds__(GD_THREADS, 2) void k_gram_left(const uint8_t* __restrict__ arena, size_t arenaStride, const GdCol* __restrict__ cols, int places, int ncb,
@@ -599,10 +599,10 @@ struct GdPlan {
 	const GdTile* tiles = nullptr;
 	int nCellTiles = 0, grid = 0;
 	size_t lds = 0;
-	// Until the block has been judged: per column its place's group and column, per cell i <= j what is left out and the terms' magnitudes (NaN: exact or zero)
+	// Until the results have been compared: per column its place's group and column, per cell i <= j what is left out and the terms' magnitudes (NaN: exact or zero)
 	std::vector<GdCol> cols;
 	std::vector<double> left, mags;
-	bool judged = false;
+	bool compared = false;
 	bool suits[2] = {false, false}; // all cells / those across groups: no further from the exact sums than the fp64 kernel's
 	~GdPlan() { if(dImg) (void) hipFree(dImg); }
 };
@@ -750,7 +750,7 @@ static int gd_build_plan(cla_block* b, GdPlan& P) {
 	// The errors are parts of the columns' largest values, a cell's terms need not be: every cell whose columns are not both free of
 	// rounding has to reach, on average over the rows, 2^-10 of the product of their largest values, whoever asks.
 	// (Six products left out of up to 2^14 2^-70 and two roundings of up to 2^-56: 2^-53.0 a row, all of one sign where a tuple has nearly all rows: up to 2^-43 of the
-	// terms' sum. Unasked a block comes here only if gd_judge finds less than in fp64.)
+	// terms' sum. Unasked a block comes here only if gd_compare finds less than in fp64.)
 	struct Tmp { void* p = nullptr; ~Tmp() { if(p) (void) hipFree(p); } } tmp;
 	const size_t sumBytes = nMag * sizeof(unsigned long long);
 	if(no_room(&tmp.p, 2 * sumBytes + digitTabs.size())) return 1;
@@ -814,7 +814,7 @@ static bool gd_pays(const cla_block* b) {
 // and other cells, Zipf(1.1) codes of 256 normal values, 100 columns: 2,000 rows 8.0e-17 / 7.9e-17 and 8.8e-18 / 2.0e-17, which stay in fp64 as up to some 20,000 rows do, 50,000 1.7e-16 / 1.1e-16 and
 // 1.0e-17 / 2.4e-17, 200,003 3.5e-16 / 8.9e-17 and 1.6e-17 / 2.3e-17, 2,000,003 2.4e-15 / 1.0e-16 and 7.5e-17 / 3.0e-17; uniform codes 10,007 rows 1.0e-16 / 5.2e-17 and
 // 4.3e-18 / 3.4e-18. One value at 5 among them stays in fp64 at 200,003 rows, three decades of values, or a tuple with 99 % of the rows far below the largest, at any number measured.)
-static int gd_judge(cla_block* b, GdPlan& P, const std::function<int(double*)>& fp64) {
+static int gd_compare(cla_block* b, GdPlan& P, const std::function<int(double*)>& fp64) {
 	const int n = b->nCols;
 	auto relative = [&](size_t at) { return P.left[at] / P.mags[at]; };
 	double sum = 0.0, most = 0.0;
@@ -854,12 +854,12 @@ static int gd_judge(cla_block* b, GdPlan& P, const std::function<int(double*)>& 
 			}
 		for(int s = 0; s < 2; s++) P.suits[s] = of[s].ours <= of[s].theirs && of[s].oursMost <= of[s].theirsMost;
 	}
-	P.judged = true;
+	P.compared = true;
 	P.cols = {}; P.left = {}; P.mags = {};
 	return 0;
 }
 
-// 0: the block goes this way (its plan is made), 1: it does not, negative: an error. across: only cells across groups are wanted of it. fp64: see gd_judge.
+// 0: the block goes this way (its plan is made), 1: it does not, negative: an error. across: only cells across groups are wanted of it. fp64: see gd_compare.
 int gram_digits_plan(cla_block* b, bool across, const std::function<int(double*)>& fp64) {
 	if(b->opt.tsmmDigits == 0 || (b->opt.tsmmDigits == 1 && !gd_pays(b))) return 1;
 	if(b->gdPlan == nullptr) {
@@ -876,14 +876,14 @@ int gram_digits_plan(cla_block* b, bool across, const std::function<int(double*)
 	}
 	GdPlan& P = *b->gdPlan;
 	if(P.rc || b->opt.tsmmDigits == 2) return P.rc;
-	if(!P.judged) {
+	if(!P.compared) {
 		hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
 		CLA_HIP(hipStreamIsCapturing(b->stream, &capturing));
 		if(capturing != hipStreamCaptureStatusNone) return 1;
 		// (its launches are not the call's)
 		const size_t stats = b->lastStats.size();
 		const NoProfile quiet(b);
-		const int rc = gd_judge(b, P, fp64);
+		const int rc = gd_compare(b, P, fp64);
 		b->lastStats.resize(stats);
 		if(rc) return rc;
 	}

@@ -271,7 +271,7 @@ static int room_failures(int& thrown) {
 }
 
 // t(X) %*% X of 64 byte-code columns, called or prepared, with each allocation of the library failing in turn while profiling is on: the next call's
-// kernels have their times. (Values that digits round: the block is judged by both kernels, whose launches are not the call's.)
+// kernels have their times. (Values that digits round: both kernels run and their results are compared; those launches are not the call's.)
 static int profile_failures(int& thrown) {
 	enum { M = 64, V = 5 };
 	std::vector<uint8_t> codes((size_t) N);
