@@ -10,17 +10,13 @@ pytestmark = pytest.mark.gpu
 
 
 def product(cla, specs, n_rows, n_cols, digits, options=()):
-    """The product, its non-zeros, and whether the integer kernel has formed it: both forms report as k_gram_tiles, their LDS differs."""
     blk = cla.build_block(n_rows, n_cols, specs)
-    lds = {}
-    for d in (0, digits):
-        for key, value in (("tsmm_digits", d), *options):
-            blk.set_option(key, value)
-        out, nnz = blk.tsmm()
-        lds[d] = [k["lds"] for k in blk.stats()["kernels"] if k["name"] == "k_gram_tiles"]
-        assert len(lds[d]) == 1
+    for key, value in (("tsmm_digits", digits), *options):
+        blk.set_option(key, value)
+    out, nnz = blk.tsmm()
+    lds = {k["lds"] for k in blk.stats()["kernels"] if k["name"] == "k_gram_tiles"}
     blk.close()
-    return out, nnz, lds[digits] != lds[0]
+    return out, nnz, lds
 
 
 @pytest.mark.parametrize("n_cols", [17, 31, 32, 33, 48, 49, 50, 52, 53, 64, 65, 68, 80, 81, 82, 84, 85, 96, 97, 99, 100, 101, 112])
@@ -29,11 +25,7 @@ def test_edges(cla, ora, n_cols, n_rows, n_vals):
     from systemds_amd import synth
     rng = np.random.default_rng(n_cols + n_rows)
     specs = columns(synth, rng, n_rows, n_cols, n_vals, np.uint8, 1)
-    if n_rows == 1:  # (values near their columns' largest: the magnitudes' rule takes the block)
-        for spec in specs:
-            spec.dict = rng.uniform(0.3, 1.0, spec.dict.shape) * rng.choice([-1.0, 1.0], spec.dict.shape)
-    out, nnz, digits = product(cla, specs, n_rows, n_cols, 2)
-    assert digits
+    out, nnz, _ = product(cla, specs, n_rows, n_cols, 2)
     D = ora.np_decompress(specs, n_rows, n_cols)
     assert np.array_equal(out, out.T)
     assert_matches_truth(out, D.T, D, what=f"{n_rows} x {n_cols}")
@@ -51,8 +43,7 @@ def test_wide_groups_constants_and_zeros(cla, ora, width, one_kernel):
     specs[1].dict[:, 0] = 0.0
     specs.append(synth.GroupSpec("const", np.array([n_cols - 3, n_cols - 1], np.int32), np.array([[2.5, -1.0]])))
     specs.append(synth.GroupSpec("const", np.array([0, 7], np.int32), np.array([[1.5, 0.25]])))
-    out, nnz, digits = product(cla, specs, n_rows, n_cols, 2, [("tsmm_one_kernel", one_kernel)])
-    assert digits
+    out, nnz, _ = product(cla, specs, n_rows, n_cols, 2, [("tsmm_one_kernel", one_kernel)])
     D = ora.np_decompress(specs, n_rows, n_cols)
     assert_matches_truth(out, D.T, D, what="constants")
     assert np.array_equal(out, out.T) and nnz == np.count_nonzero(out)
@@ -67,8 +58,7 @@ def test_largest_sums(cla, n_cols, sign):
     v = sum(sign * (127 if sign > 0 else -128) * 256.0 ** k for k in range(7)) * 2.0 ** -55 if sign > 0 else -sum(128 * 256.0 ** k for k in range(7)) * 2.0 ** -55
     code = np.zeros(n_rows, np.uint8)
     specs = [synth.GroupSpec("ddc", np.array([c], np.int32), np.array([[v], [v / 2]]), code) for c in range(n_cols)]
-    out, _, digits = product(cla, specs, n_rows, n_cols, 2)
-    assert digits
+    out, _, _ = product(cla, specs, n_rows, n_cols, 2)
     assert np.max(np.abs(out / (n_rows * v * v) - 1.0)) < 4 * 2.0 ** -53
 
 
@@ -78,8 +68,7 @@ def test_whole_numbers_are_exact(cla):
     n_rows, n_cols = 300_001, 97
     codes = rng.integers(0, 200, (n_cols, n_rows)).astype(np.uint8)
     dicts = rng.integers(-1000, 1000, (n_cols, 200)).astype(np.float64)
-    out, nnz, digits = product(cla, [synth.GroupSpec("ddc", np.array([c], np.int32), dicts[c][:, None], codes[c]) for c in range(n_cols)], n_rows, n_cols, 1)
-    assert digits
+    out, nnz, _ = product(cla, [synth.GroupSpec("ddc", np.array([c], np.int32), dicts[c][:, None], codes[c]) for c in range(n_cols)], n_rows, n_cols, 1)
     D = np.stack([dicts[c][codes[c]] for c in range(n_cols)])
     assert np.array_equal(out, D @ D.T) and nnz == np.count_nonzero(out)
 
@@ -106,9 +95,9 @@ def test_values_that_digits_do_not_suit(cla, ora, kind):
             s.dict[:, 0] = np.arange(40) == 3
     if kind == "infinite":
         specs[5].dict[3, 0] = np.inf
-    out, _, digits = product(cla, specs, n_rows, n_cols, 2)
-    want, _, _ = product(cla, specs, n_rows, n_cols, 0)
-    assert digits == (kind == "one-hot")
+    out, _, lds = product(cla, specs, n_rows, n_cols, 2)
+    want, _, fp64 = product(cla, specs, n_rows, n_cols, 0)
+    assert (lds == fp64) == (kind != "one-hot")
     if kind == "infinite":
         assert np.array_equal(np.isfinite(out), np.isfinite(want))
         return
@@ -118,6 +107,47 @@ def test_values_that_digits_do_not_suit(cla, ora, kind):
         assert np.array_equal(out, want * 1e200 * 1e200)
         return
     assert_matches_truth(out, D.T, D, what=kind)
+
+
+def on_digits(cla, specs, n_rows, n_cols, digits, options=(), plain=product):
+    """product, of the integer kernel: both forms report as k_gram_tiles, their LDS differs."""
+    out, nnz, lds = plain(cla, specs, n_rows, n_cols, digits, options)
+    assert len(lds) == 1 and lds != plain(cla, specs, n_rows, n_cols, 0, options)[2]
+    return out, nnz, lds
+
+
+@pytest.mark.parametrize("n_cols", [17, 32, 33, 49, 52, 65, 84, 97, 101, 112])
+@pytest.mark.parametrize("n_rows,n_vals", [(63, 256), (257, 7), (16449, 256), (40009, 60)])
+def test_edges_on_digits(cla, ora, monkeypatch, n_cols, n_rows, n_vals):
+    monkeypatch.setitem(globals(), "product", on_digits)
+    test_edges(cla, ora, n_cols, n_rows, n_vals)
+
+
+@pytest.mark.parametrize("n_cols", [17, 31, 32, 33, 48, 49, 50, 52, 53, 64, 65, 68, 80, 81, 82, 84, 85, 96, 97, 99, 100, 101, 112])
+def test_one_row_on_digits(cla, ora, n_cols):
+    """Values near their columns' largest: the magnitudes' rule takes the block."""
+    from systemds_amd import synth
+    rng = np.random.default_rng(n_cols)
+    specs = columns(synth, rng, 1, n_cols, 3, np.uint8, 1)
+    for spec in specs:
+        spec.dict = rng.uniform(0.3, 1.0, spec.dict.shape) * rng.choice([-1.0, 1.0], spec.dict.shape)
+    out, nnz, _ = on_digits(cla, specs, 1, n_cols, 2)
+    D = ora.np_decompress(specs, 1, n_cols)
+    assert np.array_equal(out, out.T) and nnz == np.count_nonzero(out)
+    assert_matches_truth(out, D.T, D, what=f"1 x {n_cols}")
+
+
+@pytest.mark.parametrize("width", [8, 40])
+@pytest.mark.parametrize("one_kernel", [0, 1])
+def test_wide_groups_on_digits(cla, ora, monkeypatch, width, one_kernel):
+    monkeypatch.setitem(globals(), "product", on_digits)
+    test_wide_groups_constants_and_zeros(cla, ora, width, one_kernel)
+
+
+def test_sums_and_whole_numbers_on_digits(cla, monkeypatch):
+    monkeypatch.setitem(globals(), "product", on_digits)
+    test_largest_sums(cla, 35, -1)
+    test_whole_numbers_are_exact(cla)
 
 
 def errors(specs, out, n_cols):
@@ -156,9 +186,9 @@ def test_no_less_precise_than_fp64(cla, kind, n_rows, n_cols, n_vals, digits):
         elif kind == "uniform":
             codes = rng.integers(0, n_vals, n_rows)
         specs.append(synth.GroupSpec("ddc", np.array([c], np.int32), d[:, None], codes.astype(np.uint8)))
-    out, _, ran = product(cla, specs, n_rows, n_cols, 1)
-    want, _, _ = product(cla, specs, n_rows, n_cols, 0)
-    assert ran == digits
+    out, _, lds = product(cla, specs, n_rows, n_cols, 1)
+    want, _, fp64 = product(cla, specs, n_rows, n_cols, 0)
+    assert (lds != fp64) == digits
     if digits:
         got, ref = (errors(specs, o, n_cols) for o in (out, want))
         assert np.sqrt((got ** 2).mean()) <= np.sqrt((ref ** 2).mean()) and got.max() <= ref.max()
